@@ -213,12 +213,14 @@ struct xcq_context_s {
   int32_t* d_shell_atom = nullptr;
   bool last_grad = false;   // the last evaluation was an EXC gradient
   double* d_zc = nullptr;   // Z coefficients per point block (in-stage mode 3), lazily
+  double* d_syr_part = nullptr;  // slice buffer of the FP64 SYR2K, lazily
   int64_t pblocks = 0;      // point blocks of the uploaded tasks
   double* d_out2 = nullptr;
   double* d_corr = nullptr;  // [nmol][kCorrBlocks] partials of the P32 correction
   double* d_rpart = nullptr;  // [nmol][kRedBlocks][2] partials of EXC/NEL
   double* d_tmax = nullptr;   // bound table: one {float, float} per function granule
   int64_t tmax_total = 0;
+  bool last_mixed = false;   // the last evaluation ran the mixed kernels
   int last_want_vxc = 0;     // the last evaluation returns VXC
   int last_vxc_eval = 0;     // the last evaluation computed VXC
 
@@ -256,6 +258,7 @@ struct xcq_context_s {
     dfree(d_counters);
     dfree(d_red);
     dfree(d_zc);
+    dfree(d_syr_part);
     dfree(d_uks);
     dfree(d_fxcu);
     pblocks = 0;
@@ -312,7 +315,7 @@ CtxView view_of(xcq_context_s* c) {
                  c->d_work,  c->d_qoff,  c->d_counters, c->timing ? c->d_tstamp : nullptr,
                  c->d_P,     c->d_Pf32,  c->d_vxc,   c->d_red,        c->d_scratch,
                  c->vxc_drop, reinterpret_cast<unsigned*>(c->d_tmax),
-                 c->max_l <= kInStageMaxL ? c->dens_in_stage : 0, c->d_shc, c->d_zc};
+                 c->max_l <= kInStageMaxL ? c->dens_in_stage : 0, c->d_shc, c->d_zc, c->d_syr_part};
 }
 
 // Heuristic per-item costs (used when no predicted task costs are set):
@@ -333,6 +336,7 @@ int build_work_lists(xcq_context_s* ctx) {
   int64_t ncounters = 0;
   const bool have_cost = ctx->cost_d.size() == (size_t)ctx->ntasks &&
                          ctx->cost_s.size() == (size_t)ctx->ntasks;
+  const bool queued = ctx->nqueues > 0;  // only then are the items' costs read
   for (auto& d : ctx->h_tasks) {
     d.nt_d = d.nbe <= ctx->dens32_max_nbe ? 32 : (d.nbe >= ctx->dens128_min_nbe ? 128 : 64);
     d.dens_cls = d.nt_d == 32    ? 0
@@ -368,7 +372,7 @@ int build_work_lists(xcq_context_s* ctx) {
         const double ci = have_cost ? ctx->cost_d[i] / nmb : heur_dens_item(d);
         for (int pb = 0; pb < nmb; ++pb) {
           W.push_back(WorkItem{i, pb, 0, 0});
-          cost.push_back(ci);
+          if (queued) cost.push_back(ci);
         }
       }
       finish_range(c.dens[v], cost);
@@ -389,16 +393,64 @@ int build_work_lists(xcq_context_s* ctx) {
         for (int it = 0; it < nt_tiles; ++it)
           for (int jt = 0; jt <= it; ++jt) {
             W.push_back(WorkItem{i, it, jt, 0});
-            cost.push_back(ci);
+            if (queued) cost.push_back(ci);
           }
       }
       finish_range(c.syr2k[v], cost);
     }
+    // FP64 SYR2K: regions and point slices.  A slice is as long as gives the
+    // chunk one item per resident workgroup (3 per CU), between 256 points
+    // (below that storing and summing slices costs what the shorter chain
+    // saves: 120 functions, 0.104 ms at 256, 0.142 at 64) and 4,096 (larger
+    // chunks start such chains first and end them before the rest; 1,024
+    // to 8,192 time the same on 24 and 150 waters).
+    constexpr int64_t kSyrItems = 768;
+    constexpr int kSliceMin = 256, kSliceMax = 4096;
+    auto syr_regions = [&](const DevTask& d, auto&& f) {
+      const int nb = (d.nbe + 15) / 16;
+      const int ni = syr_row_groups(nb), nj = syr_col_groups(nb);
+      for (int it = 0; it < ni; ++it)
+        for (int jt = 0; jt < nj; ++jt)
+          if ((it + 1) * nb / ni > jt * nb / nj) f(it | jt << 16);  // blocks below the diagonal
+    };
+    int64_t region_points = 0;
+    for (int32_t i = c.task_begin; i < c.task_end; ++i) {
+      int64_t n = 0;
+      syr_regions(ctx->h_tasks[i], [&](int) { ++n; });
+      region_points += n * ctx->h_tasks[i].npts;
+    }
+    const int32_t kslice =
+        (int32_t)std::clamp<int64_t>(region_points / kSyrItems, kSliceMin, kSliceMax);
+    std::vector<WorkItem> sums;
+    std::vector<double> cost;
+    c.syr2k_f64.off = (int64_t)W.size();
+    c.syr_slots = 0;
+    for (int32_t i = c.task_begin; i < c.task_end; ++i) {
+      const DevTask& d = ctx->h_tasks[i];
+      if (d.npts == 0) continue;
+      const int32_t ns = std::min((d.npts + kslice - 1) / kslice, 0x7fff);
+      const size_t first = W.size();
+      syr_regions(d, [&](int32_t rg) {
+        if (ns > 1) sums.push_back(WorkItem{i, rg, ns, (int32_t)c.syr_slots});
+        for (int32_t sl = 0; sl < ns; ++sl)
+          W.push_back(WorkItem{i, rg, sl | ns << 16,
+                               ns > 1 ? (int32_t)c.syr_slots++ : 0});
+      });
+      const size_t n = W.size() - first;
+      if (!queued) continue;
+      cost.insert(cost.end(), n, have_cost ? ctx->cost_s[i] / std::max<size_t>(n, 1)
+                                           : (double)d.npts / ns);
+    }
+    finish_range(c.syr2k_f64, cost);
+    c.syr2k_sum.off = (int64_t)W.size();
+    c.syr2k_sum.n = (int64_t)sums.size();
+    W.insert(W.end(), sums.begin(), sums.end());
   }
   dfree(ctx->d_work);
   dfree(ctx->d_qoff);
   dfree(ctx->d_tstamp);
   dfree(ctx->d_counters);
+  dfree(ctx->d_syr_part);
   int rc;
   if ((rc = dalloc(&ctx->d_work, W.size()))) return rc;
   if ((rc = dalloc(&ctx->d_qoff, Q.size()))) return rc;
@@ -413,6 +465,17 @@ int build_work_lists(xcq_context_s* ctx) {
     XCQ_HIP(hipMemset(ctx->d_tstamp, 0, 2 * W.size() * sizeof(int64_t)));
   ctx->drop_graph();
   return XCQ_SUCCESS;
+}
+
+// The slice buffer of the FP64 SYR2K, sized for the chunk that needs most
+// (freed with the work lists that say how much).
+int ensure_syr_part(xcq_context_s* ctx) {
+  if (ctx->d_syr_part) return XCQ_SUCCESS;
+  int64_t slots = 0;
+  for (const auto& c : ctx->chunks) slots = std::max(slots, c.syr_slots);
+  if (slots == 0) return XCQ_SUCCESS;
+  ctx->drop_graph();
+  return dalloc(&ctx->d_syr_part, (size_t)slots * kSyrBlocks * 256);
 }
 
 // Enqueue one evaluation on the context's stream.  Events are recorded only
@@ -483,11 +546,15 @@ int enqueue_pipeline(xcq_context_s* ctx, int func, int precision, int want_vxc, 
       }
       XCQ_HIP(rec(ev[7]));
       XCQ_HIP(rec(ev[8]));
-      for (int k = 0; k < 2; ++k)
-        if ((rc = launch_syr2k(v, c.syr2k[k], k == 0 ? 32 : 64, precision))) return rc;
+      if ((rc = launch_syr2k(v, c, precision))) return rc;
       XCQ_HIP(rec(ev[9]));
-      launches += 2;
-      items += c.syr2k[0].n + c.syr2k[1].n;
+      if (precision == XCQ_PREC_FP64) {
+        launches += 1;
+        items += c.syr2k_f64.n;
+      } else {
+        launches += 2;
+        items += c.syr2k[0].n + c.syr2k[1].n;
+      }
     }
   }
   const int32_t nmol = (int32_t)ctx->mols.size();
@@ -535,6 +602,7 @@ int run_pipeline(xcq_context_s* ctx, int func, int precision, int want_vxc) {
     if (rc) return rc;
     ctx->pf32_valid = true;
   }
+  ctx->last_mixed = precision == XCQ_PREC_MIXED;
   ctx->last_want_vxc = want_vxc;
   ctx->last_uks = false;
   ctx->last_fxc = false;
@@ -548,6 +616,8 @@ int run_pipeline(xcq_context_s* ctx, int func, int precision, int want_vxc) {
     if (rc) return rc;
     ctx->drop_graph();
   }
+  if (want_vxc && precision == XCQ_PREC_FP64)
+    if (int rc = ensure_syr_part(ctx)) return rc;
   ctx->last_vxc_eval = want_vxc;
   if (!ctx->use_graph) {
     ctx->last_graph = false;
@@ -1123,7 +1193,11 @@ int xcq_task_times(xcq_context ctx, double* dens_us, double* syr2k_us) {
   };
   for (const auto& c : ctx->chunks) {
     for (int v = 0; v < 4; ++v) add(c.dens[v], dens_us);
-    for (int v = 0; v < 2; ++v) add(c.syr2k[v], syr2k_us);
+    // The list the last evaluation ran (the other keeps older stamps).
+    if (ctx->last_mixed)
+      for (int v = 0; v < 2; ++v) add(c.syr2k[v], syr2k_us);
+    else
+      add(c.syr2k_f64, syr2k_us);
   }
   return XCQ_SUCCESS;
 }
@@ -1384,6 +1458,7 @@ void ssf_molmeta(int32_t natoms, const double* atom_xyz, std::vector<double>& ra
 // The per-point buffers of the UKS, FXC and gradient paths (freed with the
 // task set, whose point-block count sizes them).
 int ensure_point_buffers(xcq_context_s* ctx) {
+  if (int rc = ensure_syr_part(ctx)) return rc;
   if (ctx->d_uks) return XCQ_SUCCESS;
   return dalloc(&ctx->d_uks, (size_t)5 * 256 * std::max<int64_t>(ctx->pblocks, 1));
 }
@@ -1425,9 +1500,7 @@ int z_and_vxc(xcq_context_s* ctx, CtxView v, const Chunk& c, int mode, int gga,
     if ((rc = z_from_point_coeffs(ctx, v, c, mode, gga, coef))) return rc;
     v.tmax = nullptr;
   }
-  for (int k = 0; k < 2; ++k)
-    if ((rc = launch_syr2k(v, c.syr2k[k], k == 0 ? 32 : 64, XCQ_PREC_FP64))) return rc;
-  return XCQ_SUCCESS;
+  return launch_syr2k(v, c, XCQ_PREC_FP64);
 }
 
 // One UKS evaluation on the context's stream (FP64; in-stage basis
@@ -1517,6 +1590,7 @@ int xcq_exc_vxc_uks(xcq_context ctx, int functional, int want_vxc) {
   int rc;
   if ((rc = ensure_point_buffers(ctx))) return rc;
   if (!ctx->d_vxcz && (rc = dalloc(&ctx->d_vxcz, (size_t)ctx->p_total))) return rc;
+  ctx->last_mixed = false;
   ctx->last_want_vxc = want_vxc ? 1 : 0;
   ctx->last_vxc_eval = want_vxc ? 1 : 0;
   ctx->last_graph = false;
@@ -1623,6 +1697,7 @@ int xcq_fxc_contraction(xcq_context ctx, int functional) {
   XCQ_HIP(hipSetDevice(ctx->device));
   int rc;
   if ((rc = ensure_point_buffers(ctx))) return rc;
+  ctx->last_mixed = false;
   ctx->last_want_vxc = 0;
   ctx->last_vxc_eval = 0;
   ctx->last_graph = false;
@@ -1721,10 +1796,12 @@ int xcq_fxc_contraction_uks(xcq_context ctx, int functional) {
               "xcq_upload_trial_density_z)");
   XCQ_HIP(hipSetDevice(ctx->device));
   int rc;
+  if ((rc = ensure_syr_part(ctx))) return rc;
   if (!ctx->d_fxcu &&
       (rc = dalloc(&ctx->d_fxcu, (size_t)6 * 256 * std::max<int64_t>(ctx->pblocks, 1))))
     return rc;
   if (!ctx->d_vxcz && (rc = dalloc(&ctx->d_vxcz, (size_t)ctx->p_total))) return rc;
+  ctx->last_mixed = false;
   ctx->last_want_vxc = 0;
   ctx->last_vxc_eval = 0;
   ctx->last_graph = false;
@@ -1967,6 +2044,7 @@ int grad_prepare(xcq_context_s* ctx, int functional, int32_t natoms, const doubl
     XCQ_HIP(hipMemcpy(ctx->d_gnbr_r, hnr.data(), 8 * hnr.size(), hipMemcpyHostToDevice));
   }
   if ((rc = ensure_point_buffers(ctx))) return rc;
+  ctx->last_mixed = false;
   ctx->last_want_vxc = 0;
   ctx->last_vxc_eval = 0;
   ctx->last_graph = false;

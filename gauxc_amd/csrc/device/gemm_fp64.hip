@@ -2,17 +2,17 @@
 // (v_mfma_f64_16x16x4_f64).
 //
 //  (X = fac B P_sub, the density reduction and Z live in density.hip.)
-//  k_syr2k    : V = B^T Z + Z^T B for lower-triangle 64x64 tiles with the
-//               scatter-add into VXC fused into the epilogue (GauXC: DSYR2K
-//               per task + sym_inc_by_submat, scheme1_base.cxx:1712-1766).
+//  k_syr2k    : V = B^T Z + Z^T B, lower triangle, with the scatter-add
+//               into VXC fused into the epilogue (GauXC: DSYR2K per task +
+//               sym_inc_by_submat, scheme1_base.cxx:1712-1766).
 //
-// Workgroup: 256 threads = 4 waves in a 2x2 arrangement.  K advances 16 per
-// LDS stage.
 // MFMA operand layout (16x16x4 f64, measured on gfx950): lane l holds
 // A[l%16][l/16] and B[l/16][l%16]; accumulator register r of lane l is
 // D[4*r + l/16][l%16] (rows interleave across the four 16-lane groups,
 // unlike the FP32-output MFMAs whose register r holds row 4*(l/16) + r).
 #include "internal.hpp"
+
+#include <type_traits>
 
 namespace xcq {
 
@@ -22,162 +22,279 @@ __device__ __forceinline__ v4d mfma_f64(double a, double b, v4d c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
+// Region of an FP64 SYR2K work item: blocks of 16 functions, rows [r0, r1)
+// and columns [c0, c1), without the rows above and the columns right of its
+// part on or below the diagonal, so c0 <= r0 and c1 <= r1.
+struct SyrRegion {
+  int r0, r1, c0, c1;
+};
+__device__ __forceinline__ SyrRegion syr_region(const DevTask& t, int a, int b) {
+  const int nb = (t.nbe + 15) / 16;
+  const int ni = syr_row_groups(nb), nj = syr_col_groups(nb);
+  const int r1 = (a + 1) * nb / ni, c0 = b * nb / nj;
+  return SyrRegion{max(a * nb / ni, c0), r1, c0, min((b + 1) * nb / nj, r1)};
+}
+
+// The region's wanted blocks, bit (row - r0) * (c1 - c0) + column - c0: on or
+// below the diagonal, and not negligible by the bound table, |sum_p B_pi
+// Z_pj| <= npts max|B_i| max|Z_j| (1.01 covers the rounding of the stored
+// maxima and of the products).  Lane l of a wave decides bit l (a region has
+// at most 64 blocks).
+__device__ __forceinline__ uint64_t syr_mask(const DevTask& t, const SyrRegion& s, int lane,
+                                             const unsigned* tmax, double drop) {
+  const int nc = s.c1 - s.c0;
+  const int rb = s.r0 + lane / nc, cb = s.c0 + lane % nc;
+  bool want = rb < s.r1 && rb >= cb;
+  if (want && tmax) {
+    const unsigned* tm = tmax + 2 * t.tmax_off;
+    const int gi = 16 * rb / kGran, gj = 16 * cb / kGran;
+    const double bound =
+        1.01 * (double)t.npts *
+        ((double)__uint_as_float(tm[2 * gi]) * (double)__uint_as_float(tm[2 * gj + 1]) +
+         (double)__uint_as_float(tm[2 * gi + 1]) * (double)__uint_as_float(tm[2 * gj]));
+    want = !(bound < drop);
+  }
+  return __builtin_amdgcn_ballot_w64(want);
+}
+
+// One 1 KiB fragment from memory into LDS: lane l's 16 bytes at base + off
+// go to lds + 16 l.  Inline asm (as the density stage's operand ring) so
+// that the compiler's wait insertion, which cannot tell the two stages
+// apart, adds no wait for it before LDS reads; the K loop waits itself.
+__device__ __forceinline__ void frag_to_lds(const double* base, unsigned off, const double* lds) {
+  const unsigned m0 = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)lds);
+  asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(m0) : "memory");
+}
+
 // ---------------------------------------------------------------------------
-// Templated on the function tile NT (32 or 64); each wave owns an
-// (NT/2) x (NT/2) sub-tile = BI x BI MFMA blocks.  Loader: thread
-// (p = tid & 15, f = tid >> 4) moves point k0 + p of rows f, f+16, ... of
-// each panel; 16 lanes cover 16 consecutive points (128 B) of one row.  Rows
-// past nbe are read at row nbe-1 and zeroed by a select.  The next K step is
-// loaded into registers while the current one runs on the matrix cores.
-template <int NT>
-__global__ __launch_bounds__(256) void k_syr2k(QueueArgs qa, const DevTask* __restrict__ tasks,
-                                               const int32_t* __restrict__ bfmap,
-                                               const double* __restrict__ scratch,
-                                               double* __restrict__ vxc_all, double drop,
-    const unsigned* __restrict__ tmax) {
-  constexpr int BI = NT / 32, NQ = NT / 16, LP = NT + 4;
-  __shared__ double Bi[16][LP];
-  __shared__ double Zi[16][LP];
-  __shared__ double Bj[16][LP];
-  __shared__ double Zj[16][LP];
-  const int tid = threadIdx.x, lane = tid & 63;
+// One workgroup per region of up to 7 x 6 blocks of 16 x 16 functions (up to
+// 8 x 8 when that is the whole task) and slice of the task's points.
+//
+// What bounds it: the matrix cores, once each operand is fetched few enough
+// times.  Padding to 64-wide tiles and 64 points multiplied 1.8 to 2.3 times
+// what is wanted (150 and 24 waters); a first version with one wave per 4 x
+// 3 blocks, its operands straight from memory, multiplied 1.2 times but
+// missed L2 for 28 GB per 24-water call, 4.3 TB/s, with the matrix cores 41%
+// busy.  So four waves share a region's fragments through LDS, and only
+// blocks that hold wanted elements are multiplied: below nbe, on or below
+// the diagonal, not negligible by the bound table.  The wanted blocks are
+// dealt evenly to the waves, each block anywhere in the region; at 64 cycles
+// per MFMA the four fragments a block reads for its four MFMAs take half of
+// the LDS bandwidth.
+//
+// A fragment is 16 functions x 8 points of a plane in lane order: lane (f =
+// l & 15, q = l >> 4) holds points k + 2q, k + 2q + 1 of function row f, the
+// operands of two MFMAs whose K index q stands for the points k + 2q + j.
+// (Any order of the points serves as long as both operands use it.)  It is
+// one 16-byte load per lane from memory into LDS and one 16-byte LDS read.
+// Two stages of up to 13 blocks (B and Z) fill a third of a CU's LDS: three
+// workgroups per CU, one barrier per eight points.  Now 17 GB of L2 misses
+// per 24-water call, 3.9 TB/s, and the matrix cores 61% busy.
+//
+// Stage times, 64-wide padded tiles -> this: 24 waters 8.4 -> 4.4 ms, 150
+// waters 94.6 -> 61 ms, 120 functions on 340,000 points 0.66 -> 0.10 ms, 84
+// functions on 35,000 points 0.11 -> 0.03 ms.
+//
+// The points of a task with very many of them (20,000 after merging) are cut
+// into slices, or that task would be one serial chain: on small molecules
+// that chain was the whole stage.  A slice stores its blocks to part, and
+// k_syr2k_reduce sums a task's slices in order.
+__global__ __launch_bounds__(256, 3) void k_syr2k(QueueArgs qa, const DevTask* __restrict__ tasks,
+                                                  const int32_t* __restrict__ bfmap,
+                                                  const double* __restrict__ scratch,
+                                                  double* __restrict__ vxc_all, double drop,
+                                                  const unsigned* __restrict__ tmax,
+                                                  double* __restrict__ part) {
+  typedef double v2d __attribute__((ext_vector_type(2)));
+  constexpr int kStage = 2 * kSyrStaged * 128;  // doubles per stage
+  __shared__ __attribute__((aligned(16))) double stage[2 * kStage];
+  const int tid = threadIdx.x, lane = tid & 63, lf = lane & 15, lq = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave & 1, wn = wave >> 1;
-  const int l_p = tid & 15, l_f = tid >> 4;
 
   XCQ_FOR_EACH_ITEM(qa, it) {
     const int64_t t0 = qa.tstamp ? wall_clock64() : 0;
-    const WorkItem wi = qa.items[it];
+    const WorkItem wi = qa.items[uniform64(it)];
     const DevTask t = tasks[wi.task];
-    const int i0 = wi.a * NT, j0 = wi.b * NT;
-    const bool diag = wi.a == wi.b;
-    // Tile pairs whose every element would be dropped are skipped whole
-    // (uniform across the workgroup).
-    if (tile_pair_negligible(t, tmax, i0, j0, NT, drop)) {
+    const int nbe = t.nbe, ld = t.npts_pad;
+    const SyrRegion rg = syr_region(t, wi.a & 0xffff, wi.a >> 16);
+    const int n8 = (t.npts + 7) / 8, sl = wi.b & 0xffff, ns = wi.b >> 16;
+    const int s0 = (int)((int64_t)sl * n8 / ns), s1 = (int)((int64_t)(sl + 1) * n8 / ns);
+    const uint64_t mask = syr_mask(t, rg, lane, tmax, drop);
+    if (mask == 0) {
       stamp_item(qa, it, t0);
       continue;
     }
-    const int ld = t.npts_pad;
-    const int nbe = t.nbe;
-    const int plane = nbe * ld;
-    const double* Bm = scratch + t.b_off;
-    const double* Zm = Bm + 4 * plane;
-    const int64_t ldv = t.ldp;
-    double* vxc = vxc_all + t.p_off;
-
-    int oi[NQ], oj[NQ];
-    bool ki[NQ], kj[NQ];
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      const int fi = i0 + l_f + 16 * q, fj = j0 + l_f + 16 * q;
-      ki[q] = fi < nbe;
-      kj[q] = fj < nbe;
-      oi[q] = min(fi, nbe - 1) * ld + l_p;
-      oj[q] = min(fj, nbe - 1) * ld + l_p;
+    const int count = __popcll(mask);
+    // Staged blocks: the columns, then the rows that are not among them.
+    // Staged block u is function block u + c0, or u + gap past the columns.
+    const int nc = rg.c1 - rg.c0, gap = rg.r0 > rg.c1 ? rg.r0 - rg.c1 : 0;
+    const int nst = rg.r1 - rg.c0 - gap;
+    auto block_of = [&](int u) { return rg.c0 + u + (u < nc ? 0 : gap); };
+    // The wave's blocks: ranks [w count / 4, (w + 1) count / 4) of the mask.
+    int* slots = reinterpret_cast<int*>(stage);
+    __syncthreads();  // the previous item is done with the stages
+    if (wave == 0 && (mask >> lane & 1)) {
+      const int rb = rg.r0 + lane / nc, cb = rg.c0 + lane % nc;
+      const int ur = rb < rg.c1 ? rb - rg.c0 : rb - gap - rg.c0;
+      slots[__popcll(mask & ((uint64_t(1) << lane) - 1))] = ur | (cb - rg.c0) << 8;
     }
-    // Raw prefetch registers; the row masks are applied when staged, so the
-    // loads stay in flight across the current step's matrix instructions.
-    double rbi[NQ], rzi[NQ], rbj[NQ], rzj[NQ];
-    auto load = [&](int k0) {
+    __syncthreads();
+    const int b0 = wave * count / 4, n = (wave + 1) * count / 4 - b0;
+    int ur[kSyrSlots], uc[kSyrSlots];  // staged row and column block per slot
 #pragma unroll
-      for (int q = 0; q < NQ; ++q) {
-        rbi[q] = Bm[oi[q] + k0];
-        rzi[q] = Zm[oi[q] + k0];
-      }
-      if (!diag) {
+    for (int k = 0; k < kSyrSlots; ++k) {
+      const int v = __builtin_amdgcn_readfirstlane(slots[min(b0 + k, count - 1)]);
+      ur[k] = v & 0xff;
+      uc[k] = v >> 8;
+    }
+    __syncthreads();  // slots are read: the stages may be filled
+
+    // Fragments wave, wave + 4, ... of the 2 nst of a stage (block u's B at
+    // 2u, its Z at 2u + 1).  Rows past nbe are read at row nbe - 1; their
+    // products are not stored.  Byte offsets in a task's planes end below
+    // 4 GiB.
+    constexpr int kLoads = (2 * kSyrStaged + 3) / 4;
+    const double* Bm = scratch + t.b_off;
+    const double* Zm = Bm + 4 * (int64_t)nbe * ld;
+    const double* plane = wave & 1 ? Zm : Bm;  // c = wave + 4 e has wave's parity
+    unsigned off[kLoads];
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-          rbj[q] = Bm[oj[q] + k0];
-          rzj[q] = Zm[oj[q] + k0];
+    for (int e = 0; e < kLoads; ++e)
+      off[e] = (unsigned)(min(16 * block_of(min((wave + 4 * e) >> 1, nst - 1)) + lf, nbe - 1) * ld +
+                          2 * lq) * 8u;
+    auto issue = [&](int s, int buf) {
+      const double* src = plane + 8 * s;
+#pragma unroll
+      for (int e = 0; e < kLoads; ++e)
+        if (wave + 4 * e < 2 * nst)
+          frag_to_lds(src, off[e], stage + buf * kStage + (wave + 4 * e) * 128);
+    };
+    v4d acc[kSyrSlots];
+#pragma unroll
+    for (int k = 0; k < kSyrSlots; ++k) acc[k] = v4d{0., 0., 0., 0.};
+    auto contract = [&](auto N) {
+      constexpr int kN = decltype(N)::value;
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      issue(s0, 0);
+      for (int s = s0; s < s1; ++s) {
+        const int buf = (s - s0) & 1;
+        // This wave's fragments of stage s have landed and its reads of the
+        // other stage are done; past the barrier so are the others'.
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (s + 1 < s1) issue(s + 1, buf ^ 1);
+        const double* st = stage + buf * kStage + 2 * lane;
+#pragma unroll
+        for (int k = 0; k < kN; ++k) {
+          const v2d bi = *reinterpret_cast<const v2d*>(st + ur[k] * 256);
+          const v2d zi = *reinterpret_cast<const v2d*>(st + ur[k] * 256 + 128);
+          const v2d bj = *reinterpret_cast<const v2d*>(st + uc[k] * 256);
+          const v2d zj = *reinterpret_cast<const v2d*>(st + uc[k] * 256 + 128);
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            acc[k] = mfma_f64(bi[j], zj[j], acc[k]);
+            acc[k] = mfma_f64(zi[j], bj[j], acc[k]);
+          }
         }
       }
     };
-
-    v4d acc[BI][BI];
-#pragma unroll
-    for (int i = 0; i < BI; ++i)
-#pragma unroll
-      for (int j = 0; j < BI; ++j) acc[i][j] = v4d{0., 0., 0., 0.};
-
-    load(0);
-    for (int k0 = 0; k0 < ld; k0 += 16) {
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) {
-        Bi[l_p][l_f + 16 * q] = ki[q] ? rbi[q] : 0.;
-        Zi[l_p][l_f + 16 * q] = ki[q] ? rzi[q] : 0.;
-        if (!diag) {
-          Bj[l_p][l_f + 16 * q] = kj[q] ? rbj[q] : 0.;
-          Zj[l_p][l_f + 16 * q] = kj[q] ? rzj[q] : 0.;
-        }
-      }
-      __syncthreads();
-      if (k0 + 16 < ld) load(k0 + 16);
-      const double(*BJ)[LP] = diag ? Bi : Bj;
-      const double(*ZJ)[LP] = diag ? Zi : Zj;
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        const int kr = ks * 4 + (lane >> 4);
-        double bi_[BI], zi_[BI], bj_[BI], zj_[BI];
-#pragma unroll
-        for (int q = 0; q < BI; ++q) {
-          const int ci = wm * 16 * BI + q * 16 + (lane & 15);
-          const int cj = wn * 16 * BI + q * 16 + (lane & 15);
-          bi_[q] = Bi[kr][ci];
-          zi_[q] = Zi[kr][ci];
-          bj_[q] = BJ[kr][cj];
-          zj_[q] = ZJ[kr][cj];
-        }
-#pragma unroll
-        for (int x = 0; x < BI; ++x)
-#pragma unroll
-          for (int y = 0; y < BI; ++y) {
-            acc[x][y] = mfma_f64(bi_[x], zj_[y], acc[x][y]);
-            acc[x][y] = mfma_f64(zi_[x], bj_[y], acc[x][y]);
-          }
-      }
-      __syncthreads();
+    switch (n) {
+      case 0: contract(std::integral_constant<int, 0>{}); break;
+      case 1: contract(std::integral_constant<int, 1>{}); break;
+      case 2: contract(std::integral_constant<int, 2>{}); break;
+      case 3: contract(std::integral_constant<int, 3>{}); break;
+      case 4: contract(std::integral_constant<int, 4>{}); break;
+      case 5: contract(std::integral_constant<int, 5>{}); break;
+      case 6: contract(std::integral_constant<int, 6>{}); break;
+      case 7: contract(std::integral_constant<int, 7>{}); break;
+      case 8: contract(std::integral_constant<int, 8>{}); break;
+      case 9: contract(std::integral_constant<int, 9>{}); break;
+      case 10: contract(std::integral_constant<int, 10>{}); break;
+      default: contract(std::integral_constant<int, 11>{}); break;
     }
 
-    // Scatter-add into VXC.  Element (i, j) of the tile (i >= j locally) is
-    // added at (bf[j], bf[i]) of the column-major VXC: the 16 lanes of a
-    // lane group hold 16 consecutive j, so each atomic instruction touches a
-    // few 128-byte column segments instead of 16 columns.  The
-    // symmetrisation that follows sums the two triangles, so which triangle
-    // an element lands in does not matter.
-    const int32_t* bf = bfmap + t.bf_off;
+    if (ns > 1) {
+      double* dst = part + ((int64_t)wi.c * kSyrBlocks + b0) * 256 + lane;
 #pragma unroll
-    for (int bj = 0; bj < BI; ++bj) {
-      const int j = j0 + wn * 16 * BI + bj * 16 + (lane & 15);
-      if (j < nbe) {
-        const int rj = bf[j];
+      for (int k = 0; k < kSyrSlots; ++k)
+        if (k < n) {
 #pragma unroll
-        for (int bi = 0; bi < BI; ++bi)
+          for (int r = 0; r < 4; ++r) dst[(k * 4 + r) * 64] = acc[k][r];
+        }
+    } else {
+      // Scatter-add, in transposed order: element (i, j) of the task (i >=
+      // j) is added at (bf[j], bf[i]) of the column-major VXC, so that the 16
+      // lanes of a lane group, 16 consecutive j, touch a few 128-byte column
+      // segments instead of 16 columns.  The symmetrisation that follows
+      // sums the two triangles, so which triangle an element lands in does
+      // not matter.
+      const int32_t* bf = bfmap + t.bf_off;
+      double* vxc = vxc_all + t.p_off;
+#pragma unroll
+      for (int k = 0; k < kSyrSlots; ++k)
+        if (k < n) {
+          const int j = 16 * block_of(uc[k]) + lf, i0 = 16 * block_of(ur[k]) + lq;
+          const int cj = bf[min(j, nbe - 1)];
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const int i = i0 + wm * 16 * BI + bi * 16 + 4 * r + (lane >> 4);
+            const int i = i0 + 4 * r;
             // Negligible contributions are not added (NaN still is).
-            if (i < nbe && (!diag || i >= j) && !(fabs(acc[bi][bj][r]) < drop))
-              atomicAdd(vxc + (int64_t)bf[i] * ldv + rj, acc[bi][bj][r]);
+            if (i < nbe && i >= j && !(fabs(acc[k][r]) < drop))
+              atomicAdd(vxc + (int64_t)bf[i] * t.ldp + cj, acc[k][r]);
           }
-      }
+        }
     }
     stamp_item(qa, it, t0);
   }
 }
 
+// Sums the slices of one block of a region in order and adds it to VXC.
+// Item: task, region (as above), number of slices, first slice's place in
+// part; blockIdx.y is the rank of the block among the region's wanted ones.
+__global__ __launch_bounds__(256) void k_syr2k_reduce(const WorkItem* __restrict__ items,
+                                                      const DevTask* __restrict__ tasks,
+                                                      const int32_t* __restrict__ bfmap,
+                                                      const double* __restrict__ part,
+                                                      double* __restrict__ vxc_all, double drop,
+                                                      const unsigned* __restrict__ tmax) {
+  const WorkItem wi = items[blockIdx.x];
+  const DevTask t = tasks[wi.task];
+  const int tid = threadIdx.x, lane = tid & 63, rank = blockIdx.y;
+  const SyrRegion rg = syr_region(t, wi.a & 0xffff, wi.a >> 16);
+  const uint64_t mask = syr_mask(t, rg, lane, tmax, drop);
+  if (rank >= __popcll(mask)) return;
+  const double* src = part + ((int64_t)wi.c * kSyrBlocks + rank) * 256 + tid;
+  double v = 0.;
+#pragma unroll 8
+  for (int s = 0; s < wi.b; ++s) v += src[(int64_t)s * kSyrBlocks * 256];
+  // The rank-th wanted block.
+  uint64_t m = mask;
+  for (int k = 0; k < rank; ++k) m &= m - 1;
+  const int k = __ffsll((unsigned long long)m) - 1, nc = rg.c1 - rg.c0;
+  const int i = 16 * (rg.r0 + k / nc) + 4 * (tid >> 6) + (lane >> 4);
+  const int j = 16 * (rg.c0 + k % nc) + (lane & 15);
+  const int32_t* bf = bfmap + t.bf_off;
+  if (i < t.nbe && i >= j && !(fabs(v) < drop))
+    atomicAdd(vxc_all + t.p_off + (int64_t)bf[i] * t.ldp + bf[j], v);
+}
+
 int launch_syr2k_mixed(const CtxView& v, const WorkRange& r, int nt);
 
-int launch_syr2k(const CtxView& v, const WorkRange& r, int nt, int precision) {
+int launch_syr2k(const CtxView& v, const Chunk& c, int precision) {
+  if (precision != XCQ_PREC_FP64) {
+    for (int k = 0; k < 2; ++k)
+      if (int rc = launch_syr2k_mixed(v, c.syr2k[k], k == 0 ? 32 : 64)) return rc;
+    return XCQ_SUCCESS;
+  }
+  const WorkRange& r = c.syr2k_f64;
   if (r.n == 0) return XCQ_SUCCESS;
-  if (precision != XCQ_PREC_FP64) return launch_syr2k_mixed(v, r, nt);
-  const QueueArgs qa = queue_args(v, r);
-  const double* scr = static_cast<const double*>(v.scratch);
-  if (nt == 32)
-    hipLaunchKernelGGL(k_syr2k<32>, dim3(grid_of(r)), dim3(256), 0, v.stream, qa, v.tasks,
-                       v.bfmap, scr, v.vxc, v.vxc_drop, v.vxc_drop > 0.0 ? v.tmax : nullptr);
-  else
-    hipLaunchKernelGGL(k_syr2k<64>, dim3(grid_of(r)), dim3(256), 0, v.stream, qa, v.tasks,
-                       v.bfmap, scr, v.vxc, v.vxc_drop, v.vxc_drop > 0.0 ? v.tmax : nullptr);
+  const unsigned* tm = v.vxc_drop > 0.0 ? v.tmax : nullptr;
+  hipLaunchKernelGGL(k_syr2k, dim3(grid_of(r)), dim3(256), 0, v.stream, queue_args(v, r), v.tasks,
+                     v.bfmap, static_cast<const double*>(v.scratch), v.vxc, v.vxc_drop, tm,
+                     v.syr_part);
+  if (c.syr2k_sum.n)
+    hipLaunchKernelGGL(k_syr2k_reduce, dim3((unsigned)c.syr2k_sum.n, kSyrBlocks), dim3(256), 0,
+                       v.stream, v.work + c.syr2k_sum.off, v.tasks, v.bfmap, v.syr_part, v.vxc, v.vxc_drop,
+                       tm);
   XCQ_HIP(hipGetLastError());
   return XCQ_SUCCESS;
 }

@@ -86,8 +86,8 @@ struct DevTask {
   int64_t p_off;      // offset of the molecule's P (and P slices, VXC) in elements
 };
 
-struct WorkItem {  // (task, a, b): a/b are point-block or tile indices
-  int32_t task, a, b, pad_;
+struct WorkItem {  // (task, a, b): a/b are point-block or tile indices (FP64 SYR2K: see Chunk)
+  int32_t task, a, b, c;
 };
 
 // A launchable work list: items [off, off + n) of the context's work array.
@@ -119,8 +119,31 @@ struct Chunk {
   int64_t scratch_elems = 0;  // elements of T (FP64 or FP32) used by B-family arrays
   WorkRange coll;             // all point blocks (collocation) = dens[0..3] back to back
   WorkRange dens[4];          // density blocks by class (DevTask::dens_cls)
-  WorkRange syr2k[2];         // SYR2K tiles (it >= jt) with 32- / 64-function tiles
+  WorkRange syr2k[2];         // mixed SYR2K tiles (it >= jt) with 32- / 64-function tiles
+  // FP64 SYR2K, per region and point slice: a = row group | column group <<
+  // 16, b = slice | slices << 16, c = place in the slice buffer (slices >
+  // 1); and per region with several slices: a as above, b = slices, c = the
+  // first slice's place.
+  WorkRange syr2k_f64, syr2k_sum;
+  int64_t syr_slots = 0;      // places used in the slice buffer
 };
+
+// FP64 SYR2K regions: a task's nb = ceil(nbe / 16) blocks of 16 functions are
+// one region when at most kSyrWhole of them (their triangle fits the
+// kSyrBlocks accumulators), else divided evenly over row groups of up to 7
+// and column groups of up to 6 blocks; its points evenly over its slices.
+constexpr int kSyrRows = 7, kSyrCols = 6, kSyrWhole = 8;
+constexpr int kSyrStaged = kSyrRows + kSyrCols;  // blocks staged at once
+constexpr int kSyrSlots = 11;                    // blocks per wave
+constexpr int kSyrBlocks = 4 * kSyrSlots;        // blocks per region
+static_assert(kSyrRows * kSyrCols <= kSyrBlocks && kSyrWhole <= kSyrStaged &&
+              kSyrWhole * (kSyrWhole + 1) / 2 <= kSyrBlocks, "SYR2K region");
+__host__ __device__ inline int syr_row_groups(int nb) {
+  return nb <= kSyrWhole ? 1 : (nb + kSyrRows - 1) / kSyrRows;
+}
+__host__ __device__ inline int syr_col_groups(int nb) {
+  return nb <= kSyrWhole ? 1 : (nb + kSyrCols - 1) / kSyrCols;
+}
 
 // View of a context's device buffers for the translation units that run
 // pipeline stages (defined in context.hip).
@@ -147,6 +170,7 @@ struct CtxView {
                     // FP64 path runs 3); 3 = for its fold, Z left to a separate launch
   const DevShellC* shc;
   double* zc;       // Z coefficients per point block [4][64] (in-stage mode 3)
+  double* syr_part; // slice buffer of the FP64 SYR2K, kSyrBlocks blocks per place
 };
 // Basis data of the density stage's own evaluation of B and grad B.
 struct ShellArgs {
@@ -169,6 +193,15 @@ inline QueueArgs queue_args(const CtxView& v, const WorkRange& r) {
 inline unsigned grid_of(const WorkRange& r) { return (unsigned)(r.nq ? r.nq : r.n); }
 
 constexpr int64_t kNoItem = INT64_MAX;
+
+// A value every lane of the wave holds, in scalar registers (an item index
+// drawn from a queue comes through LDS, which the compiler cannot know to be
+// uniform; without this everything derived from it would be kept per lane).
+__device__ __forceinline__ int64_t uniform64(int64_t x) {
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)x);
+  const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)((uint64_t)x >> 32));
+  return (int64_t)((uint64_t)hi << 32 | lo);
+}
 
 // Next item of this workgroup's dynamic queue, or kNoItem.  Every thread of
 // the workgroup calls it (uniform control flow): one lane takes a ticket
@@ -298,8 +331,8 @@ int launch_ssf_grad(const CtxView& v, const WorkRange& r, int natoms, const doub
                     const double* dnear, const double* wf, double* grad,
                     const int32_t* nbr_idx = nullptr, const double* nbr_r = nullptr);
 int launch_z_from_coeffs(const CtxView& v, const WorkRange& r, int gga, const double* coef);
-// B^T Z + Z^T B with the VXC scatter-add, one work range of `nt`-wide tiles.
-int launch_syr2k(const CtxView& v, const WorkRange& r, int nt, int precision);
+// B^T Z + Z^T B of a chunk with the VXC scatter-add.
+int launch_syr2k(const CtxView& v, const Chunk& c, int precision);
 int launch_P_to_f32(hipStream_t s, int64_t n, const double* P, float* out);
 int launch_fill(hipStream_t s, double* p, int64_t n);
 // Symmetrise the VXC of nmol molecules: mol_n[m] = nbf, mol_off[m] = offset.
