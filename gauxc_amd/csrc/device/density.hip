@@ -1,41 +1,30 @@
 // Density stage of the XC path: X = fac B P_sub, rho / grad rho, the
-// functional with weight folding, the EXC/NEL block sums and the Z matrix,
-// in one launch.
+// functional with weight folding, the EXC/NEL block sums and the Z matrix.
 //
 // One 256-thread workgroup owns one (task, 64-point block) and walks every
-// 64-function column tile of the task.  Per tile it forms the transposed
-// product X^T = fac P_sub B^T (64 functions x 64 points) on the matrix
-// cores, so that an accumulator register holds one function of 16
-// consecutive points across a lane group: the epilogue then reads B and
-// grad B rows with coalesced 16-point segments (the planes are stored
-// point-contiguous) and folds
+// function tile of the task.  Per tile it forms the transposed product
+// X^T = fac P_sub B^T (functions x 64 points) on the matrix cores and folds
 //   rho_p = sum_j B_pj X_pj,   grad rho_p = 2 sum_j dB_pj X_pj
-// (reference_local_host_work_driver.cxx:242-268) into per-point partials
-// kept in LDS.  After the last tile the block's 64 points are complete: the
-// functional runs in the same workgroup (host_integrator_exc_vxc.hpp:445-502)
-// and gives the Z coefficients a = w vrho / 2, c = 2 w vsigma grad rho and
-// the block's (w eps rho, w rho) sums; the tail then writes
-//   Z = a B + c . grad B        (reference_local_host_work_driver.cxx:678-713)
-// for the block's points.  X never reaches HBM.
+// (reference_local_host_work_driver.cxx:242-268) into per-point partials.
+// After the last tile the block's 64 points are complete.  FP64: the sums go
+// to memory (32 bytes per point), k_xc_points evaluates the functional
+// (host_integrator_exc_vxc.hpp:445-502) and leaves the Z coefficients a = w
+// vrho / 2, c = 2 w vsigma grad rho and the block's (w eps rho, w rho) sums,
+// and a further launch forms
+//   Z = a B + c . grad B        (reference_local_host_work_driver.cxx:678-713).
+// Mixed precision: the functional and, but for in-stage mode 3, Z follow in
+// the same workgroup.  X never reaches HBM.
 //
-// The K loop is software-pipelined: step s+1's global loads are issued into
-// registers before step s's matrix instructions, and the LDS stage is double
-// buffered so one barrier per step suffices.  Out-of-range rows/columns are
-// read at a clamped (valid) index and zeroed by a select, so the loads are
-// branch-free.  K indices are uniform across a wave, which makes the
-// basis-map lookups scalar loads.
-//
-// Both kernels are templated on the function tile NT (32 or 64): a task's
-// rows are covered by ceil(nbe / NT) tiles, so small tasks are not padded to
-// 64.  A launch either runs one workgroup per (task, block) item or, in
-// queued mode, one persistent workgroup per queue of items.
+// The K loops are software-pipelined, the LDS stages double buffered, one
+// barrier per step.  The mixed kernel is templated on the function tile NT
+// (32, 64 or 128).  A launch either runs one workgroup per (task, block)
+// item or, in queued mode, one persistent workgroup per queue of items.
 //
 // Basis evaluation mode (template argument INSTAGE): 0 reads B and grad B
 // from the planes the collocation stage stored; in the in-stage modes the
 // fold evaluates them at the block's points from the shell parameters
-// (fold_in_stage) and Z is formed either in the same kernel (mode 1,
-// z_in_stage) or by a separate launch from the Z coefficients this kernel
-// leaves (mode 3, k_z_in_stage in collocation.hip).
+// and Z is formed either in the same kernel (mode 1, z_in_stage) or by a
+// separate launch (mode 3, k_z_in_stage in collocation.hip).
 #include "internal.hpp"
 #include "functional.hpp"
 #include "shell_eval.hpp"
@@ -49,12 +38,6 @@ using v4d = double __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 namespace {
-
-constexpr int kPad64 = 68;  // FP64 stage row (doubles)
-
-
-
-
 
 __device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
@@ -606,41 +589,115 @@ __device__ __forceinline__ void z_in_stage(const DevTask& t, const ShellArgs& sa
 
 // ---------------------------------------------------------------------------
 // FP64 (v_mfma_f64_16x16x4_f64; accumulator register r of lane l holds row
-// 4r + l/16).  Waves: wm = function half (NT/2 rows = BI blocks of 16),
-// wn = point half of the 64-point block.  Loader roles: thread
-// (c = tid & 63, q = tid >> 6) loads K rows 4q..4q+3 of column c of the B^T
-// stage (point c) and, for c < NT, of the P_sub stage (function n0 + c).
-// INSTAGE = 3: the fold evaluates B and grad B itself (fold_in_stage, from
-// the X^T tile written over the stages) and the block's Z coefficients go
-// to zbuf for the separate Z launch; 0: the fold and Z read the planes the
-// collocation stage stored.  HIOCC (in-stage, 64-wide tiles): a register
-// budget for three workgroups per CU, which spills a few registers of the
-// fold and still hides more latency.
-template <int NT, bool GGA, int INSTAGE, bool HIOCC = false>
-__global__ __launch_bounds__(256, HIOCC ? 3 : 2) void k_density_f64(
+// 4r + l/16).  Function tiles of up to 64 rows, a task's blocks of 16
+// functions divided evenly over them; wave w owns 16 of the block's 64 points
+// and every row of the tile, so
+//  * rows are multiplied in steps of 16, not of a tile: the tile's number of
+//    16-row blocks picks one of four K loops;
+//  * a wave whose points all lie past npts skips its products (the point
+//    group is rotated by the block index, so that this does not always idle
+//    the same SIMD);
+//  * the B^T operand, which no other wave needs, comes straight from memory
+//    to registers, one K step of 16 ahead; only P_sub is staged in LDS.
+// P_sub rows are gathered one K step ahead into registers as well: wave w
+// fetches rows 4w .. 4w + 3 of the step, lane = function.  The rows' basis
+// functions (64 of them per vector load, a whole chunk ahead) are broadcast
+// by readlane, so no scalar load is waited for inside the K loop.
+// INSTAGE = 3: the fold evaluates B and grad B itself, from X^T written over
+// the stages and from the tile's shells, which were staged in LDS while the
+// product ran; 0: it reads the planes the collocation stage stored.
+//
+// What bounds it: on gfx950 an FP64 MFMA and another wave's vector
+// instructions do not overlap (measured: 0.45 ms of the one and 0.64 ms of
+// the other take 1.06 ms together), so the products and the fold add up (4.7
+// of the first version's 7.9 ms on 24 waters); the rest were chains of
+// dependent loads, barriers and the functional on one wave of four, with two
+// waves per SIMD to cover them.  The functional is now a launch of its own,
+// the shells come from LDS, and four waves fit a SIMD (20 registers spill;
+// three waves without spills: 6.7 ms).  24 waters: 8.9 (64-wide padded
+// tiles, 1.4 times the products wanted) -> 6.1 ms; 150 waters: 152 -> 138 ms,
+// there bound by L2 misses (890 GB, 6.5 TB/s); 84 functions: 52 -> 28 us.
+constexpr int kF64K = 16;  // K rows per stage
+
+// Shells of one tile of NT functions (at most NT + 1 of them, and one more
+// for each of the four waves' loops to end on), staged in LDS while the
+// tile's product runs.
+template <int NT>
+struct FoldShells {
+  static constexpr int kMax = NT + 5;
+  double ox[kMax], oy[kMax], oz[kMax], a0[kMax], c0[kMax];
+  int bf0[kMax], info[kMax], ish[kMax];
+  int next;  // shell holding the function after the tile
+};
+
+// As fold_in_stage, the shells from LDS: wave w takes shells w, w + 4, ...
+// until one starts at or past nhi.
+template <bool GGA, int NT>
+__device__ __forceinline__ void fold_staged(const ShellArgs& sa, const FoldShells<NT>& fs, int nlo,
+                                            int nhi, int wave, int lane, const double* xt,
+                                            double rx, double ry, double rz, double (&r)[4]) {
+  for (int j = wave;; j += 4) {
+    const int bf0 = uni(fs.bf0[j]);
+    if (bf0 >= nhi) break;
+    const int info = uni(fs.info[j]);
+    const int l = info & 0xff, nprim = info >> 16;
+    const bool pure = (info >> 8) & 1;
+    const double x = rx - fs.ox[j], y = ry - fs.oy[j], z = rz - fs.oz[j];
+    const double a0 = fs.a0[j];
+    const double r2 = x * x + y * y + z * z;
+    double R = fs.c0[j] * exp(-a0 * r2), dR = -2. * a0 * R;
+    if (nprim > 1) {
+      const DevShell* sh = sa.shells + uni(fs.ish[j]);
+      for (int k = 1; k < nprim; ++k) {
+        const double a = sh->alpha[k], e = sh->coeff[k] * exp(-a * r2);
+        R += e;
+        dR += -2. * a * e;
+      }
+    }
+    double sy = 0., sgx = 0., sgy = 0., sgz = 0.;
+    shell_functions_l<kInStageMaxL, GGA, true, true>(
+        l, x, y, z, R, dR, pure, [&](int f, double v, double gx, double gy, double gz) {
+          const int n = bf0 + f;  // uniform
+          if (n >= nlo && n < nhi) {
+            const double xv = xt[(n - nlo) * kXLd + lane];
+            sy += v * xv;
+            if constexpr (GGA) {
+              sgx += gx * xv;
+              sgy += gy * xv;
+              sgz += gz * xv;
+            }
+          }
+        });
+    r[0] += R * sy;
+    if constexpr (GGA) {
+      const double d = dR * sy;
+      r[1] += R * sgx + d * x;
+      r[2] += R * sgy + d * y;
+      r[3] += R * sgz + d * z;
+    }
+  }
+}
+
+template <bool GGA, int INSTAGE, int NT>
+__global__ __launch_bounds__(256, 4) void k_density_f64(
     QueueArgs qa, const DevTask* __restrict__ tasks, const int32_t* __restrict__ bfmap,
-    const double* __restrict__ Pall, double* __restrict__ scratch,
-    const double* __restrict__ weights, int func, double fac, int want_z,
-    double* __restrict__ red, unsigned* __restrict__ tmax, ShellArgs sa,
-    double* __restrict__ zbuf, double* __restrict__ dens_out, int x_plane) {
-  constexpr int BI = NT / 32;
-  constexpr int kPtD = 2 * 16 * (NT + 4), kStageD = kPtD + 2 * 16 * kPad64;
-  static_assert(INSTAGE == 0 || NT * kXLd <= kStageD, "X^T tile must fit the stages");
-  __shared__ double stage[kStageD];
-  // [buf][k][function]: A operand (P_sub); [buf][k][point]: B operand (B^T)
-  double(*Pt)[16][NT + 4] = reinterpret_cast<double(*)[16][NT + 4]>(stage);
-  double(*Bt)[16][kPad64] = reinterpret_cast<double(*)[16][kPad64]>(stage + kPtD);
-  __shared__ double dens[4][64][4];
-  __shared__ double zc[4][64];
-  __shared__ unsigned smax[kGranLds][2];
+    const double* __restrict__ Pall, double* __restrict__ scratch, double fac, ShellArgs sa,
+    double* __restrict__ dens_out, int x_plane) {
+  constexpr int kBI = NT / 16;
+  static_assert(NT == 64, "the tile is 64 functions");
+  constexpr int kLd = NT + 16;  // stage row: four K rows hit distinct banks
+  constexpr int kStage = kF64K * kLd;
+  constexpr int kStageD = 2 * kStage > 64 * kXLd ? 2 * kStage : 64 * kXLd;
+  __shared__ __attribute__((aligned(16))) double stage[kStageD];  // P_sub [buf][k][function]
+  // The per-point partials take the stages' place after the last tile.
+  double(*dens)[64][4] = reinterpret_cast<double(*)[64][4]>(stage);
+  __shared__ FoldShells<NT> fs;
   const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
-  const int wm = wave & 1, wn = wave >> 1;
-  const int lc = lane, lq = wave;  // loader column / K quad
-  auto frow = [&](int r) { return 4 * r + (lane >> 4); };
+  const int lf = lane & 15, lq = lane >> 4;
 
   XCQ_FOR_EACH_ITEM(qa, it) {
     const int64_t t0 = qa.tstamp ? wall_clock64() : 0;
-    const WorkItem wi = qa.items[it];
+    const WorkItem wi = qa.items[uniform64(it)];
     const DevTask t = tasks[wi.task];
     const int m0 = wi.a * kPtBlock;
     const int ld = t.npts_pad;
@@ -650,14 +707,13 @@ __global__ __launch_bounds__(256, HIOCC ? 3 : 2) void k_density_f64(
     const double* P = Pall + t.p_off;
     double* Bm = scratch + t.b_off;
     const int32_t* bf = bfmap + t.bf_off;
-    for (int i = tid; i < 4 * 64 * 4; i += 256) (&dens[0][0][0])[i] = 0.;
-    if (tid < 2 * kGranLds) (&smax[0][0])[tid] = 0u;
-    __syncthreads();
-    const double* bcol = Bm + m0 + lc;
-    const int nks = (nbe + 15) / 16;
-    // In-stage fold: this lane's point (padded points take the task's last
-    // point: finite values, which meet zero X), the shell cursor and this
-    // wave's density partials.
+    const int pg = (wave + wi.a) & 3;           // the wave's 16 points of the block
+    const int pcol = m0 + 16 * pg + lf;         // this lane's point (column)
+    const bool active = m0 + 16 * pg < t.npts;  // the wave has points
+    const int nks = (nbe + kF64K - 1) / kF64K;
+    // In-stage fold: lane = point (padded points take the task's last point:
+    // finite values, which meet zero X) and this wave's density partials; on
+    // stored planes the partials of the lane's column.
     double rx = 0., ry = 0., rz = 0.;
     if constexpr (INSTAGE != 0) {
       const int pl = min(m0 + lane, t.npts - 1);
@@ -667,135 +723,216 @@ __global__ __launch_bounds__(256, HIOCC ? 3 : 2) void k_density_f64(
     }
     int s_cur = 0;
     double part[4] = {0., 0., 0., 0.};
+    const auto rsB = __builtin_amdgcn_make_buffer_rsrc(Bm, 0, (int)((unsigned)plane * 8u), 0x00020000);
 
-    for (int n0 = 0; n0 < nbe; n0 += NT) {
-      const int ncol = n0 + lc;
-      const bool colok = lc < NT && ncol < nbe;
-      const double* Pc = P + bf[min(ncol, nbe - 1)];  // column bf[n] of P (P symmetric)
-      // Prefetch registers hold raw loads; the masks and the factor are
-      // applied when they are staged, so no load is waited for before the
-      // matrix instructions of the current step are issued.
-      double rb[4], rp[4];
-      auto load = [&](int k0) {
-        int rowp[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) rowp[e] = bf[min(k0 + 4 * lq + e, nbe - 1)];  // scalar
+    // Tiles of 16-row blocks [blk, blk + nbk).
+    const int ntile = (nks + kBI - 1) / kBI;
+    for (int tile = 0; tile < ntile; ++tile) {
+      const int blk = tile * nks / ntile, nbk = (tile + 1) * nks / ntile - blk;
+      const int n0 = 16 * blk, nhi = min(n0 + 16 * nbk, nbe);
+      // P is symmetric: P(n, k) is read as row bf[k], column bf[n], so that
+      // neighbouring lanes touch neighbouring elements.  Rows of the tile
+      // past nbe repeat the last function; their X is not used.
+      const unsigned cn = 8u * (unsigned)bf[min(n0 + lane, nbe - 1)];
+      int vrow = bf[min(lane, nbe - 1)];  // functions of the current 64 K rows
+      int vnext = bf[min(64 + lane, nbe - 1)];
+      double rp[4], rb[4];
+      auto load = [&](int s) {
+        if (s > 0 && (s & 3) == 0) {
+          vrow = vnext;
+          vnext = bf[min(16 * s + 64 + lane, nbe - 1)];
+        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int kc = min(k0 + 4 * lq + e, nbe - 1);
-          rb[e] = bcol[kc * ld];
-          rp[e] = Pc[(int64_t)rowp[e] * ldp];
+          const int row = __builtin_amdgcn_readlane(vrow, (16 * s + 4 * wave + e) & 63);
+          rp[e] = *reinterpret_cast<const double*>(
+              reinterpret_cast<const char*>(P + (int64_t)row * ldp) + cn);
+        }
+        if (16 * s + 16 <= nbe) {
+#pragma unroll
+          for (int ks = 0; ks < 4; ++ks)
+            rb[ks] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(
+                rsB, (lq * ld + pcol) * 8, (16 * s + 4 * ks) * ld * 8, 0));
+        } else {
+#pragma unroll
+          for (int ks = 0; ks < 4; ++ks)
+            rb[ks] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(
+                rsB, (min(16 * s + 4 * ks + lq, nbe - 1) * ld + pcol) * 8, 0, 0));
         }
       };
-      v4d acc[BI][2];
-#pragma unroll
-      for (int i = 0; i < BI; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = v4d{0., 0., 0., 0.};
       load(0);
-      for (int s = 0; s < nks; ++s) {
-        const int buf = s & 1;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const bool kok = 16 * s + 4 * lq + e < nbe;
-          Bt[buf][4 * lq + e][lc] = kok ? rb[e] : 0.;
-          if (lc < NT) Pt[buf][4 * lq + e][lc] = (kok && colok) ? fac * rp[e] : 0.;
-        }
-        __syncthreads();
-        if (s + 1 < nks) load(16 * (s + 1));
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-          const int kr = ks * 4 + (lane >> 4);
-          double a[BI];
-#pragma unroll
-          for (int bi = 0; bi < BI; ++bi) a[bi] = Pt[buf][kr][wm * 16 * BI + bi * 16 + (lane & 15)];
-          const double b0 = Bt[buf][kr][wn * 32 + (lane & 15)];
-          const double b1 = Bt[buf][kr][wn * 32 + 16 + (lane & 15)];
-#pragma unroll
-          for (int bi = 0; bi < BI; ++bi) {
-            acc[bi][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[bi], b0, acc[bi][0], 0, 0, 0);
-            acc[bi][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[bi], b1, acc[bi][1], 0, 0, 0);
+      if constexpr (INSTAGE != 0) {
+        // The shells of this tile's functions; the first ones past it end
+        // the fold's loops.
+        if (tid < FoldShells<NT>::kMax) {
+          const int s = s_cur + tid;
+          int f0 = INT_MAX, f1 = INT_MAX, ish = 0;
+          if (s < t.nshells) {
+            f0 = sa.lsh[t.lsh_off + s];
+            ish = sa.shell_list[t.sh_off + s];
+            if (s + 1 < t.nshells) f1 = sa.lsh[t.lsh_off + s + 1];
           }
+          const DevShellC c = sa.shc[ish];
+          fs.bf0[tid] = f0;
+          fs.ish[tid] = ish;
+          fs.info[tid] = c.info;
+          fs.ox[tid] = c.ox;
+          fs.oy[tid] = c.oy;
+          fs.oz[tid] = c.oz;
+          fs.a0[tid] = c.a0;
+          fs.c0[tid] = c.c0;
+          if (f0 <= nhi && f1 > nhi) fs.next = s;
         }
       }
-      if ((INSTAGE == 0 || !HIOCC) && x_plane >= 0) {
-        // The X tile itself into plane x_plane (row = function, column =
-        // point), for callers that contract it again (the EXC gradient; not
-        // in the three-workgroups-per-CU configuration, whose register
-        // budget it would overrun).
-        double* xo = Bm + (int64_t)x_plane * plane + m0;
+      v4d acc[kBI];
 #pragma unroll
-        for (int bi = 0; bi < BI; ++bi)
+      for (int i = 0; i < kBI; ++i) acc[i] = v4d{0., 0., 0., 0.};
+      auto contract = [&](auto NB) {
+        constexpr int BI = decltype(NB)::value;
+        for (int s = 0; s < nks; ++s) {
+          double* st = stage + (s & 1) * kStage;
+          double b[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            // P rows past nbe are zero, B rows past it repeat the last one.
+            const bool kok = 16 * s + 4 * wave + e < nbe;
+            st[(4 * wave + e) * kLd + lane] = kok ? rp[e] : 0.;
+            b[e] = rb[e];
+          }
+          __syncthreads();
+          if (s + 1 < nks) load(s + 1);
+          if (active) {
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) {
+              double a[BI];
+#pragma unroll
+              for (int i = 0; i < BI; ++i) a[i] = st[(4 * ks + lq) * kLd + 16 * i + lf];
+#pragma unroll
+              for (int i = 0; i < BI; ++i)
+                acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[ks], acc[i], 0, 0, 0);
+            }
+          }
+        }
+      };
+      switch (nbk) {
+        case 1: contract(std::integral_constant<int, 1>{}); break;
+        case 2: contract(std::integral_constant<int, 2>{}); break;
+        case 3: contract(std::integral_constant<int, 3>{}); break;
+        default: contract(std::integral_constant<int, 4>{}); break;
+      }
+#pragma unroll
+      for (int i = 0; i < kBI; ++i) acc[i] *= fac;  // 1 or 2: exact
+      if (x_plane >= 0) {
+        // The X tile itself into plane x_plane (row = function, column =
+        // point), for callers that contract it again (the EXC gradient).
+        double* xo = Bm + (int64_t)x_plane * plane + pcol;
+#pragma unroll
+        for (int i = 0; i < kBI; ++i)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const int row = n0 + wm * 16 * BI + bi * 16 + frow(r);
-            if (row < nbe) {
-#pragma unroll
-              for (int bj = 0; bj < 2; ++bj)
-                xo[(int64_t)row * ld + wn * 32 + bj * 16 + (lane & 15)] = acc[bi][bj][r];
-            }
+            const int row = n0 + 16 * i + 4 * r + lq;
+            if (row < nhi) xo[(int64_t)row * ld] = acc[i][r];
           }
       }
       if constexpr (INSTAGE != 0) {
-        double* xt = stage;
-        __syncthreads();  // every wave is done with the last K step's stage
+        __syncthreads();  // every wave is done with the stages
 #pragma unroll
-        for (int bi = 0; bi < BI; ++bi)
+        for (int i = 0; i < kBI; ++i)
 #pragma unroll
-          for (int bj = 0; bj < 2; ++bj)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              xt[(wm * 16 * BI + bi * 16 + frow(r)) * kXLd + wn * 32 + bj * 16 + (lane & 15)] =
-                  acc[bi][bj][r];
+          for (int r = 0; r < 4; ++r)
+            stage[(16 * i + 4 * r + lq) * kXLd + 16 * pg + lf] = acc[i][r];
         __syncthreads();
-        s_cur = fold_in_stage<GGA>(t, sa, s_cur, n0, min(n0 + NT, nbe), wave, lane, xt, rx, ry,
-                                   rz, part);
+        fold_staged<GGA, NT>(sa, fs, n0, nhi, wave, lane, stage, rx, ry, rz, part);
+        s_cur = uni(fs.next);
       } else {
-        double x[BI][2][4];
 #pragma unroll
-        for (int i = 0; i < BI; ++i)
+        for (int i = 0; i < kBI; ++i) {
+          if (16 * i >= nhi - n0) break;
 #pragma unroll
-          for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) x[i][j][r] = acc[i][j][r];
-        fold_tile<double, BI, GGA>(x, frow, m0, n0, wm, wn, lane, nbe, ld, plane, Bm, dens);
+          for (int r = 0; r < 4; ++r) {
+            const int j = n0 + 16 * i + 4 * r + lq, o = min(j, nbe - 1) * ld + pcol;
+            const double xv = j < nhi ? acc[i][r] : 0.;
+            part[0] += Bm[o] * xv;
+            if constexpr (GGA) {
+              part[1] += Bm[plane + o] * xv;
+              part[2] += Bm[2 * plane + o] * xv;
+              part[3] += Bm[3 * plane + o] * xv;
+            }
+          }
+        }
       }
-      // The next tile's first stage write targets buffer 0, last read at step
-      // nks-2 (or nks-1 when nks == 1), or the X^T tile; all waves pass this
-      // barrier after it.
-      __syncthreads();
+      __syncthreads();  // the next tile's first stage write is safe
     }
+    constexpr int ND = INSTAGE != 0 ? 4 : 1;
     if constexpr (INSTAGE != 0) {
 #pragma unroll
       for (int c = 0; c < 4; ++c) dens[wave][lane][c] = part[c];
-      __syncthreads();
-    }
-    if (dens_out) {
-      // One spin component of a UKS evaluation: the block's raw sums
-      // (sum B X, sum dB/dx X, ...) per point, [block][4][64]; the
-      // polarised functional runs once both components are in.
-      constexpr int ND = INSTAGE != 0 ? 4 : 2;
-      if (tid < 64) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          double v = 0.;
-#pragma unroll
-          for (int d = 0; d < ND; ++d) v += dens[d][tid][c];
-          dens_out[(t.red_off + wi.a) * 256 + c * 64 + tid] = v;
-        }
-      }
     } else {
-      finish_points<INSTAGE != 0 ? 4 : 2>(t, wi.a, tid, dens, zc, weights, func, GGA, red);
-      if (want_z) {
-        __syncthreads();
-        if constexpr (INSTAGE != 0)
-          zbuf[(t.red_off + wi.a) * 256 + tid] = (&zc[0][0])[tid];
-        else
-          write_z<double, GGA>(t, m0, tid, zc, Bm, smax, tmax ? tmax + 2 * t.tmax_off : nullptr);
+      // Sum over the four 16-lane groups (different functions, same point).
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        part[c] += __shfl_xor(part[c], 16);
+        part[c] += __shfl_xor(part[c], 32);
+        if (lane < 16) dens[0][16 * pg + lf][c] = part[c];
+      }
+    }
+    __syncthreads();
+    // The block's raw sums (sum B X, sum dB/dx X, ...) per point,
+    // [block][4][64].
+    if (tid < 64) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        double v = 0.;
+#pragma unroll
+        for (int d = 0; d < ND; ++d) v += dens[d][tid][c];
+        dens_out[(t.red_off + wi.a) * 256 + c * 64 + tid] = v;
       }
     }
     stamp_item(qa, it, t0);
     __syncthreads();
+  }
+}
+
+// Functional of the FP64 path from the density stage's raw sums, one wave
+// per point block: the Z coefficients over the sums and the block's (EXC,
+// NEL) partials.  A launch of its own: inside the density kernel it ran on
+// one wave of four, for 3 of a workgroup's 50 us, and its registers alone
+// kept that kernel at two waves per SIMD.
+__global__ __launch_bounds__(64) void k_xc_points(const WorkItem* __restrict__ items,
+                                                  const DevTask* __restrict__ tasks,
+                                                  const double* __restrict__ weights, int func,
+                                                  int gga, double* __restrict__ sums,
+                                                  double* __restrict__ red) {
+  const WorkItem wi = items[blockIdx.x];
+  const DevTask t = tasks[wi.task];
+  const int tid = threadIdx.x;
+  double* s = sums + (t.red_off + wi.a) * 256 + tid;
+  const int p = wi.a * kPtBlock + tid;
+  const double rho = s[0];
+  const double gx = 2.0 * s[64], gy = 2.0 * s[128], gz = 2.0 * s[192];
+  double e = 0., n = 0., za = 0., c = 0.;
+  if (p < t.npts) {
+    const double w = weights[t.pt_off + p];
+    n = w * rho;
+    if (func != 0) {
+      const XCOut o =
+          dev_eval_functional(func, rho, gga ? gx * gx + gy * gy + gz * gz : 0.);
+      e = w * o.e;
+      za = 0.5 * w * o.vr;
+      c = gga ? 2.0 * w * o.vs : 0.;
+    }
+  }
+  s[0] = za;
+  s[64] = c * gx;
+  s[128] = c * gy;
+  s[192] = c * gz;
+  for (int off = 32; off > 0; off >>= 1) {
+    e += __shfl_xor(e, off);
+    n += __shfl_xor(n, off);
+  }
+  if (tid == 0) {
+    red[2 * (t.red_off + wi.a)] = e;
+    red[2 * (t.red_off + wi.a) + 1] = n;
   }
 }
 
@@ -1317,20 +1454,24 @@ __global__ __launch_bounds__(64) void k_fxc_points_uks(
 }
 
 // Z = a B + c . grad B of one point block from stored coefficients
-// ([block][4][64]) and the stored FP64 planes (no screening bounds).
+// ([block][4][64]) and the stored FP64 planes, with the screening bounds when
+// tmax is given.
 template <bool GGA>
 __global__ __launch_bounds__(256) void k_z_from_coeffs(const WorkItem* __restrict__ items,
                                                        const DevTask* __restrict__ tasks,
                                                        double* __restrict__ scratch,
-                                                       const double* __restrict__ coef) {
+                                                       const double* __restrict__ coef,
+                                                       unsigned* __restrict__ tmax) {
   __shared__ double zc[4][64];
   __shared__ unsigned smax[kGranLds][2];
   const WorkItem wi = items[blockIdx.x];
   const DevTask t = tasks[wi.task];
   const int tid = threadIdx.x;
   (&zc[0][0])[tid] = coef[(t.red_off + wi.a) * 256 + tid];
+  if (tid < 2 * kGranLds) (&smax[0][0])[tid] = 0u;
   __syncthreads();
-  write_z<double, GGA>(t, wi.a * kPtBlock, tid, zc, scratch + t.b_off, smax, nullptr);
+  write_z<double, GGA>(t, wi.a * kPtBlock, tid, zc, scratch + t.b_off, smax,
+                       tmax ? tmax + 2 * t.tmax_off : nullptr);
 }
 
 int launch_uks_points(const CtxView& v, const WorkRange& r, int func, int gga, const double* ds,
@@ -1361,90 +1502,105 @@ int launch_fxc_points_uks(const CtxView& v, const WorkRange& r, int func, int gg
   return XCQ_SUCCESS;
 }
 
-int launch_z_from_coeffs(const CtxView& v, const WorkRange& r, int gga, const double* coef) {
+int launch_z_from_coeffs(const CtxView& v, const WorkRange& r, int gga, const double* coef,
+                         unsigned* tmax) {
   if (r.n == 0) return XCQ_SUCCESS;
   double* scr = static_cast<double*>(v.scratch);
-  if (gga)
-    hipLaunchKernelGGL(k_z_from_coeffs<true>, dim3((unsigned)r.n), dim3(256), 0, v.stream,
-                       v.work + r.off, v.tasks, scr, coef);
-  else
-    hipLaunchKernelGGL(k_z_from_coeffs<false>, dim3((unsigned)r.n), dim3(256), 0, v.stream,
-                       v.work + r.off, v.tasks, scr, coef);
+  auto kern = gga ? k_z_from_coeffs<true> : k_z_from_coeffs<false>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)r.n), dim3(256), 0, v.stream, v.work + r.off, v.tasks,
+                     scr, coef, tmax);
   XCQ_HIP(hipGetLastError());
   return XCQ_SUCCESS;
 }
 
-int launch_density(const CtxView& v, const WorkRange& r, int nt, bool hiocc, int precision,
-                   int func, int gga, double fac, int want_z, const double* P_override,
-                   double* dens_out, int x_plane) {
+int launch_xc_points(const CtxView& v, const WorkRange& r, int func, int gga, double* sums) {
   if (r.n == 0) return XCQ_SUCCESS;
-  XCQ_REQUIRE(x_plane < 0 || (precision == XCQ_PREC_FP64 && !hiocc && x_plane < 5),
-              XCQ_ERROR_INVALID_ARGUMENT,
-              "the X plane is stored by the FP64 kernels in their two-workgroup configuration");
+  hipLaunchKernelGGL(k_xc_points, dim3((unsigned)r.n), dim3(64), 0, v.stream, v.work + r.off,
+                     v.tasks, v.w, func, gga, sums, v.red);
+  XCQ_HIP(hipGetLastError());
+  return XCQ_SUCCESS;
+}
+
+int launch_density_f64(const CtxView& v, const Chunk& c, int gga, double fac, const double* P,
+                       double* dens_out, int x_plane) {
+  XCQ_REQUIRE(x_plane < 5, XCQ_ERROR_INVALID_ARGUMENT, "the scratch has five planes");
+  const ShellArgs sa{v.shells, v.shc, v.shell_list, v.lsh, v.px, v.py, v.pz};
+  double* scr = static_cast<double*>(v.scratch);
+  auto go = [&](auto kern, const WorkRange& r) {
+    if (r.n)
+      hipLaunchKernelGGL(kern, dim3(grid_of(r)), dim3(256), 0, v.stream, queue_args(v, r), v.tasks,
+                         v.bfmap, P, scr, fac, sa, dens_out, x_plane);
+  };
+  auto run = [&](auto kern) {
+    // One kernel serves every class; each class has queues of its own.
+    if (c.dens[0].nq || c.dens[1].nq || c.dens[2].nq || c.dens[3].nq)
+      for (const WorkRange& r : c.dens) go(kern, r);
+    else
+      go(kern, c.coll);
+  };
+  // Any in-stage mode runs the FP64 kernel's one (mode 3).
+  if (v.in_stage != 0)
+    gga ? run(k_density_f64<true, 3, 64>) : run(k_density_f64<false, 3, 64>);
+  else
+    gga ? run(k_density_f64<true, 0, 64>) : run(k_density_f64<false, 0, 64>);
+  XCQ_HIP(hipGetLastError());
+  return XCQ_SUCCESS;
+}
+
+namespace {
+int launch_density_mx(const CtxView& v, const WorkRange& r, int nt, bool hiocc, int func, int gga,
+                      double fac, int want_z) {
+  if (r.n == 0) return XCQ_SUCCESS;
   const QueueArgs qa = queue_args(v, r);
   const dim3 grid(grid_of(r)), block(256);
-  // The bound table is filled only when VXC is computed and contributions
-  // may be dropped.
   unsigned* tm = (want_z && v.vxc_drop > 0.0) ? v.tmax : nullptr;
   const ShellArgs sa{v.shells, v.shc, v.shell_list, v.lsh, v.px, v.py, v.pz};
-  if (precision == XCQ_PREC_FP64) {
-    double* scr = static_cast<double*>(v.scratch);
-    const double* P = P_override ? P_override : v.P;
-    auto go = [&](auto kern) {
-      hipLaunchKernelGGL(kern, grid, block, 0, v.stream, qa, v.tasks, v.bfmap, P, scr, v.w,
-                         func, fac, want_z, v.red, tm, sa, v.zc, dens_out, x_plane);
-    };
-    // Any in-stage mode runs the FP64 kernel's one (mode 3).
-    if (v.in_stage != 0) {
-      if (nt == 32)
-        gga ? go(k_density_f64<32, true, 3>) : go(k_density_f64<32, false, 3>);
-      else if (hiocc)
-        gga ? go(k_density_f64<64, true, 3, true>) : go(k_density_f64<64, false, 3, true>);
-      else
-        gga ? go(k_density_f64<64, true, 3>) : go(k_density_f64<64, false, 3>);
+  float* scr = static_cast<float*>(v.scratch);
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, block, 0, v.stream, qa, v.tasks, v.bfmap, v.Pf32, scr, v.w,
+                       func, fac, want_z, v.red, tm, sa, v.zc);
+  };
+  // Template arguments: tile width, GGA, high occupancy, in-stage mode.
+  auto pick = [&](auto g, auto ins) {
+    constexpr bool G = decltype(g)::value;
+    constexpr int I = decltype(ins)::value;
+    if (nt == 32) {
+      go(k_density_mx<32, G, false, I>);
+    } else if (nt == 128) {
+      go(k_density_mx<128, G, false, I>);
+    } else if constexpr (I != 1) {
+      if (hiocc) go(k_density_mx<64, G, true, I>);
+      else go(k_density_mx<64, G, false, I>);
     } else {
-      if (nt == 32)
-        gga ? go(k_density_f64<32, true, 0>) : go(k_density_f64<32, false, 0>);
-      else
-        gga ? go(k_density_f64<64, true, 0>) : go(k_density_f64<64, false, 0>);
+      // The in-stage fold with the in-kernel Z pass needs more than the
+      // 168 registers of the three-workgroups-per-CU configuration; it
+      // runs at two.
+      go(k_density_mx<64, G, false, I>);
     }
-  } else {
-    float* scr = static_cast<float*>(v.scratch);
-    auto go = [&](auto kern) {
-      hipLaunchKernelGGL(kern, grid, block, 0, v.stream, qa, v.tasks, v.bfmap, v.Pf32, scr, v.w,
-                         func, fac, want_z, v.red, tm, sa, v.zc);
-    };
-    // Template arguments: tile width, GGA, high occupancy, in-stage mode.
-    auto pick = [&](auto g, auto ins) {
-      constexpr bool G = decltype(g)::value;
-      constexpr int I = decltype(ins)::value;
-      if (nt == 32) {
-        go(k_density_mx<32, G, false, I>);
-      } else if (nt == 128) {
-        go(k_density_mx<128, G, false, I>);
-      } else if constexpr (I != 1) {
-        if (hiocc) go(k_density_mx<64, G, true, I>);
-        else go(k_density_mx<64, G, false, I>);
-      } else {
-        // The in-stage fold with the in-kernel Z pass needs more than the
-        // 168 registers of the three-workgroups-per-CU configuration; it
-        // runs at two.
-        go(k_density_mx<64, G, false, I>);
-      }
-    };
-    using T_ = std::true_type;
-    using F_ = std::false_type;
-    using M0 = std::integral_constant<int, 0>;
-    using M1 = std::integral_constant<int, 1>;
-    using M3 = std::integral_constant<int, 3>;
-    if (v.in_stage == 1)
-      gga ? pick(T_{}, M1{}) : pick(F_{}, M1{});
-    else if (v.in_stage == 3)
-      gga ? pick(T_{}, M3{}) : pick(F_{}, M3{});
-    else
-      gga ? pick(T_{}, M0{}) : pick(F_{}, M0{});
-  }
+  };
+  using T_ = std::true_type;
+  using F_ = std::false_type;
+  using M0 = std::integral_constant<int, 0>;
+  using M1 = std::integral_constant<int, 1>;
+  using M3 = std::integral_constant<int, 3>;
+  if (v.in_stage == 1)
+    gga ? pick(T_{}, M1{}) : pick(F_{}, M1{});
+  else if (v.in_stage == 3)
+    gga ? pick(T_{}, M3{}) : pick(F_{}, M3{});
+  else
+    gga ? pick(T_{}, M0{}) : pick(F_{}, M0{});
   XCQ_HIP(hipGetLastError());
+  return XCQ_SUCCESS;
+}
+
+}  // namespace
+
+int launch_density_mixed(const CtxView& v, const Chunk& c, int func, int gga, double fac,
+                         int want_z) {
+  for (int k = 0; k < 4; ++k)
+    if (int rc = launch_density_mx(v, c.dens[k], k == 0 ? 32 : (k == 3 ? 128 : 64), k == 1, func,
+                                   gga, fac, want_z))
+      return rc;
   return XCQ_SUCCESS;
 }
 

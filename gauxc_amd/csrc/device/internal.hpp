@@ -286,14 +286,17 @@ int launch_z_in_stage(hipStream_t s, const WorkItem* items, int64_t n, const Dev
                       const int32_t* lsh_first, const double* px, const double* py,
                       const double* pz, const double* zcoef, void* scratch, int precision,
                       unsigned* tmax, int gga, int lmax);
-// Density stage (X, rho/grad rho, functional, EXC/NEL, Z) of one work range
-// whose tasks use `nt`-function tiles (hiocc: the three-workgroups-per-CU
-// configuration of the mixed kernel).  FP64 only, without hiocc:
-// x_plane >= 0 also stores X = fac P_sub B into that scratch plane.
-int launch_density(const CtxView& v, const WorkRange& r, int nt, bool hiocc, int precision,
-                   int func, int gga, double fac, int want_z,
-                   const double* P_override = nullptr, double* dens_out = nullptr,
-                   int x_plane = -1);
+// Mixed density stage (X, rho/grad rho, functional, EXC/NEL, Z) of a chunk.
+int launch_density_mixed(const CtxView& v, const Chunk& c, int func, int gga, double fac,
+                         int want_z);
+// FP64 density stage of a chunk: X = fac P_sub B folded into the raw sums
+// (sum B X, sum dB/dx X, ...) per point, dens_out[block][4][64]; x_plane >= 0
+// also stores X into that scratch plane.
+int launch_density_f64(const CtxView& v, const Chunk& c, int gga, double fac, const double* P,
+                       double* dens_out, int x_plane = -1);
+// RKS functional per point block from the sums (factor 2, or 1 for func 0):
+// Z coefficients over them, (EXC, NEL) partials.
+int launch_xc_points(const CtxView& v, const WorkRange& r, int func, int gga, double* sums);
 // UKS: polarised functional and Z coefficients per point block from the two
 // density passes' raw sums; Z planes from stored coefficients.
 int launch_uks_points(const CtxView& v, const WorkRange& r, int func, int gga, const double* ds,
@@ -330,7 +333,8 @@ int launch_grad_contract_uks(const CtxView& v, const WorkRange& r, int gga,
 int launch_ssf_grad(const CtxView& v, const WorkRange& r, int natoms, const double* xyz,
                     const double* dnear, const double* wf, double* grad,
                     const int32_t* nbr_idx = nullptr, const double* nbr_r = nullptr);
-int launch_z_from_coeffs(const CtxView& v, const WorkRange& r, int gga, const double* coef);
+int launch_z_from_coeffs(const CtxView& v, const WorkRange& r, int gga, const double* coef,
+                         unsigned* tmax);
 // B^T Z + Z^T B of a chunk with the VXC scatter-add.
 int launch_syr2k(const CtxView& v, const Chunk& c, int precision);
 int launch_P_to_f32(hipStream_t s, int64_t n, const double* P, float* out);
