@@ -130,6 +130,21 @@ uint64_t space_code(const double* p) {
   return code;
 }
 
+// An n x n matrix between the caller's memory (leading dimension ld) and the
+// device's (n), on the stream.  A contiguous one is a single copy: the
+// runtime moves a two-dimensional copy of pageable memory row by row, about
+// 9 us each (1,248 functions: 11.5 ms against 0.6 ms; 7,800: 79 against 16).
+hipError_t matrix_to_device(double* d, const double* h, int64_t n, int64_t ld, hipStream_t s) {
+  if (ld == n) return hipMemcpyAsync(d, h, (size_t)(n * n) * 8, hipMemcpyHostToDevice, s);
+  return hipMemcpy2DAsync(d, (size_t)n * 8, h, (size_t)ld * 8, (size_t)n * 8, n,
+                          hipMemcpyHostToDevice, s);
+}
+hipError_t matrix_to_host(double* h, const double* d, int64_t n, int64_t ld, hipStream_t s) {
+  if (ld == n) return hipMemcpyAsync(h, d, (size_t)(n * n) * 8, hipMemcpyDeviceToHost, s);
+  return hipMemcpy2DAsync(h, (size_t)ld * 8, d, (size_t)n * 8, (size_t)n * 8, n,
+                          hipMemcpyDeviceToHost, s);
+}
+
 struct MolInfo {
   int32_t sh_begin = 0, nshells = 0, nbf = 0;
   int64_t p_off = 0;
@@ -1431,8 +1446,7 @@ int xcq_upload_density_mol(xcq_context ctx, int32_t mol, int32_t nbf, const doub
               "density dimension does not match the basis");
   XCQ_REQUIRE(ldp >= nbf, XCQ_ERROR_INVALID_ARGUMENT, "ldp < nbf");
   XCQ_HIP(hipSetDevice(ctx->device));
-  XCQ_HIP(hipMemcpy2DAsync(ctx->d_P + M.p_off, (size_t)nbf * 8, P, (size_t)ldp * 8,
-                           (size_t)nbf * 8, nbf, hipMemcpyHostToDevice, ctx->stream));
+  XCQ_HIP(matrix_to_device(ctx->d_P + M.p_off, P, nbf, ldp, ctx->stream));
   XCQ_HIP(hipStreamSynchronize(ctx->stream));
   M.have_density = true;
   ctx->pf32_valid = false;  // the FP32 copy follows the new density
@@ -1607,8 +1621,7 @@ int xcq_upload_density_z(xcq_context ctx, int32_t nbf, const double* Pz, int64_t
   XCQ_HIP(hipSetDevice(ctx->device));
   int rc;
   if (!ctx->d_Pz && (rc = dalloc(&ctx->d_Pz, (size_t)ctx->p_total))) return rc;
-  XCQ_HIP(hipMemcpy2DAsync(ctx->d_Pz, (size_t)nbf * 8, Pz, (size_t)ldp * 8, (size_t)nbf * 8, nbf,
-                           hipMemcpyHostToDevice, ctx->stream));
+  XCQ_HIP(matrix_to_device(ctx->d_Pz, Pz, nbf, ldp, ctx->stream));
   XCQ_HIP(hipStreamSynchronize(ctx->stream));
   ctx->have_pz = true;
   return XCQ_SUCCESS;
@@ -1646,8 +1659,7 @@ int xcq_download_results_uks(xcq_context ctx, double* exc, double* nel, double* 
   int rc = xcq_download_results_mol(ctx, 0, exc, nel, vxc_s, ldvxc);
   if (rc || !vxc_z) return rc;
   const MolInfo& M = ctx->mols[0];
-  XCQ_HIP(hipMemcpy2DAsync(vxc_z, (size_t)ldvxc * 8, ctx->d_vxcz, (size_t)M.nbf * 8,
-                           (size_t)M.nbf * 8, M.nbf, hipMemcpyDeviceToHost, ctx->stream));
+  XCQ_HIP(matrix_to_host(vxc_z, ctx->d_vxcz, M.nbf, ldvxc, ctx->stream));
   XCQ_HIP(hipStreamSynchronize(ctx->stream));
   return XCQ_SUCCESS;
 }
@@ -1711,8 +1723,7 @@ int xcq_upload_trial_density(xcq_context ctx, int32_t nbf, const double* tP, int
   XCQ_HIP(hipSetDevice(ctx->device));
   int rc;
   if (!ctx->d_tP && (rc = dalloc(&ctx->d_tP, (size_t)ctx->p_total))) return rc;
-  XCQ_HIP(hipMemcpy2DAsync(ctx->d_tP, (size_t)nbf * 8, tP, (size_t)ldp * 8, (size_t)nbf * 8, nbf,
-                           hipMemcpyHostToDevice, ctx->stream));
+  XCQ_HIP(matrix_to_device(ctx->d_tP, tP, nbf, ldp, ctx->stream));
   XCQ_HIP(hipStreamSynchronize(ctx->stream));
   ctx->have_tp = true;
   return XCQ_SUCCESS;
@@ -1807,8 +1818,7 @@ int xcq_upload_trial_density_z(xcq_context ctx, int32_t nbf, const double* tPz, 
   XCQ_HIP(hipSetDevice(ctx->device));
   int rc;
   if (!ctx->d_tPz && (rc = dalloc(&ctx->d_tPz, (size_t)ctx->p_total))) return rc;
-  XCQ_HIP(hipMemcpy2DAsync(ctx->d_tPz, (size_t)nbf * 8, tPz, (size_t)ldp * 8, (size_t)nbf * 8,
-                           nbf, hipMemcpyHostToDevice, ctx->stream));
+  XCQ_HIP(matrix_to_device(ctx->d_tPz, tPz, nbf, ldp, ctx->stream));
   XCQ_HIP(hipStreamSynchronize(ctx->stream));
   ctx->have_tpz = true;
   return XCQ_SUCCESS;
@@ -1858,9 +1868,7 @@ int xcq_download_fxc_uks(xcq_context ctx, double* nel, double* fxc_s, double* fx
     double* dst = c == 0 ? fxc_s : fxc_z;
     if (!dst) continue;
     XCQ_REQUIRE(ldfxc >= M.nbf, XCQ_ERROR_INVALID_ARGUMENT, "ldfxc < nbf");
-    XCQ_HIP(hipMemcpy2DAsync(dst, (size_t)ldfxc * 8, c == 0 ? ctx->d_vxc : ctx->d_vxcz,
-                             (size_t)M.nbf * 8, (size_t)M.nbf * 8, M.nbf,
-                             hipMemcpyDeviceToHost, ctx->stream));
+    XCQ_HIP(matrix_to_host(dst, c == 0 ? ctx->d_vxc : ctx->d_vxcz, M.nbf, ldfxc, ctx->stream));
   }
   XCQ_HIP(hipStreamSynchronize(ctx->stream));
   if (nel) *nel = out[1];
@@ -1876,8 +1884,7 @@ int xcq_download_fxc(xcq_context ctx, double* nel, double* fxc, int64_t ldfxc) {
   XCQ_HIP(hipMemcpyAsync(out, ctx->d_out2, 16, hipMemcpyDeviceToHost, ctx->stream));
   if (fxc) {
     XCQ_REQUIRE(ldfxc >= M.nbf, XCQ_ERROR_INVALID_ARGUMENT, "ldfxc < nbf");
-    XCQ_HIP(hipMemcpy2DAsync(fxc, (size_t)ldfxc * 8, ctx->d_vxc, (size_t)M.nbf * 8,
-                             (size_t)M.nbf * 8, M.nbf, hipMemcpyDeviceToHost, ctx->stream));
+    XCQ_HIP(matrix_to_host(fxc, ctx->d_vxc, M.nbf, ldfxc, ctx->stream));
   }
   XCQ_HIP(hipStreamSynchronize(ctx->stream));
   if (nel) *nel = out[1];
@@ -2139,8 +2146,7 @@ int xcq_download_results_mol(xcq_context ctx, int32_t mol, double* exc, double* 
   if (vxc) {
     XCQ_REQUIRE(ctx->last_want_vxc, XCQ_ERROR_STATE, "last evaluation did not compute VXC");
     XCQ_REQUIRE(ldvxc >= M.nbf, XCQ_ERROR_INVALID_ARGUMENT, "ldvxc < nbf");
-    XCQ_HIP(hipMemcpy2DAsync(vxc, (size_t)ldvxc * 8, ctx->d_vxc + M.p_off, (size_t)M.nbf * 8,
-                             (size_t)M.nbf * 8, M.nbf, hipMemcpyDeviceToHost, ctx->stream));
+    XCQ_HIP(matrix_to_host(vxc, ctx->d_vxc + M.p_off, M.nbf, ldvxc, ctx->stream));
   }
   XCQ_HIP(hipStreamSynchronize(ctx->stream));
   if (exc) *exc = out[0];
