@@ -238,7 +238,7 @@ struct xcq_context_s {
   double* d_grad = nullptr;
   int32_t* d_shell_atom = nullptr;
   bool last_grad = false;   // the last evaluation was an EXC gradient
-  double* d_zc = nullptr;   // per point block: FP64 density sums, Z coefficients; lazily
+  double* d_zc = nullptr;   // per point block: density sums, then Z coefficients; lazily
   double* d_syr_part = nullptr;  // slice buffer of the FP64 SYR2K, lazily
   int64_t pblocks = 0;      // point blocks of the uploaded tasks
   double* d_out2 = nullptr;
@@ -522,17 +522,14 @@ int ensure_syr_part(xcq_context_s* ctx) {
 
 // Enqueue one evaluation on the context's stream.  Events are recorded only
 // when `events` is set (not under graph capture).
-// The basis evaluation mode a precision runs: the FP64 kernels have the
-// stored planes (0) and the in-stage fold with a Z launch (3).
-int effective_mode(const CtxView& v, int precision) {
-  if (precision == XCQ_PREC_FP64) return v.in_stage != 0 ? 3 : 0;
-  return v.in_stage;
-}
+// The basis evaluation mode the kernels run: on stored planes (0) or in the
+// stages (3).
+int effective_mode(const CtxView& v) { return v.in_stage != 0 ? 3 : 0; }
 
 int enqueue_pipeline(xcq_context_s* ctx, int func, int precision, int want_vxc, bool events) {
   const int gga = (func == XCQ_FUNC_PBE || func == XCQ_FUNC_PBE0) ? 1 : 0;
   const CtxView v = view_of(ctx);
-  const int mode = effective_mode(v, precision);
+  const int mode = effective_mode(v);
   hipStream_t s = ctx->stream;
   const double fac = func == 0 ? 1.0 : 2.0;
   int rc;
@@ -561,37 +558,25 @@ int enqueue_pipeline(xcq_context_s* ctx, int func, int precision, int want_vxc, 
                                    gga && mode == 0, ctx->max_l);
     if (rc) return rc;
     XCQ_HIP(rec(ev[1]));
-    // Stage 1: X and the density; FP64 leaves the sums to the functional's
-    // launch (stage 2) and Z to its own (stage 3).  Mixed: the functional,
-    // EXC/NEL and, but for in-stage mode 3, Z belong to the density launches
-    // (one per tile width).
+    // Stage 1: X and the density; 2: the functional; 3: Z.
     XCQ_HIP(rec(ev[2]));
-    if (precision == XCQ_PREC_FP64)
-      rc = launch_density_f64(v, c, gga, fac, ctx->d_P, ctx->d_zc);
-    else
-      rc = launch_density_mixed(v, c, func, gga, fac, want_vxc);
-    if (rc) return rc;
+    if ((rc = launch_density(v, c, precision, gga, fac, ctx->d_zc))) return rc;
     XCQ_HIP(rec(ev[3]));
     XCQ_HIP(rec(ev[4]));
-    if (precision == XCQ_PREC_FP64 && (rc = launch_xc_points(v, c.coll, func, gga, ctx->d_zc)))
-      return rc;
+    if ((rc = launch_xc_points(v, c.coll, func, gga, ctx->d_zc))) return rc;
     XCQ_HIP(rec(ev[5]));
-    launches += precision == XCQ_PREC_FP64 ? 3 : 5;
+    launches += 3;
     items += c.coll.n;
     if (want_vxc) {
       XCQ_HIP(rec(ev[6]));
-      if (mode == 3) {
-        if ((rc = launch_z_in_stage(s, cw, c.coll.n, v.tasks, v.shells, v.shell_list, v.lsh,
-                                    v.px, v.py, v.pz, v.zc, v.scratch, precision,
-                                    v.vxc_drop > 0.0 ? v.tmax : nullptr, gga, ctx->max_l)))
-          return rc;
-        ++launches;
-      } else if (precision == XCQ_PREC_FP64) {
-        if ((rc = launch_z_from_coeffs(v, c.coll, gga, ctx->d_zc,
-                                       v.vxc_drop > 0.0 ? v.tmax : nullptr)))
-          return rc;
-        ++launches;
-      }
+      unsigned* tm = v.vxc_drop > 0.0 ? v.tmax : nullptr;
+      if (mode == 3)
+        rc = launch_z_in_stage(s, cw, c.coll.n, v.tasks, v.shells, v.shell_list, v.lsh, v.px,
+                               v.py, v.pz, v.zc, v.scratch, precision, tm, gga, ctx->max_l);
+      else
+        rc = launch_z_from_coeffs(v, c.coll, precision, gga, v.zc, tm);
+      if (rc) return rc;
+      ++launches;
       XCQ_HIP(rec(ev[7]));
       XCQ_HIP(rec(ev[8]));
       if ((rc = launch_syr2k(v, c, precision))) return rc;
@@ -659,8 +644,7 @@ int run_pipeline(xcq_context_s* ctx, int func, int precision, int want_vxc) {
   // The mixed path's EXC correction needs VXC, so EXC-only requests in that
   // precision evaluate it too (and do not return it).
   if (precision == XCQ_PREC_MIXED && func != 0) want_vxc = 1;
-  if ((precision == XCQ_PREC_FP64 ||
-       (want_vxc && effective_mode(view_of(ctx), precision) == 3)) && !ctx->d_zc) {
+  if (!ctx->d_zc) {
     int rc = dalloc(&ctx->d_zc, (size_t)256 * std::max<int64_t>(ctx->pblocks, 1));
     if (rc) return rc;
     ctx->drop_graph();
@@ -1525,7 +1509,7 @@ int derivative_mode(const xcq_context_s* ctx) { return ctx->max_l <= kInStageMax
 // Z of a chunk from per-point coefficients ([block][4][64]) into plane 4.
 int z_from_point_coeffs(xcq_context_s* ctx, const CtxView& v, const Chunk& c, int mode, int gga,
                         const double* coef) {
-  if (mode == 0) return launch_z_from_coeffs(v, c.coll, gga, coef, nullptr);
+  if (mode == 0) return launch_z_from_coeffs(v, c.coll, XCQ_PREC_FP64, gga, coef, nullptr);
   return launch_z_in_stage(ctx->stream, v.work + c.coll.off, c.coll.n, v.tasks, v.shells,
                            v.shell_list, v.lsh, v.px, v.py, v.pz, coef, v.scratch,
                            XCQ_PREC_FP64, nullptr, gga, ctx->max_l);
@@ -1589,8 +1573,8 @@ int enqueue_uks(xcq_context_s* ctx, int func, int want_vxc) {
                                       gga && mode == 0, ctx->max_l)))
       return rc;
     for (int pass = 0; pass < 2; ++pass)
-      if ((rc = launch_density_f64(v, c, gga, 1.0, pass == 0 ? ctx->d_P : ctx->d_Pz,
-                                   pass == 0 ? ds : dz)))
+      if ((rc = launch_density(v, c, XCQ_PREC_FP64, gga, 1.0, pass == 0 ? ds : dz,
+                               pass == 0 ? ctx->d_P : ctx->d_Pz)))
         return rc;
     if ((rc = launch_uks_points(v, c.coll, func, gga, ds, dz, zs, zz))) return rc;
     if (!want_vxc) continue;
@@ -1698,8 +1682,8 @@ int enqueue_fxc(xcq_context_s* ctx, int func) {
                                       gga && mode == 0, ctx->max_l)))
       return rc;
     for (int pass = 0; pass < 2; ++pass)
-      if ((rc = launch_density_f64(v, c, gga, 2.0, pass == 0 ? ctx->d_P : ctx->d_tP,
-                                   pass == 0 ? dp : dt)))
+      if ((rc = launch_density(v, c, XCQ_PREC_FP64, gga, 2.0, pass == 0 ? dp : dt,
+                               pass == 0 ? ctx->d_P : ctx->d_tP)))
         return rc;
     if ((rc = launch_fxc_points(v, c.coll, func, gga, dp, dt, zc))) return rc;
     if ((rc = z_and_vxc(ctx, v, c, mode, gga, zc))) return rc;
@@ -1789,7 +1773,7 @@ int enqueue_fxc_uks(xcq_context_s* ctx, int func) {
                                       gga && mode == 0, ctx->max_l)))
       return rc;
     for (int pass = 0; pass < 4; ++pass)
-      if ((rc = launch_density_f64(v, c, gga, 1.0, mats[pass], dd[pass])))
+      if ((rc = launch_density(v, c, XCQ_PREC_FP64, gga, 1.0, dd[pass], mats[pass])))
         return rc;
     if ((rc = launch_fxc_points_uks(v, c.coll, func, gga, dd[0], dd[1], dd[2], dd[3], zs, zz)))
       return rc;
@@ -1929,7 +1913,8 @@ int enqueue_grad(xcq_context_s* ctx, int func, int weight_derivs) {
     // X: plane 1 in the in-stage mode (no gradient planes are stored),
     // plane 4 on stored planes.
     const int x_pl = mode == 3 ? 1 : 4;
-    if ((rc = launch_density_f64(v, c, gga, 2.0, ctx->d_P, dp, gga ? x_pl : -1))) return rc;
+    if ((rc = launch_density(v, c, XCQ_PREC_FP64, gga, 2.0, dp, ctx->d_P, gga ? x_pl : -1)))
+      return rc;
     if ((rc = launch_grad_points(v, c.coll, func, gga, dp, coef, wf))) return rc;
     // Za: plane 4 (in-stage evaluation) or over grad_z B in plane 3.
     const int za_pl = mode == 3 ? 4 : 3;
@@ -1983,8 +1968,9 @@ int enqueue_grad_uks(xcq_context_s* ctx, int func, int weight_derivs) {
     // In-stage mode: the density passes leave X_N in plane 2 and X_Z in
     // plane 3 (GGA), which no gradient plane occupies.
     for (int pass = 0; pass < 2; ++pass)
-      if ((rc = launch_density_f64(v, c, gga, 1.0, pass == 0 ? ctx->d_P : ctx->d_Pz,
-                                   pass == 0 ? ds : dz, (gga && mode == 3) ? 2 + pass : -1)))
+      if ((rc = launch_density(v, c, XCQ_PREC_FP64, gga, 1.0, pass == 0 ? ds : dz,
+                               pass == 0 ? ctx->d_P : ctx->d_Pz,
+                               (gga && mode == 3) ? 2 + pass : -1)))
         return rc;
     if ((rc = launch_grad_points_uks(v, c.coll, func, gga, ds, dz, wf))) return rc;
     if (mode == 3) {

@@ -165,9 +165,8 @@ struct CtxView {
   double vxc_drop;  // B^T Z contributions with |v| < vxc_drop are not added to VXC
   unsigned* tmax;   // per granule {max |B|, max |Z|} as float bits (the density stage
                     // fills it, the B^T Z stage skips tile pairs bounded below vxc_drop)
-  int in_stage;     // density stage's basis evaluation: 0 = reads the stored B /
-                    // grad B planes; 1 = evaluates them for its fold and Z (mixed; the
-                    // FP64 path runs 3); 3 = for its fold, Z left to a separate launch
+  int in_stage;     // basis evaluation of the fold and the Z launch: 0 = the stored B /
+                    // grad B planes; else they evaluate them (1 runs as 3)
   const DevShellC* shc;
   double* zc;       // Z coefficients per point block [4][64] (in-stage mode 3)
   double* syr_part; // slice buffer of the FP64 SYR2K, kSyrBlocks blocks per place
@@ -286,14 +285,11 @@ int launch_z_in_stage(hipStream_t s, const WorkItem* items, int64_t n, const Dev
                       const int32_t* lsh_first, const double* px, const double* py,
                       const double* pz, const double* zcoef, void* scratch, int precision,
                       unsigned* tmax, int gga, int lmax);
-// Mixed density stage (X, rho/grad rho, functional, EXC/NEL, Z) of a chunk.
-int launch_density_mixed(const CtxView& v, const Chunk& c, int func, int gga, double fac,
-                         int want_z);
-// FP64 density stage of a chunk: X = fac P_sub B folded into the raw sums
-// (sum B X, sum dB/dx X, ...) per point, dens_out[block][4][64]; x_plane >= 0
-// also stores X into that scratch plane.
-int launch_density_f64(const CtxView& v, const Chunk& c, int gga, double fac, const double* P,
-                       double* dens_out, int x_plane = -1);
+// Density stage of a chunk: X = fac P_sub B folded into the raw sums (sum B
+// X, sum dB/dx X, ...) per point, dens_out[block][4][64].  FP64 only: another
+// density matrix, and x_plane >= 0 also stores X into that scratch plane.
+int launch_density(const CtxView& v, const Chunk& c, int precision, int gga, double fac,
+                   double* dens_out, const double* P_override = nullptr, int x_plane = -1);
 // RKS functional per point block from the sums (factor 2, or 1 for func 0):
 // Z coefficients over them, (EXC, NEL) partials.
 int launch_xc_points(const CtxView& v, const WorkRange& r, int func, int gga, double* sums);
@@ -333,8 +329,8 @@ int launch_grad_contract_uks(const CtxView& v, const WorkRange& r, int gga,
 int launch_ssf_grad(const CtxView& v, const WorkRange& r, int natoms, const double* xyz,
                     const double* dnear, const double* wf, double* grad,
                     const int32_t* nbr_idx = nullptr, const double* nbr_r = nullptr);
-int launch_z_from_coeffs(const CtxView& v, const WorkRange& r, int gga, const double* coef,
-                         unsigned* tmax);
+int launch_z_from_coeffs(const CtxView& v, const WorkRange& r, int precision, int gga,
+                         const double* coef, unsigned* tmax);
 // B^T Z + Z^T B of a chunk with the VXC scatter-add.
 int launch_syr2k(const CtxView& v, const Chunk& c, int precision);
 int launch_P_to_f32(hipStream_t s, int64_t n, const double* P, float* out);
