@@ -152,6 +152,11 @@ struct MolInfo {
 };
 }  // namespace
 
+// The pairs kernel pays where P does not stay in the caches beside the
+// planes (see k_density_wide): it draws level near 3,100 functions, 78 MB.
+constexpr int32_t kWideAuto = 1 << 30, kWideNbe = 256;
+constexpr int64_t kWidePBytes = int64_t(64) << 20;
+
 struct xcq_context_s {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -194,7 +199,9 @@ struct xcq_context_s {
   int64_t ncounters = 0;
   int32_t dens32_max_nbe = 48, syr2k32_max_nbe = 96;  // tile policy
   int32_t dens_hiocc_max_nbe = 0;  // 64-wide density tiles at three workgroups per CU
-  int32_t dens128_min_nbe = 1 << 30;  // 128-wide (mixed) density tiles from this nbe on
+  // FP64 density on 128-wide tiles and block pairs from this nbe on; kWideAuto:
+  // from kWideNbe on in molecules whose P exceeds kWidePBytes.
+  int32_t dens128_min_nbe = kWideAuto;
   // Mixed density stage's basis evaluation (bases up to l = 3): 1 = its
   // fold and Z evaluate B / grad B, 3 = its fold does and a separate launch
   // forms Z, 0 = both read the planes the collocation stage stores.
@@ -347,7 +354,7 @@ CtxView view_of(xcq_context_s* c) {
 // Heuristic per-item costs (used when no predicted task costs are set):
 // matrix-core work of the item, npts * rows * cols in the padded tile.
 double heur_dens_item(const DevTask& d) {
-  const double rows = std::ceil(d.nbe / double(d.nt_d)) * d.nt_d;
+  const double rows = std::ceil(d.nbe / 16.) * 16.;
   return (double)kPtBlock * rows * d.nbe;
 }
 double heur_syr2k_item(const DevTask& d) { return (double)d.npts_pad * d.nt_s * d.nt_s; }
@@ -364,10 +371,14 @@ int build_work_lists(xcq_context_s* ctx) {
                          ctx->cost_s.size() == (size_t)ctx->ntasks;
   const bool queued = ctx->nqueues > 0;  // only then are the items' costs read
   for (auto& d : ctx->h_tasks) {
-    d.nt_d = d.nbe <= ctx->dens32_max_nbe ? 32 : (d.nbe >= ctx->dens128_min_nbe ? 128 : 64);
-    d.dens_cls = d.nt_d == 32    ? 0
-                 : d.nt_d == 128 ? 3
-                                 : (d.nbe <= ctx->dens_hiocc_max_nbe ? 1 : 2);
+    // Pairs need two blocks to pair and more than 64 functions.
+    const int32_t wide = ctx->dens128_min_nbe != kWideAuto ? ctx->dens128_min_nbe
+                         : (int64_t)d.ldp * d.ldp * 8 > kWidePBytes ? kWideNbe
+                                                                    : kWideAuto;
+    d.dens_cls = d.nbe <= ctx->dens32_max_nbe                               ? 0
+                 : d.nbe >= std::max(wide, 65) && d.npts > kPtBlock         ? 3
+                 : d.nbe <= ctx->dens_hiocc_max_nbe                         ? 1
+                                                                            : 2;
     d.nt_s = d.nbe <= ctx->syr2k32_max_nbe ? 32 : 64;
   }
   auto finish_range = [&](WorkRange& r, const std::vector<double>& cost) {
@@ -403,7 +414,7 @@ int build_work_lists(xcq_context_s* ctx) {
                        return ba != bb ? ba > bb : ctx->place[a] < ctx->place[b];
                      });
   for (auto& c : ctx->chunks) {
-    for (int v = 0; v < 4; ++v) {  // density classes (DevTask::dens_cls)
+    for (int v = 3; v >= 0; --v) {  // density classes (DevTask::dens_cls)
       c.dens[v].off = (int64_t)W.size();
       std::vector<double> cost;
       for (int32_t q = c.task_begin; q < c.task_end; ++q) {
@@ -419,7 +430,23 @@ int build_work_lists(xcq_context_s* ctx) {
       }
       finish_range(c.dens[v], cost);
     }
-    c.coll.off = c.dens[0].off;
+    c.dens_pair.off = (int64_t)W.size();
+    {
+      std::vector<double> cost;
+      for (int32_t q = c.task_begin; q < c.task_end; ++q) {
+        const int32_t i = order[q];
+        const DevTask& d = ctx->h_tasks[i];
+        if (d.dens_cls != 3) continue;
+        const int npair = (d.npts_pad / kPtBlock + 1) / 2;
+        const double ci = have_cost ? ctx->cost_d[i] / npair : 2. * heur_dens_item(d);
+        for (int pr = 0; pr < npair; ++pr) {
+          W.push_back(WorkItem{i, pr, 0, 0});
+          if (queued) cost.push_back(ci);
+        }
+      }
+      finish_range(c.dens_pair, cost);
+    }
+    c.coll.off = c.dens[3].off;
     c.coll.n = c.dens[0].n + c.dens[1].n + c.dens[2].n + c.dens[3].n;
     c.coll.nq = 0;
     for (int v = 0; v < 2; ++v) {  // SYR2K tiles
@@ -1230,7 +1257,10 @@ int xcq_task_times(xcq_context ctx, double* dens_us, double* syr2k_us) {
     }
   };
   for (const auto& c : ctx->chunks) {
-    for (int v = 0; v < 4; ++v) add(c.dens[v], dens_us);
+    // FP64 runs class 3 as pairs, but on stored planes.
+    const bool pairs = !ctx->last_mixed && effective_mode(view_of(ctx)) != 0;
+    for (int v = 0; v < (pairs ? 3 : 4); ++v) add(c.dens[v], dens_us);
+    if (pairs) add(c.dens_pair, dens_us);
     // The list the last evaluation ran (the other keeps older stamps).
     if (ctx->last_mixed)
       for (int v = 0; v < 2; ++v) add(c.syr2k[v], syr2k_us);

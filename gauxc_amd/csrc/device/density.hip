@@ -208,17 +208,43 @@ constexpr int kDensTile = 64;  // functions per tile
 // Shells of one tile (at most one more than its functions, and one for each
 // of the four waves' loops to end on), staged in LDS while the tile's
 // product runs.
+template <int NT>
 struct FoldShells {
-  static constexpr int kMax = kDensTile + 5;
+  static constexpr int kMax = NT + 5;
   double ox[kMax], oy[kMax], oz[kMax], a0[kMax], c0[kMax];
   int bf0[kMax], info[kMax], ish[kMax];
   int next;  // shell holding the function after the tile
+
+  // Stages the shells from s_first on of task t's tile that ends at function
+  // nhi (threads 0 .. kMax - 1); the first ones past it end the fold's loops.
+  __device__ __forceinline__ void load(const DevTask& t, const ShellArgs& sa, int s_first, int nhi,
+                                       int tid) {
+    if (tid >= kMax) return;
+    const int s = s_first + tid;
+    int f0 = INT_MAX, f1 = INT_MAX, i = 0;
+    if (s < t.nshells) {
+      f0 = sa.lsh[t.lsh_off + s];
+      i = sa.shell_list[t.sh_off + s];
+      if (s + 1 < t.nshells) f1 = sa.lsh[t.lsh_off + s + 1];
+    }
+    const DevShellC c = sa.shc[i];
+    bf0[tid] = f0;
+    ish[tid] = i;
+    info[tid] = c.info;
+    ox[tid] = c.ox;
+    oy[tid] = c.oy;
+    oz[tid] = c.oz;
+    a0[tid] = c.a0;
+    c0[tid] = c.c0;
+    if (f0 <= nhi && f1 > nhi) next = s;
+  }
 };
 
 // Folds rows [nlo, nhi) of the X^T tile in LDS (row n - nlo, column =
 // point) into this lane's partials r: rho += B X, grad rho / 2 += grad B X.
-// Wave w takes the tile's shells w, w + 4, ... until one starts at or past
-// nhi; lane = point, so a shell is wave-uniform.  With B_f = R Y_f and grad
+// The wave takes the tile's shells first, first + step, ... until one starts
+// at or past nhi, leaving out those that end before nlo; lane = point, so a
+// shell is wave-uniform; rows of X^T are LD doubles apart.  With B_f = R Y_f and grad
 // B_f = R grad Y_f + dR r Y_f, a shell adds R sy to rho and R sg + dR r sy
 // to grad rho / 2, where sy = sum Y_f X_f and sg = sum grad Y_f X_f over its
 // functions in the range: the functions are formed from their angular
@@ -227,16 +253,17 @@ struct FoldShells {
 // misses res^T X (res = B - B32, P symmetric), a first-order term that does
 // not average out (it biased EXC by about -3e-10 relative): rho also takes
 // sum res X.
-template <bool GGA, bool RES32>
-__device__ __forceinline__ void fold_staged(const ShellArgs& sa, const FoldShells& fs, int nlo,
-                                            int nhi, int wave, int lane, const double* xt,
+template <bool GGA, bool RES32, int LD, int NT>
+__device__ __forceinline__ void fold_staged(const ShellArgs& sa, const FoldShells<NT>& fs, int nlo,
+                                            int nhi, int first, int step, const double* xt,
                                             double rx, double ry, double rz, double (&r)[4]) {
-  for (int j = wave;; j += 4) {
+  for (int j = first;; j += step) {
     const int bf0 = uni(fs.bf0[j]);
     if (bf0 >= nhi) break;
     const int info = uni(fs.info[j]);
     const int l = info & 0xff, nprim = info >> 16;
     const bool pure = (info >> 8) & 1;
+    if (NT > 64 && bf0 + (pure ? 2 * l + 1 : (l + 1) * (l + 2) / 2) <= nlo) continue;
     const double x = rx - fs.ox[j], y = ry - fs.oy[j], z = rz - fs.oz[j];
     const double a0 = fs.a0[j];
     const double r2 = x * x + y * y + z * z;
@@ -254,7 +281,7 @@ __device__ __forceinline__ void fold_staged(const ShellArgs& sa, const FoldShell
         l, x, y, z, R, dR, pure, [&](int f, double v, double gx, double gy, double gz) {
           const int n = bf0 + f;  // uniform
           if (n >= nlo && n < nhi) {
-            const double xv = xt[(n - nlo) * kXLd + lane];
+            const double xv = xt[(n - nlo) * LD];
             sy += v * xv;
             if constexpr (RES32) {
               const double b = R * v;
@@ -296,7 +323,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void k_density(
   __shared__ __attribute__((aligned(16))) double lds[kXtD];
   T* stage = reinterpret_cast<T*>(lds);
   double(*dens)[64][4] = reinterpret_cast<double(*)[64][4]>(lds);
-  __shared__ FoldShells fs;
+  __shared__ FoldShells<kDensTile> fs;
   const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
   const int lf = lane & 15, lq = lane >> 4;
   auto arow = [&](int r) { return kF32 ? 4 * lq + r : 4 * r + lq; };  // accumulator rows
@@ -372,27 +399,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void k_density(
       };
       load(0);
       if constexpr (INSTAGE != 0) {
-        // The shells of this tile's functions; the first ones past it end
-        // the fold's loops.
-        if (tid < FoldShells::kMax) {
-          const int s = s_cur + tid;
-          int f0 = INT_MAX, f1 = INT_MAX, ish = 0;
-          if (s < t.nshells) {
-            f0 = sa.lsh[t.lsh_off + s];
-            ish = sa.shell_list[t.sh_off + s];
-            if (s + 1 < t.nshells) f1 = sa.lsh[t.lsh_off + s + 1];
-          }
-          const DevShellC c = sa.shc[ish];
-          fs.bf0[tid] = f0;
-          fs.ish[tid] = ish;
-          fs.info[tid] = c.info;
-          fs.ox[tid] = c.ox;
-          fs.oy[tid] = c.oy;
-          fs.oz[tid] = c.oz;
-          fs.a0[tid] = c.a0;
-          fs.c0[tid] = c.c0;
-          if (f0 <= nhi && f1 > nhi) fs.next = s;
-        }
+        fs.load(t, sa, s_cur, nhi, tid);
       }
       v4d acc[kBI];
 #pragma unroll
@@ -467,7 +474,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void k_density(
           for (int r = 0; r < 4; ++r)
             lds[(16 * i + arow(r)) * kXLd + 16 * pg + lf] = acc[i][r];
         __syncthreads();
-        fold_staged<GGA, kF32>(sa, fs, n0, nhi, wave, lane, lds, rx, ry, rz, part);
+        fold_staged<GGA, kF32, kXLd>(sa, fs, n0, nhi, wave, 4, lds + lane, rx, ry, rz, part);
         s_cur = uni(fs.next);
       } else {
         const unsigned short* lo = lo_plane(Bm, plane);
@@ -515,6 +522,192 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void k_density(
         for (int d = 0; d < ND; ++d) v += dens[d][tid][c];
         dens_out[(t.red_off + wi.a) * 256 + c * 64 + tid] = v;
       }
+    }
+    stamp_item(qa, it, t0);
+    __syncthreads();
+  }
+}
+
+// The same in FP64 for tasks of many functions of large molecules: one
+// workgroup per (task, pair of 64-point blocks), tiles of up to 128
+// functions, each wave 32 points and every row of the tile.  On 150 waters
+// the kernel above is bound by L2 misses (890 GB, 6.5 TB/s): P_sub of a task
+// (2 MB and more) and the blocks' B panels do not stay in L2, P_sub is
+// gathered once per point block and B read once per tile.  Twice the points
+// and twice the functions per workgroup halve both, at two waves per SIMD
+// (128 accumulator registers).  Density stage: 150 waters 137 -> 117 ms, 90
+// waters 33.3 -> 30.0, 60 waters 18.6 -> 18.0, 40 waters 8.8 -> 9.1, 24 waters
+// 6.1 -> 6.8; mixed precision (64-function tiles, half the bytes) lost at
+// every size (150 waters 88 -> 95).  Lane (f, q) holds the adjacent points 2f,
+// 2f + 1 of its wave's 32: one 16-byte load of B serves two MFMA columns.
+template <bool GGA>
+__global__ __launch_bounds__(256, 2) void k_density_wide(
+    QueueArgs qa, const DevTask* __restrict__ tasks, const int32_t* __restrict__ bfmap,
+    const double* __restrict__ Pall, double* __restrict__ scratch, double fac, ShellArgs sa,
+    double* __restrict__ dens_out, int x_plane) {
+  typedef double v2d __attribute__((ext_vector_type(2)));
+  constexpr int NT = 128;
+  constexpr int kBI = NT / 16;
+  constexpr int kK = 16;
+  constexpr int kKQ = kK / 4;
+  constexpr int kLd = NT + 16;
+  constexpr int kStage = kK * kLd;
+  constexpr int kXL = 2 * kPtBlock + 2;  // X^T row (128 points) in doubles
+  constexpr int kXtD = 64 * kXL;         // 64 rows at a time
+  static_assert(2 * kStage <= kXtD, "LDS is shared");
+  __shared__ __attribute__((aligned(16))) double lds[kXtD];
+  double* stage = lds;
+  double(*dens)[128][4] = reinterpret_cast<double(*)[128][4]>(lds);
+  __shared__ FoldShells<NT> fs;
+  const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
+  const int lf = lane & 15, lq = lane >> 4;
+
+  XCQ_FOR_EACH_ITEM(qa, it) {
+    const int64_t t0 = qa.tstamp ? wall_clock64() : 0;
+    const WorkItem wi = qa.items[uniform64(it)];
+    const DevTask t = tasks[wi.task];
+    const int m0 = 2 * wi.a * kPtBlock;
+    const int ld = t.npts_pad;
+    const int nbe = t.nbe;
+    const int plane = nbe * ld;
+    const int64_t ldp = t.ldp;
+    const double* P = Pall + t.p_off;
+    double* Bm = scratch + t.b_off;
+    const int32_t* bf = bfmap + t.bf_off;
+    const int pg = (wave + wi.a) & 3;           // the wave's 32 points of the pair
+    const int pcol = m0 + 32 * pg + 2 * lf;     // this lane's first point (column)
+    const bool active = m0 + 32 * pg < t.npts;  // the wave has points
+    const int nks = (nbe + kK - 1) / kK, nblk = (nbe + 15) / 16;
+    // Fold: waves 0, 2 take the first 64 points, waves 1, 3 the others.
+    const int ph = wave & 1;
+    const int pl = min(m0 + kPtBlock * ph + lane, t.npts - 1);
+    const double rx = sa.px[t.pt_off + pl], ry = sa.py[t.pt_off + pl], rz = sa.pz[t.pt_off + pl];
+    int s_cur = 0;
+    double part[4] = {0., 0., 0., 0.};
+    const auto rsB = __builtin_amdgcn_make_buffer_rsrc(
+        Bm, 0, (int)((unsigned)plane * 8u), 0x00020000);
+    auto ldB = [&](int vo, int so) {  // element offsets: lane, scalar
+      return __builtin_bit_cast(v2d,
+                                __builtin_amdgcn_raw_buffer_load_b128(rsB, vo * 8, so * 8, 0));
+    };
+
+    const int ntile = (nblk + kBI - 1) / kBI;
+    for (int tile = 0; tile < ntile; ++tile) {
+      const int blk = tile * nblk / ntile, nbk = (tile + 1) * nblk / ntile - blk;
+      const int n0 = 16 * blk, nhi = min(n0 + 16 * nbk, nbe);
+      const unsigned c0 = 8u * (unsigned)bf[min(n0 + lane, nbe - 1)];
+      const unsigned c1 = 8u * (unsigned)bf[min(n0 + 64 + lane, nbe - 1)];
+      int vrow = bf[min(lane, nbe - 1)];
+      int vnext = bf[min(64 + lane, nbe - 1)];
+      double rp[kKQ][2];
+      v2d rb[kKQ];
+#pragma unroll
+      for (int ks = 0; ks < kKQ; ++ks) rb[ks] = v2d{0., 0.};
+      auto load = [&](int s) {
+        if (s > 0 && s % (64 / kK) == 0) {
+          vrow = vnext;
+          vnext = bf[min(kK * s + 64 + lane, nbe - 1)];
+        }
+#pragma unroll
+        for (int e = 0; e < kKQ; ++e) {
+          const int row = __builtin_amdgcn_readlane(vrow, (kK * s + kKQ * wave + e) & 63);
+          const char* Pr = reinterpret_cast<const char*>(P + (int64_t)row * ldp);
+          rp[e][0] = *reinterpret_cast<const double*>(Pr + c0);
+          rp[e][1] = *reinterpret_cast<const double*>(Pr + c1);
+        }
+      };
+      // Row block ks of the B rows of step s.
+      auto loadB = [&](int s, int ks) {
+        if (!active) return;
+        if (kK * (s + 1) <= nbe) rb[ks] = ldB(lq * ld + pcol, (kK * s + 4 * ks) * ld);
+        else rb[ks] = ldB(min(kK * s + 4 * ks + lq, nbe - 1) * ld + pcol, 0);
+      };
+      load(0);
+#pragma unroll
+      for (int ks = 0; ks < kKQ; ++ks) loadB(0, ks);
+      fs.load(t, sa, s_cur, nhi, tid);
+      v4d acc[kBI][2];
+#pragma unroll
+      for (int i = 0; i < kBI; ++i) acc[i][0] = acc[i][1] = v4d{0., 0., 0., 0.};
+      auto contract = [&](auto NB) {
+        constexpr int BI = decltype(NB)::value;
+        for (int s = 0; s < nks; ++s) {
+          double* st = stage + (s & 1) * kStage;
+#pragma unroll
+          for (int e = 0; e < kKQ; ++e) {
+            // P rows past nbe are zero, B rows past it repeat the last one.
+            const bool kok = kK * s + kKQ * wave + e < nbe;
+            st[(kKQ * wave + e) * kLd + lane] = kok ? rp[e][0] : 0.;
+            st[(kKQ * wave + e) * kLd + 64 + lane] = kok ? rp[e][1] : 0.;
+          }
+          __syncthreads();
+          const bool more = s + 1 < nks;
+          if (more) load(s + 1);
+          if (active) {
+#pragma unroll
+            for (int ks = 0; ks < kKQ; ++ks) {
+              double a[BI];
+#pragma unroll
+              for (int i = 0; i < BI; ++i) a[i] = st[(4 * ks + lq) * kLd + 16 * i + lf];
+#pragma unroll
+              for (int i = 0; i < BI; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                  acc[i][j] =
+                      __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], rb[ks][j], acc[i][j], 0, 0, 0);
+              if (more) loadB(s + 1, ks);
+            }
+          }
+        }
+      };
+      // Tasks of this kernel have at least five blocks, so a tile has four.
+      switch (nbk) {
+        case 4: contract(std::integral_constant<int, 4>{}); break;
+        case 5: contract(std::integral_constant<int, 5>{}); break;
+        case 6: contract(std::integral_constant<int, 6>{}); break;
+        case 7: contract(std::integral_constant<int, 7>{}); break;
+        default: contract(std::integral_constant<int, 8>{}); break;
+      }
+#pragma unroll
+      for (int i = 0; i < kBI; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] *= fac;  // 1 or 2: exact
+      if (x_plane >= 0 && active) {
+        double* xo = Bm + (int64_t)x_plane * plane + pcol;
+#pragma unroll
+        for (int i = 0; i < kBI; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int row = n0 + 16 * i + 4 * r + lq;
+            if (row < nhi)
+              *reinterpret_cast<v2d*>(xo + (int64_t)row * ld) = v2d{acc[i][0][r], acc[i][1][r]};
+          }
+      }
+#pragma unroll
+      for (int h = 0; h < NT / 64; ++h) {
+        if (64 * h >= nhi - n0) break;
+        __syncthreads();  // every wave is done with the stages (or the last rows)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            *reinterpret_cast<v2d*>(lds + (16 * i + 4 * r + lq) * kXL + 32 * pg + 2 * lf) =
+                v2d{acc[4 * h + i][0][r], acc[4 * h + i][1][r]};
+        __syncthreads();
+        fold_staged<GGA, false, kXL>(sa, fs, n0 + 64 * h, min(n0 + 64 * h + 64, nhi), wave >> 1, 2,
+                                    lds + kPtBlock * ph + lane, rx, ry, rz, part);
+      }
+      s_cur = uni(fs.next);
+      __syncthreads();  // the next tile's first stage write is safe
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) dens[wave >> 1][kPtBlock * ph + lane][c] = part[c];
+    __syncthreads();
+    if (tid < 128 && m0 + (tid & 64) < ld) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        dens_out[(t.red_off + 2 * wi.a + (tid >> 6)) * 256 + c * 64 + (tid & 63)] =
+            dens[0][tid][c] + dens[1][tid][c];
     }
     stamp_item(qa, it, t0);
     __syncthreads();
@@ -889,25 +1082,37 @@ int launch_density(const CtxView& v, const Chunk& c, int precision, int gga, dou
                    double* dens_out, const double* P_override, int x_plane) {
   XCQ_REQUIRE(x_plane < 5, XCQ_ERROR_INVALID_ARGUMENT, "the scratch has five planes");
   const ShellArgs sa{v.shells, v.shc, v.shell_list, v.lsh, v.px, v.py, v.pz};
-  auto run = [&](auto kern, const auto* P, auto* scr) {
-    auto go = [&](const WorkRange& r) {
-      if (r.n)
-        hipLaunchKernelGGL(kern, dim3(grid_of(r)), dim3(256), 0, v.stream, queue_args(v, r),
-                           v.tasks, v.bfmap, P, scr, fac, sa, dens_out, x_plane);
-    };
-    // One kernel serves every class; each class has queues of its own.
-    if (c.dens[0].nq || c.dens[1].nq || c.dens[2].nq || c.dens[3].nq)
-      for (const WorkRange& r : c.dens) go(r);
-    else
-      go(c.coll);
+  auto go = [&](auto kern, const WorkRange& r, const auto* P, auto* scr) {
+    if (r.n)
+      hipLaunchKernelGGL(kern, dim3(grid_of(r)), dim3(256), 0, v.stream, queue_args(v, r), v.tasks,
+                         v.bfmap, P, scr, fac, sa, dens_out, x_plane);
   };
-  // Any in-stage mode is the kernel's one (3).
+  // Classes [0, n): one launch, but for queues, which each class has of its
+  // own.  The classes' items lie one after the other, the highest first.
+  auto run = [&](auto kern, const auto* P, auto* scr, int n) {
+    if (c.dens[0].nq || c.dens[1].nq || c.dens[2].nq || c.dens[3].nq) {
+      for (int k = n - 1; k >= 0; --k) go(kern, c.dens[k], P, scr);
+    } else {
+      WorkRange r = c.coll;
+      if (n == 3) {
+        r.off += c.dens[3].n;
+        r.n -= c.dens[3].n;
+      }
+      go(kern, r, P, scr);
+    }
+  };
+  // Any in-stage mode is the kernels' one (3).  FP64 runs class 3 as pairs.
   auto pick = [&](const auto* P, auto* scr) {
     using T = std::remove_pointer_t<decltype(scr)>;
-    if (v.in_stage != 0)
-      gga ? run(k_density<T, true, 3>, P, scr) : run(k_density<T, false, 3>, P, scr);
-    else
-      gga ? run(k_density<T, true, 0>, P, scr) : run(k_density<T, false, 0>, P, scr);
+    if (v.in_stage == 0) {
+      gga ? run(k_density<T, true, 0>, P, scr, 4) : run(k_density<T, false, 0>, P, scr, 4);
+      return;
+    }
+    if constexpr (sizeof(T) == 8)
+      gga ? go(k_density_wide<true>, c.dens_pair, P, scr)
+          : go(k_density_wide<false>, c.dens_pair, P, scr);
+    constexpr int n = sizeof(T) == 8 ? 3 : 4;
+    gga ? run(k_density<T, true, 3>, P, scr, n) : run(k_density<T, false, 3>, P, scr, n);
   };
   if (precision == XCQ_PREC_FP64)
     pick(P_override ? P_override : v.P, static_cast<double*>(v.scratch));
