@@ -120,12 +120,17 @@ void xcd_queue_layout(std::vector<WorkItem>& v, size_t b, size_t e, const std::v
   }
 }
 
-// Place of a point on a space-filling (Morton) curve of 1 bohr cells.
+// Place of a point on a space-filling (Morton) curve of 1 bohr cells, 39 bits:
+// 13 bits of each coordinate, spread three apart.
 uint64_t space_code(const double* p) {
   uint64_t code = 0;
   for (int d = 0; d < 3; ++d) {
-    const uint64_t c = (uint64_t)std::clamp(p[d] + 32768.0, 0.0, 65535.0);
-    for (int b = 0; b < 16; ++b) code |= (c >> b & 1) << (3 * b + d);
+    uint64_t c = (uint64_t)std::clamp(p[d] + 4096.0, 0.0, 8191.0);
+    c = (c | c << 16) & 0x0000ff0000ff;
+    c = (c | c << 8) & 0x00f00f00f00f;
+    c = (c | c << 4) & 0x0c30c30c30c3;
+    c = (c | c << 2) & 0x249249249249;
+    code |= c << d;
   }
   return code;
 }
@@ -404,21 +409,19 @@ int build_work_lists(xcq_context_s* ctx) {
   // ones.  (150 waters: FP64 density 166 ms by cost, 135 by place alone, 138
   // in steps of 64, mixed 110, 109 and 100 ms; 24 waters: 6.3, 6.6 and 6.1.)
   constexpr int kPlaceNbe = 64;
-  std::vector<int32_t> order(ctx->ntasks);
-  std::iota(order.begin(), order.end(), 0);
+  std::vector<std::pair<uint64_t, int32_t>> order(ctx->ntasks);
+  for (int32_t i = 0; i < ctx->ntasks; ++i) {
+    const uint64_t step = std::min(ctx->h_tasks[i].nbe / kPlaceNbe, 1023);
+    order[i] = {(1023 - step) << 54 | ctx->place[i], i};
+  }
   for (const auto& c : ctx->chunks)
-    std::stable_sort(order.begin() + c.task_begin, order.begin() + c.task_end,
-                     [&](int32_t a, int32_t b) {
-                       const int ba = ctx->h_tasks[a].nbe / kPlaceNbe;
-                       const int bb = ctx->h_tasks[b].nbe / kPlaceNbe;
-                       return ba != bb ? ba > bb : ctx->place[a] < ctx->place[b];
-                     });
+    std::sort(order.begin() + c.task_begin, order.begin() + c.task_end);
   for (auto& c : ctx->chunks) {
     for (int v = 3; v >= 0; --v) {  // density classes (DevTask::dens_cls)
       c.dens[v].off = (int64_t)W.size();
       std::vector<double> cost;
       for (int32_t q = c.task_begin; q < c.task_end; ++q) {
-        const int32_t i = order[q];
+        const int32_t i = order[q].second;
         const DevTask& d = ctx->h_tasks[i];
         if (d.dens_cls != v) continue;
         const int nmb = d.npts_pad / kPtBlock;
@@ -434,7 +437,7 @@ int build_work_lists(xcq_context_s* ctx) {
     {
       std::vector<double> cost;
       for (int32_t q = c.task_begin; q < c.task_end; ++q) {
-        const int32_t i = order[q];
+        const int32_t i = order[q].second;
         const DevTask& d = ctx->h_tasks[i];
         if (d.dens_cls != 3) continue;
         const int npair = (d.npts_pad / kPtBlock + 1) / 2;
@@ -1092,7 +1095,7 @@ int xcq_upload_tasks_batched(xcq_context ctx, int32_t ntasks, const xcq_task* ta
   ctx->place.resize(ntasks);
   for (int32_t i = 0; i < ntasks; ++i) {
     const double* p = ht[i].npts ? points + 3 * ht[i].pt_off : nullptr;
-    ctx->place[i] = (uint64_t)ht[i].mol << 48 | (p ? space_code(p) : 0);
+    ctx->place[i] = (uint64_t)std::min(ht[i].mol, 0x7fff) << 39 | (p ? space_code(p) : 0);
   }
   ctx->h_tasks = std::move(ht);
   ctx->chunks = std::move(chunks);
