@@ -248,6 +248,7 @@ struct xcq_context_s {
   bool ssf_lists = true;          // xcq_set_ssf_neighbour_lists
   bool grad_lists = false;        // the last gradient's weight part uses the lists
   double* d_grad = nullptr;
+  double* d_grad_part = nullptr;  // kGradCopies partial sums
   int32_t* d_shell_atom = nullptr;
   bool last_grad = false;   // the last evaluation was an EXC gradient
   double* d_zc = nullptr;   // per point block: density sums, then Z coefficients; lazily
@@ -337,6 +338,7 @@ struct xcq_context_s {
     dfree(d_gnbr_idx);
     dfree(d_gnbr_r);
     dfree(d_grad);
+    dfree(d_grad_part);
     dfree(d_shell_atom);
     dfree(d_out2);
     dfree(d_corr);
@@ -1933,7 +1935,8 @@ int enqueue_grad(xcq_context_s* ctx, int func, int weight_derivs) {
   double* coef = dp + blk;
   double* wf = coef + blk;
   int rc;
-  if ((rc = launch_fill(s, ctx->d_grad, 3 * (int64_t)ctx->grad_natoms))) return rc;
+  const int64_t gs = grad_stride(ctx->grad_natoms);
+  if ((rc = launch_fill(s, ctx->d_grad_part, kGradCopies * gs))) return rc;
   if (ctx->ncounters &&
       (rc = launch_fill(s, reinterpret_cast<double*>(ctx->d_counters), ctx->ncounters)))
     return rc;
@@ -1954,15 +1957,16 @@ int enqueue_grad(xcq_context_s* ctx, int func, int weight_derivs) {
     if (mode == 3) rc = z_from_point_coeffs(ctx, v, c, mode, gga, coef);
     else rc = launch_grad_zpair(v, c.coll, gga, coef, nullptr, 3, -1);
     if (rc || (rc = launch_plane_product(v, c.coll, za_pl, 2))) return rc;
-    if ((rc = launch_grad_contract(v, c.coll, gga, ctx->d_shell_atom, coef, weight_derivs,
-                                   ctx->d_grad, x_pl, 2, ctx->max_l)))
+    if ((rc = launch_grad_contract(v, c.coll, gga, ctx->d_shell_atom, coef, nullptr,
+                                   weight_derivs, ctx->d_grad_part, gs, x_pl, 2, ctx->max_l)))
       return rc;
     if (weight_derivs &&
         (rc = launch_ssf_grad(v, c.coll, ctx->grad_natoms, ctx->d_gxyz, ctx->d_dnear, wf,
-                              ctx->d_grad, ctx->grad_lists ? ctx->d_gnbr_idx : nullptr,
+                              ctx->d_grad_part, gs, ctx->grad_lists ? ctx->d_gnbr_idx : nullptr,
                               ctx->grad_lists ? ctx->d_gnbr_r : nullptr)))
       return rc;
   }
+  if ((rc = launch_grad_sum(s, ctx->grad_natoms, ctx->d_grad_part, gs, ctx->d_grad))) return rc;
   return launch_reduce_sums(s, 1, ctx->d_mol_blk, ctx->d_red, ctx->d_rpart, nullptr, 1.0,
                             ctx->d_out2);
 }
@@ -1988,7 +1992,8 @@ int enqueue_grad_uks(xcq_context_s* ctx, int func, int weight_derivs) {
   double* dz = ds + blk;
   double* wf = dz + blk;
   int rc;
-  if ((rc = launch_fill(s, ctx->d_grad, 3 * (int64_t)ctx->grad_natoms))) return rc;
+  const int64_t gs = grad_stride(ctx->grad_natoms);
+  if ((rc = launch_fill(s, ctx->d_grad_part, kGradCopies * gs))) return rc;
   if (ctx->ncounters &&
       (rc = launch_fill(s, reinterpret_cast<double*>(ctx->d_counters), ctx->ncounters)))
     return rc;
@@ -2022,15 +2027,16 @@ int enqueue_grad_uks(xcq_context_s* ctx, int func, int weight_derivs) {
                   (rc = launch_plane_product(v, c.coll, 0, 3, ctx->d_Pz, 1.0, 0))))
         return rc;
     }
-    if ((rc = launch_grad_contract_uks(v, c.coll, gga, ctx->d_shell_atom, ds, dz, weight_derivs,
-                                       ctx->d_grad, ctx->max_l)))
+    if ((rc = launch_grad_contract(v, c.coll, gga, ctx->d_shell_atom, ds, dz, weight_derivs,
+                                   ctx->d_grad_part, gs, 2, 1, ctx->max_l)))
       return rc;
     if (weight_derivs &&
         (rc = launch_ssf_grad(v, c.coll, ctx->grad_natoms, ctx->d_gxyz, ctx->d_dnear, wf,
-                              ctx->d_grad, ctx->grad_lists ? ctx->d_gnbr_idx : nullptr,
+                              ctx->d_grad_part, gs, ctx->grad_lists ? ctx->d_gnbr_idx : nullptr,
                               ctx->grad_lists ? ctx->d_gnbr_r : nullptr)))
       return rc;
   }
+  if ((rc = launch_grad_sum(s, ctx->grad_natoms, ctx->d_grad_part, gs, ctx->d_grad))) return rc;
   return launch_reduce_sums(s, 1, ctx->d_mol_blk, ctx->d_red, ctx->d_rpart, nullptr, 1.0,
                             ctx->d_out2);
 }
@@ -2074,12 +2080,14 @@ int grad_prepare(xcq_context_s* ctx, int functional, int32_t natoms, const doubl
     dfree(ctx->d_gxyz);
     dfree(ctx->d_dnear);
     dfree(ctx->d_grad);
+    dfree(ctx->d_grad_part);
     dfree(ctx->d_gnbr_idx);
     dfree(ctx->d_gnbr_r);
     ctx->grad_natoms = 0;
     if ((rc = dalloc(&ctx->d_gxyz, 3 * (size_t)natoms)) ||
         (rc = dalloc(&ctx->d_dnear, (size_t)natoms)) ||
-        (rc = dalloc(&ctx->d_grad, 3 * (size_t)natoms)))
+        (rc = dalloc(&ctx->d_grad, 3 * (size_t)natoms)) ||
+        (rc = dalloc(&ctx->d_grad_part, (size_t)(kGradCopies * grad_stride(natoms)))))
       return rc;
     ctx->grad_natoms = natoms;
   }

@@ -38,6 +38,8 @@
 #include "functional.hpp"
 #include "shell_eval.hpp"
 
+#include <type_traits>
+
 namespace xcq {
 
 // ---- per-point coefficients ------------------------------------------------
@@ -306,278 +308,152 @@ __global__ __launch_bounds__(256) void k_plane_product(const WorkItem* __restric
   }
 }
 
-// ---- gradient and Hessian-vector product of a shell's functions ------------
-// For B = R(r^2) m(r) with R1 = -2 sum a c e^{-a r^2} and R2 = 4 sum a^2 c
-// e^{-a r^2} (so d_i R = x_i R1, d_i d_j R = delta_ij R1 + x_i x_j R2):
-//   d_i B = d_i m R + m x_i R1,
-//   (H c)_i = R d_i(c . grad m) + R1 (d_i m (r . c) + x_i (c . grad m))
-//           + m (c_i R1 + x_i (r . c) R2).
-// Calls sink(f, gx, gy, gz, hx, hy, hz) per function (CCA order; spherical
-// outputs one at a time from their nonzero Cartesian terms).
-template <int L, typename Sink>
-__device__ __forceinline__ void shell_grad_hc(double x, double y, double z, double R, double R1,
-                                              double R2, double cx, double cy, double cz,
-                                              bool pure, Sink&& sink) {
-  double xp[L + 1], yp[L + 1], zp[L + 1];
-  xp[0] = yp[0] = zp[0] = 1.;
-#pragma unroll
-  for (int k = 1; k <= L; ++k) {
-    xp[k] = xp[k - 1] * x;
-    yp[k] = yp[k - 1] * y;
-    zp[k] = zp[k - 1] * z;
-  }
-  const double rc = x * cx + y * cy + z * cz;
-  // x^n and its first and second derivatives (0 where the power is negative).
-  auto pw = [](const double* t, int n) { return n < 0 ? 0. : t[n < 0 ? 0 : n]; };
-  auto term = [&](int a, int b, double* o) {
-    const int c = L - a - b;
-    const double m = xp[a] * yp[b] * zp[c];
-    const double mx = a * pw(xp, a - 1) * yp[b] * zp[c];
-    const double my = b * xp[a] * pw(yp, b - 1) * zp[c];
-    const double mz = c * xp[a] * yp[b] * pw(zp, c - 1);
-    const double mxx = a * (a - 1) * pw(xp, a - 2) * yp[b] * zp[c];
-    const double myy = b * (b - 1) * xp[a] * pw(yp, b - 2) * zp[c];
-    const double mzz = c * (c - 1) * xp[a] * yp[b] * pw(zp, c - 2);
-    const double mxy = a * b * pw(xp, a - 1) * pw(yp, b - 1) * zp[c];
-    const double mxz = a * c * pw(xp, a - 1) * yp[b] * pw(zp, c - 1);
-    const double myz = b * c * xp[a] * pw(yp, b - 1) * pw(zp, c - 1);
-    const double cm = cx * mx + cy * my + cz * mz;
-    o[0] = mx * R + m * x * R1;
-    o[1] = my * R + m * y * R1;
-    o[2] = mz * R + m * z * R1;
-    o[3] = R * (cx * mxx + cy * mxy + cz * mxz) + R1 * (mx * rc + x * cm) + m * (cx * R1 + x * rc * R2);
-    o[4] = R * (cx * mxy + cy * myy + cz * myz) + R1 * (my * rc + y * cm) + m * (cy * R1 + y * rc * R2);
-    o[5] = R * (cx * mxz + cy * myz + cz * mzz) + R1 * (mz * rc + z * cm) + m * (cz * R1 + z * rc * R2);
-  };
-  if (pure) {
-#pragma unroll
-    for (int mo = 0; mo < 2 * L + 1; ++mo) {
-      double acc[6] = {0., 0., 0., 0., 0., 0.};
-      int ic = 0;
-#pragma unroll
-      for (int a = L; a >= 0; --a) {
-#pragma unroll
-        for (int b = L - a; b >= 0; --b) {
-          const double cf = kSph.c[L][mo][ic];
-          if (cf != 0.) {
-            double o[6];
-            term(a, b, o);
-#pragma unroll
-            for (int q = 0; q < 6; ++q) acc[q] += cf * o[q];
-          }
-          ++ic;
-        }
-      }
-      sink(mo, acc[0], acc[1], acc[2], acc[3], acc[4], acc[5]);
-    }
-  } else {
-    int ic = 0;
-#pragma unroll
-    for (int a = L; a >= 0; --a) {
-#pragma unroll
-      for (int b = L - a; b >= 0; --b) {
-        double o[6];
-        term(a, b, o);
-        sink(ic, o[0], o[1], o[2], o[3], o[4], o[5]);
-        ++ic;
-      }
-    }
-  }
-}
-
-// Gradient and full Hessian of a shell's functions:
-//   d_i d_j B = R d_i d_j m + R1 (d_i m x_j + d_j m x_i) + m (delta_ij R1 + x_i x_j R2).
-// Calls sink(f, gx, gy, gz, h) with h = (xx, xy, xz, yy, yz, zz).
-template <int L, typename Sink>
-__device__ __forceinline__ void shell_grad_hess(double x, double y, double z, double R,
-                                                double R1, double R2, bool pure, Sink&& sink) {
-  double xp[L + 1], yp[L + 1], zp[L + 1];
-  xp[0] = yp[0] = zp[0] = 1.;
-#pragma unroll
-  for (int k = 1; k <= L; ++k) {
-    xp[k] = xp[k - 1] * x;
-    yp[k] = yp[k - 1] * y;
-    zp[k] = zp[k - 1] * z;
-  }
-  auto pw = [](const double* t, int n) { return n < 0 ? 0. : t[n < 0 ? 0 : n]; };
-  auto term = [&](int a, int b, double* o) {
-    const int c = L - a - b;
-    const double m = xp[a] * yp[b] * zp[c];
-    const double mx = a * pw(xp, a - 1) * yp[b] * zp[c];
-    const double my = b * xp[a] * pw(yp, b - 1) * zp[c];
-    const double mz = c * xp[a] * yp[b] * pw(zp, c - 1);
-    const double mxx = a * (a - 1) * pw(xp, a - 2) * yp[b] * zp[c];
-    const double myy = b * (b - 1) * xp[a] * pw(yp, b - 2) * zp[c];
-    const double mzz = c * (c - 1) * xp[a] * yp[b] * pw(zp, c - 2);
-    const double mxy = a * b * pw(xp, a - 1) * pw(yp, b - 1) * zp[c];
-    const double mxz = a * c * pw(xp, a - 1) * yp[b] * pw(zp, c - 1);
-    const double myz = b * c * xp[a] * pw(yp, b - 1) * pw(zp, c - 1);
-    o[0] = mx * R + m * x * R1;
-    o[1] = my * R + m * y * R1;
-    o[2] = mz * R + m * z * R1;
-    o[3] = R * mxx + 2. * R1 * mx * x + m * (R1 + x * x * R2);
-    o[4] = R * mxy + R1 * (mx * y + my * x) + m * x * y * R2;
-    o[5] = R * mxz + R1 * (mx * z + mz * x) + m * x * z * R2;
-    o[6] = R * myy + 2. * R1 * my * y + m * (R1 + y * y * R2);
-    o[7] = R * myz + R1 * (my * z + mz * y) + m * y * z * R2;
-    o[8] = R * mzz + 2. * R1 * mz * z + m * (R1 + z * z * R2);
-  };
-  if (pure) {
-#pragma unroll
-    for (int mo = 0; mo < 2 * L + 1; ++mo) {
-      double acc[9] = {0., 0., 0., 0., 0., 0., 0., 0., 0.};
-      int ic = 0;
-#pragma unroll
-      for (int a = L; a >= 0; --a) {
-#pragma unroll
-        for (int b = L - a; b >= 0; --b) {
-          const double cf = kSph.c[L][mo][ic];
-          if (cf != 0.) {
-            double o[9];
-            term(a, b, o);
-#pragma unroll
-            for (int q = 0; q < 9; ++q) acc[q] += cf * o[q];
-          }
-          ++ic;
-        }
-      }
-      sink(mo, acc[0], acc[1], acc[2], acc + 3);
-    }
-  } else {
-    int ic = 0;
-#pragma unroll
-    for (int a = L; a >= 0; --a) {
-#pragma unroll
-      for (int b = L - a; b >= 0; --b) {
-        double o[9];
-        term(a, b, o);
-        sink(ic, o[0], o[1], o[2], o + 3);
-        ++ic;
-      }
-    }
-  }
-}
-
-// The highest angular momentum a contraction kernel instantiates: the
-// kernels are compiled for LMAX = 3 (the register budget of f functions)
-// and LMAX = 4, and the launchers pick by the basis.
-template <int LMAX>
-constexpr int kTopL = LMAX > 3 ? 4 : 3;
-
 // ---- basis-function part of the gradient -----------------------------------
-// One (task, 64-point block) per 256-thread workgroup; lane = point, wave w
-// takes the task's shells w, w + 4, ...  Per shell (with the weight
-// derivatives: on an atom other than the parent): sum over its functions and the block's points of
-// grad B . Y + X (H c) (X only for GGAs), reduced over the wave; runs of
-// shells on one atom are added to that atom with one set of atomics, the
-// parent's share (weight derivatives only) once per wave at the end.
-template <bool GGA, int LMAX>
-__global__ __launch_bounds__(256, 2) void k_grad_contract(
-    const WorkItem* __restrict__ items, const DevTask* __restrict__ tasks,
-    const DevShell* __restrict__ shells, const int32_t* __restrict__ shell_list,
-    const int32_t* __restrict__ lsh_first, const int32_t* __restrict__ shell_atom,
-    const double* __restrict__ px, const double* __restrict__ py,
-    const double* __restrict__ pz, const double* __restrict__ scratch,
-    const double* __restrict__ coef, int weight_derivs, double* __restrict__ grad, int x_pl,
-    int y_pl) {
-  const WorkItem wi = items[blockIdx.x];
-  const DevTask t = tasks[wi.task];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int p = wi.a * kPtBlock + lane;
-  const bool valid = p < t.npts;
-  const int pc = min(p, t.npts - 1);
-  const double gx = px[t.pt_off + pc], gy = py[t.pt_off + pc], gz = pz[t.pt_off + pc];
-  const int64_t b = t.red_off + wi.a;
-  double cx = 0., cy = 0., cz = 0.;
-  if (GGA && valid) {
-    cx = coef[b * 256 + 64 + lane];
-    cy = coef[b * 256 + 128 + lane];
-    cz = coef[b * 256 + 192 + lane];
+// A shell's contribution at a point,
+//   s_i = sum_f [ Y_f d_i B_f + sum_j c_j X_f d_i d_j B_f ],
+// for B_f = R(r^2) m_f with R1 = -2 sum a c e^{-a r^2}, R2 = 4 sum a^2 c
+// e^{-a r^2} (so d_i R = x_i R1, d_i d_j R = delta_ij R1 + x_i x_j R2).  The
+// sums over f go into the polynomials y = sum_f Y_f m_f and p = sum_f X_f
+// m_f, collected by Cartesian coefficient (7 functions of an f shell into 10
+// coefficients, two terms each), which are then differentiated once per
+// shell instead of each m_f by itself:
+//   s_i = R d_i y + x_i R1 y
+//       + R d_i (c . grad p) + R1 (d_i p (r . c) + x_i (c . grad p))
+//       + p (c_i R1 + x_i (r . c) R2).
+template <int L>
+constexpr int kCart = (L + 1) * (L + 2) / 2;
+
+// q[cart] = sum_f v_f C_f,cart; get(f) gives v_f.
+template <int L, typename Get>
+__device__ __forceinline__ void cart_coeffs(bool pure, double (&q)[kCart<L>], Get&& get) {
+  if (!pure) {
+#pragma unroll
+    for (int ic = 0; ic < kCart<L>; ++ic) q[ic] = get(ic);
+    return;
   }
-  const int64_t ld = t.npts_pad;
-  const int64_t plane = (int64_t)t.nbe * ld;
-  const int64_t m0 = (int64_t)wi.a * kPtBlock + lane;
-  const double* Xp = scratch + t.b_off + x_pl * plane + m0;
-  const double* Yp = scratch + t.b_off + y_pl * plane + m0;
-  int cur = -1;                            // atom of the running sum (uniform)
-  double run[3] = {0., 0., 0.}, par[3] = {0., 0., 0.};
-  auto flush = [&]() {
-    if (cur >= 0 && lane == 0) {
 #pragma unroll
-      for (int d = 0; d < 3; ++d) atomicAdd(grad + 3 * cur + d, -2.0 * run[d]);
-    }
-  };
-  for (int k = wave; k < t.nshells; k += 4) {
-    const int ish = __builtin_amdgcn_readfirstlane(shell_list[t.sh_off + k]);
-    const int at = __builtin_amdgcn_readfirstlane(shell_atom[ish]);
-    if (at < 0 || (weight_derivs && at == t.iparent)) continue;
-    const int bf0 = __builtin_amdgcn_readfirstlane(lsh_first[t.lsh_off + k]);
-    const DevShell* sh = shells + ish;
-    const int l = sh->l, nprim = sh->nprim;
-    const bool pure = sh->pure != 0;
-    const double x = gx - sh->O[0], y = gy - sh->O[1], z = gz - sh->O[2];
-    const double r2 = x * x + y * y + z * z;
-    double R = 0., R1 = 0., R2 = 0.;
-    for (int q = 0; q < nprim; ++q) {
-      const double a = sh->alpha[q], e = sh->coeff[q] * exp(-a * r2);
-      R += e;
-      R1 -= 2. * a * e;
-      R2 += 4. * a * a * e;
-    }
-    double s[3] = {0., 0., 0.};
-    auto put = [&](int f, double bx, double by, double bz, double hx, double hy, double hz) {
-      const int64_t r = (int64_t)(bf0 + f) * ld;
-      const double Y = valid ? Yp[r] : 0.;
-      s[0] = fma(bx, Y, s[0]);
-      s[1] = fma(by, Y, s[1]);
-      s[2] = fma(bz, Y, s[2]);
-      if constexpr (GGA) {
-        const double X = valid ? Xp[r] : 0.;
-        s[0] = fma(X, hx, s[0]);
-        s[1] = fma(X, hy, s[1]);
-        s[2] = fma(X, hz, s[2]);
-      }
-    };
-    if (l == 0) shell_grad_hc<0>(x, y, z, R, R1, R2, cx, cy, cz, pure, put);
-    else if (l == 1) shell_grad_hc<1>(x, y, z, R, R1, R2, cx, cy, cz, pure, put);
-    else if (l == 2) shell_grad_hc<2>(x, y, z, R, R1, R2, cx, cy, cz, pure, put);
-    else if (l == 3) shell_grad_hc<3>(x, y, z, R, R1, R2, cx, cy, cz, pure, put);
-    else shell_grad_hc<kTopL<LMAX>>(x, y, z, R, R1, R2, cx, cy, cz, pure, put);
+  for (int ic = 0; ic < kCart<L>; ++ic) q[ic] = 0.;
 #pragma unroll
-    for (int d = 0; d < 3; ++d)
-      for (int off = 32; off > 0; off >>= 1) s[d] += __shfl_xor(s[d], off);
-    if (at != cur) {
-      flush();
-      cur = at;
+  for (int m = 0; m < 2 * L + 1; ++m) {
+    const double v = get(m);
 #pragma unroll
-      for (int d = 0; d < 3; ++d) run[d] = 0.;
-    }
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      run[d] += s[d];
-      par[d] += s[d];
-    }
-  }
-  flush();
-  if (weight_derivs && lane == 0 && cur >= 0) {
-#pragma unroll
-    for (int d = 0; d < 3; ++d) atomicAdd(grad + 3 * t.iparent + d, 2.0 * par[d]);
+    for (int ic = 0; ic < kCart<L>; ++ic)
+      if (kSph.c[L][m][ic] != 0.) q[ic] = fma(kSph.c[L][m][ic], v, q[ic]);
   }
 }
 
-// UKS basis-function part: as k_grad_contract with Y in plane 1, X_N in
-// plane 2 and X_Z in plane 3; per function grad B . Y + H (X_N c_s + X_Z c_z)
-// (the Hessian term for GGAs only).
-template <bool GGA, int LMAX>
-__global__ __launch_bounds__(256, 2) void k_grad_contract_uks(
+// Powers 0 .. L of a displacement; 0 where the exponent is negative.
+template <int L>
+struct Powers {
+  double x[L + 1], y[L + 1], z[L + 1];
+  __device__ __forceinline__ Powers(double px, double py, double pz) {
+    x[0] = y[0] = z[0] = 1.;
+#pragma unroll
+    for (int k = 1; k <= L; ++k) {
+      x[k] = x[k - 1] * px;
+      y[k] = y[k - 1] * py;
+      z[k] = z[k - 1] * pz;
+    }
+  }
+  // d^i/dx^i d^j/dy^j d^k/dz^k of x^a y^b z^c, i + j + k <= 2.
+  __device__ __forceinline__ double mono(int a, int b, int c, int i, int j, int k) const {
+    auto f = [](int n, int d) { return d == 0 ? 1 : d == 1 ? n : n * (n - 1); };
+    const int w = f(a, i) * f(b, j) * f(c, k);
+    if (w == 0) return 0.;
+    return (double)w * (x[a - i] * y[b - j] * z[c - k]);
+  }
+};
+
+// s += R grad y + R1 r y for the polynomial y with coefficients q.
+template <int L>
+__device__ __forceinline__ void add_value(const Powers<L>& pw, const double (&q)[kCart<L>],
+                                          double x, double y, double z, double R, double R1,
+                                          double (&s)[3]) {
+  double v = 0., g[3] = {0., 0., 0.};
+  int ic = 0;
+#pragma unroll
+  for (int a = L; a >= 0; --a)
+#pragma unroll
+    for (int b = L - a; b >= 0; --b, ++ic) {
+      const int c = L - a - b;
+      v = fma(q[ic], pw.mono(a, b, c, 0, 0, 0), v);
+      if (a) g[0] = fma(q[ic], pw.mono(a, b, c, 1, 0, 0), g[0]);
+      if (b) g[1] = fma(q[ic], pw.mono(a, b, c, 0, 1, 0), g[1]);
+      if (c) g[2] = fma(q[ic], pw.mono(a, b, c, 0, 0, 1), g[2]);
+    }
+  v *= R1;
+  s[0] += R * g[0] + x * v;
+  s[1] += R * g[1] + y * v;
+  s[2] += R * g[2] + z * v;
+}
+
+// s += the Hessian of R p times (cx, cy, cz), p with coefficients q.
+template <int L>
+__device__ __forceinline__ void add_hessian(const Powers<L>& pw, const double (&q)[kCart<L>],
+                                            double x, double y, double z, double R, double R1,
+                                            double R2, double cx, double cy, double cz,
+                                            double (&s)[3]) {
+  double v = 0., g[3] = {0., 0., 0.}, h[6] = {0., 0., 0., 0., 0., 0.};  // xx xy xz yy yz zz
+  int ic = 0;
+#pragma unroll
+  for (int a = L; a >= 0; --a)
+#pragma unroll
+    for (int b = L - a; b >= 0; --b, ++ic) {
+      const int c = L - a - b;
+      v = fma(q[ic], pw.mono(a, b, c, 0, 0, 0), v);
+      if (a) g[0] = fma(q[ic], pw.mono(a, b, c, 1, 0, 0), g[0]);
+      if (b) g[1] = fma(q[ic], pw.mono(a, b, c, 0, 1, 0), g[1]);
+      if (c) g[2] = fma(q[ic], pw.mono(a, b, c, 0, 0, 1), g[2]);
+      if (a > 1) h[0] = fma(q[ic], pw.mono(a, b, c, 2, 0, 0), h[0]);
+      if (a && b) h[1] = fma(q[ic], pw.mono(a, b, c, 1, 1, 0), h[1]);
+      if (a && c) h[2] = fma(q[ic], pw.mono(a, b, c, 1, 0, 1), h[2]);
+      if (b > 1) h[3] = fma(q[ic], pw.mono(a, b, c, 0, 2, 0), h[3]);
+      if (b && c) h[4] = fma(q[ic], pw.mono(a, b, c, 0, 1, 1), h[4]);
+      if (c > 1) h[5] = fma(q[ic], pw.mono(a, b, c, 0, 0, 2), h[5]);
+    }
+  const double rc = x * cx + y * cy + z * cz;
+  const double cg = cx * g[0] + cy * g[1] + cz * g[2];
+  const double t = R1 * cg + v * rc * R2;  // along r
+  const double u = v * R1;                 // along c
+  s[0] += R * (cx * h[0] + cy * h[1] + cz * h[2]) + R1 * g[0] * rc + x * t + cx * u;
+  s[1] += R * (cx * h[1] + cy * h[3] + cz * h[4]) + R1 * g[1] * rc + y * t + cy * u;
+  s[2] += R * (cx * h[2] + cy * h[4] + cz * h[5]) + R1 * g[2] * rc + z * t + cz * u;
+}
+
+// One (task, 64-point block) per 256-thread workgroup; lane = point, wave w
+// takes the task's shells w, w + 4, ..., their parameters staged in LDS 64
+// at a time.  Per shell (with the weight derivatives: on an atom other than
+// the parent) the sums above, reduced over the wave; runs of shells on one
+// atom are added to that atom with one set of atomics, the parent's share
+// (weight derivatives only) once per wave at the end.  NX = 1 (RKS): Y in
+// plane y_pl, X in plane x_pl with the coefficients coef_s (GGA); NX = 2
+// (UKS): X_N and X_Z in planes x_pl and x_pl + 1 with coef_s and coef_z.
+// What bounds it: FP64 vector work and the reads of Y and X.  On 13 waters
+// (883,000 points, PBE) it takes 0.85 ms.  4.1 ms of atomic additions to one
+// gradient had hidden the arithmetic (kGradCopies).
+__device__ __forceinline__ void reduce_lanes(double (&v)[3]) {
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+    for (int off = 32; off > 0; off >>= 1) v[d] += __shfl_xor(v[d], off);
+}
+
+struct GradShells {
+  static constexpr int kMax = 64, kPrims = 4;
+  double ox[kMax], oy[kMax], oz[kMax], a[kPrims][kMax], c[kPrims][kMax];
+  int bf0[kMax], info[kMax], ish[kMax], atom[kMax];
+};
+
+template <bool GGA, int LMAX, int NX>
+__global__ __launch_bounds__(256, LMAX > 3 || NX > 1 ? 2 : 3) void k_grad_contract(
     const WorkItem* __restrict__ items, const DevTask* __restrict__ tasks,
     const DevShell* __restrict__ shells, const int32_t* __restrict__ shell_list,
     const int32_t* __restrict__ lsh_first, const int32_t* __restrict__ shell_atom,
     const double* __restrict__ px, const double* __restrict__ py,
     const double* __restrict__ pz, const double* __restrict__ scratch,
     const double* __restrict__ coef_s, const double* __restrict__ coef_z, int weight_derivs,
-    double* __restrict__ grad) {
+    double* __restrict__ grad, int64_t gstride, int x_pl, int y_pl) {
+  __shared__ GradShells st;
+  grad += (int64_t)(blockIdx.x % kGradCopies) * gstride;
   const WorkItem wi = items[blockIdx.x];
   const DevTask t = tasks[wi.task];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -592,93 +468,111 @@ __global__ __launch_bounds__(256, 2) void k_grad_contract_uks(
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
       cs[d] = coef_s[b * 256 + (1 + d) * 64 + lane];
-      cz[d] = coef_z[b * 256 + (1 + d) * 64 + lane];
+      if (NX > 1) cz[d] = coef_z[b * 256 + (1 + d) * 64 + lane];
     }
   }
   const int64_t ld = t.npts_pad;
   const int64_t plane = (int64_t)t.nbe * ld;
   const int64_t m0 = (int64_t)wi.a * kPtBlock + lane;
-  const double* Yp = scratch + t.b_off + plane + m0;
-  const double* XNp = scratch + t.b_off + 2 * plane + m0;
-  const double* XZp = scratch + t.b_off + 3 * plane + m0;
-  int cur = -1;
+  const double* Yp = scratch + t.b_off + y_pl * plane + m0;
+  const double* Xp = scratch + t.b_off + x_pl * plane + m0;
+  int cur = -1;                            // atom of the running sum (uniform)
   double run[3] = {0., 0., 0.}, par[3] = {0., 0., 0.};
-  auto flush = [&]() {
-    if (cur >= 0 && lane == 0) {
-#pragma unroll
-      for (int d = 0; d < 3; ++d) atomicAdd(grad + 3 * cur + d, -2.0 * run[d]);
-    }
+  auto add = [&](int at, double fac, double v0, double v1, double v2) {
+    const double val = lane == 0 ? v0 : lane == 1 ? v1 : v2;
+    if (lane < 3) atomicAdd(grad + 3 * (int64_t)at + lane, fac * val);
   };
-  for (int k = wave; k < t.nshells; k += 4) {
-    const int ish = __builtin_amdgcn_readfirstlane(shell_list[t.sh_off + k]);
-    const int at = __builtin_amdgcn_readfirstlane(shell_atom[ish]);
-    if (at < 0 || (weight_derivs && at == t.iparent)) continue;
-    const int bf0 = __builtin_amdgcn_readfirstlane(lsh_first[t.lsh_off + k]);
-    const DevShell* sh = shells + ish;
-    const int l = sh->l, nprim = sh->nprim;
-    const bool pure = sh->pure != 0;
-    const double x = gx - sh->O[0], y = gy - sh->O[1], z = gz - sh->O[2];
-    const double r2 = x * x + y * y + z * z;
-    double R = 0., R1 = 0., R2 = 0.;
-    for (int q = 0; q < nprim; ++q) {
-      const double a = sh->alpha[q], e = sh->coeff[q] * exp(-a * r2);
-      R += e;
-      R1 -= 2. * a * e;
-      R2 += 4. * a * a * e;
-    }
-    double s[3] = {0., 0., 0.};
-    auto put = [&](int f, double bx, double by, double bz, const double* h) {
-      const int64_t r = (int64_t)(bf0 + f) * ld;
-      const double Y = valid ? Yp[r] : 0.;
-      s[0] = fma(bx, Y, s[0]);
-      s[1] = fma(by, Y, s[1]);
-      s[2] = fma(bz, Y, s[2]);
-      if constexpr (GGA) {
-        const double xn = valid ? XNp[r] : 0., xz = valid ? XZp[r] : 0.;
-        const double vx = xn * cs[0] + xz * cz[0], vy = xn * cs[1] + xz * cz[1],
-                     vz = xn * cs[2] + xz * cz[2];
-        s[0] += h[0] * vx + h[1] * vy + h[2] * vz;
-        s[1] += h[1] * vx + h[3] * vy + h[4] * vz;
-        s[2] += h[2] * vx + h[4] * vy + h[5] * vz;
+  auto flush = [&]() {
+    if (cur >= 0) add(cur, -2.0, run[0], run[1], run[2]);
+  };
+  for (int pass = 0; pass < t.nshells; pass += GradShells::kMax) {
+    const int nsh = min(GradShells::kMax, t.nshells - pass);
+    __syncthreads();  // the previous pass is done with the staged shells
+    if (tid < nsh) {
+      const int ish = shell_list[t.sh_off + pass + tid];
+      const DevShell* sh = shells + ish;
+      st.ish[tid] = ish;
+      st.atom[tid] = shell_atom[ish];
+      st.bf0[tid] = lsh_first[t.lsh_off + pass + tid];
+      st.info[tid] = sh->l | (sh->pure ? 1 << 8 : 0) | (sh->nprim << 16);
+      st.ox[tid] = sh->O[0];
+      st.oy[tid] = sh->O[1];
+      st.oz[tid] = sh->O[2];
+      const int np = min(sh->nprim, GradShells::kPrims);
+      for (int k = 0; k < np; ++k) {
+        st.a[k][tid] = sh->alpha[k];
+        st.c[k][tid] = sh->coeff[k];
       }
-    };
-    if constexpr (GGA) {
-      if (l == 0) shell_grad_hess<0>(x, y, z, R, R1, R2, pure, put);
-      else if (l == 1) shell_grad_hess<1>(x, y, z, R, R1, R2, pure, put);
-      else if (l == 2) shell_grad_hess<2>(x, y, z, R, R1, R2, pure, put);
-      else if (l == 3) shell_grad_hess<3>(x, y, z, R, R1, R2, pure, put);
-      else shell_grad_hess<kTopL<LMAX>>(x, y, z, R, R1, R2, pure, put);
-    } else {
-      // LDA needs only grad B: the Hessian-vector form with c = 0.
-      auto put3 = [&](int f, double bx, double by, double bz, double, double, double) {
-        const double h0[6] = {0., 0., 0., 0., 0., 0.};
-        put(f, bx, by, bz, h0);
+    }
+    __syncthreads();
+    for (int k = wave; k < nsh; k += 4) {
+      const int at = __builtin_amdgcn_readfirstlane(st.atom[k]);
+      if (at < 0 || (weight_derivs && at == t.iparent)) continue;
+      const int bf0 = __builtin_amdgcn_readfirstlane(st.bf0[k]);
+      const int info = __builtin_amdgcn_readfirstlane(st.info[k]);
+      const int l = info & 0xff, nprim = info >> 16;
+      const bool pure = (info >> 8) & 1;
+      const double x = gx - st.ox[k], y = gy - st.oy[k], z = gz - st.oz[k];
+      const double r2 = x * x + y * y + z * z;
+      double R = 0., R1 = 0., R2 = 0.;
+      auto prim = [&](double a, double c) {
+        const double e = c * exp(-a * r2);
+        R += e;
+        R1 -= 2. * a * e;
+        R2 += 4. * a * a * e;
       };
-      if (l == 0) shell_grad_hc<0>(x, y, z, R, R1, R2, 0., 0., 0., pure, put3);
-      else if (l == 1) shell_grad_hc<1>(x, y, z, R, R1, R2, 0., 0., 0., pure, put3);
-      else if (l == 2) shell_grad_hc<2>(x, y, z, R, R1, R2, 0., 0., 0., pure, put3);
-      else if (l == 3) shell_grad_hc<3>(x, y, z, R, R1, R2, 0., 0., 0., pure, put3);
-      else shell_grad_hc<kTopL<LMAX>>(x, y, z, R, R1, R2, 0., 0., 0., pure, put3);
-    }
+      for (int q = 0; q < min(nprim, GradShells::kPrims); ++q) prim(st.a[q][k], st.c[q][k]);
+      if (nprim > GradShells::kPrims) {
+        const DevShell* sh = shells + __builtin_amdgcn_readfirstlane(st.ish[k]);
+        for (int q = GradShells::kPrims; q < nprim; ++q) prim(sh->alpha[q], sh->coeff[q]);
+      }
+      double s[3] = {0., 0., 0.};
+      auto shell = [&](auto LC) {
+        constexpr int L = decltype(LC)::value;
+        const Powers<L> pw(x, y, z);
+        double q[kCart<L>];
+        const int64_t r0 = (int64_t)bf0 * ld;
+        auto get = [&](const double* pl) {
+          return [=](int f) { return valid ? pl[r0 + f * ld] : 0.; };
+        };
+        cart_coeffs<L>(pure, q, get(Yp));
+        add_value<L>(pw, q, x, y, z, R, R1, s);
+        if constexpr (GGA) {
+          cart_coeffs<L>(pure, q, get(Xp));
+          add_hessian<L>(pw, q, x, y, z, R, R1, R2, cs[0], cs[1], cs[2], s);
+          if constexpr (NX > 1) {
+            cart_coeffs<L>(pure, q, get(Xp + plane));
+            add_hessian<L>(pw, q, x, y, z, R, R1, R2, cz[0], cz[1], cz[2], s);
+          }
+        }
+      };
+      if (l == 0) shell(std::integral_constant<int, 0>{});
+      else if (l == 1) shell(std::integral_constant<int, 1>{});
+      else if (l == 2) shell(std::integral_constant<int, 2>{});
+      else if (l == 3 || LMAX == 3) shell(std::integral_constant<int, 3>{});
+      else shell(std::integral_constant<int, LMAX>{});
+      if (at != cur) {
+        // The running sums are per lane; they are reduced when their atom's
+        // run of shells ends.
+        reduce_lanes(run);
+        flush();
+        cur = at;
 #pragma unroll
-    for (int d = 0; d < 3; ++d)
-      for (int off = 32; off > 0; off >>= 1) s[d] += __shfl_xor(s[d], off);
-    if (at != cur) {
-      flush();
-      cur = at;
+        for (int d = 0; d < 3; ++d) {
+          par[d] += run[d];
+          run[d] = 0.;
+        }
+      }
 #pragma unroll
-      for (int d = 0; d < 3; ++d) run[d] = 0.;
-    }
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      run[d] += s[d];
-      par[d] += s[d];
+      for (int d = 0; d < 3; ++d) run[d] += s[d];
     }
   }
+  reduce_lanes(run);
   flush();
-  if (weight_derivs && lane == 0 && cur >= 0) {
+  if (weight_derivs && cur >= 0) {
 #pragma unroll
-    for (int d = 0; d < 3; ++d) atomicAdd(grad + 3 * t.iparent + d, 2.0 * par[d]);
+    for (int d = 0; d < 3; ++d) par[d] += run[d];
+    add(t.iparent, 2.0, par[0], par[1], par[2]);
   }
 }
 
@@ -692,32 +586,43 @@ __global__ __launch_bounds__(256, 2) void k_grad_contract_uks(
 //   1 - g(v) = (1 - v)^4 (5 v^3 + 20 v^2 + 29 v + 16) / 16,  g'(v) = 35 (1 - v^2)^3 / 16,
 //   t(mu) = 35 (1 + v)^3 / ((mu - a)(5 v^3 + 20 v^2 + 29 v + 16)),  v = mu / a,
 // which stays accurate up to the |mu| < a - 1e-4 bound the contraction uses.
-// One thread per point (lane of a 64-point block); distances are recomputed
-// where needed.  Without neighbour lists every loop runs over all atoms,
-// O(natoms^2) per point.  With them (nbr_idx / nbr_r: row A holds every atom
-// in order of increasing R_AB, A itself first) the loops stop where the
-// triangle inequality makes every remaining term vanish, as in the weights
-// kernel: a factor s(mu_BC) differs from 1, and |mu_BC| can fall below a,
-// only for R_BC < 2 d_B / (1 - a); P_B > 0 only for d_B <= (1 + a)/(1 - a)
-// d_min; so the parent's list is read up to max(2 d_A / (1 - a),
-// d_A + that bound) and each B's list up to 2 d_B / (1 - a), all widened by
-// a relative 1e-10.  The terms skipped are exactly zero (factors exactly 1).
+// With neighbour lists (nbr_idx / nbr_r: row A holds every atom in order of
+// increasing R_AB, A itself first) the loops stop where the triangle
+// inequality makes every remaining term vanish, as in the weights kernel: a
+// factor s(mu_BC) differs from 1, and |mu_BC| can fall below a, only for
+// R_BC < 2 d_B / (1 - a); P_B > 0 only for d_B <= (1 + a)/(1 - a) d_min; so
+// the parent's list is read up to max(2 d_A / (1 - a), d_A + that bound) and
+// each B's list up to 2 d_B / (1 - a), all widened by a relative 1e-10.  The
+// terms skipped are exactly zero (factors exactly 1).  Without lists every
+// loop runs over all atoms.
+//
+// One wave per 64-point block, lane = point.  All loops are uniform: they
+// run as far as any lane needs, so indices and atoms are read by scalar
+// loads and lanes that need less multiply by exact ones.  The first pass
+// forms sum_B P_B and keeps the products of the first kSsfKeep atoms with
+// P_B > kSsfTol in any lane; the second takes A (with P_A - sum in P_B's
+// place, from dw/dR_C of w's numerator and denominator together) and those
+// atoms, and forms for each neighbour C the derivative of s(mu_BC).  What
+// falls on C is summed over the wave, four C at a time (a transposing
+// reduction: 21 exchanges where 12 separate sums take 72); what falls on B
+// and on A stays in registers and is summed once.
+// What bounds it: FP64 vector work.  On 13 waters (883,000 points) 1.4 ms;
+// with every thread's own loop bounds and one atomic addition per thread and
+// term 6.4 ms.
 constexpr double kSsfA = 0.64;
 constexpr double kSsfTol = 1e-13;
 
-__device__ __forceinline__ double ssf_s(double mu) {
-  if (mu <= -kSsfA) return 1.;
-  if (mu >= kSsfA) return 0.;
-  const double v = mu / kSsfA, v2 = v * v;
-  const double g = v * (35. + v2 * (-35. + v2 * (21. - 5. * v2))) / 16.;
+constexpr int kSsfKeep = 12;
+
+// s at v = mu / a: the limits +-1 give exactly 0 and 1.
+__device__ __forceinline__ double ssf_s(double v) {
+  v = fmin(fmax(v, -1.), 1.);
+  const double v2 = v * v;
+  const double g = v * (35. + v2 * (-35. + v2 * (21. - 5. * v2))) * 0.0625;
   return 0.5 * (1. - g);
 }
-__device__ __forceinline__ double ssf_t(double mu) {
-  const double v = mu / kSsfA;
-  return 35. * (1. + v) * (1. + v) * (1. + v) /
-         ((mu - kSsfA) * (((5. * v + 20.) * v + 29.) * v + 16.));
-}
 
+template <bool LISTS>
 __global__ __launch_bounds__(64) void k_ssf_grad(const WorkItem* __restrict__ items,
                                                  const DevTask* __restrict__ tasks,
                                                  const double* __restrict__ px,
@@ -726,154 +631,188 @@ __global__ __launch_bounds__(64) void k_ssf_grad(const WorkItem* __restrict__ it
                                                  const double* __restrict__ xyz,
                                                  const double* __restrict__ dnear,
                                                  const double* __restrict__ wf,
-                                                 double* __restrict__ grad,
+                                                 double* __restrict__ grad, int64_t gstride,
                                                  const int32_t* __restrict__ nbr_idx,
                                                  const double* __restrict__ nbr_r) {
+  __shared__ double keep[kSsfKeep][64];
   const WorkItem wi = items[blockIdx.x];
   const DevTask t = tasks[wi.task];
   const int lane = threadIdx.x;
   const int p = wi.a * kPtBlock + lane;
-  if (p >= t.npts) return;
+  const int pc = min(p, t.npts - 1);
   const double f = wf[(t.red_off + wi.a) * 64 + lane];
-  if (fabs(f) < 1e-12) return;
-  const double r[3] = {px[t.pt_off + p], py[t.pt_off + p], pz[t.pt_off + p]};
-  auto X = [&](int at, int d) { return xyz[3 * at + d]; };
-  auto dist = [&](int at) {
-    const double dx = r[0] - X(at, 0), dy = r[1] - X(at, 1), dz = r[2] - X(at, 2);
-    return sqrt(dx * dx + dy * dy + dz * dz);
-  };
-  auto rab = [&](int a, int b) {
-    const double dx = X(a, 0) - X(b, 0), dy = X(a, 1) - X(b, 1), dz = X(a, 2) - X(b, 2);
-    return sqrt(dx * dx + dy * dy + dz * dz);
-  };
+  const double rx = px[t.pt_off + pc], ry = py[t.pt_off + pc], rz = pz[t.pt_off + pc];
   const int A = t.iparent;
+  auto X = [&](int at, int d) { return xyz[3 * (int64_t)at + d]; };
+  auto dist = [&](int at) {
+    const double dx = rx - X(at, 0), dy = ry - X(at, 1), dz = rz - X(at, 2);
+    return sqrt(dx * dx + dy * dy + dz * dz);
+  };
+  // Entry q of B's list (atom, R_BC); lists start with B itself at q = 0.
+  auto nbr_at = [&](int B, int q) { return LISTS ? nbr_idx[(int64_t)B * natoms + q] : q; };
+  auto nbr_d = [&](int B, int q) {
+    if (LISTS) return nbr_r[(int64_t)B * natoms + q];
+    const double dx = X(B, 0) - X(q, 0), dy = X(B, 1) - X(q, 1), dz = X(B, 2) - X(q, 2);
+    return sqrt(dx * dx + dy * dy + dz * dz);
+  };
+  constexpr double kWiden = 1.0 + 1e-10, kInvA = 1.0 / kSsfA;
+  constexpr double bound = kSsfA - 1e-4;
   const double dA = dist(A);
-  if (dA < 0.5 * (1. - kSsfA) * dnear[A]) return;
-  const double bound = kSsfA - 1e-4;
-  if (nbr_idx) {
-    constexpr double kWiden = 1.0 + 1e-10;
-    const int32_t* an = nbr_idx + (size_t)A * natoms;
-    const double* ar = nbr_r + (size_t)A * natoms;
-    // Nearest atom (R_AB* <= 2 d_A) and the candidate bound.
+  const bool on = p < t.npts && !(fabs(f) < 1e-12) && !(dA < 0.5 * (1. - kSsfA) * dnear[A]);
+  if (!__any(on)) return;
+  // Nearest atom (R_AB* <= 2 d_A) and the candidate bound.
+  double cbound = INFINITY, rmax = INFINITY;
+  if (LISTS) {
     double dmin = dA;
-    for (int k = 1; k < natoms && ar[k] <= 2.0 * dA * kWiden; ++k) dmin = fmin(dmin, dist(an[k]));
-    const double cbound = (1.0 + kSsfA) / (1.0 - kSsfA) * dmin * kWiden + 1e-12;
-    const double rmax = fmax(2.0 * dA / (1.0 - kSsfA), dA + cbound) * kWiden;
-    // P_B over B's list (factors beyond 2 d_B / (1 - a) are exactly 1).
-    auto part_l = [&](int B, double dB) {
-      if (dB > cbound) return 0.;
-      const int32_t* bn = nbr_idx + (size_t)B * natoms;
-      const double* br = nbr_r + (size_t)B * natoms;
-      const double rf = 2.0 * dB / (1.0 - kSsfA) * kWiden;
-      double v = 1.;
-      for (int q = 1; q < natoms && br[q] < rf && v > 0.; ++q)
-        v *= ssf_s((dB - dist(bn[q])) / br[q]);
-      return v;
-    };
-    double sum = 0.;
-    for (int k = 0; k < natoms && ar[k] <= rmax; ++k) {
-      const int B = an[k];
-      sum += part_l(B, k == 0 ? dA : dist(B));
-    }
-    const double pA = part_l(A, dA);
-    double gA[3] = {0., 0., 0.};
-    for (int k = 1; k < natoms && ar[k] <= rmax; ++k) {
-      const int B = an[k];
-      const double dB = dist(B);
-      double gb[3] = {0., 0., 0.};
-      const double rAB = ar[k];
-      const double muAB = (dA - dB) / rAB;
-      if (fabs(muAB) < bound) {
-        const double c1 = ssf_t(muAB) / rAB * (pA - sum) / sum * f / dB;
-#pragma unroll
-        for (int d = 0; d < 3; ++d)
-          gb[d] = c1 * ((X(B, d) - r[d]) + muAB * (X(B, d) - X(A, d)) / rAB * dB);
-      }
-      const double pB = part_l(B, dB);
-      if (pB > kSsfTol) {
-        const int32_t* bn = nbr_idx + (size_t)B * natoms;
-        const double* br = nbr_r + (size_t)B * natoms;
-        const double rf = 2.0 * dB / (1.0 - kSsfA) * kWiden;
-        for (int q = 1; q < natoms && br[q] < rf; ++q) {
-          const int C = bn[q];
-          const double rBC = br[q], dC = dist(C);
-          const double muBC = (dB - dC) / rBC;
-          if (fabs(muBC) >= bound) continue;
-          const double c = pB * ssf_t(muBC) / rBC / sum * f;
-#pragma unroll
-          for (int d = 0; d < 3; ++d)
-            gb[d] -= c * ((X(B, d) - r[d]) / dB - muBC * (X(B, d) - X(C, d)) / rBC);
-          if (C != A) {
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-              const double gc = c * ((X(C, d) - r[d]) / dC + muBC * (X(C, d) - X(B, d)) / rBC);
-              atomicAdd(grad + 3 * C + d, gc);
-              gA[d] -= gc;
-            }
-          }
-        }
-      }
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        if (gb[d] != 0.) atomicAdd(grad + 3 * B + d, gb[d]);
-        gA[d] -= gb[d];
-      }
-    }
-#pragma unroll
-    for (int d = 0; d < 3; ++d) atomicAdd(grad + 3 * A + d, gA[d]);
-    return;
+    for (int k = 1; k < natoms && __any(on && nbr_d(A, k) <= 2.0 * dA * kWiden); ++k)
+      dmin = fmin(dmin, dist(nbr_at(A, k)));
+    cbound = (1.0 + kSsfA) / (1.0 - kSsfA) * dmin * kWiden + 1e-12;
+    rmax = fmax(2.0 * dA / (1.0 - kSsfA), dA + cbound) * kWiden;
   }
+  auto reach = [&](double dB) { return 2.0 * dB / (1.0 - kSsfA) * kWiden; };
+  constexpr int q0 = LISTS ? 1 : 0;
+  // P_B, 0 in lanes that are off or beyond the candidate bound.
   auto part = [&](int B, double dB) {
-    double v = 1.;
-    for (int C = 0; C < natoms && v > 0.; ++C)
-      if (C != B) v *= ssf_s((dB - dist(C)) / rab(B, C));
+    double v = on && dB <= cbound ? 1. : 0.;
+    const double rf = reach(dB);
+    if (!__any(v > 0.)) return v;
+    for (int q = q0; q < natoms; q += 4) {
+      int C[4];
+      double R[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int qj = min(q + j, natoms - 1);
+        C[j] = nbr_at(B, qj);
+        R[j] = nbr_d(B, qj);
+      }
+      if (!__any(v > 0. && (!LISTS || R[0] < rf))) break;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (q + j < natoms && C[j] != B) v *= ssf_s((dB - dist(C[j])) / (kSsfA * R[j]));
+    }
     return v;
   };
-  double sum = 0.;
-  for (int B = 0; B < natoms; ++B) sum += part(B, B == A ? dA : dist(B));
-  const double pA = part(A, dA);
-  double gA[3] = {0., 0., 0.};
-  for (int B = 0; B < natoms; ++B) {
-    if (B == A) continue;
-    const double dB = dist(B);
-    double gb[3] = {0., 0., 0.};
-    const double rAB = rab(A, B);
-    const double muAB = (dA - dB) / rAB;
-    if (fabs(muAB) < bound) {
-      const double c1 = ssf_t(muAB) / rAB * (pA - sum) / sum * f / dB;
+  double sum = 0., pA = 0.;
+  int nkeep = 0, kover = natoms, kept[kSsfKeep];
+  for (int k = 0; k < natoms && (!LISTS || __any(on && nbr_d(A, k) <= rmax)); ++k) {
+    const int B = nbr_at(A, k);
+    const double pB = part(B, dist(B));
+    sum += pB;
+    if (B == A) pA = pB;
+    else if (__any(pB > kSsfTol) && kover == natoms) {
+      if (nkeep == kSsfKeep) kover = k;
+      else {
+        keep[nkeep][lane] = pB;
 #pragma unroll
-      for (int d = 0; d < 3; ++d)
-        gb[d] = c1 * ((X(B, d) - r[d]) + muAB * (X(B, d) - X(A, d)) / rAB * dB);
-    }
-    const double pB = part(B, dB);
-    if (pB > kSsfTol) {
-      for (int C = 0; C < natoms; ++C) {
-        if (C == B) continue;
-        const double rBC = rab(B, C), dC = dist(C);
-        const double muBC = (dB - dC) / rBC;
-        if (fabs(muBC) >= bound) continue;
-        const double c = pB * ssf_t(muBC) / rBC / sum * f;
-#pragma unroll
-        for (int d = 0; d < 3; ++d)
-          gb[d] -= c * ((X(B, d) - r[d]) / dB - muBC * (X(B, d) - X(C, d)) / rBC);
-        if (C != A) {
-#pragma unroll
-          for (int d = 0; d < 3; ++d) {
-            const double gc = c * ((X(C, d) - r[d]) / dC + muBC * (X(C, d) - X(B, d)) / rBC);
-            atomicAdd(grad + 3 * C + d, gc);
-            gA[d] -= gc;
-          }
-        }
+        for (int i = 0; i < kSsfKeep; ++i)
+          if (i == nkeep) kept[i] = B;
+        ++nkeep;
       }
     }
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      if (gb[d] != 0.) atomicAdd(grad + 3 * B + d, gb[d]);
-      gA[d] -= gb[d];
-    }
   }
+  grad += (int64_t)(blockIdx.x % kGradCopies) * gstride;
+  const double fs = on ? f / sum : 0.;
+  double gA[3] = {0., 0., 0.};
+  // The derivatives of B's factors, weighted by cf.
+  auto derivs = [&](int B, double cf, bool act) {
+    const double dB = dist(B), rf = reach(dB);
+    const double iB = act && dB > 0. ? cf / dB : 0.;
+    const double ub[3] = {(X(B, 0) - rx) * iB, (X(B, 1) - ry) * iB, (X(B, 2) - rz) * iB};
+    double gb[3] = {0., 0., 0.};
+    for (int q = q0; q < natoms; q += 4) {
+      int C[4];
+      double R[4], g[4][3];
 #pragma unroll
-  for (int d = 0; d < 3; ++d) atomicAdd(grad + 3 * A + d, gA[d]);
+      for (int j = 0; j < 4; ++j) {
+        const int qj = min(q + j, natoms - 1);
+        C[j] = nbr_at(B, qj);
+        R[j] = nbr_d(B, qj);
+      }
+      if (LISTS && !__any(act && R[0] < rf)) break;
+      bool any = false;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const double dC = dist(C[j]);
+        const double iR = 1. / R[j];
+        const double mu = (dB - dC) * iR;
+        const bool in = q + j < natoms && C[j] != B && act && fabs(mu) < bound;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) g[j][d] = 0.;
+        if (!__any(in)) continue;
+        const double v = mu * kInvA, v1 = 1. + v;
+        const double tm = 35. * (v1 * v1 * v1) /
+                          ((mu - kSsfA) * (((5. * v + 20.) * v + 29.) * v + 16.)) * iR;
+        const double tt = in ? tm : 0.;
+        const double e = cf * tt * mu * iR;
+        const double iC = in ? cf * tt / dC : 0.;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          const double s = e * (X(C[j], d) - X(B, d));
+          gb[d] -= tt * ub[d] + s;
+          const double r = d == 0 ? rx : d == 1 ? ry : rz;
+          g[j][d] = C[j] == A ? 0. : iC * (X(C[j], d) - r) + s;
+          gA[d] -= g[j][d];
+        }
+        any = any || C[j] != A;
+      }
+      if (!any) continue;
+      // Sums over the wave: lanes of 16-lane group j end with those of C[j].
+      double u[2][3], w[3];
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+          u[j][d] = (lane & 32 ? g[j + 2][d] : g[j][d]) +
+                    __shfl_xor(lane & 32 ? g[j][d] : g[j + 2][d], 32);
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        w[d] = (lane & 16 ? u[1][d] : u[0][d]) + __shfl_xor(lane & 16 ? u[0][d] : u[1][d], 16);
+#pragma unroll
+        for (int off = 8; off > 0; off >>= 1) w[d] += __shfl_xor(w[d], off);
+      }
+      const int at = lane & 32 ? (lane & 16 ? C[3] : C[2]) : (lane & 16 ? C[1] : C[0]);
+      const int d = lane & 15;
+      const double val = d == 0 ? w[0] : d == 1 ? w[1] : w[2];
+      if (d < 3 && val != 0.) atomicAdd(grad + 3 * (int64_t)at + d, val);
+    }
+    if (B == A) return;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) gA[d] -= gb[d];
+    reduce_lanes(gb);
+    const double val = lane == 0 ? gb[0] : lane == 1 ? gb[1] : gb[2];
+    if (lane < 3) atomicAdd(grad + 3 * (int64_t)B + lane, val);
+  };
+  derivs(A, (pA - sum) * fs, on);
+  for (int i = 0; i < nkeep; ++i) {
+    int B = 0;
+#pragma unroll
+    for (int q = 0; q < kSsfKeep; ++q)
+      if (q == i) B = kept[q];
+    const double pB = keep[i][lane];
+    derivs(B, pB * fs, pB > kSsfTol);
+  }
+  // Atoms beyond the kept ones (many comparable distances): formed again.
+  for (int k = kover; k < natoms && (!LISTS || __any(on && nbr_d(A, k) <= rmax)); ++k) {
+    const int B = nbr_at(A, k);
+    if (B == A) continue;
+    const double pB = part(B, dist(B));
+    if (__any(pB > kSsfTol)) derivs(B, pB * fs, pB > kSsfTol);
+  }
+  reduce_lanes(gA);
+  const double val = lane == 0 ? gA[0] : lane == 1 ? gA[1] : gA[2];
+  if (lane < 3) atomicAdd(grad + 3 * (int64_t)A + lane, val);
+}
+
+// The gradient's kGradCopies partial sums, added in order.
+__global__ __launch_bounds__(256) void k_grad_sum(int n, int64_t gstride,
+                                                  const double* __restrict__ part,
+                                                  double* __restrict__ grad) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  double s = 0.;
+#pragma unroll 16
+  for (int c = 0; c < kGradCopies; ++c) s += part[c * gstride + i];
+  grad[i] = s;
 }
 
 // ---- launchers ------------------------------------------------------------------
@@ -922,43 +861,43 @@ int launch_plane_product(const CtxView& v, const WorkRange& r, int in_pl, int ou
 }
 
 int launch_grad_contract(const CtxView& v, const WorkRange& r, int gga,
-                         const int32_t* shell_atom, const double* coef, int weight_derivs,
-                         double* grad, int x_pl, int y_pl, int lmax) {
-  if (r.n == 0) return XCQ_SUCCESS;
-  auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3((unsigned)r.n), dim3(256), 0, v.stream, v.work + r.off,
-                       v.tasks, v.shells, v.shell_list, v.lsh, shell_atom, v.px, v.py, v.pz,
-                       static_cast<const double*>(v.scratch), coef, weight_derivs, grad, x_pl,
-                       y_pl);
-  };
-  if (lmax <= 3) gga ? go(k_grad_contract<true, 3>) : go(k_grad_contract<false, 3>);
-  else gga ? go(k_grad_contract<true, 4>) : go(k_grad_contract<false, 4>);
-  XCQ_HIP(hipGetLastError());
-  return XCQ_SUCCESS;
-}
-
-int launch_grad_contract_uks(const CtxView& v, const WorkRange& r, int gga,
-                             const int32_t* shell_atom, const double* coef_s,
-                             const double* coef_z, int weight_derivs, double* grad, int lmax) {
+                         const int32_t* shell_atom, const double* coef_s, const double* coef_z,
+                         int weight_derivs, double* part, int64_t gstride, int x_pl, int y_pl,
+                         int lmax) {
   if (r.n == 0) return XCQ_SUCCESS;
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, dim3((unsigned)r.n), dim3(256), 0, v.stream, v.work + r.off,
                        v.tasks, v.shells, v.shell_list, v.lsh, shell_atom, v.px, v.py, v.pz,
                        static_cast<const double*>(v.scratch), coef_s, coef_z, weight_derivs,
-                       grad);
+                       part, gstride, x_pl, y_pl);
   };
-  if (lmax <= 3) gga ? go(k_grad_contract_uks<true, 3>) : go(k_grad_contract_uks<false, 3>);
-  else gga ? go(k_grad_contract_uks<true, 4>) : go(k_grad_contract_uks<false, 4>);
+  auto pick = [&](auto LM) {
+    constexpr int L = decltype(LM)::value;
+    if (!coef_z) gga ? go(k_grad_contract<true, L, 1>) : go(k_grad_contract<false, L, 1>);
+    else gga ? go(k_grad_contract<true, L, 2>) : go(k_grad_contract<false, L, 2>);
+  };
+  if (lmax <= 3) pick(std::integral_constant<int, 3>{});
+  else pick(std::integral_constant<int, 4>{});
   XCQ_HIP(hipGetLastError());
   return XCQ_SUCCESS;
 }
 
 int launch_ssf_grad(const CtxView& v, const WorkRange& r, int natoms, const double* xyz,
-                    const double* dnear, const double* wf, double* grad,
+                    const double* dnear, const double* wf, double* part, int64_t gstride,
                     const int32_t* nbr_idx, const double* nbr_r) {
   if (r.n == 0) return XCQ_SUCCESS;
-  hipLaunchKernelGGL(k_ssf_grad, dim3((unsigned)r.n), dim3(64), 0, v.stream, v.work + r.off,
-                     v.tasks, v.px, v.py, v.pz, natoms, xyz, dnear, wf, grad, nbr_idx, nbr_r);
+  hipLaunchKernelGGL(nbr_idx ? k_ssf_grad<true> : k_ssf_grad<false>, dim3((unsigned)r.n),
+                     dim3(64), 0, v.stream, v.work + r.off, v.tasks, v.px, v.py, v.pz, natoms,
+                     xyz, dnear, wf, part, gstride, nbr_idx, nbr_r);
+  XCQ_HIP(hipGetLastError());
+  return XCQ_SUCCESS;
+}
+
+int launch_grad_sum(hipStream_t s, int natoms, const double* part, int64_t gstride,
+                    double* grad) {
+  const int n = 3 * natoms;
+  hipLaunchKernelGGL(k_grad_sum, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, gstride,
+                     part, grad);
   XCQ_HIP(hipGetLastError());
   return XCQ_SUCCESS;
 }

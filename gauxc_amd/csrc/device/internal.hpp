@@ -311,23 +311,31 @@ int launch_grad_points(const CtxView& v, const WorkRange& r, int func, int gga, 
                        double* coef, double* wf);
 int launch_plane_product(const CtxView& v, const WorkRange& r, int in_pl, int out_pl,
                          const double* P = nullptr, double fac = 2.0, int accumulate = 0);
+// The gradient's contributions go to kGradCopies partial sums (workgroup i to
+// i % kGradCopies) that k_grad_sum adds up: one atomic target per component
+// is what the contraction of 13 waters waited for (4.4 ms).  As the copies
+// are a multiple of the 8 XCDs, to which workgroups go in turn, each copy is
+// written from one XCD.
+constexpr int kGradCopies = 64;
+inline int64_t grad_stride(int natoms) { return (3 * (int64_t)natoms + 15) / 16 * 16; }
+// Y in plane y_pl; X in x_pl, or (UKS: coef_z given) X_N in x_pl and X_Z in
+// x_pl + 1.
 int launch_grad_contract(const CtxView& v, const WorkRange& r, int gga,
-                         const int32_t* shell_atom, const double* coef, int weight_derivs,
-                         double* grad, int x_pl, int y_pl, int lmax);
+                         const int32_t* shell_atom, const double* coef_s, const double* coef_z,
+                         int weight_derivs, double* part, int64_t gstride, int x_pl, int y_pl,
+                         int lmax);
 // Za = a B + c . grad B from [block][4][64] coefficients into plane pl_s
 // (and, with coef_z, a second one into pl_z; planes 3 and 4 only).  UKS:
-// coefficients written over the P_s / P_z sums; contraction with Y
-// (plane 1), X_N (2), X_Z (3).
+// coefficients written over the P_s / P_z sums.
 int launch_grad_points_uks(const CtxView& v, const WorkRange& r, int func, int gga, double* ds,
                            double* dz, double* wf);
 int launch_grad_zpair(const CtxView& v, const WorkRange& r, int gga, const double* coef_s,
                       const double* coef_z, int pl_s, int pl_z);
-int launch_grad_contract_uks(const CtxView& v, const WorkRange& r, int gga,
-                             const int32_t* shell_atom, const double* coef_s,
-                             const double* coef_z, int weight_derivs, double* grad, int lmax);
 int launch_ssf_grad(const CtxView& v, const WorkRange& r, int natoms, const double* xyz,
-                    const double* dnear, const double* wf, double* grad,
-                    const int32_t* nbr_idx = nullptr, const double* nbr_r = nullptr);
+                    const double* dnear, const double* wf, double* part, int64_t gstride,
+                    const int32_t* nbr_idx, const double* nbr_r);
+int launch_grad_sum(hipStream_t s, int natoms, const double* part, int64_t gstride,
+                    double* grad);
 int launch_z_from_coeffs(const CtxView& v, const WorkRange& r, int precision, int gga,
                          const double* coef, unsigned* tmax);
 // B^T Z + Z^T B of a chunk with the VXC scatter-add.
