@@ -21,7 +21,8 @@
 // Basis evaluation mode (template argument INSTAGE): 0 reads B and grad B
 // from the planes the collocation stage stored, and so does the Z launch
 // (k_z_from_coeffs); 3 evaluates them at the block's points from the shell
-// parameters, as does k_z_in_stage (collocation.hip).
+// parameters, as does k_z_in_stage (collocation.hip).  kProductOnly stops at
+// the product, of any stored plane, for the EXC gradient.
 #include "internal.hpp"
 #include "functional.hpp"
 #include "shell_eval.hpp"
@@ -203,7 +204,13 @@ __device__ __forceinline__ void write_z(const DevTask& t, int m0, int tid, doubl
 // spill: 4.9 and 96).  The kernel it replaces, with tiles of 32, 64 and 128
 // functions padded to, a ring of direct-to-LDS dword loads and the
 // functional inside, took 6.6 and 100 ms.
+//
+// INSTAGE = kProductOnly: X = fac P_sub B, with any stored plane for B, goes to
+// plane x_plane (is added to it with accumulate) and nothing else is done (13
+// waters: 1.35 ms; on 64-function padded tiles with both operands through LDS
+// 2.0).
 constexpr int kDensTile = 64;  // functions per tile
+constexpr int kProductOnly = -1;
 
 // Shells of one tile (at most one more than its functions, and one for each
 // of the four waves' loops to end on), staged in LDS while the tile's
@@ -309,7 +316,7 @@ template <typename T, bool GGA, int INSTAGE>
 __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void k_density(
     QueueArgs qa, const DevTask* __restrict__ tasks, const int32_t* __restrict__ bfmap,
     const T* __restrict__ Pall, T* __restrict__ scratch, double fac, ShellArgs sa,
-    double* __restrict__ dens_out, int x_plane) {
+    double* __restrict__ dens_out, int x_plane, int b_plane, int accumulate) {
   constexpr bool kF32 = sizeof(T) == 4;
   constexpr int kBI = kDensTile / 16;
   constexpr int kK = kF32 ? 32 : 16;      // K rows per stage
@@ -317,6 +324,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void k_density(
   constexpr int kLd = kDensTile + 16;     // stage row: four K rows hit distinct banks
   constexpr int kStage = kK * kLd;
   constexpr int kXtD = kDensTile * kXLd;  // X^T in doubles
+  constexpr bool kFold = INSTAGE != kProductOnly, kEval = INSTAGE > 0;
   static_assert(2 * kStage * sizeof(T) <= kXtD * 8 && 4 * 64 * 4 <= kXtD, "LDS is shared");
   // P_sub stages [buf][k][function]; X^T and the per-point partials take
   // their place.
@@ -348,7 +356,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void k_density(
     // finite values, which meet zero X) and this wave's density partials; on
     // stored planes the partials of the lane's column.
     double rx = 0., ry = 0., rz = 0.;
-    if constexpr (INSTAGE != 0) {
+    if constexpr (kEval) {
       const int pl = min(m0 + lane, t.npts - 1);
       rx = sa.px[t.pt_off + pl];
       ry = sa.py[t.pt_off + pl];
@@ -357,7 +365,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void k_density(
     int s_cur = 0;
     double part[4] = {0., 0., 0., 0.};
     const auto rsB = __builtin_amdgcn_make_buffer_rsrc(
-        Bm, 0, (int)((unsigned)plane * (unsigned)sizeof(T)), 0x00020000);
+        Bm + (kFold ? 0 : (int64_t)b_plane * plane), 0, (int)((unsigned)plane * (unsigned)sizeof(T)), 0x00020000);
     auto ldB = [&](int vo, int so) -> T {  // element offsets: lane, scalar
       if constexpr (kF32)
         return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(rsB, vo * 4, so * 4, 0));
@@ -398,7 +406,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void k_density(
         }
       };
       load(0);
-      if constexpr (INSTAGE != 0) {
+      if constexpr (kEval) {
         fs.load(t, sa, s_cur, nhi, tid);
       }
       v4d acc[kBI];
@@ -463,10 +471,13 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void k_density(
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const int row = n0 + 16 * i + arow(r);
-            if (row < nhi) xo[(int64_t)row * ld] = (T)acc[i][r];
+            if (row < nhi) {
+              T* o = xo + (int64_t)row * ld;
+              *o = !kFold && accumulate ? (T)(*o + acc[i][r]) : (T)acc[i][r];
+            }
           }
       }
-      if constexpr (INSTAGE != 0) {
+      if constexpr (kEval) {
         __syncthreads();  // every wave is done with the stages
 #pragma unroll
         for (int i = 0; i < kBI; ++i)
@@ -476,7 +487,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void k_density(
         __syncthreads();
         fold_staged<GGA, kF32, kXLd>(sa, fs, n0, nhi, wave, 4, lds + lane, rx, ry, rz, part);
         s_cur = uni(fs.next);
-      } else {
+      } else if constexpr (kFold) {
         const unsigned short* lo = lo_plane(Bm, plane);
 #pragma unroll
         for (int i = 0; i < kBI; ++i) {
@@ -498,8 +509,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void k_density(
       }
       __syncthreads();  // the next tile's first stage write is safe
     }
-    constexpr int ND = INSTAGE != 0 ? 4 : 1;
-    if constexpr (INSTAGE != 0) {
+    if constexpr (!kFold) continue;
+    constexpr int ND = kEval ? 4 : 1;
+    if constexpr (kEval) {
 #pragma unroll
       for (int c = 0; c < 4; ++c) dens[wave][lane][c] = part[c];
     } else {
@@ -1085,7 +1097,13 @@ int launch_density(const CtxView& v, const Chunk& c, int precision, int gga, dou
   auto go = [&](auto kern, const WorkRange& r, const auto* P, auto* scr) {
     if (r.n)
       hipLaunchKernelGGL(kern, dim3(grid_of(r)), dim3(256), 0, v.stream, queue_args(v, r), v.tasks,
-                         v.bfmap, P, scr, fac, sa, dens_out, x_plane);
+                         v.bfmap, P, scr, fac, sa, dens_out, x_plane, 0, 0);
+  };
+  auto go_wide = [&](auto kern, const auto* P, auto* scr) {
+    if (c.dens_pair.n)
+      hipLaunchKernelGGL(kern, dim3(grid_of(c.dens_pair)), dim3(256), 0, v.stream,
+                         queue_args(v, c.dens_pair), v.tasks, v.bfmap, P, scr, fac, sa, dens_out,
+                         x_plane);
   };
   // Classes [0, n): one launch, but for queues, which each class has of its
   // own.  The classes' items lie one after the other, the highest first.
@@ -1109,8 +1127,7 @@ int launch_density(const CtxView& v, const Chunk& c, int precision, int gga, dou
       return;
     }
     if constexpr (sizeof(T) == 8)
-      gga ? go(k_density_wide<true>, c.dens_pair, P, scr)
-          : go(k_density_wide<false>, c.dens_pair, P, scr);
+      gga ? go_wide(k_density_wide<true>, P, scr) : go_wide(k_density_wide<false>, P, scr);
     constexpr int n = sizeof(T) == 8 ? 3 : 4;
     gga ? run(k_density<T, true, 3>, P, scr, n) : run(k_density<T, false, 3>, P, scr, n);
   };
@@ -1118,6 +1135,17 @@ int launch_density(const CtxView& v, const Chunk& c, int precision, int gga, dou
     pick(P_override ? P_override : v.P, static_cast<double*>(v.scratch));
   else
     pick(v.Pf32, static_cast<float*>(v.scratch));
+  XCQ_HIP(hipGetLastError());
+  return XCQ_SUCCESS;
+}
+
+int launch_plane_product(const CtxView& v, const WorkRange& r, int in_pl, int out_pl,
+                         const double* P, double fac, int accumulate) {
+  if (r.n == 0) return XCQ_SUCCESS;
+  hipLaunchKernelGGL((k_density<double, false, kProductOnly>), dim3((unsigned)r.n), dim3(256), 0,
+                     v.stream, queue_args(v, r), v.tasks, v.bfmap, P ? P : v.P,
+                     static_cast<double*>(v.scratch), fac, ShellArgs{}, nullptr, out_pl, in_pl,
+                     accumulate);
   XCQ_HIP(hipGetLastError());
   return XCQ_SUCCESS;
 }
