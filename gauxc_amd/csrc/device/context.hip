@@ -364,7 +364,6 @@ double heur_dens_item(const DevTask& d) {
   const double rows = std::ceil(d.nbe / 16.) * 16.;
   return (double)kPtBlock * rows * d.nbe;
 }
-double heur_syr2k_item(const DevTask& d) { return (double)d.npts_pad * d.nt_s * d.nt_s; }
 
 // Rebuild the work lists and queue tables of every chunk from the current
 // tile policy and schedule, and upload them.
@@ -386,7 +385,6 @@ int build_work_lists(xcq_context_s* ctx) {
                  : d.nbe >= std::max(wide, 65) && d.npts > kPtBlock         ? 3
                  : d.nbe <= ctx->dens_hiocc_max_nbe                         ? 1
                                                                             : 2;
-    d.nt_s = d.nbe <= ctx->syr2k32_max_nbe ? 32 : 64;
   }
   auto finish_range = [&](WorkRange& r, const std::vector<double>& cost) {
     r.n = (int64_t)W.size() - r.off;
@@ -454,71 +452,60 @@ int build_work_lists(xcq_context_s* ctx) {
     c.coll.off = c.dens[3].off;
     c.coll.n = c.dens[0].n + c.dens[1].n + c.dens[2].n + c.dens[3].n;
     c.coll.nq = 0;
-    for (int v = 0; v < 2; ++v) {  // SYR2K tiles
-      const int nt = v == 0 ? 32 : 64;
-      c.syr2k[v].off = (int64_t)W.size();
+    // SYR2K: regions and point slices.  A slice is as long as gives the chunk
+    // one item per resident workgroup (3 per CU), between 256 points (below
+    // that storing and summing slices costs what the shorter chain saves: 120
+    // functions, FP64 0.104 ms at 256, 0.142 at 64) and 4,096 (larger chunks
+    // start such chains first and end them before the rest; 1,024 to 8,192
+    // time the same on 24 and 150 waters).
+    c.syr_slots = 0;
+    auto syr2k = [&](auto MX) {
+      constexpr bool kMx = decltype(MX)::value;
+      constexpr int64_t kSyrItems = 768;
+      constexpr int kSliceMin = 256, kSliceMax = 4096;
+      auto regions = [&](const DevTask& d, auto&& f) {
+        const int nb = (d.nbe + 15) / 16;
+        const int ni = syr_row_groups<kMx>(nb), nj = syr_col_groups<kMx>(nb);
+        for (int it = 0; it < ni; ++it)
+          for (int jt = 0; jt < nj; ++jt)  // with blocks below the diagonal
+            if ((it + 1) * nb / ni > jt * nb / nj) f(it | jt << 16);
+      };
+      int64_t region_points = 0;
+      for (int32_t i = c.task_begin; i < c.task_end; ++i) {
+        int64_t n = 0;
+        regions(ctx->h_tasks[i], [&](int) { ++n; });
+        region_points += n * ctx->h_tasks[i].npts;
+      }
+      const int32_t kslice =
+          (int32_t)std::clamp<int64_t>(region_points / kSyrItems, kSliceMin, kSliceMax);
+      std::vector<WorkItem> sums;
       std::vector<double> cost;
+      WorkRange &r = c.syr2k[kMx], &rs = c.syr2k_sum[kMx];
+      r.off = (int64_t)W.size();
+      int64_t slots = 0;
       for (int32_t i = c.task_begin; i < c.task_end; ++i) {
         const DevTask& d = ctx->h_tasks[i];
-        if (d.nt_s != nt) continue;
-        const int nt_tiles = (d.nbe + nt - 1) / nt;
-        const int npairs = nt_tiles * (nt_tiles + 1) / 2;
-        const double ci = have_cost ? ctx->cost_s[i] / npairs : heur_syr2k_item(d);
-        for (int it = 0; it < nt_tiles; ++it)
-          for (int jt = 0; jt <= it; ++jt) {
-            W.push_back(WorkItem{i, it, jt, 0});
-            if (queued) cost.push_back(ci);
-          }
+        if (d.npts == 0) continue;
+        const int32_t ns = std::min((d.npts + kslice - 1) / kslice, 0x7fff);
+        const size_t first = W.size();
+        regions(d, [&](int32_t rg) {
+          if (ns > 1) sums.push_back(WorkItem{i, rg, ns, (int32_t)slots});
+          for (int32_t sl = 0; sl < ns; ++sl)
+            W.push_back(WorkItem{i, rg, sl | ns << 16, ns > 1 ? (int32_t)slots++ : 0});
+        });
+        const size_t n = W.size() - first;
+        if (!queued) continue;
+        cost.insert(cost.end(), n, have_cost ? ctx->cost_s[i] / std::max<size_t>(n, 1)
+                                             : (double)d.npts / ns);
       }
-      finish_range(c.syr2k[v], cost);
-    }
-    // FP64 SYR2K: regions and point slices.  A slice is as long as gives the
-    // chunk one item per resident workgroup (3 per CU), between 256 points
-    // (below that storing and summing slices costs what the shorter chain
-    // saves: 120 functions, 0.104 ms at 256, 0.142 at 64) and 4,096 (larger
-    // chunks start such chains first and end them before the rest; 1,024
-    // to 8,192 time the same on 24 and 150 waters).
-    constexpr int64_t kSyrItems = 768;
-    constexpr int kSliceMin = 256, kSliceMax = 4096;
-    auto syr_regions = [&](const DevTask& d, auto&& f) {
-      const int nb = (d.nbe + 15) / 16;
-      const int ni = syr_row_groups(nb), nj = syr_col_groups(nb);
-      for (int it = 0; it < ni; ++it)
-        for (int jt = 0; jt < nj; ++jt)
-          if ((it + 1) * nb / ni > jt * nb / nj) f(it | jt << 16);  // blocks below the diagonal
+      finish_range(r, cost);
+      rs.off = (int64_t)W.size();
+      rs.n = (int64_t)sums.size();
+      W.insert(W.end(), sums.begin(), sums.end());
+      c.syr_slots = std::max(c.syr_slots, slots);
     };
-    int64_t region_points = 0;
-    for (int32_t i = c.task_begin; i < c.task_end; ++i) {
-      int64_t n = 0;
-      syr_regions(ctx->h_tasks[i], [&](int) { ++n; });
-      region_points += n * ctx->h_tasks[i].npts;
-    }
-    const int32_t kslice =
-        (int32_t)std::clamp<int64_t>(region_points / kSyrItems, kSliceMin, kSliceMax);
-    std::vector<WorkItem> sums;
-    std::vector<double> cost;
-    c.syr2k_f64.off = (int64_t)W.size();
-    c.syr_slots = 0;
-    for (int32_t i = c.task_begin; i < c.task_end; ++i) {
-      const DevTask& d = ctx->h_tasks[i];
-      if (d.npts == 0) continue;
-      const int32_t ns = std::min((d.npts + kslice - 1) / kslice, 0x7fff);
-      const size_t first = W.size();
-      syr_regions(d, [&](int32_t rg) {
-        if (ns > 1) sums.push_back(WorkItem{i, rg, ns, (int32_t)c.syr_slots});
-        for (int32_t sl = 0; sl < ns; ++sl)
-          W.push_back(WorkItem{i, rg, sl | ns << 16,
-                               ns > 1 ? (int32_t)c.syr_slots++ : 0});
-      });
-      const size_t n = W.size() - first;
-      if (!queued) continue;
-      cost.insert(cost.end(), n, have_cost ? ctx->cost_s[i] / std::max<size_t>(n, 1)
-                                           : (double)d.npts / ns);
-    }
-    finish_range(c.syr2k_f64, cost);
-    c.syr2k_sum.off = (int64_t)W.size();
-    c.syr2k_sum.n = (int64_t)sums.size();
-    W.insert(W.end(), sums.begin(), sums.end());
+    syr2k(std::false_type{});
+    syr2k(std::true_type{});
   }
   dfree(ctx->d_work);
   dfree(ctx->d_qoff);
@@ -541,7 +528,7 @@ int build_work_lists(xcq_context_s* ctx) {
   return XCQ_SUCCESS;
 }
 
-// The slice buffer of the FP64 SYR2K, sized for the chunk that needs most
+// The slice buffer of the SYR2K, sized for the chunk that needs most
 // (freed with the work lists that say how much).
 int ensure_syr_part(xcq_context_s* ctx) {
   if (ctx->d_syr_part) return XCQ_SUCCESS;
@@ -613,13 +600,8 @@ int enqueue_pipeline(xcq_context_s* ctx, int func, int precision, int want_vxc, 
       XCQ_HIP(rec(ev[8]));
       if ((rc = launch_syr2k(v, c, precision))) return rc;
       XCQ_HIP(rec(ev[9]));
-      if (precision == XCQ_PREC_FP64) {
-        launches += 1;
-        items += c.syr2k_f64.n;
-      } else {
-        launches += 2;
-        items += c.syr2k[0].n + c.syr2k[1].n;
-      }
+      launches += 1;
+      items += c.syr2k[precision != XCQ_PREC_FP64].n;
     }
   }
   const int32_t nmol = (int32_t)ctx->mols.size();
@@ -681,7 +663,7 @@ int run_pipeline(xcq_context_s* ctx, int func, int precision, int want_vxc) {
     if (rc) return rc;
     ctx->drop_graph();
   }
-  if (want_vxc && precision == XCQ_PREC_FP64)
+  if (want_vxc)
     if (int rc = ensure_syr_part(ctx)) return rc;
   ctx->last_vxc_eval = want_vxc;
   if (!ctx->use_graph) {
@@ -1267,10 +1249,7 @@ int xcq_task_times(xcq_context ctx, double* dens_us, double* syr2k_us) {
     for (int v = 0; v < (pairs ? 3 : 4); ++v) add(c.dens[v], dens_us);
     if (pairs) add(c.dens_pair, dens_us);
     // The list the last evaluation ran (the other keeps older stamps).
-    if (ctx->last_mixed)
-      for (int v = 0; v < 2; ++v) add(c.syr2k[v], syr2k_us);
-    else
-      add(c.syr2k_f64, syr2k_us);
+    add(c.syr2k[ctx->last_mixed], syr2k_us);
   }
   return XCQ_SUCCESS;
 }

@@ -10,7 +10,7 @@
 // A[l%16][l/16] and B[l/16][l%16]; accumulator register r of lane l is
 // D[4*r + l/16][l%16] (rows interleave across the four 16-lane groups,
 // unlike the FP32-output MFMAs whose register r holds row 4*(l/16) + r).
-#include "internal.hpp"
+#include "syr2k.hpp"
 
 #include <type_traits>
 
@@ -20,41 +20,6 @@ using v4d = double __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ v4d mfma_f64(double a, double b, v4d c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-
-// Region of an FP64 SYR2K work item: blocks of 16 functions, rows [r0, r1)
-// and columns [c0, c1), without the rows above and the columns right of its
-// part on or below the diagonal, so c0 <= r0 and c1 <= r1.
-struct SyrRegion {
-  int r0, r1, c0, c1;
-};
-__device__ __forceinline__ SyrRegion syr_region(const DevTask& t, int a, int b) {
-  const int nb = (t.nbe + 15) / 16;
-  const int ni = syr_row_groups(nb), nj = syr_col_groups(nb);
-  const int r1 = (a + 1) * nb / ni, c0 = b * nb / nj;
-  return SyrRegion{max(a * nb / ni, c0), r1, c0, min((b + 1) * nb / nj, r1)};
-}
-
-// The region's wanted blocks, bit (row - r0) * (c1 - c0) + column - c0: on or
-// below the diagonal, and not negligible by the bound table, |sum_p B_pi
-// Z_pj| <= npts max|B_i| max|Z_j| (1.01 covers the rounding of the stored
-// maxima and of the products).  Lane l of a wave decides bit l (a region has
-// at most 64 blocks).
-__device__ __forceinline__ uint64_t syr_mask(const DevTask& t, const SyrRegion& s, int lane,
-                                             const unsigned* tmax, double drop) {
-  const int nc = s.c1 - s.c0;
-  const int rb = s.r0 + lane / nc, cb = s.c0 + lane % nc;
-  bool want = rb < s.r1 && rb >= cb;
-  if (want && tmax) {
-    const unsigned* tm = tmax + 2 * t.tmax_off;
-    const int gi = 16 * rb / kGran, gj = 16 * cb / kGran;
-    const double bound =
-        1.01 * (double)t.npts *
-        ((double)__uint_as_float(tm[2 * gi]) * (double)__uint_as_float(tm[2 * gj + 1]) +
-         (double)__uint_as_float(tm[2 * gi + 1]) * (double)__uint_as_float(tm[2 * gj]));
-    want = !(bound < drop);
-  }
-  return __builtin_amdgcn_ballot_w64(want);
 }
 
 // One 1 KiB fragment from memory into LDS: lane l's 16 bytes at base + off
@@ -106,6 +71,7 @@ __global__ __launch_bounds__(256, 3) void k_syr2k(QueueArgs qa, const DevTask* _
                                                   const unsigned* __restrict__ tmax,
                                                   double* __restrict__ part) {
   typedef double v2d __attribute__((ext_vector_type(2)));
+  constexpr int kSyrSlots = kSyr<false>.slots, kSyrStaged = kSyr<false>.staged();
   constexpr int kStage = 2 * kSyrStaged * 128;  // doubles per stage
   __shared__ __attribute__((aligned(16))) double stage[2 * kStage];
   const int tid = threadIdx.x, lane = tid & 63, lf = lane & 15, lq = lane >> 4;
@@ -116,7 +82,7 @@ __global__ __launch_bounds__(256, 3) void k_syr2k(QueueArgs qa, const DevTask* _
     const WorkItem wi = qa.items[uniform64(it)];
     const DevTask t = tasks[wi.task];
     const int nbe = t.nbe, ld = t.npts_pad;
-    const SyrRegion rg = syr_region(t, wi.a & 0xffff, wi.a >> 16);
+    const SyrRegion rg = syr_region<false>(t, wi.a & 0xffff, wi.a >> 16);
     const int n8 = (t.npts + 7) / 8, sl = wi.b & 0xffff, ns = wi.b >> 16;
     const int s0 = (int)((int64_t)sl * n8 / ns), s1 = (int)((int64_t)(sl + 1) * n8 / ns);
     const uint64_t mask = syr_mask(t, rg, lane, tmax, drop);
@@ -250,6 +216,7 @@ __global__ __launch_bounds__(256, 3) void k_syr2k(QueueArgs qa, const DevTask* _
 // Sums the slices of one block of a region in order and adds it to VXC.
 // Item: task, region (as above), number of slices, first slice's place in
 // part; blockIdx.y is the rank of the block among the region's wanted ones.
+template <bool MX>
 __global__ __launch_bounds__(256) void k_syr2k_reduce(const WorkItem* __restrict__ items,
                                                       const DevTask* __restrict__ tasks,
                                                       const int32_t* __restrict__ bfmap,
@@ -259,42 +226,41 @@ __global__ __launch_bounds__(256) void k_syr2k_reduce(const WorkItem* __restrict
   const WorkItem wi = items[blockIdx.x];
   const DevTask t = tasks[wi.task];
   const int tid = threadIdx.x, lane = tid & 63, rank = blockIdx.y;
-  const SyrRegion rg = syr_region(t, wi.a & 0xffff, wi.a >> 16);
-  const uint64_t mask = syr_mask(t, rg, lane, tmax, drop);
-  if (rank >= __popcll(mask)) return;
+  const SyrRegion rg = syr_region<MX>(t, wi.a & 0xffff, wi.a >> 16);
+  uint64_t m = syr_mask(t, rg, lane, tmax, drop);
+  if (rank >= __popcll(m)) return;
+  for (int k = 0; k < rank; ++k) m &= m - 1;
+  const int k = __ffsll((unsigned long long)m) - 1, nc = rg.c1 - rg.c0;  // the rank-th one
+  const int rb = rg.r0 + k / nc, cb = rg.c0 + k % nc;
   const double* src = part + ((int64_t)wi.c * kSyrBlocks + rank) * 256 + tid;
   double v = 0.;
 #pragma unroll 8
   for (int s = 0; s < wi.b; ++s) v += src[(int64_t)s * kSyrBlocks * 256];
-  // The rank-th wanted block.
-  uint64_t m = mask;
-  for (int k = 0; k < rank; ++k) m &= m - 1;
-  const int k = __ffsll((unsigned long long)m) - 1, nc = rg.c1 - rg.c0;
-  const int i = 16 * (rg.r0 + k / nc) + 4 * (tid >> 6) + (lane >> 4);
-  const int j = 16 * (rg.c0 + k % nc) + (lane & 15);
+  const int r = tid >> 6, lq = lane >> 4;
+  const int i = 16 * rb + (MX ? 4 * lq + r : 4 * r + lq), j = 16 * cb + (lane & 15);
   const int32_t* bf = bfmap + t.bf_off;
   if (i < t.nbe && i >= j && !(fabs(v) < drop))
     atomicAdd(vxc_all + t.p_off + (int64_t)bf[i] * t.ldp + bf[j], v);
 }
 
-int launch_syr2k_mixed(const CtxView& v, const WorkRange& r, int nt);
+int launch_syr2k_mixed(const CtxView& v, const WorkRange& r, const unsigned* tm);
 
 int launch_syr2k(const CtxView& v, const Chunk& c, int precision) {
-  if (precision != XCQ_PREC_FP64) {
-    for (int k = 0; k < 2; ++k)
-      if (int rc = launch_syr2k_mixed(v, c.syr2k[k], k == 0 ? 32 : 64)) return rc;
-    return XCQ_SUCCESS;
-  }
-  const WorkRange& r = c.syr2k_f64;
+  const int mx = precision != XCQ_PREC_FP64;
+  const WorkRange &r = c.syr2k[mx], &sum = c.syr2k_sum[mx];
   if (r.n == 0) return XCQ_SUCCESS;
   const unsigned* tm = v.vxc_drop > 0.0 ? v.tmax : nullptr;
-  hipLaunchKernelGGL(k_syr2k, dim3(grid_of(r)), dim3(256), 0, v.stream, queue_args(v, r), v.tasks,
-                     v.bfmap, static_cast<const double*>(v.scratch), v.vxc, v.vxc_drop, tm,
-                     v.syr_part);
-  if (c.syr2k_sum.n)
-    hipLaunchKernelGGL(k_syr2k_reduce, dim3((unsigned)c.syr2k_sum.n, kSyrBlocks), dim3(256), 0,
-                       v.stream, v.work + c.syr2k_sum.off, v.tasks, v.bfmap, v.syr_part, v.vxc, v.vxc_drop,
-                       tm);
+  if (mx) {
+    if (int rc = launch_syr2k_mixed(v, r, tm)) return rc;
+  } else {
+    hipLaunchKernelGGL(k_syr2k, dim3(grid_of(r)), dim3(256), 0, v.stream, queue_args(v, r),
+                       v.tasks, v.bfmap, static_cast<const double*>(v.scratch), v.vxc, v.vxc_drop,
+                       tm, v.syr_part);
+  }
+  if (sum.n)
+    hipLaunchKernelGGL(mx ? k_syr2k_reduce<true> : k_syr2k_reduce<false>,
+                       dim3((unsigned)sum.n, mx ? kSyr<true>.blocks() : kSyr<false>.blocks()), dim3(256), 0, v.stream,
+                       v.work + sum.off, v.tasks, v.bfmap, v.syr_part, v.vxc, v.vxc_drop, tm);
   XCQ_HIP(hipGetLastError());
   return XCQ_SUCCESS;
 }

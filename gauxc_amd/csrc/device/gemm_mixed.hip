@@ -6,10 +6,9 @@
 //    stored as FP32 plus a bfloat16 residual (plane 5 of the task scratch),
 //    about 32 significant bits: FP32 rounding of B was the largest error
 //    term of the EXC/VXC budget.
-//  * P is held as three bfloat16 slices p0 + p1 + p2 (24 significant bits).
-//    Each FP32 operand element is split on the fly into three bfloat16
-//    slices (exact: 3 x 8 bits cover the FP32 significand); B's residual is
-//    its fourth slice b3.
+//  * For B^T Z each FP32 operand element is split on the fly into three
+//    bfloat16 slices (exact: 3 x 8 bits cover the FP32 significand); B's
+//    residual is its fourth slice b3.
 //  * A product is formed from the leading slice product (one MFMA, its own
 //    FP32 accumulator, so the large partial sum is rounded once per K block)
 //    and six correction products (b0 z1, b1 z0, b0 z2, b1 z1, b2 z0, b3 z0;
@@ -19,12 +18,12 @@
 //    2e4 in the B^T Z product).
 //  * Densities, the functional, EXC/NEL and VXC accumulate in FP64.
 //
-// Kernels mirror the FP64 ones (gemm_fp64.hip; the density stage is in
-// density.hip): k_syr2k_mx fuses the scatter-add into VXC into the
-// B^T Z + Z^T B epilogue.  Operand layout of the MFMA (measured on gfx950): lane l holds
+// The regions of the B^T Z + Z^T B product are those of the FP64 kernel, with
+// limits of their own (syr2k.hpp); the density stage is in density.hip.
+// Operand layout of the MFMA (measured on gfx950): lane l holds
 // A[l%16][8(l/16) .. 8(l/16)+7] and B[8(l/16) .. +7][l%16]; accumulator
 // register r of lane l is D[4(l/16)+r][l%16].
-#include "internal.hpp"
+#include "syr2k.hpp"
 
 #include <type_traits>
 
@@ -32,14 +31,9 @@ namespace xcq {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
-typedef unsigned short us8 __attribute__((ext_vector_type(8)));
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
 constexpr int kKB = 32;    // K block = MFMA depth
-constexpr int kRow = 40;   // LDS row length in bf16 (32 + 8 pad, 80 B: 16-B aligned)
-
-__device__ __forceinline__ unsigned short bf_bits(__bf16 v) {
-  return __builtin_bit_cast(unsigned short, v);
-}
 
 // Splits two FP32 values into three bfloat16 slices each (round to nearest
 // even at every step, so x = a + b + c exactly); the slices of the pair come
@@ -55,10 +49,6 @@ __device__ __forceinline__ void split3f_pair(f2v x, unsigned& a, unsigned& b, un
   a = __builtin_bit_cast(unsigned, h1);
   b = __builtin_bit_cast(unsigned, h2);
   c = __builtin_bit_cast(unsigned, h3);
-}
-
-__device__ __forceinline__ bf16x8 ldfrag(const unsigned short* p) {
-  return __builtin_bit_cast(bf16x8, *reinterpret_cast<const us8*>(p));
 }
 
 __device__ __forceinline__ v4f mfma_v(bf16x8 a, bf16x8 b, v4f c) {
@@ -84,219 +74,234 @@ __global__ __launch_bounds__(256) void k_P_to_f32(int64_t n, const double* __res
 }
 
 // ---------------------------------------------------------------------------
-// B^T Z + Z^T B with the VXC scatter-add (mirrors k_syr2k of the FP64 path),
-// templated on the function tile NT.  Loader: thread (g = tid & 3,
-// f = tid >> 2) moves points k0+8g..k0+8g+7 of one row (four lanes cover a
-// row's 128 B): for NT = 64 row f of the i and j panels, for NT = 32 row
-// f & 31 of the i panels (f < 32) or of the j panels (f >= 32).  Rows past
-// nbe are read at row nbe-1 and zeroed by a select.
-template <int NT, int PF = 1>
-__global__ __launch_bounds__(256, NT == 32 ? 4 : 2) void k_syr2k_mx(QueueArgs qa,
-                                                  const DevTask* __restrict__ tasks,
-                                                  const int32_t* __restrict__ bfmap,
-                                                  const float* __restrict__ scratch,
-                                                  double* __restrict__ vxc_all, double drop,
-    const unsigned* __restrict__ tmax) {
-  constexpr int BI = NT / 32;
-  __shared__ __attribute__((aligned(16))) unsigned short Bi[4][NT][kRow];
-  __shared__ __attribute__((aligned(16))) unsigned short Zi[3][NT][kRow];
-  __shared__ __attribute__((aligned(16))) unsigned short Bj[4][NT][kRow];
-  __shared__ __attribute__((aligned(16))) unsigned short Zj[3][NT][kRow];
-  const int tid = threadIdx.x, lane = tid & 63;
+// B^T Z + Z^T B with the VXC scatter-add.  One 256-thread workgroup per region
+// (up to 6 x 5 blocks of 16 functions, or a whole task of up to 7) and slice
+// of the task's points, K blocks of 32 points.
+//
+// Per K block the region's blocks are split into bfloat16 slices once (wave w
+// takes blocks w, w + 4, ...; four lanes cover 128 bytes of a row) and staged
+// in LDS as fragments, 1 KiB per block and slice; then each wave multiplies
+// its share of the wanted blocks (below nbe, on or below the diagonal, not
+// negligible; in row order, so that a row's seven fragments stay in registers
+// while its columns pass).  Rows past nbe lie past the end of the plane and
+// are read as zeros by the buffer loads.
+// A fragment's 16 bytes of (function f, points 8q .. 8q + 7) are at unit 16 q +
+// (f ^ 2q), which keeps the loader's writes (lane 4f + q) and the waves' reads
+// (lane 16 q + f) free of bank conflicts.
+//
+// What bounds it: reading B and Z, 10 bytes per function and point.  24 waters
+// miss L2 for 12.4 GB, about what the planes hold, at 3.5 TB/s, with the
+// matrix cores 18% and the vector units 26% busy.  Tiles of 64 functions,
+// padded and with both triangles of the diagonal ones, read and split twice
+// as much: 24 waters 4.7 -> 3.5 ms, 150 waters 58 -> 51 ms.  Regions of 4 x 4
+// blocks take 3.7 and 53 ms, of 4 x 3 at three workgroups per CU 3.9 and 55;
+// blocks in row pairs that share a column's fragments, or fragments loaded a
+// block ahead, spill registers in the K loop (6.5 and 3.9 ms).  The raw
+// operands of the next K block wait in registers; they are local to the loop,
+// so that they are not carried from item to item (18 registers spill, none
+// in the K loops; carried 79).
+// Slices and their order as in the FP64 kernel (k_syr2k).
+__global__ __launch_bounds__(256, 2) void k_syr2k_mx(QueueArgs qa,
+                                                     const DevTask* __restrict__ tasks,
+                                                     const int32_t* __restrict__ bfmap,
+                                                     const float* __restrict__ scratch,
+                                                     double* __restrict__ vxc_all, double drop,
+                                                     const unsigned* __restrict__ tmax,
+                                                     double* __restrict__ part) {
+  constexpr int kSlots = kSyr<true>.slots, kStaged = kSyr<true>.staged();
+  constexpr int kLoads = (kStaged + 3) / 4;
+  __shared__ v4u stage[kStaged * 7 * 64];  // [block][b0 b1 b2 b3 z0 z1 z2][16 q + (f ^ 2q)]
+  const int tid = threadIdx.x, lane = tid & 63, lf = lane & 15, lq = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave & 1, wn = wave >> 1;
-  const int pg = tid & 3, f = tid >> 2;
-  const int frow = NT == 64 ? f : (f & 31);
-  const int kk = 8 * (lane >> 4);
+  const int wf = lane >> 2, wq = lane & 3;               // loader: function, point group
+  const int wpos = 16 * wq + (wf ^ (wq << 1)), rpos = 16 * lq + (lf ^ (lq << 1));
 
   XCQ_FOR_EACH_ITEM(qa, it) {
     const int64_t t0 = qa.tstamp ? wall_clock64() : 0;
-    const WorkItem wi = qa.items[it];
+    const WorkItem wi = qa.items[uniform64(it)];
     const DevTask t = tasks[wi.task];
-    const int i0 = wi.a * NT, j0 = wi.b * NT;
-    const bool diag = wi.a == wi.b;
-    // Tile pairs whose every element would be dropped are skipped whole
-    // (uniform across the workgroup).
-    if (tile_pair_negligible(t, tmax, i0, j0, NT, drop)) {
+    const int nbe = t.nbe, ld = t.npts_pad;
+    const SyrRegion rg = syr_region<true>(t, wi.a & 0xffff, wi.a >> 16);
+    const int n32 = (t.npts + kKB - 1) / kKB, sl = wi.b & 0xffff, ns = wi.b >> 16;
+    const int s0 = (int)((int64_t)sl * n32 / ns), s1 = (int)((int64_t)(sl + 1) * n32 / ns);
+    const uint64_t mask = syr_mask(t, rg, lane, tmax, drop);
+    if (mask == 0) {
       stamp_item(qa, it, t0);
       continue;
     }
-    const int ld = t.npts_pad;
-    const int nbe = t.nbe;
-    const int plane = nbe * ld;
-    const float* Bm = scratch + t.b_off_mx;
-    const float* Zm = Bm + 4 * plane;
-    // bfloat16 residual of the value plane (plane 5, 2 bytes per element)
-    const unsigned short* Lm = reinterpret_cast<const unsigned short*>(Bm + 5 * (int64_t)plane);
-    const int64_t ldv = t.ldp;
-    double* vxc = vxc_all + t.p_off;
-    const int fi = i0 + frow, fj = j0 + frow;
-    const bool ki = fi < nbe, kj = fj < nbe;
-    const int oi = min(fi, nbe - 1) * ld + 8 * pg, oj = min(fj, nbe - 1) * ld + 8 * pg;
-
-    double acc[BI][BI][4];
+    const int count = __popcll(mask);
+    // Staged blocks: the columns, then the rows that are not among them.
+    // Staged block u is function block u + c0, or u + gap past the columns.
+    const int nc = rg.c1 - rg.c0, gap = rg.r0 > rg.c1 ? rg.r0 - rg.c1 : 0;
+    const int nst = rg.r1 - rg.c0 - gap;
+    auto block_of = [&](int u) { return rg.c0 + u + (u < nc ? 0 : gap); };
+    // The wave's blocks: ranks [w count / 4, (w + 1) count / 4) of the mask.
+    int* slots = reinterpret_cast<int*>(stage);
+    __syncthreads();  // the previous item is done with the stage
+    if (wave == 0 && (mask >> lane & 1)) {
+      const int rb = rg.r0 + lane / nc, cb = rg.c0 + lane % nc;
+      const int ur = rb < rg.c1 ? rb - rg.c0 : rb - gap - rg.c0;
+      slots[__popcll(mask & ((uint64_t(1) << lane) - 1))] = ur | (cb - rg.c0) << 8;
+    }
+    __syncthreads();
+    const int b0 = wave * count / 4, n = (wave + 1) * count / 4 - b0;
+    int ur[kSlots], uc[kSlots];  // staged row and column block per slot
 #pragma unroll
-    for (int a = 0; a < BI; ++a)
-#pragma unroll
-      for (int b = 0; b < BI; ++b)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[a][b][r] = 0.;
-
-    // Raw prefetch registers, a ring of PF K blocks (PF = 3 for 32-wide
-    // tiles: two blocks stay in flight while one is staged and multiplied;
-    // 64-wide tiles have no register room for more than one).  The row
-    // masks are applied when staged, so the loads stay in flight across the
-    // matrix instructions.
-    // Panel sides this thread loads: both (i then j) for 64-wide tiles, one
-    // (i for f < 32, j otherwise) for 32-wide ones; the j side is skipped on
-    // diagonal tiles (it equals the i side).
-    constexpr int SIDES = NT == 64 ? 2 : 1;
-    auto side_id = [&](int sd) { return NT == 64 ? sd : (f < 32 ? 0 : 1); };
-    auto side_on = [&](int sd) { return side_id(sd) == 0 || !diag; };
-    float4 pre[PF][SIDES][2][2];  // [slot][side][B, Z][two float4]
-    uint4 prel[PF][SIDES];        // residuals of B (8 bfloat16)
-    auto load = [&](int k0, auto S) {
-      constexpr int sl = decltype(S)::value;
-#pragma unroll
-      for (int sd = 0; sd < SIDES; ++sd) {
-        if (!side_on(sd)) continue;
-        const int o = (side_id(sd) == 0 ? oi : oj) + k0;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          pre[sl][sd][0][h] = *reinterpret_cast<const float4*>(Bm + o + 4 * h);
-          pre[sl][sd][1][h] = *reinterpret_cast<const float4*>(Zm + o + 4 * h);
-        }
-        prel[sl][sd] = *reinterpret_cast<const uint4*>(Lm + o);
-      }
-    };
-    auto stage = [&](const float4 (&v)[2], bool ok, unsigned short (*dst)[NT][kRow]) {
-      const float* pv = reinterpret_cast<const float*>(&v[0]);  // 8 consecutive points
-      uint4 s1, s2, s3;
-      unsigned* w1 = reinterpret_cast<unsigned*>(&s1);
-      unsigned* w2 = reinterpret_cast<unsigned*>(&s2);
-      unsigned* w3 = reinterpret_cast<unsigned*>(&s3);
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        split3f_pair(f2v{ok ? pv[2 * e] : 0.f, ok ? pv[2 * e + 1] : 0.f}, w1[e], w2[e], w3[e]);
-      *reinterpret_cast<uint4*>(&dst[0][frow][pg * 8]) = s1;
-      *reinterpret_cast<uint4*>(&dst[1][frow][pg * 8]) = s2;
-      *reinterpret_cast<uint4*>(&dst[2][frow][pg * 8]) = s3;
-    };
-
-    auto stage_lo = [&](const uint4& l, bool ok, unsigned short (*dst)[NT][kRow]) {
-      *reinterpret_cast<uint4*>(&dst[3][frow][pg * 8]) = ok ? l : make_uint4(0u, 0u, 0u, 0u);
-    };
-
-    // One K block: stage ring slot S, refill it with block k0 + PF * kKB,
-    // multiply.
-    auto step = [&](int k0, auto S) {
-      constexpr int sl = decltype(S)::value;
-#pragma unroll
-      for (int sd = 0; sd < SIDES; ++sd) {
-        if (!side_on(sd)) continue;
-        const bool i_side = side_id(sd) == 0;
-        const bool ok = i_side ? ki : kj;
-        unsigned short(*db)[NT][kRow] = i_side ? Bi : Bj;
-        unsigned short(*dz)[NT][kRow] = i_side ? Zi : Zj;
-        stage(pre[sl][sd][0], ok, db);
-        stage_lo(prel[sl][sd], ok, db);
-        stage(pre[sl][sd][1], ok, dz);
-      }
-      __syncthreads();
-      if (k0 + PF * kKB < ld) load(k0 + PF * kKB, S);
-      unsigned short(*BJ)[NT][kRow] = diag ? Bi : Bj;
-      unsigned short(*ZJ)[NT][kRow] = diag ? Zi : Zj;
-      bf16x8 fbi[BI][4], fzi[BI][3], fbj[BI][4], fzj[BI][3];
-#pragma unroll
-      for (int q = 0; q < BI; ++q)
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          const int ra = wm * 16 * BI + q * 16 + (lane & 15);
-          const int rb = wn * 16 * BI + q * 16 + (lane & 15);
-          fbi[q][s] = ldfrag(&Bi[s][ra][kk]);
-          fbj[q][s] = ldfrag(&BJ[s][rb][kk]);
-          if (s < 3) {
-            fzi[q][s] = ldfrag(&Zi[s][ra][kk]);
-            fzj[q][s] = ldfrag(&ZJ[s][rb][kk]);
-          }
-        }
-      __syncthreads();
-      // Leading products b0 z0 in one FP32 accumulator, the corrections
-      // (b0 z1, b1 z0, b0 z2, b1 z1, b2 z0, b3 z0; b3 = stored residual) in
-      // another, for B_i^T Z_j and Z_i^T B_j alike.
-      v4f cm[BI][BI], cc[BI][BI];
-#pragma unroll
-      for (int bi = 0; bi < BI; ++bi)
-#pragma unroll
-        for (int bj = 0; bj < BI; ++bj) {
-          cm[bi][bj] = mfma_v(fbi[bi][0], fzj[bj][0], v4f{0.f, 0.f, 0.f, 0.f});
-          cm[bi][bj] = mfma_v(fzi[bi][0], fbj[bj][0], cm[bi][bj]);
-          cc[bi][bj] = v4f{0.f, 0.f, 0.f, 0.f};
-        }
-#pragma unroll
-      for (int pr = 0; pr < 6; ++pr) {
-        const int sb = corr_b(pr), sz = corr_z(pr);
-#pragma unroll
-        for (int bi = 0; bi < BI; ++bi)
-#pragma unroll
-          for (int bj = 0; bj < BI; ++bj) {
-            cc[bi][bj] = mfma_v(fbi[bi][sb], fzj[bj][sz], cc[bi][bj]);  // B_i^T Z_j
-            cc[bi][bj] = mfma_v(fzi[bi][sz], fbj[bj][sb], cc[bi][bj]);  // Z_i^T B_j
-          }
-      }
-#pragma unroll
-      for (int bi = 0; bi < BI; ++bi)
-#pragma unroll
-        for (int bj = 0; bj < BI; ++bj)
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            acc[bi][bj][r] += (double)cm[bi][bj][r] + (double)cc[bi][bj][r];
-    };
-
-    using I0 = std::integral_constant<int, 0>;
-    using I1 = std::integral_constant<int, (PF > 1 ? 1 : 0)>;
-    using I2 = std::integral_constant<int, (PF > 2 ? 2 : 0)>;
-    load(0, I0{});
-    if (PF > 1 && kKB < ld) load(kKB, I1{});
-    if (PF > 2 && 2 * kKB < ld) load(2 * kKB, I2{});
-    for (int k0 = 0; k0 < ld; k0 += PF * kKB) {
-      step(k0, I0{});
-      if (PF > 1 && k0 + kKB < ld) step(k0 + kKB, I1{});
-      if (PF > 2 && k0 + 2 * kKB < ld) step(k0 + 2 * kKB, I2{});
+    for (int k = 0; k < kSlots; ++k) {
+      const int v = __builtin_amdgcn_readfirstlane(slots[min(b0 + k, count - 1)]);
+      ur[k] = v & 0xff;
+      uc[k] = v >> 8;
     }
 
-    // Scatter-add into VXC in transposed order (see k_syr2k).
-    const int32_t* bf = bfmap + t.bf_off;
+    const unsigned plane = (unsigned)nbe * (unsigned)ld;
+    const float* Bm = scratch + t.b_off_mx;
+    const auto rsB = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(Bm), 0,
+                                                       (int)(plane * 4u), 0x00020000);
+    const auto rsZ = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(Bm + 4 * (int64_t)plane), 0, (int)(plane * 4u), 0x00020000);
+    const auto rsL = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(Bm + 5 * (int64_t)plane), 0, (int)(plane * 2u), 0x00020000);
+    int off[kLoads];  // element of the loader's row and point group
 #pragma unroll
-    for (int bj = 0; bj < BI; ++bj) {
-      const int j = j0 + wn * 16 * BI + bj * 16 + (lane & 15);
-      if (j < nbe) {
-        const int rj = bf[j];
+    for (int e = 0; e < kLoads; ++e)
+      off[e] = (16 * block_of(min(wave + 4 * e, nst - 1)) + wf) * ld + 8 * wq;
+    struct Raw {
+      v4u b[2], z[2], lo;
+    };
+    auto load = [&](Raw (&raw)[kLoads], int s) {
+      const int so = s * kKB;
 #pragma unroll
-        for (int bi = 0; bi < BI; ++bi)
+      for (int e = 0; e < kLoads; ++e) {
+        if (wave + 4 * e >= nst) break;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          raw[e].b[h] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(
+                                                 rsB, off[e] * 4 + 16 * h, so * 4, 0));
+          raw[e].z[h] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(
+                                                 rsZ, off[e] * 4 + 16 * h, so * 4, 0));
+        }
+        raw[e].lo = __builtin_bit_cast(
+            v4u, __builtin_amdgcn_raw_buffer_load_b128(rsL, off[e] * 2, so * 2, 0));
+      }
+    };
+    auto split = [&](const v4u (&x)[2], v4u* dst) {
+      v4u a, b, c;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        // (Copies: a bit cast of a vector's element itself reads element 0.)
+        const unsigned x0 = x[e >> 1][2 * (e & 1)], x1 = x[e >> 1][2 * (e & 1) + 1];
+        const f2v v{__builtin_bit_cast(float, x0), __builtin_bit_cast(float, x1)};
+        unsigned a1, b1, c1;
+        split3f_pair(v, a1, b1, c1);
+        a[e] = a1;
+        b[e] = b1;
+        c[e] = c1;
+      }
+      dst[0] = a;
+      dst[64] = b;
+      dst[128] = c;
+    };
+    double acc[kSlots][4];
+#pragma unroll
+    for (int k = 0; k < kSlots; ++k)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[k][r] = 0.;
+    struct Frags {
+      bf16x8 b[4], z[3];
+    };
+    auto frags = [&](Frags& f, int u) {
+      const v4u* st = stage + u * 7 * 64 + rpos;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) f.b[q] = __builtin_bit_cast(bf16x8, st[64 * q]);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) f.z[q] = __builtin_bit_cast(bf16x8, st[64 * (4 + q)]);
+    };
+    auto contract = [&](auto N) {
+      constexpr int kN = decltype(N)::value;
+      Raw raw[kLoads];
+      if (s0 < s1) load(raw, s0);
+      for (int s = s0; s < s1; ++s) {
+        __syncthreads();  // the stage's previous reads are done
+#pragma unroll
+        for (int e = 0; e < kLoads; ++e) {
+          if (wave + 4 * e >= nst) break;
+          v4u* dst = stage + (wave + 4 * e) * 7 * 64 + wpos;
+          split(raw[e].b, dst);
+          dst[3 * 64] = raw[e].lo;
+          split(raw[e].z, dst + 4 * 64);
+        }
+        __syncthreads();
+        if (s + 1 < s1) load(raw, s + 1);
+        Frags row;
+#pragma unroll
+        for (int k = 0; k < kN; ++k) {
+          Frags col;
+          frags(col, uc[k]);
+          if (k == 0 || ur[k] != ur[k - 1]) frags(row, ur[k]);
+          // Leading products b0 z0 in one FP32 accumulator, the corrections
+          // (b0 z1, b1 z0, b0 z2, b1 z1, b2 z0, b3 z0; b3 = stored residual)
+          // in another, for B_i^T Z_j and Z_i^T B_j alike.
+          v4f cm = mfma_v(row.b[0], col.z[0], v4f{0.f, 0.f, 0.f, 0.f});
+          v4f cc = v4f{0.f, 0.f, 0.f, 0.f};
+          cm = mfma_v(row.z[0], col.b[0], cm);
+#pragma unroll
+          for (int pr = 0; pr < 6; ++pr) {
+            const int sb = corr_b(pr), sz = corr_z(pr);
+            cc = mfma_v(row.b[sb], col.z[sz], cc);  // B_i^T Z_j
+            cc = mfma_v(row.z[sz], col.b[sb], cc);  // Z_i^T B_j
+          }
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[k][r] += (double)cm[r] + (double)cc[r];
+        }
+      }
+    };
+    __syncthreads();  // slots are read: the stage may be filled
+    switch (n) {
+      case 0: contract(std::integral_constant<int, 0>{}); break;
+      case 1: contract(std::integral_constant<int, 1>{}); break;
+      case 2: contract(std::integral_constant<int, 2>{}); break;
+      case 3: contract(std::integral_constant<int, 3>{}); break;
+      case 4: contract(std::integral_constant<int, 4>{}); break;
+      case 5: contract(std::integral_constant<int, 5>{}); break;
+      case 6: contract(std::integral_constant<int, 6>{}); break;
+      case 7: contract(std::integral_constant<int, 7>{}); break;
+      default: contract(std::integral_constant<int, 8>{}); break;
+    }
+
+    if (ns > 1) {
+      double* dst = part + ((int64_t)wi.c * kSyrBlocks + b0) * 256 + lane;
+#pragma unroll
+      for (int k = 0; k < kSlots; ++k)
+        if (k < n) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) dst[(k * 4 + r) * 64] = acc[k][r];
+        }
+    } else {
+      // Scatter-add into VXC in transposed order (see k_syr2k).
+      const int32_t* bf = bfmap + t.bf_off;
+      double* vxc = vxc_all + t.p_off;
+#pragma unroll
+      for (int k = 0; k < kSlots; ++k)
+        if (k < n) {
+          const int j = 16 * block_of(uc[k]) + lf, i0 = 16 * block_of(ur[k]) + 4 * lq;
+          const int cj = bf[min(j, nbe - 1)];
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const int i = i0 + wm * 16 * BI + bi * 16 + 4 * (lane >> 4) + r;
+            const int i = i0 + r;
             // Negligible contributions are not added (NaN still is).
-            if (i < nbe && (!diag || i >= j) && !(fabs(acc[bi][bj][r]) < drop))
-              atomicAdd(vxc + (int64_t)bf[i] * ldv + rj, acc[bi][bj][r]);
+            if (i < nbe && i >= j && !(fabs(acc[k][r]) < drop))
+              atomicAdd(vxc + (int64_t)bf[i] * t.ldp + cj, acc[k][r]);
           }
-      }
+        }
     }
     stamp_item(qa, it, t0);
   }
 }
 
-int launch_syr2k_mixed(const CtxView& v, const WorkRange& r, int nt) {
-  if (r.n == 0) return XCQ_SUCCESS;
-  const QueueArgs qa = queue_args(v, r);
-  const float* scr = static_cast<const float*>(v.scratch);
-  if (nt == 32)
-    hipLaunchKernelGGL(k_syr2k_mx<32>, dim3(grid_of(r)), dim3(256), 0, v.stream, qa, v.tasks,
-                       v.bfmap, scr, v.vxc, v.vxc_drop, v.vxc_drop > 0.0 ? v.tmax : nullptr);
-  else
-    hipLaunchKernelGGL(k_syr2k_mx<64>, dim3(grid_of(r)), dim3(256), 0, v.stream, qa, v.tasks,
-                       v.bfmap, scr, v.vxc, v.vxc_drop, v.vxc_drop > 0.0 ? v.tmax : nullptr);
+int launch_syr2k_mixed(const CtxView& v, const WorkRange& r, const unsigned* tm) {
+  hipLaunchKernelGGL(k_syr2k_mx, dim3(grid_of(r)), dim3(256), 0, v.stream, queue_args(v, r),
+                     v.tasks, v.bfmap, static_cast<const float*>(v.scratch), v.vxc, v.vxc_drop,
+                     tm, v.syr_part);
   XCQ_HIP(hipGetLastError());
   return XCQ_SUCCESS;
 }

@@ -66,7 +66,6 @@ struct DevTask {
   int32_t npts_pad;   // npts rounded up to kPtBlock
   int32_t mol;        // molecule of the task
   int32_t ldp;        // nbf of the molecule = leading dimension of its P and VXC
-  int32_t nt_s;       // function tile of the SYR2K kernel (32 or 64)
   int32_t dens_cls;   // density work list: 0 to 2 by the tile policy's thresholds, 3 =
                       // 128-wide tiles on pairs of point blocks
   int64_t pt_off;     // points (SoA) / weights
@@ -84,7 +83,7 @@ struct DevTask {
   int64_t p_off;      // offset of the molecule's P (and P slices, VXC) in elements
 };
 
-struct WorkItem {  // (task, a, b): a/b are point-block or tile indices (FP64 SYR2K: see Chunk)
+struct WorkItem {  // (task, a, b): a/b are point-block or pair indices (SYR2K: see Chunk)
   int32_t task, a, b, c;
 };
 
@@ -118,30 +117,40 @@ struct Chunk {
   WorkRange coll;             // all point blocks (collocation) = dens[3..0] back to back
   WorkRange dens[4];          // density blocks by class (DevTask::dens_cls)
   WorkRange dens_pair;        // pairs of density blocks of class 3
-  WorkRange syr2k[2];         // mixed SYR2K tiles (it >= jt) with 32- / 64-function tiles
-  // FP64 SYR2K, per region and point slice: a = row group | column group <<
-  // 16, b = slice | slices << 16, c = place in the slice buffer (slices >
-  // 1); and per region with several slices: a as above, b = slices, c = the
-  // first slice's place.
-  WorkRange syr2k_f64, syr2k_sum;
+  // SYR2K (FP64, mixed), per region and point slice: a = row group | column
+  // group << 16, b = slice | slices << 16, c = place in the slice buffer
+  // (slices > 1); and per region with several slices: a as above, b =
+  // slices, c = the first slice's place.
+  WorkRange syr2k[2], syr2k_sum[2];
   int64_t syr_slots = 0;      // places used in the slice buffer
 };
 
-// FP64 SYR2K regions: a task's nb = ceil(nbe / 16) blocks of 16 functions are
-// one region when at most kSyrWhole of them (their triangle fits the
-// kSyrBlocks accumulators), else divided evenly over row groups of up to 7
-// and column groups of up to 6 blocks; its points evenly over its slices.
-constexpr int kSyrRows = 7, kSyrCols = 6, kSyrWhole = 8;
-constexpr int kSyrStaged = kSyrRows + kSyrCols;  // blocks staged at once
-constexpr int kSyrSlots = 11;                    // blocks per wave
-constexpr int kSyrBlocks = 4 * kSyrSlots;        // blocks per region
-static_assert(kSyrRows * kSyrCols <= kSyrBlocks && kSyrWhole <= kSyrStaged &&
-              kSyrWhole * (kSyrWhole + 1) / 2 <= kSyrBlocks, "SYR2K region");
+// SYR2K regions: a task's nb = ceil(nbe / 16) blocks of 16 functions are one
+// region when at most `whole` of them (their triangle fits the accumulators),
+// else divided evenly over row groups of up to `rows` and column groups of up
+// to `cols` blocks; its points evenly over its slices.
+struct SyrLimits {
+  int rows, cols, whole;
+  int slots;                                            // blocks per wave
+  constexpr int staged() const { return rows + cols; }  // blocks staged at once
+  constexpr int blocks() const { return 4 * slots; }    // blocks per region
+  constexpr bool ok() const {
+    return rows * cols <= blocks() && whole <= staged() && whole * (whole + 1) / 2 <= blocks() &&
+           whole * whole <= 64 && rows * cols <= 64;
+  }
+};
+template <bool MX>
+constexpr SyrLimits kSyr = MX ? SyrLimits{6, 5, 7, 8} : SyrLimits{7, 6, 8, 11};
+static_assert(kSyr<false>.ok() && kSyr<true>.ok() &&
+              kSyr<true>.blocks() <= kSyr<false>.blocks(), "SYR2K region");
+constexpr int kSyrBlocks = kSyr<false>.blocks();  // blocks per place of the slice buffer
+template <bool MX>
 __host__ __device__ inline int syr_row_groups(int nb) {
-  return nb <= kSyrWhole ? 1 : (nb + kSyrRows - 1) / kSyrRows;
+  return nb <= kSyr<MX>.whole ? 1 : (nb + kSyr<MX>.rows - 1) / kSyr<MX>.rows;
 }
+template <bool MX>
 __host__ __device__ inline int syr_col_groups(int nb) {
-  return nb <= kSyrWhole ? 1 : (nb + kSyrCols - 1) / kSyrCols;
+  return nb <= kSyr<MX>.whole ? 1 : (nb + kSyr<MX>.cols - 1) / kSyr<MX>.cols;
 }
 
 // View of a context's device buffers for the translation units that run
@@ -163,12 +172,12 @@ struct CtxView {
   void* scratch;
   double vxc_drop;  // B^T Z contributions with |v| < vxc_drop are not added to VXC
   unsigned* tmax;   // per granule {max |B|, max |Z|} as float bits (the density stage
-                    // fills it, the B^T Z stage skips tile pairs bounded below vxc_drop)
+                    // fills it, the B^T Z stage skips blocks bounded below vxc_drop)
   int in_stage;     // basis evaluation of the fold and the Z launch: 0 = the stored B /
                     // grad B planes; else they evaluate them (1 runs as 3)
   const DevShellC* shc;
   double* zc;       // Z coefficients per point block [4][64] (in-stage mode 3)
-  double* syr_part; // slice buffer of the FP64 SYR2K, kSyrBlocks blocks per place
+  double* syr_part; // slice buffer of the SYR2K, kSyrBlocks blocks per place
 };
 // Basis data of the density stage's own evaluation of B and grad B.
 struct ShellArgs {
@@ -226,29 +235,6 @@ __device__ __forceinline__ int64_t next_ticket(const QueueArgs& qa) {
   for (int64_t it_var = (qa).qoff ? next_ticket(qa) : (int64_t)blockIdx.x,            \
                it_end_ = (qa).qoff ? kNoItem : it_var + 1;                             \
        it_var < it_end_; it_var = (qa).qoff ? next_ticket(qa) : it_var + 1)
-
-// True when every element of the B^T Z + Z^T B tile pair (rows i0.., columns
-// j0.., nt wide) of task t is bounded below `drop` by the granule maxima the
-// density stage recorded: |sum_p B_pi Z_pj| <= npts max|B_i| max|Z_j|.
-// The factor 1.01 covers the rounding of the stored maxima and of the
-// products.
-__device__ __forceinline__ bool tile_pair_negligible(const DevTask& t, const unsigned* tmax,
-                                                     int i0, int j0, int nt, double drop) {
-  if (!tmax) return false;
-  const unsigned* tm = tmax + 2 * t.tmax_off;
-  const int ng = (t.nbe + kGran - 1) / kGran;
-  float bi = 0.f, zi = 0.f, bj = 0.f, zj = 0.f;
-  for (int g = i0 / kGran; g < min((i0 + nt) / kGran, ng); ++g) {
-    bi = fmaxf(bi, __uint_as_float(tm[2 * g]));
-    zi = fmaxf(zi, __uint_as_float(tm[2 * g + 1]));
-  }
-  for (int g = j0 / kGran; g < min((j0 + nt) / kGran, ng); ++g) {
-    bj = fmaxf(bj, __uint_as_float(tm[2 * g]));
-    zj = fmaxf(zj, __uint_as_float(tm[2 * g + 1]));
-  }
-  const double bound = 1.01 * (double)t.npts * ((double)bi * zj + (double)zi * bj);
-  return bound < drop;
-}
 
 __device__ __forceinline__ void stamp_item(const QueueArgs& qa, int64_t it, int64_t t0) {
   if (qa.tstamp && threadIdx.x == 0) {
