@@ -1470,12 +1470,12 @@ namespace {
 // launches build; above it they loop over every atom.
 constexpr int32_t kSsfNbrMaxAtoms = 8192;
 
-// Per atom A, every atom in order of increasing R_AB with A itself first
-// (row-major natoms x natoms), for k_ssf's bounded loops.
+// Per atom A, every atom in order of increasing R_AB with A itself first,
+// and 1 / (0.64 R_AB) (row-major natoms x natoms), for k_ssf's bounded loops.
 void ssf_neighbours(int32_t natoms, const std::vector<double>& rab, std::vector<int32_t>& idx,
-                    std::vector<double>& r) {
+                    std::vector<double>& inv) {
   idx.resize((size_t)natoms * natoms);
-  r.resize(idx.size());
+  inv.resize(idx.size());
   std::vector<int32_t> ord(natoms);
   for (int32_t A = 0; A < natoms; ++A) {
     const double* col = rab.data() + (size_t)A * natoms;  // R_AB = rab[B + A * natoms]
@@ -1485,7 +1485,7 @@ void ssf_neighbours(int32_t natoms, const std::vector<double>& rab, std::vector<
                      [&](int32_t u, int32_t v) { return col[u] < col[v]; });
     for (int32_t k = 0; k < natoms; ++k) {
       idx[(size_t)A * natoms + k] = ord[k];
-      r[(size_t)A * natoms + k] = k == 0 ? 0.0 : col[ord[k]];
+      inv[(size_t)A * natoms + k] = k == 0 ? INFINITY : 1.0 / (0.64 * col[ord[k]]);
     }
   }
 }

@@ -37,6 +37,7 @@
 #include "internal.hpp"
 #include "functional.hpp"
 #include "shell_eval.hpp"
+#include "ssf.hpp"
 
 #include <type_traits>
 
@@ -484,8 +485,8 @@ __global__ __launch_bounds__(256, LMAX > 3 || NX > 1 ? 2 : 3) void k_grad_contra
 //   1 - g(v) = (1 - v)^4 (5 v^3 + 20 v^2 + 29 v + 16) / 16,  g'(v) = 35 (1 - v^2)^3 / 16,
 //   t(mu) = 35 (1 + v)^3 / ((mu - a)(5 v^3 + 20 v^2 + 29 v + 16)),  v = mu / a,
 // which stays accurate up to the |mu| < a - 1e-4 bound the contraction uses.
-// With neighbour lists (nbr_idx / nbr_r: row A holds every atom in order of
-// increasing R_AB, A itself first) the loops stop where the triangle
+// With neighbour lists (nbr_idx / nbr_i: row A holds every atom in order of
+// increasing R_AB, A itself first, and 1 / (a R_AB)) the loops stop where the triangle
 // inequality makes every remaining term vanish, as in the weights kernel: a
 // factor s(mu_BC) differs from 1, and |mu_BC| can fall below a, only for
 // R_BC < 2 d_B / (1 - a); P_B > 0 only for d_B <= (1 + a)/(1 - a) d_min; so
@@ -504,21 +505,12 @@ __global__ __launch_bounds__(256, LMAX > 3 || NX > 1 ? 2 : 3) void k_grad_contra
 // falls on C is summed over the wave, four C at a time (a transposing
 // reduction: 21 exchanges where 12 separate sums take 72); what falls on B
 // and on A stays in registers and is summed once.
-// What bounds it: FP64 vector work.  On 13 waters (883,000 points) 1.4 ms;
+// What bounds it: FP64 vector work.  On 13 waters (883,000 points) 1.25 ms;
 // with every thread's own loop bounds and one atomic addition per thread and
 // term 6.4 ms.
-constexpr double kSsfA = 0.64;
 constexpr double kSsfTol = 1e-13;
 
 constexpr int kSsfKeep = 12;
-
-// s at v = mu / a: the limits +-1 give exactly 0 and 1.
-__device__ __forceinline__ double ssf_s(double v) {
-  v = fmin(fmax(v, -1.), 1.);
-  const double v2 = v * v;
-  const double g = v * (35. + v2 * (-35. + v2 * (21. - 5. * v2))) * 0.0625;
-  return 0.5 * (1. - g);
-}
 
 template <bool LISTS>
 __global__ __launch_bounds__(64) void k_ssf_grad(const WorkItem* __restrict__ items,
@@ -531,7 +523,7 @@ __global__ __launch_bounds__(64) void k_ssf_grad(const WorkItem* __restrict__ it
                                                  const double* __restrict__ wf,
                                                  double* __restrict__ grad, int64_t gstride,
                                                  const int32_t* __restrict__ nbr_idx,
-                                                 const double* __restrict__ nbr_r) {
+                                                 const double* __restrict__ nbr_i) {
   __shared__ double keep[kSsfKeep][64];
   const WorkItem wi = items[blockIdx.x];
   const DevTask t = tasks[wi.task];
@@ -546,53 +538,55 @@ __global__ __launch_bounds__(64) void k_ssf_grad(const WorkItem* __restrict__ it
     const double dx = rx - X(at, 0), dy = ry - X(at, 1), dz = rz - X(at, 2);
     return sqrt(dx * dx + dy * dy + dz * dz);
   };
-  // Entry q of B's list (atom, R_BC); lists start with B itself at q = 0.
+  // Entry q of B's list: atom C and 1 / (a R_BC); lists start with B itself.
   auto nbr_at = [&](int B, int q) { return LISTS ? nbr_idx[(int64_t)B * natoms + q] : q; };
-  auto nbr_d = [&](int B, int q) {
-    if (LISTS) return nbr_r[(int64_t)B * natoms + q];
+  auto nbr_inv = [&](int B, int q) {
+    if (LISTS) return nbr_i[(int64_t)B * natoms + q];
     const double dx = X(B, 0) - X(q, 0), dy = X(B, 1) - X(q, 1), dz = X(B, 2) - X(q, 2);
-    return sqrt(dx * dx + dy * dy + dz * dz);
+    return 1. / (kSsfA * sqrt(dx * dx + dy * dy + dz * dz));
   };
-  constexpr double kWiden = 1.0 + 1e-10, kInvA = 1.0 / kSsfA;
+  constexpr double kWiden = 1.0 + 1e-10;
   constexpr double bound = kSsfA - 1e-4;
   const double dA = dist(A);
   const bool on = p < t.npts && !(fabs(f) < 1e-12) && !(dA < 0.5 * (1. - kSsfA) * dnear[A]);
   if (!__any(on)) return;
   // Nearest atom (R_AB* <= 2 d_A) and the candidate bound.
-  double cbound = INFINITY, rmax = INFINITY;
+  double cbound = INFINITY, imax = 0.;  // imax: 1 / (a R) at the list's end
   if (LISTS) {
     double dmin = dA;
-    for (int k = 1; k < natoms && __any(on && nbr_d(A, k) <= 2.0 * dA * kWiden); ++k)
+    const double i2 = 1.0 / (kSsfA * 2.0 * dA * kWiden);
+    for (int k = 1; k < natoms && __any(on && nbr_inv(A, k) >= i2); ++k)
       dmin = fmin(dmin, dist(nbr_at(A, k)));
     cbound = (1.0 + kSsfA) / (1.0 - kSsfA) * dmin * kWiden + 1e-12;
-    rmax = fmax(2.0 * dA / (1.0 - kSsfA), dA + cbound) * kWiden;
+    imax = 1.0 / (kSsfA * fmax(2.0 * dA / (1.0 - kSsfA), dA + cbound) * kWiden);
   }
-  auto reach = [&](double dB) { return 2.0 * dB / (1.0 - kSsfA) * kWiden; };
+  // 1 / (a R) where B's list ends.
+  auto reach = [&](double dB) { return (1.0 - kSsfA) / (kSsfA * 2.0 * dB * kWiden); };
   constexpr int q0 = LISTS ? 1 : 0;
   // P_B, 0 in lanes that are off or beyond the candidate bound.
   auto part = [&](int B, double dB) {
     double v = on && dB <= cbound ? 1. : 0.;
-    const double rf = reach(dB);
     if (!__any(v > 0.)) return v;
+    const double rf = reach(dB);
     for (int q = q0; q < natoms; q += 4) {
       int C[4];
-      double R[4];
+      double I[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int qj = min(q + j, natoms - 1);
         C[j] = nbr_at(B, qj);
-        R[j] = nbr_d(B, qj);
+        I[j] = nbr_inv(B, qj);
       }
-      if (!__any(v > 0. && (!LISTS || R[0] < rf))) break;
+      if (!__any(v > 0. && (!LISTS || I[0] > rf))) break;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        if (q + j < natoms && C[j] != B) v *= ssf_s((dB - dist(C[j])) / (kSsfA * R[j]));
+        if (q + j < natoms && C[j] != B) v *= ssf_s((dB - dist(C[j])) * I[j]);
     }
     return v;
   };
   double sum = 0., pA = 0.;
   int nkeep = 0, kover = natoms, kept[kSsfKeep];
-  for (int k = 0; k < natoms && (!LISTS || __any(on && nbr_d(A, k) <= rmax)); ++k) {
+  for (int k = 0; k < natoms && (!LISTS || __any(on && nbr_inv(A, k) >= imax)); ++k) {
     const int B = nbr_at(A, k);
     const double pB = part(B, dist(B));
     sum += pB;
@@ -619,25 +613,24 @@ __global__ __launch_bounds__(64) void k_ssf_grad(const WorkItem* __restrict__ it
     double gb[3] = {0., 0., 0.};
     for (int q = q0; q < natoms; q += 4) {
       int C[4];
-      double R[4], g[4][3];
+      double I[4], g[4][3];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int qj = min(q + j, natoms - 1);
         C[j] = nbr_at(B, qj);
-        R[j] = nbr_d(B, qj);
+        I[j] = nbr_inv(B, qj);
       }
-      if (LISTS && !__any(act && R[0] < rf)) break;
+      if (LISTS && !__any(act && I[0] > rf)) break;
       bool any = false;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const double dC = dist(C[j]);
-        const double iR = 1. / R[j];
-        const double mu = (dB - dC) * iR;
+        const double v = (dB - dC) * I[j], mu = kSsfA * v, iR = kSsfA * I[j];
         const bool in = q + j < natoms && C[j] != B && act && fabs(mu) < bound;
 #pragma unroll
         for (int d = 0; d < 3; ++d) g[j][d] = 0.;
         if (!__any(in)) continue;
-        const double v = mu * kInvA, v1 = 1. + v;
+        const double v1 = 1. + v;
         const double tm = 35. * (v1 * v1 * v1) /
                           ((mu - kSsfA) * (((5. * v + 20.) * v + 29.) * v + 16.)) * iR;
         const double tt = in ? tm : 0.;
@@ -690,7 +683,7 @@ __global__ __launch_bounds__(64) void k_ssf_grad(const WorkItem* __restrict__ it
     derivs(B, pB * fs, pB > kSsfTol);
   }
   // Atoms beyond the kept ones (many comparable distances): formed again.
-  for (int k = kover; k < natoms && (!LISTS || __any(on && nbr_d(A, k) <= rmax)); ++k) {
+  for (int k = kover; k < natoms && (!LISTS || __any(on && nbr_inv(A, k) >= imax)); ++k) {
     const int B = nbr_at(A, k);
     if (B == A) continue;
     const double pB = part(B, dist(B));
@@ -772,11 +765,11 @@ int launch_grad_contract(const CtxView& v, const WorkRange& r, int gga,
 
 int launch_ssf_grad(const CtxView& v, const WorkRange& r, int natoms, const double* xyz,
                     const double* dnear, const double* wf, double* part, int64_t gstride,
-                    const int32_t* nbr_idx, const double* nbr_r) {
+                    const int32_t* nbr_idx, const double* nbr_i) {
   if (r.n == 0) return XCQ_SUCCESS;
   hipLaunchKernelGGL(nbr_idx ? k_ssf_grad<true> : k_ssf_grad<false>, dim3((unsigned)r.n),
                      dim3(64), 0, v.stream, v.work + r.off, v.tasks, v.px, v.py, v.pz, natoms,
-                     xyz, dnear, wf, part, gstride, nbr_idx, nbr_r);
+                     xyz, dnear, wf, part, gstride, nbr_idx, nbr_i);
   XCQ_HIP(hipGetLastError());
   return XCQ_SUCCESS;
 }
