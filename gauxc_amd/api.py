@@ -605,14 +605,13 @@ class DeviceContext:
 
     def set_density_basis_eval(self, mode):
         """3 (default) = the density stage evaluates basis values/gradients
-        for its fold and a separate launch for Z; 1 = the mixed density stage
-        for both (FP64 runs 3); 0 (or False) = both read the planes the
-        collocation stage stored."""
+        for its fold and a separate launch for Z; 1 runs as 3; 0 (or False) =
+        both read the planes the collocation stage stored."""
         N.xcq_check(self.lib.xcq_set_density_basis_eval(self.h, int(mode)),
                     "xcq_set_density_basis_eval")
 
     def density_basis_eval(self):
-        """The basis evaluation mode in effect (see set_density_basis_eval)."""
+        """The basis evaluation mode set (see set_density_basis_eval)."""
         m = ctypes.c_int32(0)
         N.xcq_check(self.lib.xcq_get_density_basis_eval(self.h, ctypes.byref(m)),
                     "xcq_get_density_basis_eval")

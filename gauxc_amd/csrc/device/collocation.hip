@@ -215,9 +215,10 @@ __global__ __launch_bounds__(256, coll_waves(LMAX, GRAD, sizeof(T) == 8)) void k
 // bounds.  Five waves per SIMD: with the gradient folded along the
 // coefficient vector (shell_functions_z) up to f needs 114 registers; at
 // five waves 8 spill and the launch is still faster (24 waters, FP32 Z
-// 1.30 -> 1.20 ms, FP64 1.63 -> 1.49 ms).
+// 1.30 -> 1.20 ms, FP64 1.63 -> 1.49 ms).  With g functions 40 would spill:
+// four.
 template <bool GGA, int LMAX, typename T>
-__global__ __launch_bounds__(256, 5) void k_z_in_stage(const WorkItem* __restrict__ blocks,
+__global__ __launch_bounds__(256, LMAX > 3 ? 4 : 5) void k_z_in_stage(const WorkItem* __restrict__ blocks,
                                                       const DevTask* __restrict__ tasks,
                                                       const DevShell* __restrict__ shells,
                                                       const int32_t* __restrict__ shell_list,
@@ -316,8 +317,8 @@ int launch_z_in_stage(hipStream_t s, const WorkItem* items, int64_t n, const Dev
                       const double* pz, const double* zcoef, void* scratch, int precision,
                       unsigned* tmax, int gga, int lmax) {
   if (n == 0) return XCQ_SUCCESS;
-  XCQ_REQUIRE(lmax >= 0 && lmax <= kInStageMaxL, XCQ_ERROR_INVALID_ARGUMENT,
-              "in-stage Z: angular momentum out of range");
+  XCQ_REQUIRE(lmax >= 0 && lmax <= (precision == XCQ_PREC_FP64 ? 4 : 3),
+              XCQ_ERROR_INVALID_ARGUMENT, "in-stage Z: angular momentum out of range");
   auto go = [&](auto kern, auto* scr) {
     hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(256), 0, s, items, tasks, shells,
                        shell_list, lsh_first, px, py, pz, zcoef, scr, tmax);
@@ -326,10 +327,12 @@ int launch_z_in_stage(hipStream_t s, const WorkItem* items, int64_t n, const Dev
     using T = std::remove_pointer_t<decltype(scr)>;
     if (gga) {
       if (lmax <= 2) go(k_z_in_stage<true, 2, T>, scr);
-      else go(k_z_in_stage<true, 3, T>, scr);
+      else if (sizeof(T) == 4 || lmax == 3) go(k_z_in_stage<true, 3, T>, scr);
+      else if constexpr (sizeof(T) == 8) go(k_z_in_stage<true, 4, T>, scr);
     } else {
       if (lmax <= 2) go(k_z_in_stage<false, 2, T>, scr);
-      else go(k_z_in_stage<false, 3, T>, scr);
+      else if (sizeof(T) == 4 || lmax == 3) go(k_z_in_stage<false, 3, T>, scr);
+      else if constexpr (sizeof(T) == 8) go(k_z_in_stage<false, 4, T>, scr);
     }
   };
   if (precision == XCQ_PREC_FP64) pick(static_cast<double*>(scratch));

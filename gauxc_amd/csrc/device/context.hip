@@ -355,7 +355,7 @@ CtxView view_of(xcq_context_s* c) {
                  c->d_work,  c->d_qoff,  c->d_counters, c->timing ? c->d_tstamp : nullptr,
                  c->d_P,     c->d_Pf32,  c->d_vxc,   c->d_red,        c->d_scratch,
                  c->vxc_drop, reinterpret_cast<unsigned*>(c->d_tmax),
-                 c->max_l <= kInStageMaxL ? c->dens_in_stage : 0, c->d_shc, c->d_zc, c->d_syr_part};
+                 c->dens_in_stage, c->max_l, c->d_shc, c->d_zc, c->d_syr_part};
 }
 
 // Heuristic per-item costs (used when no predicted task costs are set):
@@ -541,14 +541,20 @@ int ensure_syr_part(xcq_context_s* ctx) {
 
 // Enqueue one evaluation on the context's stream.  Events are recorded only
 // when `events` is set (not under graph capture).
-// The basis evaluation mode the kernels run: on stored planes (0) or in the
-// stages (3).
-int effective_mode(const CtxView& v) { return v.in_stage != 0 ? 3 : 0; }
+// The basis evaluation mode an energy evaluation runs: on stored planes (0) or
+// in the stages (3).  Mixed precision with g functions stays on stored planes:
+// the stages' FP64 values in place of the stored FP32 ones move VXC by up to
+// 1e-9 (in place of the FP32 rounding, 6e-9 from FP64), while FP64 agrees to
+// 2e-16 (4 waters with g functions, 0.66 -> 0.42 ms).
+int effective_mode(const xcq_context_s* ctx, int precision) {
+  return ctx->dens_in_stage == 0 || (precision != XCQ_PREC_FP64 && ctx->max_l > 3) ? 0 : 3;
+}
 
 int enqueue_pipeline(xcq_context_s* ctx, int func, int precision, int want_vxc, bool events) {
   const int gga = (func == XCQ_FUNC_PBE || func == XCQ_FUNC_PBE0) ? 1 : 0;
-  const CtxView v = view_of(ctx);
-  const int mode = effective_mode(v);
+  CtxView v = view_of(ctx);
+  const int mode = effective_mode(ctx, precision);
+  v.in_stage = mode;
   hipStream_t s = ctx->stream;
   const double fac = func == 0 ? 1.0 : 2.0;
   int rc;
@@ -1174,7 +1180,7 @@ int xcq_set_density_basis_eval(xcq_context ctx, int32_t in_stage) {
 
 int xcq_get_density_basis_eval(xcq_context ctx, int32_t* mode) {
   XCQ_REQUIRE(ctx && mode, XCQ_ERROR_INVALID_ARGUMENT, "null argument");
-  *mode = ctx->max_l <= kInStageMaxL ? ctx->dens_in_stage : 0;
+  *mode = ctx->dens_in_stage;
   return XCQ_SUCCESS;
 }
 
@@ -1245,7 +1251,7 @@ int xcq_task_times(xcq_context ctx, double* dens_us, double* syr2k_us) {
   };
   for (const auto& c : ctx->chunks) {
     // FP64 runs class 3 as pairs, but on stored planes.
-    const bool pairs = !ctx->last_mixed && effective_mode(view_of(ctx)) != 0;
+    const bool pairs = !ctx->last_mixed && effective_mode(ctx, XCQ_PREC_FP64) != 0;
     for (int v = 0; v < (pairs ? 3 : 4); ++v) add(c.dens[v], dens_us);
     if (pairs) add(c.dens_pair, dens_us);
     // The list the last evaluation ran (the other keeps older stamps).
@@ -1325,7 +1331,7 @@ int xcq_autotune(xcq_context ctx, int functional, int precision, int32_t* dens32
       double ms;
     };
     std::vector<int32_t> modes;
-    if (ctx->max_l <= kInStageMaxL) modes.push_back(3);
+    if (precision == XCQ_PREC_FP64 || ctx->max_l <= 3) modes.push_back(3);
     modes.push_back(0);
     Pol best{ctx->dens_in_stage, best_d, ctx->dens_hiocc_max_nbe, ctx->dens128_min_nbe, 1e300};
     for (int32_t mode : modes) {
@@ -1514,57 +1520,40 @@ int ensure_point_buffers(xcq_context_s* ctx) {
   return dalloc(&ctx->d_uks, (size_t)5 * 256 * std::max<int64_t>(ctx->pblocks, 1));
 }
 
-// Basis-evaluation mode of the FP64 UKS and FXC paths: in-stage (3: the
-// density stage evaluates B and grad B itself and Z is formed by
-// k_z_in_stage from the per-point coefficients, so collocation stores the
-// value plane only) up to kInStageMaxL, stored planes (0) above.
-int derivative_mode(const xcq_context_s* ctx) { return ctx->max_l <= kInStageMaxL ? 3 : 0; }
-
 // Z of a chunk from per-point coefficients ([block][4][64]) into plane 4.
-int z_from_point_coeffs(xcq_context_s* ctx, const CtxView& v, const Chunk& c, int mode, int gga,
-                        const double* coef) {
-  if (mode == 0) return launch_z_from_coeffs(v, c.coll, XCQ_PREC_FP64, gga, coef, nullptr);
+int z_from_point_coeffs(xcq_context_s* ctx, const CtxView& v, const Chunk& c, int gga,
+                        const double* coef, unsigned* tm = nullptr) {
   return launch_z_in_stage(ctx->stream, v.work + c.coll.off, c.coll.n, v.tasks, v.shells,
                            v.shell_list, v.lsh, v.px, v.py, v.pz, coef, v.scratch,
-                           XCQ_PREC_FP64, nullptr, gga, ctx->max_l);
+                           XCQ_PREC_FP64, tm, gga, ctx->max_l);
 }
 
 // Z from per-point coefficients, then its B^T Z + Z^T B scattered into
-// v.vxc.  In the in-stage mode with a drop tolerance the Z launch also
-// records the granule maxima of |B| and |Z| (the bound table, cleared
-// first), and the contraction skips negligible tile pairs and drops
-// negligible elements as the energy path does; on stored planes only the
-// element drop applies.
-int z_and_vxc(xcq_context_s* ctx, CtxView v, const Chunk& c, int mode, int gga,
-              const double* coef) {
+// v.vxc.  With a drop tolerance the Z launch also records the granule maxima
+// of |B| and |Z| (the bound table, cleared first), and the contraction skips
+// negligible blocks and drops negligible elements as the energy path does.
+int z_and_vxc(xcq_context_s* ctx, CtxView v, const Chunk& c, int gga, const double* coef) {
   int rc;
-  unsigned* tm = reinterpret_cast<unsigned*>(ctx->d_tmax);
   v.vxc_drop = ctx->vxc_drop;
-  if (mode == 3 && v.vxc_drop > 0.0 && tm) {
-    if ((rc = launch_fill(ctx->stream, ctx->d_tmax, ctx->tmax_total)) ||
-        (rc = launch_z_in_stage(ctx->stream, v.work + c.coll.off, c.coll.n, v.tasks, v.shells,
-                                v.shell_list, v.lsh, v.px, v.py, v.pz, coef, v.scratch,
-                                XCQ_PREC_FP64, tm, gga, ctx->max_l)))
-      return rc;
-    v.tmax = tm;
-  } else {
-    if ((rc = z_from_point_coeffs(ctx, v, c, mode, gga, coef))) return rc;
-    v.tmax = nullptr;
-  }
+  v.tmax = v.vxc_drop > 0.0 ? reinterpret_cast<unsigned*>(ctx->d_tmax) : nullptr;
+  if (v.tmax && (rc = launch_fill(ctx->stream, ctx->d_tmax, ctx->tmax_total))) return rc;
+  if ((rc = z_from_point_coeffs(ctx, v, c, gga, coef, v.tmax))) return rc;
   return launch_syr2k(v, c, XCQ_PREC_FP64);
 }
 
-// One UKS evaluation on the context's stream (FP64; in-stage basis
-// evaluation up to f functions, stored planes above): per chunk,
+// The UKS, FXC and gradient paths evaluate the basis in the stages (mode 3):
+// the density stage evaluates B and grad B itself and Z is formed from the
+// per-point coefficients, so collocation stores the value plane only.
+
+// One UKS evaluation on the context's stream (FP64): per chunk,
 // collocation; the density stage twice (P_s, then P_z; factor 1) leaving
 // raw per-point sums; the polarised functional and Z coefficients per
 // point; Z_s into the chunk's Z plane and its B^T Z + Z^T B into VXC_s; then
 // Z_z into VXC_z, both with the energy path's drop screening (z_and_vxc).
 int enqueue_uks(xcq_context_s* ctx, int func, int want_vxc) {
   const int gga = (func == XCQ_FUNC_PBE || func == XCQ_FUNC_PBE0) ? 1 : 0;
-  const int mode = derivative_mode(ctx);
   CtxView v = view_of(ctx);
-  v.in_stage = mode;
+  v.in_stage = 3;
   v.tmax = nullptr;
   v.vxc_drop = 0.0;
   hipStream_t s = ctx->stream;
@@ -1584,7 +1573,7 @@ int enqueue_uks(xcq_context_s* ctx, int func, int want_vxc) {
     const WorkItem* cw = v.work + c.coll.off;
     if ((rc = launch_collocation_fp64(s, cw, c.coll.n, v.tasks, v.shells, v.shell_list, v.lsh,
                                       v.px, v.py, v.pz, static_cast<double*>(v.scratch),
-                                      gga && mode == 0, ctx->max_l)))
+                                      0, ctx->max_l)))
       return rc;
     for (int pass = 0; pass < 2; ++pass)
       if ((rc = launch_density(v, c, XCQ_PREC_FP64, gga, 1.0, pass == 0 ? ds : dz,
@@ -1595,7 +1584,7 @@ int enqueue_uks(xcq_context_s* ctx, int func, int want_vxc) {
     for (int comp = 0; comp < 2; ++comp) {
       CtxView vc = v;
       vc.vxc = comp == 0 ? ctx->d_vxc : ctx->d_vxcz;
-      if ((rc = z_and_vxc(ctx, vc, c, mode, gga, comp == 0 ? zs : zz))) return rc;
+      if ((rc = z_and_vxc(ctx, vc, c, gga, comp == 0 ? zs : zz))) return rc;
     }
   }
   if (want_vxc) {
@@ -1665,8 +1654,7 @@ int xcq_download_results_uks(xcq_context ctx, double* exc, double* nel, double* 
 // ---- FXC contraction (GauXC's eval_fxc_contraction(P, tP)) ------------------
 namespace {
 
-// One RKS FXC contraction on the context's stream (FP64; in-stage basis
-// evaluation up to f functions, stored planes above): per chunk,
+// One RKS FXC contraction on the context's stream (FP64): per chunk,
 // collocation; the density stage twice (P, then the trial density; factor
 // 2) leaving raw per-point sums; the second-derivative kernel and Z
 // coefficients per point; Z into the chunk's Z plane and its B^T Z + Z^T B
@@ -1674,9 +1662,8 @@ namespace {
 // symmetrised.
 int enqueue_fxc(xcq_context_s* ctx, int func) {
   const int gga = (func == XCQ_FUNC_PBE || func == XCQ_FUNC_PBE0) ? 1 : 0;
-  const int mode = derivative_mode(ctx);
   CtxView v = view_of(ctx);
-  v.in_stage = mode;
+  v.in_stage = 3;
   v.tmax = nullptr;
   v.vxc_drop = 0.0;
   hipStream_t s = ctx->stream;
@@ -1693,14 +1680,14 @@ int enqueue_fxc(xcq_context_s* ctx, int func) {
     const WorkItem* cw = v.work + c.coll.off;
     if ((rc = launch_collocation_fp64(s, cw, c.coll.n, v.tasks, v.shells, v.shell_list, v.lsh,
                                       v.px, v.py, v.pz, static_cast<double*>(v.scratch),
-                                      gga && mode == 0, ctx->max_l)))
+                                      0, ctx->max_l)))
       return rc;
     for (int pass = 0; pass < 2; ++pass)
       if ((rc = launch_density(v, c, XCQ_PREC_FP64, gga, 2.0, pass == 0 ? dp : dt,
                                pass == 0 ? ctx->d_P : ctx->d_tP)))
         return rc;
     if ((rc = launch_fxc_points(v, c.coll, func, gga, dp, dt, zc))) return rc;
-    if ((rc = z_and_vxc(ctx, v, c, mode, gga, zc))) return rc;
+    if ((rc = z_and_vxc(ctx, v, c, gga, zc))) return rc;
   }
   if ((rc = launch_symmetrize(s, 1, ctx->max_nbf, ctx->d_mol_n, ctx->d_mol_off, ctx->d_vxc)))
     return rc;
@@ -1762,9 +1749,8 @@ namespace {
 // screening (z_and_vxc); symmetrised.
 int enqueue_fxc_uks(xcq_context_s* ctx, int func) {
   const int gga = (func == XCQ_FUNC_PBE || func == XCQ_FUNC_PBE0) ? 1 : 0;
-  const int mode = derivative_mode(ctx);
   CtxView v = view_of(ctx);
-  v.in_stage = mode;
+  v.in_stage = 3;
   v.tmax = nullptr;
   v.vxc_drop = 0.0;
   hipStream_t s = ctx->stream;
@@ -1784,7 +1770,7 @@ int enqueue_fxc_uks(xcq_context_s* ctx, int func) {
     const WorkItem* cw = v.work + c.coll.off;
     if ((rc = launch_collocation_fp64(s, cw, c.coll.n, v.tasks, v.shells, v.shell_list, v.lsh,
                                       v.px, v.py, v.pz, static_cast<double*>(v.scratch),
-                                      gga && mode == 0, ctx->max_l)))
+                                      0, ctx->max_l)))
       return rc;
     for (int pass = 0; pass < 4; ++pass)
       if ((rc = launch_density(v, c, XCQ_PREC_FP64, gga, 1.0, dd[pass], mats[pass])))
@@ -1794,7 +1780,7 @@ int enqueue_fxc_uks(xcq_context_s* ctx, int func) {
     for (int comp = 0; comp < 2; ++comp) {
       CtxView vc = v;
       vc.vxc = comp == 0 ? ctx->d_vxc : ctx->d_vxcz;
-      if ((rc = z_and_vxc(ctx, vc, c, mode, gga, comp == 0 ? zs : zz))) return rc;
+      if ((rc = z_and_vxc(ctx, vc, c, gga, comp == 0 ? zs : zz))) return rc;
     }
   }
   for (double* m : {ctx->d_vxc, ctx->d_vxcz})
@@ -1897,15 +1883,11 @@ namespace {
 // for GGAs, its X = 2 P_sub B in a plane; per-point Za coefficients and
 // w eps rho; Za; Y = 2 P_sub Za into plane 2; the basis-function part and
 // the grid-weight part into d_grad (the latter only with weight_derivs).
-// Up to f functions the basis is evaluated in-stage (collocation stores the
-// value plane only; X in plane 1, Za by k_z_in_stage into plane 4); with g
-// functions on stored planes (B and grad B; X in plane 4, Za over grad_z B
-// in plane 3).
+// Planes: X in 1, Za (k_z_in_stage) in 4.
 int enqueue_grad(xcq_context_s* ctx, int func, int weight_derivs) {
   const int gga = (func == XCQ_FUNC_PBE || func == XCQ_FUNC_PBE0) ? 1 : 0;
-  const int mode = derivative_mode(ctx);
   CtxView v = view_of(ctx);
-  v.in_stage = mode;
+  v.in_stage = 3;
   v.tmax = nullptr;
   v.vxc_drop = 0.0;
   hipStream_t s = ctx->stream;
@@ -1923,21 +1905,16 @@ int enqueue_grad(xcq_context_s* ctx, int func, int weight_derivs) {
     const WorkItem* cw = v.work + c.coll.off;
     if ((rc = launch_collocation_fp64(s, cw, c.coll.n, v.tasks, v.shells, v.shell_list, v.lsh,
                                       v.px, v.py, v.pz, static_cast<double*>(v.scratch),
-                                      gga && mode == 0, ctx->max_l)))
+                                      0, ctx->max_l)))
       return rc;
-    // X: plane 1 in the in-stage mode (no gradient planes are stored),
-    // plane 4 on stored planes.
-    const int x_pl = mode == 3 ? 1 : 4;
-    if ((rc = launch_density(v, c, XCQ_PREC_FP64, gga, 2.0, dp, ctx->d_P, gga ? x_pl : -1)))
+    if ((rc = launch_density(v, c, XCQ_PREC_FP64, gga, 2.0, dp, ctx->d_P, gga ? 1 : -1)))
       return rc;
     if ((rc = launch_grad_points(v, c.coll, func, gga, dp, coef, wf))) return rc;
-    // Za: plane 4 (in-stage evaluation) or over grad_z B in plane 3.
-    const int za_pl = mode == 3 ? 4 : 3;
-    if (mode == 3) rc = z_from_point_coeffs(ctx, v, c, mode, gga, coef);
-    else rc = launch_grad_zpair(v, c.coll, gga, coef, nullptr, 3, -1);
-    if (rc || (rc = launch_plane_product(v, c.coll, za_pl, 2))) return rc;
+    if ((rc = z_from_point_coeffs(ctx, v, c, gga, coef)) ||
+        (rc = launch_plane_product(v, c.coll, 4, 2)))
+      return rc;
     if ((rc = launch_grad_contract(v, c.coll, gga, ctx->d_shell_atom, coef, nullptr,
-                                   weight_derivs, ctx->d_grad_part, gs, x_pl, 2, ctx->max_l)))
+                                   weight_derivs, ctx->d_grad_part, gs, 1, 2, ctx->max_l)))
       return rc;
     if (weight_derivs &&
         (rc = launch_ssf_grad(v, c.coll, ctx->grad_natoms, ctx->d_gxyz, ctx->d_dnear, wf,
@@ -1952,17 +1929,13 @@ int enqueue_grad(xcq_context_s* ctx, int func, int weight_derivs) {
 
 // One UKS EXC gradient: per chunk, collocation; the density stage twice (P_s,
 // then P_z; factor 1); the polarised functional's coefficients written over
-// the sums, w eps rho; Y = P_s Za_s + P_z Za_z into plane 1, X_N = P_s B
-// into plane 2 and X_Z = P_z B into plane 3 (GGA); the basis-function and
-// grid-weight parts.  In-stage mode (up to f functions): X_N and X_Z come
-// from the density passes, Za_s and Za_z in turn from k_z_in_stage through
-// plane 4.  Stored planes (g functions): Za_s into plane 4 and Za_z over
-// grad_z B in plane 3, X_N and X_Z by plane products after Y.
+// the sums, w eps rho; Za_s, then Za_z (k_z_in_stage) through plane 4: Y = P_s
+// Za_s + P_z Za_z in plane 1; the basis-function and grid-weight parts.  The
+// density passes leave X_N = P_s B in plane 2 and X_Z = P_z B in plane 3 (GGA).
 int enqueue_grad_uks(xcq_context_s* ctx, int func, int weight_derivs) {
   const int gga = (func == XCQ_FUNC_PBE || func == XCQ_FUNC_PBE0) ? 1 : 0;
-  const int mode = derivative_mode(ctx);
   CtxView v = view_of(ctx);
-  v.in_stage = mode;
+  v.in_stage = 3;
   v.tmax = nullptr;
   v.vxc_drop = 0.0;
   hipStream_t s = ctx->stream;
@@ -1980,32 +1953,19 @@ int enqueue_grad_uks(xcq_context_s* ctx, int func, int weight_derivs) {
     const WorkItem* cw = v.work + c.coll.off;
     if ((rc = launch_collocation_fp64(s, cw, c.coll.n, v.tasks, v.shells, v.shell_list, v.lsh,
                                       v.px, v.py, v.pz, static_cast<double*>(v.scratch),
-                                      gga && mode == 0, ctx->max_l)))
+                                      0, ctx->max_l)))
       return rc;
-    // In-stage mode: the density passes leave X_N in plane 2 and X_Z in
-    // plane 3 (GGA), which no gradient plane occupies.
     for (int pass = 0; pass < 2; ++pass)
       if ((rc = launch_density(v, c, XCQ_PREC_FP64, gga, 1.0, pass == 0 ? ds : dz,
                                pass == 0 ? ctx->d_P : ctx->d_Pz,
-                               (gga && mode == 3) ? 2 + pass : -1)))
+                               gga ? 2 + pass : -1)))
         return rc;
     if ((rc = launch_grad_points_uks(v, c.coll, func, gga, ds, dz, wf))) return rc;
-    if (mode == 3) {
-      // Za_s, then Za_z, through plane 4: Y = P_s Za_s + P_z Za_z in plane 1.
-      if ((rc = z_from_point_coeffs(ctx, v, c, mode, gga, ds)) ||
-          (rc = launch_plane_product(v, c.coll, 4, 1, ctx->d_P, 1.0, 0)) ||
-          (rc = z_from_point_coeffs(ctx, v, c, mode, gga, dz)) ||
-          (rc = launch_plane_product(v, c.coll, 4, 1, ctx->d_Pz, 1.0, 1)))
-        return rc;
-    } else {
-      if ((rc = launch_grad_zpair(v, c.coll, gga, ds, dz, 4, 3))) return rc;
-      if ((rc = launch_plane_product(v, c.coll, 4, 1, ctx->d_P, 1.0, 0)) ||
-          (rc = launch_plane_product(v, c.coll, 3, 1, ctx->d_Pz, 1.0, 1)))
-        return rc;
-      if (gga && ((rc = launch_plane_product(v, c.coll, 0, 2, ctx->d_P, 1.0, 0)) ||
-                  (rc = launch_plane_product(v, c.coll, 0, 3, ctx->d_Pz, 1.0, 0))))
-        return rc;
-    }
+    if ((rc = z_from_point_coeffs(ctx, v, c, gga, ds)) ||
+        (rc = launch_plane_product(v, c.coll, 4, 1, ctx->d_P, 1.0, 0)) ||
+        (rc = z_from_point_coeffs(ctx, v, c, gga, dz)) ||
+        (rc = launch_plane_product(v, c.coll, 4, 1, ctx->d_Pz, 1.0, 1)))
+      return rc;
     if ((rc = launch_grad_contract(v, c.coll, gga, ctx->d_shell_atom, ds, dz, weight_derivs,
                                    ctx->d_grad_part, gs, 2, 1, ctx->max_l)))
       return rc;

@@ -20,8 +20,9 @@
 //
 // Basis evaluation mode (template argument INSTAGE): 0 reads B and grad B
 // from the planes the collocation stage stored, and so does the Z launch
-// (k_z_from_coeffs); 3 evaluates them at the block's points from the shell
-// parameters, as does k_z_in_stage (collocation.hip).  kProductOnly stops at
+// (k_z_from_coeffs); 3 and 4 evaluate them (up to that angular momentum) at
+// the block's points from the shell parameters, as does k_z_in_stage
+// (collocation.hip).  kProductOnly stops at
 // the product, of any stored plane, for the EXC gradient.
 #include "internal.hpp"
 #include "functional.hpp"
@@ -174,7 +175,7 @@ __device__ __forceinline__ void write_z(const DevTask& t, int m0, int tid, doubl
 // fetches rows 4w .. 4w + 3 of the step, lane = function.  The rows' basis
 // functions (64 of them per vector load, a whole chunk ahead) are broadcast
 // by readlane, so no scalar load is waited for inside the K loop.
-// INSTAGE = 3: the fold evaluates B and grad B itself, from X^T written over
+// INSTAGE > 0: the fold evaluates B and grad B itself, from X^T written over
 // the stages and from the tile's shells, which were staged in LDS while the
 // product ran; 0: it reads the planes the collocation stage stored.
 //
@@ -260,7 +261,7 @@ struct FoldShells {
 // misses res^T X (res = B - B32, P symmetric), a first-order term that does
 // not average out (it biased EXC by about -3e-10 relative): rho also takes
 // sum res X.
-template <bool GGA, bool RES32, int LD, int NT>
+template <bool GGA, bool RES32, int LD, int LMAX, int NT>
 __device__ __forceinline__ void fold_staged(const ShellArgs& sa, const FoldShells<NT>& fs, int nlo,
                                             int nhi, int first, int step, const double* xt,
                                             double rx, double ry, double rz, double (&r)[4]) {
@@ -284,7 +285,7 @@ __device__ __forceinline__ void fold_staged(const ShellArgs& sa, const FoldShell
       }
     }
     double sy = 0., sgx = 0., sgy = 0., sgz = 0., sres = 0.;
-    shell_functions_l<kInStageMaxL, GGA, true, true>(
+    shell_functions_l<LMAX, GGA, true, true>(
         l, x, y, z, R, dR, pure, [&](int f, double v, double gx, double gy, double gz) {
           const int n = bf0 + f;  // uniform
           if (n >= nlo && n < nhi) {
@@ -485,7 +486,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void k_density(
           for (int r = 0; r < 4; ++r)
             lds[(16 * i + arow(r)) * kXLd + 16 * pg + lf] = acc[i][r];
         __syncthreads();
-        fold_staged<GGA, kF32, kXLd>(sa, fs, n0, nhi, wave, 4, lds + lane, rx, ry, rz, part);
+        fold_staged<GGA, kF32, kXLd, INSTAGE>(sa, fs, n0, nhi, wave, 4, lds + lane, rx, ry, rz, part);
         s_cur = uni(fs.next);
       } else if constexpr (kFold) {
         const unsigned short* lo = lo_plane(Bm, plane);
@@ -552,7 +553,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void k_density(
 // 6.1 -> 6.8; mixed precision (64-function tiles, half the bytes) lost at
 // every size (150 waters 88 -> 95).  Lane (f, q) holds the adjacent points 2f,
 // 2f + 1 of its wave's 32: one 16-byte load of B serves two MFMA columns.
-template <bool GGA>
+template <bool GGA, int LMAX>
 __global__ __launch_bounds__(256, 2) void k_density_wide(
     QueueArgs qa, const DevTask* __restrict__ tasks, const int32_t* __restrict__ bfmap,
     const double* __restrict__ Pall, double* __restrict__ scratch, double fac, ShellArgs sa,
@@ -706,7 +707,7 @@ __global__ __launch_bounds__(256, 2) void k_density_wide(
             *reinterpret_cast<v2d*>(lds + (16 * i + 4 * r + lq) * kXL + 32 * pg + 2 * lf) =
                 v2d{acc[4 * h + i][0][r], acc[4 * h + i][1][r]};
         __syncthreads();
-        fold_staged<GGA, false, kXL>(sa, fs, n0 + 64 * h, min(n0 + 64 * h + 64, nhi), wave >> 1, 2,
+        fold_staged<GGA, false, kXL, LMAX>(sa, fs, n0 + 64 * h, min(n0 + 64 * h + 64, nhi), wave >> 1, 2,
                                     lds + kPtBlock * ph + lane, rx, ry, rz, part);
       }
       s_cur = uni(fs.next);
@@ -1126,10 +1127,16 @@ int launch_density(const CtxView& v, const Chunk& c, int precision, int gga, dou
       gga ? run(k_density<T, true, 0>, P, scr, 4) : run(k_density<T, false, 0>, P, scr, 4);
       return;
     }
-    if constexpr (sizeof(T) == 8)
-      gga ? go_wide(k_density_wide<true>, P, scr) : go_wide(k_density_wide<false>, P, scr);
-    constexpr int n = sizeof(T) == 8 ? 3 : 4;
-    gga ? run(k_density<T, true, 3>, P, scr, n) : run(k_density<T, false, 3>, P, scr, n);
+    auto eval = [&](auto L) {
+      constexpr int l = decltype(L)::value;
+      if constexpr (sizeof(T) == 8)
+        gga ? go_wide(k_density_wide<true, l>, P, scr) : go_wide(k_density_wide<false, l>, P, scr);
+      constexpr int n = sizeof(T) == 8 ? 3 : 4;
+      gga ? run(k_density<T, true, l>, P, scr, n) : run(k_density<T, false, l>, P, scr, n);
+    };
+    // Mixed precision evaluates up to f functions (effective_mode).
+    if (sizeof(T) == 4 || v.max_l <= 3) eval(std::integral_constant<int, 3>{});
+    else if constexpr (sizeof(T) == 8) eval(std::integral_constant<int, 4>{});
   };
   if (precision == XCQ_PREC_FP64)
     pick(P_override ? P_override : v.P, static_cast<double*>(v.scratch));

@@ -15,10 +15,10 @@
 // so a task needs two plane products (X = 2 P_sub B for the Hessian term of
 // GGAs, Y = 2 P_sub Za) instead of four, and
 //   g_mu = grad B_mu . Y_mu + X_mu (H_mu c),  c = 2 w vgamma grad rho.
-// grad B and H c are evaluated where they are used (k_grad_contract), so the
-// chunk scratch's five planes suffice: B and grad B (collocation), X stored
-// by the density stage itself into plane 4 (GGA), Za over grad_z B in
-// plane 3 once the coefficients exist, then Y = 2 P_sub Za into plane 2.
+// grad B and H c are evaluated where they are used (k_grad_contract), and so
+// is grad B in the density stage and in Za, so of the chunk scratch's five
+// planes collocation fills only B (0); X, stored by the density stage itself,
+// goes to 1 (GGA), Za to 4, Y = 2 P_sub Za to 2.
 // The grid-weight part contracts the SSF weight derivatives with w eps rho
 // per point (k_ssf_grad).
 //
@@ -32,8 +32,7 @@
 //   c_s = g1 grad n + g2 grad m,  c_z = g2 grad n + g3 grad m,
 // g1 = (v_aa + v_ab + v_bb)/2, g2 = (v_aa - v_bb)/2, g3 = (v_aa - v_ab + v_bb)/2
 // (w vsigma folded in), and f = w eps (rho_a + rho_b) for the weight part.
-// Planes: Za_s -> 4 and Za_z -> 3 (k_grad_zpair), Y -> 1, then X_N -> 2 and
-// X_Z -> 3.
+// Planes: X_N -> 2 and X_Z -> 3, Za_s and Za_z in turn -> 4, Y -> 1.
 #include "internal.hpp"
 #include "functional.hpp"
 #include "shell_eval.hpp"
@@ -164,46 +163,6 @@ __global__ __launch_bounds__(64) void k_grad_points_uks(const WorkItem* __restri
   if (tid == 0) {
     red[2 * b] = e;
     red[2 * b + 1] = n;
-  }
-}
-
-// Za_s = a_s B + c_s . grad B into plane pl_s and, when coef_z is given,
-// Za_z = a_z B + c_z . grad B into plane pl_z (planes 3 or 4: each thread
-// reads its element's B and grad B before it writes, so plane 3 may be
-// overwritten in place) for one (task, 64-point block): lane = point, the
-// four waves take rows w, w + 4, ...
-template <bool GGA>
-__global__ __launch_bounds__(256) void k_grad_zpair(const WorkItem* __restrict__ items,
-                                                    const DevTask* __restrict__ tasks,
-                                                    double* __restrict__ scratch,
-                                                    const double* __restrict__ coef_s,
-                                                    const double* __restrict__ coef_z, int pl_s,
-                                                    int pl_z) {
-  const WorkItem wi = items[blockIdx.x];
-  const DevTask t = tasks[wi.task];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t b = t.red_off + wi.a;
-  const bool two = coef_z != nullptr;
-  double cs[4], cz[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    cs[c] = coef_s[b * 256 + c * 64 + lane];
-    cz[c] = two ? coef_z[b * 256 + c * 64 + lane] : 0.;
-  }
-  const int64_t ld = t.npts_pad;
-  const int64_t plane = (int64_t)t.nbe * ld;
-  double* B = scratch + t.b_off + (int64_t)wi.a * kPtBlock + lane;
-  for (int j = wave; j < t.nbe; j += 4) {
-    const int64_t o = (int64_t)j * ld;
-    const double bv = B[o];
-    double zs = cs[0] * bv, zz = cz[0] * bv;
-    if constexpr (GGA) {
-      const double x = B[plane + o], y = B[2 * plane + o], z = B[3 * plane + o];
-      zs += cs[1] * x + cs[2] * y + cs[3] * z;
-      zz += cz[1] * x + cz[2] * y + cz[3] * z;
-    }
-    B[pl_s * plane + o] = zs;
-    if (two) B[pl_z * plane + o] = zz;
   }
 }
 
@@ -721,22 +680,6 @@ int launch_grad_points_uks(const CtxView& v, const WorkRange& r, int func, int g
   if (r.n == 0) return XCQ_SUCCESS;
   hipLaunchKernelGGL(k_grad_points_uks, dim3((unsigned)r.n), dim3(64), 0, v.stream,
                      v.work + r.off, v.tasks, v.w, func, gga, ds, dz, v.red, wf);
-  XCQ_HIP(hipGetLastError());
-  return XCQ_SUCCESS;
-}
-
-int launch_grad_zpair(const CtxView& v, const WorkRange& r, int gga, const double* coef_s,
-                      const double* coef_z, int pl_s, int pl_z) {
-  if (r.n == 0) return XCQ_SUCCESS;
-  XCQ_REQUIRE((pl_s == 3 || pl_s == 4) && (!coef_z || ((pl_z == 3 || pl_z == 4) && pl_z != pl_s)),
-              XCQ_ERROR_INVALID_ARGUMENT, "Za planes must be 3 or 4");
-  double* scr = static_cast<double*>(v.scratch);
-  if (gga)
-    hipLaunchKernelGGL(k_grad_zpair<true>, dim3((unsigned)r.n), dim3(256), 0, v.stream,
-                       v.work + r.off, v.tasks, scr, coef_s, coef_z, pl_s, pl_z);
-  else
-    hipLaunchKernelGGL(k_grad_zpair<false>, dim3((unsigned)r.n), dim3(256), 0, v.stream,
-                       v.work + r.off, v.tasks, scr, coef_s, coef_z, pl_s, pl_z);
   XCQ_HIP(hipGetLastError());
   return XCQ_SUCCESS;
 }

@@ -175,6 +175,7 @@ struct CtxView {
                     // fills it, the B^T Z stage skips blocks bounded below vxc_drop)
   int in_stage;     // basis evaluation of the fold and the Z launch: 0 = the stored B /
                     // grad B planes; else they evaluate them (1 runs as 3)
+  int max_l;        // highest angular momentum of the basis
   const DevShellC* shc;
   double* zc;       // Z coefficients per point block [4][64] (in-stage mode 3)
   double* syr_part; // slice buffer of the SYR2K, kSyrBlocks blocks per place
@@ -187,7 +188,6 @@ struct ShellArgs {
   const int32_t* lsh;           // first local function of each task shell (ascending)
   const double *px, *py, *pz;   // point coordinates
 };
-constexpr int kInStageMaxL = 3;  // highest angular momentum it evaluates
 
 constexpr int kGran = 32;      // functions per granule of the bound table
 constexpr int kGranLds = 64;   // granules a density workgroup reduces in LDS (nbe <= 2048)
@@ -310,13 +310,9 @@ int launch_grad_contract(const CtxView& v, const WorkRange& r, int gga,
                          const int32_t* shell_atom, const double* coef_s, const double* coef_z,
                          int weight_derivs, double* part, int64_t gstride, int x_pl, int y_pl,
                          int lmax);
-// Za = a B + c . grad B from [block][4][64] coefficients into plane pl_s
-// (and, with coef_z, a second one into pl_z; planes 3 and 4 only).  UKS:
-// coefficients written over the P_s / P_z sums.
+// UKS: coefficients written over the P_s / P_z sums.
 int launch_grad_points_uks(const CtxView& v, const WorkRange& r, int func, int gga, double* ds,
                            double* dz, double* wf);
-int launch_grad_zpair(const CtxView& v, const WorkRange& r, int gga, const double* coef_s,
-                      const double* coef_z, int pl_s, int pl_z);
 int launch_ssf_grad(const CtxView& v, const WorkRange& r, int natoms, const double* xyz,
                     const double* dnear, const double* wf, double* part, int64_t gstride,
                     const int32_t* nbr_idx, const double* nbr_r);

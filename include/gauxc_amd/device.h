@@ -131,14 +131,14 @@ int xcq_set_density_wide(xcq_context ctx, int32_t wide_min_nbe);
 /* Where the rho fold and Z get the basis functions' values and gradients
  * (GauXC stores B and grad B, collocation_device_masked_combined_kernel_deriv1,
  * and reads them back in its rho and Z kernels): 3 (default) = the density
- * stage evaluates them at its points for the fold and leaves Z to a
- * separate launch that evaluates them again; 1 = the mixed density stage
- * evaluates them for both (the FP64 path runs mode 3); 0 = both read the
- * planes the collocation stage stores.  In modes 1 and 3 the collocation
- * stage stores only the value plane.  Bases with angular momentum above 3
- * always use the stored planes.  Other values: error. */
+ * stage evaluates them at its points for the fold and a separate launch
+ * evaluates them again for Z, so that the collocation stage stores only the
+ * value plane; 0 = both read the planes the collocation stage stores; 1 runs
+ * as 3.  Mixed precision with angular momentum above 3 always uses the stored
+ * planes; the UKS, FXC and gradient paths always run as 3.  Other values:
+ * error. */
 int xcq_set_density_basis_eval(xcq_context ctx, int32_t in_stage);
-/* The basis evaluation mode in effect (0 when the basis exceeds l = 3). */
+/* The basis evaluation mode set (as above). */
 int xcq_get_density_basis_eval(xcq_context ctx, int32_t* mode);
 /* B^T Z contributions with |v| < tol are not scattered into VXC (each
  * scatter-add is an FP64 atomic; on large diffuse systems most are of
