@@ -10,8 +10,8 @@ Workload (one "step" = one full EXC+VXC evaluation over every task):
   basis) are resident in HBM before the timed region; VXC stays in HBM.
 
 Both precisions run on the same resident inputs.  Before timing, the device
-autotuner picks the tile thresholds and queue count for each precision
-(untimed); the timed steps replay the captured graph of the evaluation.
+autotuner picks the basis evaluation mode, (FP64) the block-pair threshold and
+the queue count for each precision (untimed); the timed steps replay the captured graph of the evaluation.
 ``value`` is the mixed-precision rate; the FP64 rate, the speed-up and the
 mixed-vs-FP64 |dEXC| / max|dVXC| are reported beside it.
 
@@ -42,9 +42,8 @@ PEAK_BF16_TFLOPS = 2500.0
 MIXED_PEAK = {"density": PEAK_FP32_TFLOPS, "syr2k_scatter": PEAK_BF16_TFLOPS}
 PEAK_HBM_GBS = 8000.0
 STAGES = ["collocation", "density", "functional", "zmat", "syr2k_scatter", "symmetrize"]
-# Kernels of each stage (the names rocprofv3 reports); the mixed path's
-# kernels depend on its basis evaluation mode (0: stored planes, 1 / 3:
-# evaluated in the density stage, 3 with Z from its own launch).
+# Kernels of each stage (the names rocprofv3 reports) by basis evaluation mode
+# (0: stored planes, 3: evaluated in the density and Z stages).
 
 
 def stage_kernels(stage, prec, mode=0):
@@ -52,16 +51,14 @@ def stage_kernels(stage, prec, mode=0):
     if stage == "collocation":
         return [f"k_collocation<{'true' if mode == 0 else 'false'}, {t}, 3>"]
     if stage == "zmat":
-        return [f"k_z_in_stage<true, 3, {t}>"] if mode == 3 else []
-    if prec == "fp64":
-        return {"density": [f"k_density_f64<{nt}, true, {mode}>" for nt in (32, 64)],
-                "syr2k_scatter": ["k_syr2k<32>", "k_syr2k<64>"]}.get(stage, [])
+        return [f"k_z_in_stage<true, 3, {t}>" if mode == 3 else f"k_z_from_coeffs<{t}, true>"]
     if stage == "density":
-        return [f"k_density_mx<{nt}, true, {hi}, {mode}>"
-                for nt, hi in ((32, "false"), (64, "false"), (64, "true"), (128, "false"))
-                if not (hi == "true" and mode == 1)]
+        wide = ["k_density_wide<true, 3>"] if prec == "fp64" and mode == 3 else []
+        return [f"k_density<{t}, true, {mode}>"] + wide
+    if stage == "functional":
+        return ["k_xc_points"]
     if stage == "syr2k_scatter":
-        return ["k_syr2k_mx<32, 1>", "k_syr2k_mx<64, 1>"]
+        return ["k_syr2k" if prec == "fp64" else "k_syr2k_mx"]
     return []
 
 
@@ -170,10 +167,9 @@ def main():
                          "derivatives), the RKS FXC contraction and the UKS EXC/VXC on the "
                          "same workload")
     ap.add_argument("--tile-policy", default=None,
-                    help="D,S,Q[,H[,W[,M]]]: fixed density / SYR2K 32-wide thresholds, "
-                         "queue count, (mixed) density high-occupancy threshold, 128-wide "
-                         "minimum nbe and basis evaluation mode for every precision "
-                         "(skips the autotuner)")
+                    help="D,S,Q[,H[,W[,M]]]: queue count Q, FP64 block-pair minimum nbe W and "
+                         "basis evaluation mode M for every precision (D, S and H are kept "
+                         "and have no effect; skips the autotuner)")
     ap.add_argument("--copy-calibration", action="store_true",
                     help="run only a plain 1 GiB device copy (calibrates rocprofv3 "
                          "FETCH_SIZE/WRITE_SIZE against a known byte count)")
@@ -246,9 +242,8 @@ def main():
             tuned = ctx.autotune("PBE", prec)
             pol = ctx.tile_policy()
             tuned = tuned + (pol[2], pol[4], ctx.density_basis_eval())
-            log(f"{prec}: autotune -> dens32<=nbe {tuned[0]}, syr2k32<=nbe {tuned[1]}, "
-                f"queues {tuned[2]}, density hi-occupancy<=nbe {pol[2]}, "
-                f"128-wide>=nbe {pol[4]}, basis evaluation mode {tuned[6]} "
+            log(f"{prec}: autotune -> queues {tuned[2]}, block pairs from nbe {pol[4]}, "
+                f"basis evaluation mode {tuned[6]} "
                 f"({tuned[3]:.2f} ms; {time.perf_counter() - tic:.1f}s)")
         # Eager steps: per-stage HIP-event times of the kernels.
         ctx.use_graph(False)

@@ -589,6 +589,7 @@ class DeviceContext:
 
     # ---- scheduling, timing and graph controls ----
     def set_tile_policy(self, dens32_max_nbe, syr2k32_max_nbe):
+        """Thresholds of earlier kernels: kept and reported, without effect."""
         N.xcq_check(self.lib.xcq_set_tile_policy(self.h, int(dens32_max_nbe),
                                                  int(syr2k32_max_nbe)), "xcq_set_tile_policy")
 
@@ -618,10 +619,13 @@ class DeviceContext:
         return int(m.value)
 
     def set_density_wide(self, wide_min_nbe):
+        """From how many functions on FP64 density tasks run on pairs of point
+        blocks (2**30: the default rule, see xcq_set_density_wide)."""
         N.xcq_check(self.lib.xcq_set_density_wide(self.h, int(wide_min_nbe)),
                     "xcq_set_density_wide")
 
     def set_density_occupancy(self, hiocc_max_nbe):
+        """Threshold of an earlier kernel: kept and reported, without effect."""
         N.xcq_check(self.lib.xcq_set_density_occupancy(self.h, int(hiocc_max_nbe)),
                     "xcq_set_density_occupancy")
 
@@ -651,8 +655,8 @@ class DeviceContext:
         N.xcq_check(self.lib.xcq_use_graph(self.h, int(bool(on))), "xcq_use_graph")
 
     def autotune(self, func="PBE", precision="mixed"):
-        """Device autotuner (xcq_autotune): returns the chosen
-        (dens32_max_nbe, syr2k32_max_nbe, nqueues, best total ms)."""
+        """Device autotuner (xcq_autotune): returns (dens32_max_nbe,
+        syr2k32_max_nbe, nqueues, best total ms)."""
         d, s, q = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int32()
         ms = ctypes.c_double()
         N.xcq_check(self.lib.xcq_autotune(self.h, N.XCQ_FUNC[func], N.XCQ_PREC[precision],

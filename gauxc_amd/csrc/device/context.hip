@@ -202,14 +202,14 @@ struct xcq_context_s {
   int32_t* d_qoff = nullptr;
   unsigned long long* d_counters = nullptr;  // ticket counters of the dynamic queues
   int64_t ncounters = 0;
-  int32_t dens32_max_nbe = 48, syr2k32_max_nbe = 96;  // tile policy
-  int32_t dens_hiocc_max_nbe = 0;  // 64-wide density tiles at three workgroups per CU
+  // Settings of kernels that are gone (tile widths, occupancy): kept and
+  // reported, without effect.
+  int32_t dens32_max_nbe = 48, syr2k32_max_nbe = 96, dens_hiocc_max_nbe = 0;
   // FP64 density on 128-wide tiles and block pairs from this nbe on; kWideAuto:
   // from kWideNbe on in molecules whose P exceeds kWidePBytes.
   int32_t dens128_min_nbe = kWideAuto;
-  // Mixed density stage's basis evaluation (bases up to l = 3): 1 = its
-  // fold and Z evaluate B / grad B, 3 = its fold does and a separate launch
-  // forms Z, 0 = both read the planes the collocation stage stores.
+  // Basis evaluation of the density fold and Z: 3 (1 runs as 3) = in the
+  // stages, 0 = both read the planes the collocation stage stores.
   int32_t dens_in_stage = 3;
   double vxc_drop = kDefaultVxcDrop;  // see xcq_set_vxc_drop_tolerance
   int32_t nqueues = 0;                                 // 0: one workgroup per item
@@ -381,10 +381,7 @@ int build_work_lists(xcq_context_s* ctx) {
     const int32_t wide = ctx->dens128_min_nbe != kWideAuto ? ctx->dens128_min_nbe
                          : (int64_t)d.ldp * d.ldp * 8 > kWidePBytes ? kWideNbe
                                                                     : kWideAuto;
-    d.dens_cls = d.nbe <= ctx->dens32_max_nbe                               ? 0
-                 : d.nbe >= std::max(wide, 65) && d.npts > kPtBlock         ? 3
-                 : d.nbe <= ctx->dens_hiocc_max_nbe                         ? 1
-                                                                            : 2;
+    d.wide = d.nbe >= std::max(wide, 65) && d.npts > kPtBlock;
   }
   auto finish_range = [&](WorkRange& r, const std::vector<double>& cost) {
     r.n = (int64_t)W.size() - r.off;
@@ -417,13 +414,13 @@ int build_work_lists(xcq_context_s* ctx) {
   for (const auto& c : ctx->chunks)
     std::sort(order.begin() + c.task_begin, order.begin() + c.task_end);
   for (auto& c : ctx->chunks) {
-    for (int v = 3; v >= 0; --v) {  // density classes (DevTask::dens_cls)
+    for (int v = 1; v >= 0; --v) {
       c.dens[v].off = (int64_t)W.size();
       std::vector<double> cost;
       for (int32_t q = c.task_begin; q < c.task_end; ++q) {
         const int32_t i = order[q].second;
         const DevTask& d = ctx->h_tasks[i];
-        if (d.dens_cls != v) continue;
+        if (d.wide != v) continue;
         const int nmb = d.npts_pad / kPtBlock;
         const double ci = have_cost ? ctx->cost_d[i] / nmb : heur_dens_item(d);
         for (int pb = 0; pb < nmb; ++pb) {
@@ -439,7 +436,7 @@ int build_work_lists(xcq_context_s* ctx) {
       for (int32_t q = c.task_begin; q < c.task_end; ++q) {
         const int32_t i = order[q].second;
         const DevTask& d = ctx->h_tasks[i];
-        if (d.dens_cls != 3) continue;
+        if (!d.wide) continue;
         const int npair = (d.npts_pad / kPtBlock + 1) / 2;
         const double ci = have_cost ? ctx->cost_d[i] / npair : 2. * heur_dens_item(d);
         for (int pr = 0; pr < npair; ++pr) {
@@ -449,8 +446,8 @@ int build_work_lists(xcq_context_s* ctx) {
       }
       finish_range(c.dens_pair, cost);
     }
-    c.coll.off = c.dens[3].off;
-    c.coll.n = c.dens[0].n + c.dens[1].n + c.dens[2].n + c.dens[3].n;
+    c.coll.off = c.dens[1].off;
+    c.coll.n = c.dens[0].n + c.dens[1].n;
     c.coll.nq = 0;
     // SYR2K: regions and point slices.  A slice is as long as gives the chunk
     // one item per resident workgroup (3 per CU), between 256 points (below
@@ -1115,15 +1112,8 @@ int xcq_upload_tasks(xcq_context ctx, int32_t ntasks, const xcq_task* tasks, int
 
 int xcq_set_tile_policy(xcq_context ctx, int32_t dens32_max_nbe, int32_t syr2k32_max_nbe) {
   XCQ_REQUIRE(ctx, XCQ_ERROR_INVALID_ARGUMENT, "null context");
-  XCQ_HIP(hipSetDevice(ctx->device));
-  XCQ_HIP(hipStreamSynchronize(ctx->stream));
   ctx->dens32_max_nbe = dens32_max_nbe;
   ctx->syr2k32_max_nbe = syr2k32_max_nbe;
-  if (ctx->ntasks == 0) return XCQ_SUCCESS;
-  int rc = build_work_lists(ctx);
-  if (rc) return rc;
-  XCQ_HIP(hipMemcpy(ctx->d_tasks, ctx->h_tasks.data(), ctx->h_tasks.size() * sizeof(DevTask),
-                    hipMemcpyHostToDevice));
   return XCQ_SUCCESS;
 }
 
@@ -1186,14 +1176,7 @@ int xcq_get_density_basis_eval(xcq_context ctx, int32_t* mode) {
 
 int xcq_set_density_occupancy(xcq_context ctx, int32_t hiocc_max_nbe) {
   XCQ_REQUIRE(ctx, XCQ_ERROR_INVALID_ARGUMENT, "null context");
-  XCQ_HIP(hipSetDevice(ctx->device));
-  XCQ_HIP(hipStreamSynchronize(ctx->stream));
   ctx->dens_hiocc_max_nbe = hiocc_max_nbe;
-  if (ctx->ntasks == 0) return XCQ_SUCCESS;
-  int rc = build_work_lists(ctx);
-  if (rc) return rc;
-  XCQ_HIP(hipMemcpy(ctx->d_tasks, ctx->h_tasks.data(), ctx->h_tasks.size() * sizeof(DevTask),
-                    hipMemcpyHostToDevice));
   return XCQ_SUCCESS;
 }
 
@@ -1250,10 +1233,10 @@ int xcq_task_times(xcq_context ctx, double* dens_us, double* syr2k_us) {
     }
   };
   for (const auto& c : ctx->chunks) {
-    // FP64 runs class 3 as pairs, but on stored planes.
+    // FP64 runs wide tasks as pairs, but on stored planes.
     const bool pairs = !ctx->last_mixed && effective_mode(ctx, XCQ_PREC_FP64) != 0;
-    for (int v = 0; v < (pairs ? 3 : 4); ++v) add(c.dens[v], dens_us);
-    if (pairs) add(c.dens_pair, dens_us);
+    add(c.dens[0], dens_us);
+    add(pairs ? c.dens_pair : c.dens[1], dens_us);
     // The list the last evaluation ran (the other keeps older stamps).
     add(c.syr2k[ctx->last_mixed], syr2k_us);
   }
@@ -1276,9 +1259,10 @@ int xcq_autotune(xcq_context ctx, int functional, int precision, int32_t* dens32
   const bool graph = ctx->use_graph;
   ctx->use_graph = false;  // stage timing needs the eager path
   ctx->drop_graph();
-  // Median of three timed runs of (density, B^T Z) stage times.
-  auto measure = [&](double* dens_ms, double* syr_ms, double* tot_ms) -> int {
-    std::vector<double> d, sy, tt;
+  // Median of three timed runs: collocation + density + Z (the basis
+  // evaluation mode moves work between them), and everything.
+  auto measure = [&](double* dens_ms, double* tot_ms) -> int {
+    std::vector<double> d, tt;
     for (int rep = 0; rep < 4; ++rep) {
       int rc = run_pipeline(ctx, functional, precision, 1);
       if (rc) return rc;
@@ -1286,7 +1270,6 @@ int xcq_autotune(xcq_context ctx, int functional, int precision, int32_t* dens32
       xcq_stage_times(ctx, st, kStages + 1);
       if (rep == 0) continue;  // warm-up
       d.push_back(st[0] + st[1] + st[3]);
-      sy.push_back(st[4]);
       tt.push_back(st[kStages]);
     }
     auto med = [](std::vector<double>& v) {
@@ -1294,117 +1277,38 @@ int xcq_autotune(xcq_context ctx, int functional, int precision, int32_t* dens32
       return v[v.size() / 2];
     };
     *dens_ms = med(d);
-    *syr_ms = med(sy);
     *tot_ms = med(tt);
     return XCQ_SUCCESS;
   };
-  const int32_t cand[] = {0, 32, 48, 64, 96, 128, 192, 256, 1 << 30};
-  int32_t best_d = ctx->dens32_max_nbe, best_s = ctx->syr2k32_max_nbe;
-  double bd = 1e300, bs = 1e300, tot = 0.;
   int rc;
-  // The density-side times below are collocation + density + the Z launch:
-  // the basis evaluation mode moves work between them.  The two stages' tile
-  // thresholds are disjoint: sweep both at once and keep the best of each.
-  for (int32_t c : cand) {
-    if ((rc = xcq_set_tile_policy(ctx, c, c))) return rc;
-    double dm, sm;
-    if ((rc = measure(&dm, &sm, &tot))) return rc;
-    if (dm < bd) {
-      bd = dm;
-      best_d = c;
-    }
-    if (sm < bs) {
-      bs = sm;
-      best_s = c;
-    }
-  }
-  if ((rc = xcq_set_tile_policy(ctx, best_d, best_s))) return rc;
-  {
-    // Per basis evaluation mode (in-stage first, when the basis allows it):
-    // the 32-wide threshold, which 64-wide tasks run at three workgroups per
-    // CU (mixed precision, and the FP64 in-stage kernel) and, for mixed
-    // precision, from which nbe on 128-wide tiles are used; the mode with
-    // the best collocation + density (+ Z launch) time wins.
-    const bool mixed = precision == XCQ_PREC_MIXED;
-    struct Pol {
-      int32_t mode, d, h, w;
-      double ms;
-    };
-    std::vector<int32_t> modes;
-    if (precision == XCQ_PREC_FP64 || ctx->max_l <= 3) modes.push_back(3);
-    modes.push_back(0);
-    Pol best{ctx->dens_in_stage, best_d, ctx->dens_hiocc_max_nbe, ctx->dens128_min_nbe, 1e300};
-    for (int32_t mode : modes) {
-      if ((rc = xcq_set_density_basis_eval(ctx, mode))) return rc;
-      Pol p{mode, best_d, 0, 1 << 30, 1e300};
-      if ((rc = xcq_set_density_occupancy(ctx, 0))) return rc;
-      if ((rc = xcq_set_density_wide(ctx, 1 << 30))) return rc;
-      for (int32_t c : cand) {
-        if ((rc = xcq_set_tile_policy(ctx, c, best_s))) return rc;
-        double dm, sm;
-        if ((rc = measure(&dm, &sm, &tot))) return rc;
-        if (dm < p.ms) {
-          p.ms = dm;
-          p.d = c;
-        }
+  // Per basis evaluation mode, and for FP64 in the stages per threshold of the
+  // block-pair kernel; the fastest pair wins.
+  struct {
+    int32_t mode, wide;
+    double ms = 1e300;
+  } best{ctx->dens_in_stage, ctx->dens128_min_nbe};
+  const bool fp64 = precision == XCQ_PREC_FP64;
+  if (fp64 && (rc = xcq_set_density_wide(ctx, kWideAuto))) return rc;
+  for (int32_t mode : {3, 0}) {
+    if (mode == 3 && !fp64 && ctx->max_l > 3) continue;  // always on stored planes
+    if ((rc = xcq_set_density_basis_eval(ctx, mode))) return rc;
+    for (int32_t wide : {kWideAuto, INT32_MAX, 128, 192, 256, 384, 512}) {
+      if (wide != kWideAuto) {
+        if (!fp64 || mode == 0) break;  // the kernels of these do not depend on it
+        if ((rc = xcq_set_density_wide(ctx, wide))) return rc;
       }
-      if ((rc = xcq_set_tile_policy(ctx, p.d, best_s))) return rc;
-      if ((mixed && mode != 1) || (!mixed && mode == 3)) {
-        for (int32_t c : cand) {
-          if ((rc = xcq_set_density_occupancy(ctx, c))) return rc;
-          double dm, sm;
-          if ((rc = measure(&dm, &sm, &tot))) return rc;
-          if (dm < p.ms) {
-            p.ms = dm;
-            p.h = c;
-          }
-        }
-        if ((rc = xcq_set_density_occupancy(ctx, p.h))) return rc;
-      }
-      for (int32_t c : {128, 192, 256, 384, 512, 1 << 30}) {
-        if (!mixed) break;
-        if ((rc = xcq_set_density_wide(ctx, c))) return rc;
-        double dm, sm;
-        if ((rc = measure(&dm, &sm, &tot))) return rc;
-        if (dm < p.ms) {
-          p.ms = dm;
-          p.w = c;
-        }
-      }
-      if (p.ms < best.ms) best = p;
-    }
-    // A second pass over the 32-wide and the occupancy thresholds in the
-    // winning mode, the other settings at their chosen values: the first
-    // pass picked the 32-wide threshold with every 64-wide task at two
-    // workgroups per CU, and the two thresholds interact.
-    if ((rc = xcq_set_density_basis_eval(ctx, best.mode))) return rc;
-    if ((rc = xcq_set_density_occupancy(ctx, best.h))) return rc;
-    if ((rc = xcq_set_density_wide(ctx, best.w))) return rc;
-    for (int32_t c : cand) {
-      if ((rc = xcq_set_tile_policy(ctx, c, best_s))) return rc;
-      double dm, sm;
-      if ((rc = measure(&dm, &sm, &tot))) return rc;
+      double dm, tot;
+      if ((rc = measure(&dm, &tot))) return rc;
       if (dm < best.ms) {
+        best.mode = mode;
+        best.wide = wide;
         best.ms = dm;
-        best.d = c;
       }
     }
-    if ((rc = xcq_set_tile_policy(ctx, best.d, best_s))) return rc;
-    if ((mixed && best.mode != 1) || (!mixed && best.mode == 3)) {
-      for (int32_t c : cand) {
-        if ((rc = xcq_set_density_occupancy(ctx, c))) return rc;
-        double dm, sm;
-        if ((rc = measure(&dm, &sm, &tot))) return rc;
-        if (dm < best.ms) {
-          best.ms = dm;
-          best.h = c;
-        }
-      }
-    }
-    best_d = best.d;
-    if ((rc = xcq_set_tile_policy(ctx, best.d, best_s))) return rc;
-    if ((rc = xcq_set_density_occupancy(ctx, best.h))) return rc;
+    if (fp64 && (rc = xcq_set_density_wide(ctx, kWideAuto))) return rc;
   }
+  if ((rc = xcq_set_density_basis_eval(ctx, best.mode))) return rc;
+  if (fp64 && (rc = xcq_set_density_wide(ctx, best.wide))) return rc;
   // Persistent workgroups on dynamic queues (at least as many as any stage
   // kernel keeps resident per CU; surplus ones find the queues empty)
   // against one workgroup per item.
@@ -1421,8 +1325,8 @@ int xcq_autotune(xcq_context ctx, int functional, int precision, int32_t* dens32
     if ((rc = xcq_set_schedule(ctx, q, keep_d.empty() ? nullptr : keep_d.data(),
                                keep_s.empty() ? nullptr : keep_s.data())))
       return rc;
-    double dm, sm, tm;
-    if ((rc = measure(&dm, &sm, &tm))) return rc;
+    double dm, tm;
+    if ((rc = measure(&dm, &tm))) return rc;
     if (tm < bt) {
       bt = tm;
       best_q = q;
@@ -1432,8 +1336,8 @@ int xcq_autotune(xcq_context ctx, int functional, int precision, int32_t* dens32
                              keep_s.empty() ? nullptr : keep_s.data())))
     return rc;
   ctx->use_graph = graph;
-  if (dens32_max_nbe) *dens32_max_nbe = best_d;
-  if (syr2k32_max_nbe) *syr2k32_max_nbe = best_s;
+  if (dens32_max_nbe) *dens32_max_nbe = ctx->dens32_max_nbe;
+  if (syr2k32_max_nbe) *syr2k32_max_nbe = ctx->syr2k32_max_nbe;
   if (nqueues) *nqueues = best_q;
   if (best_ms) *best_ms = bt;
   return XCQ_SUCCESS;

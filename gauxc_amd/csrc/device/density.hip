@@ -1106,33 +1106,29 @@ int launch_density(const CtxView& v, const Chunk& c, int precision, int gga, dou
                          queue_args(v, c.dens_pair), v.tasks, v.bfmap, P, scr, fac, sa, dens_out,
                          x_plane);
   };
-  // Classes [0, n): one launch, but for queues, which each class has of its
-  // own.  The classes' items lie one after the other, the highest first.
-  auto run = [&](auto kern, const auto* P, auto* scr, int n) {
-    if (c.dens[0].nq || c.dens[1].nq || c.dens[2].nq || c.dens[3].nq) {
-      for (int k = n - 1; k >= 0; --k) go(kern, c.dens[k], P, scr);
+  // The blocks of all tasks, or without the wide ones: one launch, but for
+  // queues, which each list has of its own.
+  auto run = [&](auto kern, const auto* P, auto* scr, bool all) {
+    if (c.dens[0].nq || c.dens[1].nq) {
+      if (all) go(kern, c.dens[1], P, scr);
+      go(kern, c.dens[0], P, scr);
     } else {
-      WorkRange r = c.coll;
-      if (n == 3) {
-        r.off += c.dens[3].n;
-        r.n -= c.dens[3].n;
-      }
-      go(kern, r, P, scr);
+      go(kern, all ? c.coll : c.dens[0], P, scr);
     }
   };
-  // Any in-stage mode is the kernels' one (3).  FP64 runs class 3 as pairs.
+  // In-stage, FP64 runs the wide tasks as pairs.
   auto pick = [&](const auto* P, auto* scr) {
     using T = std::remove_pointer_t<decltype(scr)>;
     if (v.in_stage == 0) {
-      gga ? run(k_density<T, true, 0>, P, scr, 4) : run(k_density<T, false, 0>, P, scr, 4);
+      gga ? run(k_density<T, true, 0>, P, scr, true) : run(k_density<T, false, 0>, P, scr, true);
       return;
     }
     auto eval = [&](auto L) {
       constexpr int l = decltype(L)::value;
       if constexpr (sizeof(T) == 8)
         gga ? go_wide(k_density_wide<true, l>, P, scr) : go_wide(k_density_wide<false, l>, P, scr);
-      constexpr int n = sizeof(T) == 8 ? 3 : 4;
-      gga ? run(k_density<T, true, l>, P, scr, n) : run(k_density<T, false, l>, P, scr, n);
+      constexpr bool all = sizeof(T) == 4;
+      gga ? run(k_density<T, true, l>, P, scr, all) : run(k_density<T, false, l>, P, scr, all);
     };
     // Mixed precision evaluates up to f functions (effective_mode).
     if (sizeof(T) == 4 || v.max_l <= 3) eval(std::integral_constant<int, 3>{});

@@ -66,8 +66,7 @@ struct DevTask {
   int32_t npts_pad;   // npts rounded up to kPtBlock
   int32_t mol;        // molecule of the task
   int32_t ldp;        // nbf of the molecule = leading dimension of its P and VXC
-  int32_t dens_cls;   // density work list: 0 to 2 by the tile policy's thresholds, 3 =
-                      // 128-wide tiles on pairs of point blocks
+  int32_t wide;       // FP64 density on pairs of point blocks (k_density_wide)
   int64_t pt_off;     // points (SoA) / weights
   int64_t sh_off;     // shell list
   int64_t bf_off;     // local -> molecule basis function map (nbe entries)
@@ -114,9 +113,9 @@ struct QueueArgs {
 struct Chunk {
   int32_t task_begin = 0, task_end = 0;
   int64_t scratch_elems = 0;  // elements of T (FP64 or FP32) used by B-family arrays
-  WorkRange coll;             // all point blocks (collocation) = dens[3..0] back to back
-  WorkRange dens[4];          // density blocks by class (DevTask::dens_cls)
-  WorkRange dens_pair;        // pairs of density blocks of class 3
+  WorkRange coll;             // all point blocks (collocation) = dens[1], dens[0] back to back
+  WorkRange dens[2];          // density blocks by DevTask::wide
+  WorkRange dens_pair;        // pairs of density blocks of the wide tasks
   // SYR2K (FP64, mixed), per region and point slice: a = row group | column
   // group << 16, b = slice | slices << 16, c = place in the slice buffer
   // (slices > 1); and per region with several slices: a as above, b =

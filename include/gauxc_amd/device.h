@@ -116,17 +116,15 @@ int xcq_download_results_mol(xcq_context ctx, int32_t mol, double* exc, double* 
 
 /* ---- scheduling (no GauXC counterpart beyond the task sort of
  *      incore_replicated_xc_device_integrator_exc_vxc.hpp:253-257) ----
- * Tile policy: tasks with nbe <= dens32_max_nbe run the density stage with
- * 32-function tiles (else 64); likewise syr2k32_max_nbe for B^T Z. */
+ * Tile thresholds and density occupancy of earlier kernels: kept and reported,
+ * without effect (the kernels now take as many 16-function blocks as a task
+ * has). */
 int xcq_set_tile_policy(xcq_context ctx, int32_t dens32_max_nbe, int32_t syr2k32_max_nbe);
-/* Density tasks with 64-function tiles and nbe <= hiocc_max_nbe run in
- * the kernel configuration that fits three workgroups per CU (mixed: a
- * two-block operand ring; FP64: the in-stage kernel's register budget);
- * larger ones keep two workgroups per CU.  0 (default) disables it. */
 int xcq_set_density_occupancy(xcq_context ctx, int32_t hiocc_max_nbe);
-/* Mixed precision: density tasks with nbe >= wide_min_nbe (and above the
- * 32-wide threshold) use 128-function tiles (the FP64 path keeps 64).
- * Default: off (2^30). */
+/* FP64 density tasks with nbe >= wide_min_nbe (at least 65, and more than 64
+ * points) run on pairs of 64-point blocks with 128-function tiles.  Default
+ * (2^30): from 256 functions on in molecules whose P exceeds 64 MB, where the
+ * smaller tiles are bound by L2 misses.  Mixed precision does not use it. */
 int xcq_set_density_wide(xcq_context ctx, int32_t wide_min_nbe);
 /* Where the rho fold and Z get the basis functions' values and gradients
  * (GauXC stores B and grad B, collocation_device_masked_combined_kernel_deriv1,
@@ -176,15 +174,12 @@ int xcq_task_times(xcq_context ctx, double* dens_us, double* syr2k_us);
  * Stage times then report only the total (stage 6). */
 int xcq_use_graph(xcq_context ctx, int enable);
 /* Autotuner: times the uploaded workload on the device and keeps the
- * fastest settings.  Sweeps the 32/64 tile thresholds of the density and
- * B^T Z stages (nbe buckets {0, 32, 48, 64, 96, 128, 192, 256, all}); per
- * basis evaluation mode (3 when the basis allows it, then 0) the density
- * 32-wide threshold and, for mixed precision, the occupancy threshold over
- * the same buckets and the 128-wide threshold over {128, 192, 256, 384,
- * 512, off}, keeping the mode with the fastest collocation + density + Z
- * launch; then the persistent-queue count {0, 2, 4 per CU}.  Leaves the context on the best and reports the 32-wide
- * thresholds and queue count (any output pointer may be NULL;
- * xcq_get_tile_policy and xcq_get_density_basis_eval return the rest). */
+ * fastest settings: the basis evaluation mode (3, then 0) by collocation +
+ * density + Z, for FP64 in mode 3 with the block-pair threshold (default, off,
+ * 128, 192, 256, 384, 512); then the persistent-queue count {0, 4, 8 per CU}
+ * by the whole evaluation.  Reports the queue count and, unchanged, the tile
+ * thresholds (any output pointer may be NULL; xcq_get_tile_policy and
+ * xcq_get_density_basis_eval return the rest). */
 int xcq_autotune(xcq_context ctx, int functional, int precision, int32_t* dens32_max_nbe,
                  int32_t* syr2k32_max_nbe, int32_t* nqueues, double* best_ms);
 
