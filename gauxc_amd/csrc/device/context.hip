@@ -6,17 +6,18 @@
 //   shells      DevShell[nshells] of every molecule, molecule after molecule
 //   px/py/pz/w  SoA points and weights of all tasks, in upload order
 //   shell list, local->molecule basis map, local shell -> first function
-//   work        per chunk: [density items, 32-wide | 64-wide]
-//                          [SYR2K tiles,   32-wide | 64-wide]
+//   work        per chunk: [density blocks, wide tasks | others]
+//                          [pairs of blocks of the wide tasks]
+//                          [SYR2K regions x slices, slice sums; FP64 | mixed]
 //   qoff        queue tables of the persistent launches
 //   P, VXC      per molecule nbf x nbf, column-major, ld = nbf, concatenated
 //   P (FP32)    FP32 copy of P (mixed precision), same offsets
 //   red         (w eps rho, w rho) per point block, molecule-major
 // Chunk scratch (reused by every chunk): per task [5][nbe][npts_pad]
 // (B, dB/dx, dB/dy, dB/dz, Z).  Tasks are grouped greedily into chunks that
-// fit the arena; each chunk is one launch per stage and tile width, so every
-// launch carries thousands of workgroups (or one persistent workgroup per
-// queue).
+// fit the arena; each chunk is one launch per stage (two where FP64 density
+// has wide tasks), so every launch carries thousands of workgroups (or one
+// persistent workgroup per queue).
 #include "internal.hpp"
 
 #include <algorithm>

@@ -71,7 +71,7 @@ using Vec4 = T __attribute__((ext_vector_type(4)));
 // block's points (B with its residual; float bits, so unsigned max orders
 // them): LDS atomics into smax, then one device atomic per granule into the
 // task's bound table (direct device atomics when the task has more granules
-// than smax holds).  The B^T Z stage skips a tile pair when
+// than smax holds).  The B^T Z stage leaves out a block when
 // npts * (max|B_i| max|Z_j| + max|Z_i| max|B_j|) is below the drop tolerance.
 template <typename T, bool GGA, int kZRows = sizeof(T) == 4 ? 4 : 2>
 __device__ __forceinline__ void write_z(const DevTask& t, int m0, int tid, double (*zc)[64],

@@ -161,10 +161,10 @@ __global__ __launch_bounds__(256, 2) void k_syr2k_mx(QueueArgs qa,
         const_cast<float*>(Bm + 4 * (int64_t)plane), 0, (int)(plane * 4u), 0x00020000);
     const auto rsL = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float*>(Bm + 5 * (int64_t)plane), 0, (int)(plane * 2u), 0x00020000);
-    int off[kLoads];  // element of the loader's row and point group
+    unsigned off[kLoads];  // element of the loader's row and point group
 #pragma unroll
     for (int e = 0; e < kLoads; ++e)
-      off[e] = (16 * block_of(min(wave + 4 * e, nst - 1)) + wf) * ld + 8 * wq;
+      off[e] = (unsigned)(16 * block_of(min(wave + 4 * e, nst - 1)) + wf) * (unsigned)ld + 8 * wq;
     struct Raw {
       v4u b[2], z[2], lo;
     };
@@ -176,12 +176,12 @@ __global__ __launch_bounds__(256, 2) void k_syr2k_mx(QueueArgs qa,
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           raw[e].b[h] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(
-                                                 rsB, off[e] * 4 + 16 * h, so * 4, 0));
+                                                 rsB, (int)(off[e] * 4u + 16u * h), so * 4, 0));
           raw[e].z[h] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(
-                                                 rsZ, off[e] * 4 + 16 * h, so * 4, 0));
+                                                 rsZ, (int)(off[e] * 4u + 16u * h), so * 4, 0));
         }
         raw[e].lo = __builtin_bit_cast(
-            v4u, __builtin_amdgcn_raw_buffer_load_b128(rsL, off[e] * 2, so * 2, 0));
+            v4u, __builtin_amdgcn_raw_buffer_load_b128(rsL, (int)(off[e] * 2u), so * 2, 0));
       }
     };
     auto split = [&](const v4u (&x)[2], v4u* dst) {
