@@ -51,7 +51,8 @@ def stage_kernels(stage, prec, mode=0):
     if stage == "collocation":
         return [f"k_collocation<{'true' if mode == 0 else 'false'}, {t}, 3>"]
     if stage == "zmat":
-        return [f"k_z_in_stage<true, 3, {t}>" if mode == 3 else f"k_z_from_coeffs<{t}, true>"]
+        # (Mode 0 counts Z's work with the density stage.)
+        return [f"k_z_in_stage<true, 3, {t}>"] if mode == 3 else []
     if stage == "density":
         wide = ["k_density_wide<true, 3>"] if prec == "fp64" and mode == 3 else []
         return [f"k_density<{t}, true, {mode}>"] + wide
