@@ -202,7 +202,6 @@ struct xcq_context_s {
   WorkItem* d_work = nullptr;
   int32_t* d_qoff = nullptr;
   unsigned long long* d_counters = nullptr;  // ticket counters of the dynamic queues
-  int64_t ncounters = 0;
   // Settings of kernels that are gone (tile widths, occupancy): kept and
   // reported, without effect.
   int32_t dens32_max_nbe = 48, syr2k32_max_nbe = 96, dens_hiocc_max_nbe = 0;
@@ -513,8 +512,12 @@ int build_work_lists(xcq_context_s* ctx) {
   int rc;
   if ((rc = dalloc(&ctx->d_work, W.size()))) return rc;
   if ((rc = dalloc(&ctx->d_qoff, Q.size()))) return rc;
-  ctx->ncounters = ncounters;
-  if (ncounters && (rc = dalloc(&ctx->d_counters, (size_t)ncounters))) return rc;
+  // Zero once (the bits of 0.0): every queued launch leaves its counters at
+  // zero (next_ticket).
+  if (ncounters &&
+      ((rc = dalloc(&ctx->d_counters, (size_t)ncounters)) ||
+       (rc = launch_fill(ctx->stream, reinterpret_cast<double*>(ctx->d_counters), ncounters))))
+    return rc;
   if (ctx->timing && (rc = dalloc(&ctx->d_tstamp, 2 * W.size()))) return rc;
   if (!W.empty())
     XCQ_HIP(hipMemcpy(ctx->d_work, W.data(), W.size() * sizeof(WorkItem), hipMemcpyHostToDevice));
@@ -558,12 +561,6 @@ int enqueue_pipeline(xcq_context_s* ctx, int func, int precision, int want_vxc, 
   int rc;
   if (want_vxc && (rc = launch_fill(s, ctx->d_vxc, ctx->p_total))) return rc;
   if (want_vxc && (rc = launch_fill(s, ctx->d_tmax, ctx->tmax_total))) return rc;
-  // Ticket counters of the dynamic queues start at zero (a fill kernel, not
-  // a memset node, so graph replays reset them too; zero has the same bits
-  // as 0.0).
-  if (ctx->ncounters &&
-      (rc = launch_fill(s, reinterpret_cast<double*>(ctx->d_counters), ctx->ncounters)))
-    return rc;
   int64_t launches = want_vxc ? 1 : 0, items = 0;
   auto rec = [&](hipEvent_t e) { return events ? hipEventRecord(e, s) : hipSuccess; };
   for (size_t ci = 0; ci < ctx->chunks.size(); ++ci) {
@@ -1471,9 +1468,6 @@ int enqueue_uks(xcq_context_s* ctx, int func, int want_vxc) {
   if (want_vxc && ((rc = launch_fill(s, ctx->d_vxc, ctx->p_total)) ||
                    (rc = launch_fill(s, ctx->d_vxcz, ctx->p_total))))
     return rc;
-  if (ctx->ncounters &&
-      (rc = launch_fill(s, reinterpret_cast<double*>(ctx->d_counters), ctx->ncounters)))
-    return rc;
   for (const Chunk& c : ctx->chunks) {
     const WorkItem* cw = v.work + c.coll.off;
     if ((rc = launch_collocation_fp64(s, cw, c.coll.n, v.tasks, v.shells, v.shell_list, v.lsh,
@@ -1578,9 +1572,6 @@ int enqueue_fxc(xcq_context_s* ctx, int func) {
   double* zc = dt + blk;
   int rc;
   if ((rc = launch_fill(s, ctx->d_vxc, ctx->p_total))) return rc;
-  if (ctx->ncounters &&
-      (rc = launch_fill(s, reinterpret_cast<double*>(ctx->d_counters), ctx->ncounters)))
-    return rc;
   for (const Chunk& c : ctx->chunks) {
     const WorkItem* cw = v.work + c.coll.off;
     if ((rc = launch_collocation_fp64(s, cw, c.coll.n, v.tasks, v.shells, v.shell_list, v.lsh,
@@ -1667,9 +1658,6 @@ int enqueue_fxc_uks(xcq_context_s* ctx, int func) {
   int rc;
   if ((rc = launch_fill(s, ctx->d_vxc, ctx->p_total)) ||
       (rc = launch_fill(s, ctx->d_vxcz, ctx->p_total)))
-    return rc;
-  if (ctx->ncounters &&
-      (rc = launch_fill(s, reinterpret_cast<double*>(ctx->d_counters), ctx->ncounters)))
     return rc;
   for (const Chunk& c : ctx->chunks) {
     const WorkItem* cw = v.work + c.coll.off;
@@ -1803,9 +1791,6 @@ int enqueue_grad(xcq_context_s* ctx, int func, int weight_derivs) {
   int rc;
   const int64_t gs = grad_stride(ctx->grad_natoms);
   if ((rc = launch_fill(s, ctx->d_grad_part, kGradCopies * gs))) return rc;
-  if (ctx->ncounters &&
-      (rc = launch_fill(s, reinterpret_cast<double*>(ctx->d_counters), ctx->ncounters)))
-    return rc;
   for (const Chunk& c : ctx->chunks) {
     const WorkItem* cw = v.work + c.coll.off;
     if ((rc = launch_collocation_fp64(s, cw, c.coll.n, v.tasks, v.shells, v.shell_list, v.lsh,
@@ -1851,9 +1836,6 @@ int enqueue_grad_uks(xcq_context_s* ctx, int func, int weight_derivs) {
   int rc;
   const int64_t gs = grad_stride(ctx->grad_natoms);
   if ((rc = launch_fill(s, ctx->d_grad_part, kGradCopies * gs))) return rc;
-  if (ctx->ncounters &&
-      (rc = launch_fill(s, reinterpret_cast<double*>(ctx->d_counters), ctx->ncounters)))
-    return rc;
   for (const Chunk& c : ctx->chunks) {
     const WorkItem* cw = v.work + c.coll.off;
     if ((rc = launch_collocation_fp64(s, cw, c.coll.n, v.tasks, v.shells, v.shell_list, v.lsh,
