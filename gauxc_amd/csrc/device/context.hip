@@ -260,6 +260,7 @@ struct xcq_context_s {
   double* d_tmax = nullptr;   // bound table: one {float, float} per function granule
   int64_t tmax_total = 0;
   bool last_mixed = false;   // the last evaluation ran the mixed kernels
+  int last_mode = 3;         // basis evaluation mode the last evaluation ran in
   int last_want_vxc = 0;     // the last evaluation returns VXC
   int last_vxc_eval = 0;     // the last evaluation computed VXC
 
@@ -651,6 +652,7 @@ int run_pipeline(xcq_context_s* ctx, int func, int precision, int want_vxc) {
     ctx->pf32_valid = true;
   }
   ctx->last_mixed = precision == XCQ_PREC_MIXED;
+  ctx->last_mode = effective_mode(ctx, precision);
   ctx->last_want_vxc = want_vxc;
   ctx->last_uks = false;
   ctx->last_fxc = false;
@@ -1231,8 +1233,8 @@ int xcq_task_times(xcq_context ctx, double* dens_us, double* syr2k_us) {
     }
   };
   for (const auto& c : ctx->chunks) {
-    // FP64 runs wide tasks as pairs, but on stored planes.
-    const bool pairs = !ctx->last_mixed && effective_mode(ctx, XCQ_PREC_FP64) != 0;
+    // FP64 runs wide tasks as pairs, but not on stored planes.
+    const bool pairs = !ctx->last_mixed && ctx->last_mode != 0;
     add(c.dens[0], dens_us);
     add(pairs ? c.dens_pair : c.dens[1], dens_us);
     // The list the last evaluation ran (the other keeps older stamps).
@@ -1527,6 +1529,7 @@ int xcq_exc_vxc_uks(xcq_context ctx, int functional, int want_vxc) {
   if ((rc = ensure_point_buffers(ctx))) return rc;
   if (!ctx->d_vxcz && (rc = dalloc(&ctx->d_vxcz, (size_t)ctx->p_total))) return rc;
   ctx->last_mixed = false;
+  ctx->last_mode = 3;
   ctx->last_want_vxc = want_vxc ? 1 : 0;
   ctx->last_vxc_eval = want_vxc ? 1 : 0;
   ctx->last_graph = false;
@@ -1625,6 +1628,7 @@ int xcq_fxc_contraction(xcq_context ctx, int functional) {
   int rc;
   if ((rc = ensure_point_buffers(ctx))) return rc;
   ctx->last_mixed = false;
+  ctx->last_mode = 3;
   ctx->last_want_vxc = 0;
   ctx->last_vxc_eval = 0;
   ctx->last_graph = false;
@@ -1722,6 +1726,7 @@ int xcq_fxc_contraction_uks(xcq_context ctx, int functional) {
     return rc;
   if (!ctx->d_vxcz && (rc = dalloc(&ctx->d_vxcz, (size_t)ctx->p_total))) return rc;
   ctx->last_mixed = false;
+  ctx->last_mode = 3;
   ctx->last_want_vxc = 0;
   ctx->last_vxc_eval = 0;
   ctx->last_graph = false;
@@ -1932,6 +1937,7 @@ int grad_prepare(xcq_context_s* ctx, int functional, int32_t natoms, const doubl
   }
   if ((rc = ensure_point_buffers(ctx))) return rc;
   ctx->last_mixed = false;
+  ctx->last_mode = 3;
   ctx->last_want_vxc = 0;
   ctx->last_vxc_eval = 0;
   ctx->last_graph = false;
