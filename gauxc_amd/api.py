@@ -612,7 +612,9 @@ class DeviceContext:
                     "xcq_set_density_basis_eval")
 
     def density_basis_eval(self):
-        """The basis evaluation mode set (see set_density_basis_eval)."""
+        """The basis evaluation mode in effect for the precision of the last
+        evaluation (see set_density_basis_eval; mixed precision with g
+        functions: 0)."""
         m = ctypes.c_int32(0)
         N.xcq_check(self.lib.xcq_get_density_basis_eval(self.h, ctypes.byref(m)),
                     "xcq_get_density_basis_eval")

@@ -1170,7 +1170,8 @@ int xcq_set_density_basis_eval(xcq_context ctx, int32_t in_stage) {
 
 int xcq_get_density_basis_eval(xcq_context ctx, int32_t* mode) {
   XCQ_REQUIRE(ctx && mode, XCQ_ERROR_INVALID_ARGUMENT, "null argument");
-  *mode = ctx->dens_in_stage;
+  const int precision = ctx->last_mixed ? XCQ_PREC_MIXED : XCQ_PREC_FP64;
+  *mode = effective_mode(ctx, precision) == 0 ? 0 : ctx->dens_in_stage;
   return XCQ_SUCCESS;
 }
 

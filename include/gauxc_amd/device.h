@@ -136,7 +136,9 @@ int xcq_set_density_wide(xcq_context ctx, int32_t wide_min_nbe);
  * planes; the UKS, FXC and gradient paths always run as 3.  Other values:
  * error. */
 int xcq_set_density_basis_eval(xcq_context ctx, int32_t in_stage);
-/* The basis evaluation mode set (as above). */
+/* The basis evaluation mode in effect for the precision of the last evaluation
+ * (FP64 before the first): the mode set, but 0 for mixed precision with angular
+ * momentum above 3. */
 int xcq_get_density_basis_eval(xcq_context ctx, int32_t* mode);
 /* B^T Z contributions with |v| < tol are not scattered into VXC (each
  * scatter-add is an FP64 atomic; on large diffuse systems most are of
