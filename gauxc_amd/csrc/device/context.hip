@@ -1290,8 +1290,11 @@ int xcq_autotune(xcq_context ctx, int functional, int precision, int32_t* dens32
   } best{ctx->dens_in_stage, ctx->dens128_min_nbe};
   const bool fp64 = precision == XCQ_PREC_FP64;
   if (fp64 && (rc = xcq_set_density_wide(ctx, kWideAuto))) return rc;
+  // Mixed precision with g functions runs on stored planes whatever the mode:
+  // nothing to choose, and the mode set stays for FP64 evaluations.
+  const bool fixed = !fp64 && ctx->max_l > 3;
   for (int32_t mode : {3, 0}) {
-    if (mode == 3 && !fp64 && ctx->max_l > 3) continue;  // always on stored planes
+    if (fixed) break;
     if ((rc = xcq_set_density_basis_eval(ctx, mode))) return rc;
     for (int32_t wide : {kWideAuto, INT32_MAX, 128, 192, 256, 384, 512}) {
       if (wide != kWideAuto) {

@@ -179,8 +179,9 @@ int xcq_use_graph(xcq_context ctx, int enable);
  * fastest settings: the basis evaluation mode (3, then 0) by collocation +
  * density + Z, for FP64 in mode 3 with the block-pair threshold (default, off,
  * 128, 192, 256, 384, 512); then the persistent-queue count {0, 4, 8 per CU}
- * by the whole evaluation.  Reports the queue count and, unchanged, the tile
- * thresholds (any output pointer may be NULL; xcq_get_tile_policy and
+ * by the whole evaluation.  Mixed precision with angular momentum above 3 has
+ * no mode to choose and leaves the one set.  Reports the queue count and,
+ * unchanged, the tile thresholds (any output pointer may be NULL; xcq_get_tile_policy and
  * xcq_get_density_basis_eval return the rest). */
 int xcq_autotune(xcq_context ctx, int functional, int precision, int32_t* dens32_max_nbe,
                  int32_t* syr2k32_max_nbe, int32_t* nqueues, double* best_ms);

@@ -1,4 +1,4 @@
-"""Which basis evaluation mode a context with g functions reports:
+"""Which basis evaluation mode a context with g functions reports and keeps:
 mixed precision always runs on stored planes (0), FP64 as set."""
 import numpy as np
 import pytest
@@ -26,5 +26,14 @@ def test_mode_in_effect_with_g_functions(ctx):
         ctx.set_density_basis_eval(mode)
         ctx.exc_vxc("PBE", "mixed")
         assert ctx.density_basis_eval() == 0
+        ctx.exc_vxc("PBE", "fp64")
+        assert ctx.density_basis_eval() == mode
+
+
+def test_mixed_autotune_leaves_the_mode_of_fp64(ctx):
+    for mode in (3, 1, 0):
+        print(f"mixed autotuner, mode {mode}", flush=True)
+        ctx.set_density_basis_eval(mode)
+        ctx.autotune("PBE", "mixed")
         ctx.exc_vxc("PBE", "fp64")
         assert ctx.density_basis_eval() == mode
