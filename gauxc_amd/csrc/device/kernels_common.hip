@@ -7,6 +7,8 @@
 #include "functional.hpp"
 #include "ssf.hpp"
 
+#include <type_traits>
+
 namespace xcq {
 
 // ---------------------------------------------------------------------------
@@ -45,10 +47,14 @@ namespace xcq {
 // per factor).  The points of a wave nearly always have one parent: then
 // every loop is uniform, runs as far as any lane needs and takes lists and
 // atoms by scalar loads, two factors at a time; lanes that need less
-// multiply by exact ones.  A wave with two parents takes them in turn, one
-// with more follows each lane's own lists.  72 atoms, 4.2 million points: 4.7
-// ms when each thread ran its own loops, 3.8 so, 2.95 with 1 / (a R) in the
-// lists instead of a division per factor.
+// multiply by exact ones.  Where a wave holds several parents each lane runs
+// loops of its own.  72 atoms, 4.2 million points of one parent per wave: 4.7 ms
+// when each thread ran its own loops, 3.8 so, 2.95 with 1 / (a R) in the lists
+// instead of a division per factor.  Calls with 2^20 points around 72 and 450
+// atoms, copies included: one parent per wave 7.0 and 40 ms (own loops 7.9 and
+// 49); two 8.1 and 50 (the two in turn 10.0 and 55); a parent of its own for
+// every point 8.5 and 54 (uniform loops over each lane's own lists, where every
+// lane reads as long as any needs to, 15.3 and 216).
 __global__ __launch_bounds__(256) void k_ssf(int32_t natoms, const double* __restrict__ xyz,
                                              const double* __restrict__ rab,
                                              const double* __restrict__ dnear, int64_t npts,
@@ -81,14 +87,19 @@ __global__ __launch_bounds__(256) void k_ssf(int32_t natoms, const double* __res
   constexpr double kWiden = 1.0 + 1e-10;
   if (nbr_idx) {
     constexpr double kNegligible = 0x1p-70;
-    // The points in lanes with act, of parent P.
-    auto points = [&](int P, bool act) {
+    // The points in lanes with act, of parent P: the loops run as far as any
+    // lane needs (one parent in all of them), or each lane's by itself.
+    auto points = [&](auto UNIFORM, int P, bool act) {
+      auto any = [](bool b) {
+        if constexpr (decltype(UNIFORM)::value) return (bool)__any(b);
+        else return b;
+      };
       const int32_t* np = nbr_idx + (size_t)P * natoms;
       const double* ni = nbr_i + (size_t)P * natoms;
       double dmin = dpar;
       int inear = P;
       const double i2 = 1.0 / (a * 2.0 * dpar * kWiden);
-      for (int k = 1; k < natoms && __any(act && ni[k] >= i2); ++k) {
+      for (int k = 1; k < natoms && any(act && ni[k] >= i2); ++k) {
         const int B = np[k];
         const double d = dist(B);
         if (d < dmin) {
@@ -114,7 +125,7 @@ __global__ __launch_bounds__(256) void k_ssf(int32_t natoms, const double* __res
             C[j] = ap[qj];
             I[j] = ai[qj];
           }
-          if (!__any(v > floor_ && I[0] > ifac)) break;
+          if (!any(v > floor_ && I[0] > ifac)) break;
 #pragma unroll
           for (int j = 0; j < 2; ++j)
             if (q + j < natoms) v *= ssf_s((dA - dist(C[j])) * I[j]);
@@ -124,27 +135,23 @@ __global__ __launch_bounds__(256) void k_ssf(int32_t natoms, const double* __res
       const double ppar = product(P, dpar, 0.0, act && dpar <= bound);
       const bool some = act && ppar != 0.0;
       double sum = ppar;
-      for (int k = 1; k < natoms && __any(some && ni[k] >= icand); ++k) {
+      for (int k = 1; k < natoms && any(some && ni[k] >= icand); ++k) {
         const int A = np[k];
         const double dA = dist(A);
         bool use = some && dA <= bound;
-        if (!__any(use)) continue;
+        if (!any(use)) continue;
         const double floor_ = kNegligible * sum;
         if (use && A != inear)
           use = ssf_s((dA - dmin) / (a * rab[(size_t)A + (size_t)inear * natoms])) > floor_;
-        if (__any(use)) sum += product(A, dA, floor_, use);
+        if (any(use)) sum += product(A, dA, floor_, use);
       }
       if (act) w[ip] *= some ? ppar / sum : 0.0;
     };
-    uint64_t left = __builtin_amdgcn_ballot_w64(on);
-    for (int pass = 0; pass < 2 && left; ++pass) {
-      const int P = __builtin_amdgcn_readlane(par, __ffsll((unsigned long long)left) - 1);
-      const bool act = on && par == P;
-      points(P, act);
-      on = on && !act;
-      left = __builtin_amdgcn_ballot_w64(on);
-    }
-    if (left) points(par, on);
+    const uint64_t lanes = __builtin_amdgcn_ballot_w64(on);
+    if (lanes == 0) return;
+    const int P = __builtin_amdgcn_readlane(par, __ffsll((unsigned long long)lanes) - 1);
+    if (!__any(on && par != P)) points(std::true_type{}, P, on);
+    else if (on) points(std::false_type{}, par, true);
     return;
   }
   if (!on) return;
