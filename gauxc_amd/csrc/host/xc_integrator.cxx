@@ -47,13 +47,15 @@ int xcq_func_id(const functional_type& f) {
 }
 // Touches every page of an m x m output matrix while the device computes:
 // the pages of a freshly allocated one are otherwise first mapped by the copy
-// that fills it, one after the other (7,800 functions: 25 ms).  Values stay
-// as they are.
+// that fills it (7,800 functions: 245 ms a call against 225).  One thread ends
+// long before the device does; a team of threads was no faster and, started
+// right after the caller's own threads had run, kept the call waiting (first
+// calls of 468 functions, UKS: 4.9 ms so, 14 to 20 with 16 threads, 4.9
+// without touching).  Values stay as they are.
 void touch_pages(double* a, int64_t m, int64_t ld) {
   constexpr int64_t kPage = 4096 / sizeof(double);
   const int64_t n = m ? (m - 1) * ld + m : 0;
   if (n < 256 * kPage) return;
-#pragma omp parallel for schedule(static)
   for (int64_t i = 0; i < n; i += kPage) {
     if (i % ld >= m) continue;  // not the matrix's
     volatile double* p = a + i;
