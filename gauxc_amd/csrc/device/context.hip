@@ -69,15 +69,39 @@ void dfree(T*& p) {
 // the list's large-first order at the granularity of 8 * kXcdRun items.
 // The final partial group keeps its natural order.
 constexpr size_t kXcds = 8, kXcdRun = 16;
-void xcd_interleave(std::vector<WorkItem>& v, size_t b, size_t e) {
+void xcd_interleave(std::vector<WorkItem>& v, size_t b, size_t e, std::vector<WorkItem>& tmp) {
   constexpr size_t G = kXcds * kXcdRun;
   const size_t n = e - b, full = n / G * G;
   if (full == 0) return;
-  std::vector<WorkItem> tmp(v.begin() + b, v.begin() + b + full);
+  tmp.assign(v.begin() + b, v.begin() + b + full);
   for (size_t i = 0; i < full; ++i) {
     const size_t g = i / G, o = i % G, x = o / kXcdRun, q = o % kXcdRun;
     v[b + g * G + q * kXcds + x] = tmp[i];
   }
+}
+
+// The numbers 0 .. n - 1 in ascending order of their keys, equal keys in
+// ascending order: by a radix sort, 12 bits a pass, without the passes in which
+// all keys agree; below some 500 keys its counters cost more than comparisons.
+std::vector<int32_t> sorted_by_key(const std::vector<uint64_t>& key) {
+  constexpr int kBits = 12;
+  const size_t n = key.size();
+  std::vector<int32_t> v(n), tmp(n);
+  std::iota(v.begin(), v.end(), 0);
+  if (n < 512) {
+    std::stable_sort(v.begin(), v.end(), [&](int32_t a, int32_t b) { return key[a] < key[b]; });
+    return v;
+  }
+  for (int shift = 0; shift < 64; shift += kBits) {
+    std::vector<size_t> at((size_t(1) << kBits) + 1, 0);
+    auto digit = [&](int32_t i) { return key[i] >> shift & ((1u << kBits) - 1); };
+    for (int32_t i : v) ++at[digit(i) + 1];
+    if (std::find(at.begin(), at.end(), n) != at.end()) continue;
+    for (size_t d = 1; d < at.size(); ++d) at[d] += at[d - 1];
+    for (int32_t i : v) tmp[at[digit(i)]++] = i;
+    v.swap(tmp);
+  }
+  return v;
 }
 
 // Dynamic-queue layout of items [b, e) of v (item costs c): nx sub-lists
@@ -100,13 +124,20 @@ void xcd_queue_layout(std::vector<WorkItem>& v, size_t b, size_t e, const std::v
     groups.back().count++;
     groups.back().cost += c[i - b];
   }
-  std::stable_sort(groups.begin(), groups.end(),
-                   [](const Group& x, const Group& y) { return x.cost > y.cost; });
+  // Descending costs: the bits of a double, ordered as the values are.
+  std::vector<uint64_t> key;
+  for (const auto& g : groups) {
+    uint64_t k;
+    const double c0 = g.cost + 0.;  // -0 as 0
+    std::memcpy(&k, &c0, 8);
+    key.push_back(~(k >> 63 ? ~k : k | uint64_t(1) << 63));
+  }
   using QE = std::pair<double, int>;  // (load, sub-list)
   std::priority_queue<QE, std::vector<QE>, std::greater<QE>> heap;
   for (int q = 0; q < nx; ++q) heap.push({0.0, q});
   std::vector<std::vector<WorkItem>> qs(nx);
-  for (const auto& g : groups) {
+  for (int32_t i : sorted_by_key(key)) {
+    const Group& g = groups[i];
     QE top = heap.top();
     heap.pop();
     for (size_t k = 0; k < g.count; ++k) qs[top.second].push_back(v[g.first + k]);
@@ -214,7 +245,7 @@ struct xcq_context_s {
   double vxc_drop = kDefaultVxcDrop;  // see xcq_set_vxc_drop_tolerance
   int32_t nqueues = 0;                                 // 0: one workgroup per item
   std::vector<double> cost_d, cost_s;                  // per-task predicted costs
-  std::vector<uint64_t> place;  // per task: molecule and place of its points in space
+  std::vector<int32_t> order;  // tasks in the order of the density items, chunk by chunk
   bool timing = false;
   int64_t* d_tstamp = nullptr;
 
@@ -384,6 +415,7 @@ int build_work_lists(xcq_context_s* ctx) {
                                                                     : kWideAuto;
     d.wide = d.nbe >= std::max(wide, 65) && d.npts > kPtBlock;
   }
+  std::vector<WorkItem> tmp;
   auto finish_range = [&](WorkRange& r, const std::vector<double>& cost) {
     r.n = (int64_t)W.size() - r.off;
     r.nq = 0;
@@ -398,28 +430,16 @@ int build_work_lists(xcq_context_s* ctx) {
       ncounters += r.nx;
       xcd_queue_layout(W, (size_t)r.off, W.size(), cost, r.nx, Q);
     } else {
-      xcd_interleave(W, (size_t)r.off, W.size());
+      xcd_interleave(W, (size_t)r.off, W.size(), tmp);
     }
   };
-  // Density (and collocation, Z) items follow the tasks' places in space
-  // (neighbouring tasks gather nearly the same part of P), tasks of many
-  // functions first, in steps of kPlaceNbe, so that the launch ends on small
-  // ones.  (150 waters: FP64 density 166 ms by cost, 135 by place alone, 138
-  // in steps of 64, mixed 110, 109 and 100 ms; 24 waters: 6.3, 6.6 and 6.1.)
-  constexpr int kPlaceNbe = 64;
-  std::vector<std::pair<uint64_t, int32_t>> order(ctx->ntasks);
-  for (int32_t i = 0; i < ctx->ntasks; ++i) {
-    const uint64_t step = std::min(ctx->h_tasks[i].nbe / kPlaceNbe, 1023);
-    order[i] = {(1023 - step) << 54 | ctx->place[i], i};
-  }
-  for (const auto& c : ctx->chunks)
-    std::sort(order.begin() + c.task_begin, order.begin() + c.task_end);
+  std::vector<std::vector<int32_t>> region_lists[2];  // by number of blocks
   for (auto& c : ctx->chunks) {
     for (int v = 1; v >= 0; --v) {
       c.dens[v].off = (int64_t)W.size();
       std::vector<double> cost;
       for (int32_t q = c.task_begin; q < c.task_end; ++q) {
-        const int32_t i = order[q].second;
+        const int32_t i = ctx->order[q];
         const DevTask& d = ctx->h_tasks[i];
         if (d.wide != v) continue;
         const int nmb = d.npts_pad / kPtBlock;
@@ -435,7 +455,7 @@ int build_work_lists(xcq_context_s* ctx) {
     {
       std::vector<double> cost;
       for (int32_t q = c.task_begin; q < c.task_end; ++q) {
-        const int32_t i = order[q].second;
+        const int32_t i = ctx->order[q];
         const DevTask& d = ctx->h_tasks[i];
         if (!d.wide) continue;
         const int npair = (d.npts_pad / kPtBlock + 1) / 2;
@@ -461,18 +481,23 @@ int build_work_lists(xcq_context_s* ctx) {
       constexpr bool kMx = decltype(MX)::value;
       constexpr int64_t kSyrItems = 768;
       constexpr int kSliceMin = 256, kSliceMax = 4096;
-      auto regions = [&](const DevTask& d, auto&& f) {
+      // The regions of tasks of nb blocks of 16 functions.
+      auto regions = [&](const DevTask& d) -> const std::vector<int32_t>& {
         const int nb = (d.nbe + 15) / 16;
-        const int ni = syr_row_groups<kMx>(nb), nj = syr_col_groups<kMx>(nb);
-        for (int it = 0; it < ni; ++it)
-          for (int jt = 0; jt < nj; ++jt)  // with blocks below the diagonal
-            if ((it + 1) * nb / ni > jt * nb / nj) f(it | jt << 16);
+        auto& list = region_lists[kMx];
+        if (nb >= (int)list.size()) list.resize(nb + 1);
+        if (list[nb].empty()) {
+          const int ni = syr_row_groups<kMx>(nb), nj = syr_col_groups<kMx>(nb);
+          for (int it = 0; it < ni; ++it)
+            for (int jt = 0; jt < nj; ++jt)  // with blocks below the diagonal
+              if ((it + 1) * nb / ni > jt * nb / nj) list[nb].push_back(it | jt << 16);
+        }
+        return list[nb];
       };
       int64_t region_points = 0;
       for (int32_t i = c.task_begin; i < c.task_end; ++i) {
-        int64_t n = 0;
-        regions(ctx->h_tasks[i], [&](int) { ++n; });
-        region_points += n * ctx->h_tasks[i].npts;
+        const DevTask& d = ctx->h_tasks[i];
+        region_points += (int64_t)regions(d).size() * d.npts;
       }
       const int32_t kslice =
           (int32_t)std::clamp<int64_t>(region_points / kSyrItems, kSliceMin, kSliceMax);
@@ -486,11 +511,11 @@ int build_work_lists(xcq_context_s* ctx) {
         if (d.npts == 0) continue;
         const int32_t ns = std::min((d.npts + kslice - 1) / kslice, 0x7fff);
         const size_t first = W.size();
-        regions(d, [&](int32_t rg) {
+        for (int32_t rg : regions(d)) {
           if (ns > 1) sums.push_back(WorkItem{i, rg, ns, (int32_t)slots});
           for (int32_t sl = 0; sl < ns; ++sl)
             W.push_back(WorkItem{i, rg, sl | ns << 16, ns > 1 ? (int32_t)slots++ : 0});
-        });
+        }
         const size_t n = W.size() - first;
         if (!queued) continue;
         cost.insert(cost.end(), n, have_cost ? ctx->cost_s[i] / std::max<size_t>(n, 1)
@@ -1079,10 +1104,22 @@ int xcq_upload_tasks_batched(xcq_context ctx, int32_t ntasks, const xcq_task* ta
   ctx->ev.resize(chunks.size() * kStages * 2);
   for (auto& e : ctx->ev) XCQ_HIP(hipEventCreate(&e));
 
-  ctx->place.resize(ntasks);
-  for (int32_t i = 0; i < ntasks; ++i) {
-    const double* p = ht[i].npts ? points + 3 * ht[i].pt_off : nullptr;
-    ctx->place[i] = (uint64_t)std::min(ht[i].mol, 0x7fff) << 39 | (p ? space_code(p) : 0);
+  // Density (and collocation, Z) items follow the tasks' places in space
+  // (neighbouring tasks gather nearly the same part of P), tasks of many
+  // functions first, in steps of kPlaceNbe, so that the launch ends on small
+  // ones.  (150 waters: FP64 density 166 ms by cost, 135 by place alone, 138
+  // in steps of 64, mixed 110, 109 and 100 ms; 24 waters: 6.3, 6.6 and 6.1.)
+  constexpr int kPlaceNbe = 64;
+  ctx->order.clear();
+  for (const auto& c : chunks) {
+    std::vector<uint64_t> key;
+    for (int32_t i = c.task_begin; i < c.task_end; ++i) {
+      const DevTask& d = ht[i];
+      const uint64_t step = std::min(d.nbe / kPlaceNbe, 1023);
+      key.push_back((1023 - step) << 54 | (uint64_t)std::min(d.mol, 0x7fff) << 39 |
+                    (d.npts ? space_code(points + 3 * d.pt_off) : 0));
+    }
+    for (int32_t k : sorted_by_key(key)) ctx->order.push_back(c.task_begin + k);
   }
   ctx->h_tasks = std::move(ht);
   ctx->chunks = std::move(chunks);
