@@ -1067,7 +1067,6 @@ int xcq_upload_tasks_batched(xcq_context ctx, int32_t ntasks, const xcq_task* ta
   if ((rc = dalloc(&ctx->d_pz, npts_total))) return rc;
   if ((rc = dalloc(&ctx->d_w, npts_total))) return rc;
   if ((rc = dalloc(&ctx->d_shell_list, (size_t)nshell_entries))) return rc;
-  bfmap.resize(bfmap.size() + kBfPad, 0);
   if ((rc = dalloc(&ctx->d_bfmap, bfmap.size()))) return rc;
   if ((rc = dalloc(&ctx->d_lsh, lsh.size()))) return rc;
   if ((rc = dalloc(&ctx->d_red, (size_t)2 * std::max<int64_t>(pblocks, 1)))) return rc;

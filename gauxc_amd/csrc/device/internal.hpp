@@ -41,8 +41,6 @@ constexpr int kPtBlock = 64;      // points per collocation / density block (npt
 // diffuse systems are of such negligible pairs (about three in four on a
 // 150-water cluster), and each is an FP64 atomic.
 constexpr double kDefaultVxcDrop = 1e-18;
-constexpr int kBfPad = 32;        // zero entries after the last task's basis map: K blocks
-                                  // of 32 rows read up to 31 entries past a task's nbe
 
 struct DevShell {
   double alpha[32];
@@ -51,8 +49,8 @@ struct DevShell {
   int32_t nprim, l, pure, size;
 };
 
-// Compact copy of a shell's centre, first primitive and shape (48 bytes),
-// which the density stage's basis evaluation loads 64 shells at a time.
+// Compact copy of a shell's centre, first primitive and shape (48 bytes), from
+// which the density stage stages a tile's shells in LDS (FoldShells).
 struct DevShellC {
   double ox, oy, oz, a0, c0;
   int32_t info;  // l | pure << 8 | nprim << 16
