@@ -194,6 +194,10 @@ struct MolInfo {
 constexpr int32_t kWideAuto = 1 << 30, kWideNbe = 256;
 constexpr int64_t kWidePBytes = int64_t(64) << 20;
 
+// Sets of ticket counters: launches of one work list in an evaluation (the UKS FXC
+// contraction's density stage runs once per matrix, four times).
+constexpr int kTicketSets = 4;
+
 struct xcq_context_s {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -232,7 +236,8 @@ struct xcq_context_s {
   std::vector<int32_t> h_qoff;
   WorkItem* d_work = nullptr;
   int32_t* d_qoff = nullptr;
-  unsigned long long* d_counters = nullptr;  // ticket counters of the dynamic queues
+  unsigned long long* d_counters = nullptr;  // ticket counters of the queues, kTicketSets sets
+  int64_t ncounters = 0;                     // of one set
   // Settings of kernels that are gone (tile widths, occupancy): kept and
   // reported, without effect.
   int32_t dens32_max_nbe = 48, syr2k32_max_nbe = 96, dens_hiocc_max_nbe = 0;
@@ -538,12 +543,8 @@ int build_work_lists(xcq_context_s* ctx) {
   int rc;
   if ((rc = dalloc(&ctx->d_work, W.size()))) return rc;
   if ((rc = dalloc(&ctx->d_qoff, Q.size()))) return rc;
-  // Zero once (the bits of 0.0): every queued launch leaves its counters at
-  // zero (next_ticket).
-  if (ncounters &&
-      ((rc = dalloc(&ctx->d_counters, (size_t)ncounters)) ||
-       (rc = launch_fill(ctx->stream, reinterpret_cast<double*>(ctx->d_counters), ncounters))))
-    return rc;
+  ctx->ncounters = ncounters;
+  if (ncounters && (rc = dalloc(&ctx->d_counters, (size_t)(kTicketSets * ncounters)))) return rc;
   if (ctx->timing && (rc = dalloc(&ctx->d_tstamp, 2 * W.size()))) return rc;
   if (!W.empty())
     XCQ_HIP(hipMemcpy(ctx->d_work, W.data(), W.size() * sizeof(WorkItem), hipMemcpyHostToDevice));
@@ -566,8 +567,19 @@ int ensure_syr_part(xcq_context_s* ctx) {
   return dalloc(&ctx->d_syr_part, (size_t)slots * kSyrBlocks * 256);
 }
 
-// Enqueue one evaluation on the context's stream.  Events are recorded only
-// when `events` is set (not under graph capture).
+// Zeroes every set of ticket counters (a fill kernel, not a memset node, so graph
+// replays reset them too; zero has the same bits as 0.0).
+int clear_tickets(xcq_context_s* ctx) {
+  return launch_fill(ctx->stream, reinterpret_cast<double*>(ctx->d_counters),
+                     kTicketSets * ctx->ncounters);
+}
+
+// The view with the counters of the pass-th launch of each list.
+CtxView ticket_view(const xcq_context_s* ctx, CtxView v, int pass) {
+  v.counters = ctx->d_counters + pass * ctx->ncounters;
+  return v;
+}
+
 // The basis evaluation mode an energy evaluation runs: on stored planes (0) or
 // in the stages (3).  Mixed precision with g functions stays on stored planes:
 // the stages' FP64 values in place of the stored FP32 ones move VXC by up to
@@ -577,6 +589,8 @@ int effective_mode(const xcq_context_s* ctx, int precision) {
   return ctx->dens_in_stage == 0 || (precision != XCQ_PREC_FP64 && ctx->max_l > 3) ? 0 : 3;
 }
 
+// Enqueue one evaluation on the context's stream.  Events are recorded only
+// when `events` is set (not under graph capture).
 int enqueue_pipeline(xcq_context_s* ctx, int func, int precision, int want_vxc, bool events) {
   const int gga = (func == XCQ_FUNC_PBE || func == XCQ_FUNC_PBE0) ? 1 : 0;
   CtxView v = view_of(ctx);
@@ -587,6 +601,7 @@ int enqueue_pipeline(xcq_context_s* ctx, int func, int precision, int want_vxc, 
   int rc;
   if (want_vxc && (rc = launch_fill(s, ctx->d_vxc, ctx->p_total))) return rc;
   if (want_vxc && (rc = launch_fill(s, ctx->d_tmax, ctx->tmax_total))) return rc;
+  if ((rc = clear_tickets(ctx))) return rc;
   int64_t launches = want_vxc ? 1 : 0, items = 0;
   auto rec = [&](hipEvent_t e) { return events ? hipEventRecord(e, s) : hipSuccess; };
   for (size_t ci = 0; ci < ctx->chunks.size(); ++ci) {
@@ -1510,6 +1525,7 @@ int enqueue_uks(xcq_context_s* ctx, int func, int want_vxc) {
   if (want_vxc && ((rc = launch_fill(s, ctx->d_vxc, ctx->p_total)) ||
                    (rc = launch_fill(s, ctx->d_vxcz, ctx->p_total))))
     return rc;
+  if ((rc = clear_tickets(ctx))) return rc;
   for (const Chunk& c : ctx->chunks) {
     const WorkItem* cw = v.work + c.coll.off;
     if ((rc = launch_collocation_fp64(s, cw, c.coll.n, v.tasks, v.shells, v.shell_list, v.lsh,
@@ -1517,13 +1533,13 @@ int enqueue_uks(xcq_context_s* ctx, int func, int want_vxc) {
                                       0, ctx->max_l)))
       return rc;
     for (int pass = 0; pass < 2; ++pass)
-      if ((rc = launch_density(v, c, XCQ_PREC_FP64, gga, 1.0, pass == 0 ? ds : dz,
-                               pass == 0 ? ctx->d_P : ctx->d_Pz)))
+      if ((rc = launch_density(ticket_view(ctx, v, pass), c, XCQ_PREC_FP64, gga, 1.0,
+                               pass == 0 ? ds : dz, pass == 0 ? ctx->d_P : ctx->d_Pz)))
         return rc;
     if ((rc = launch_uks_points(v, c.coll, func, gga, ds, dz, zs, zz))) return rc;
     if (!want_vxc) continue;
     for (int comp = 0; comp < 2; ++comp) {
-      CtxView vc = v;
+      CtxView vc = ticket_view(ctx, v, comp);
       vc.vxc = comp == 0 ? ctx->d_vxc : ctx->d_vxcz;
       if ((rc = z_and_vxc(ctx, vc, c, gga, comp == 0 ? zs : zz))) return rc;
     }
@@ -1615,6 +1631,7 @@ int enqueue_fxc(xcq_context_s* ctx, int func) {
   double* zc = dt + blk;
   int rc;
   if ((rc = launch_fill(s, ctx->d_vxc, ctx->p_total))) return rc;
+  if ((rc = clear_tickets(ctx))) return rc;
   for (const Chunk& c : ctx->chunks) {
     const WorkItem* cw = v.work + c.coll.off;
     if ((rc = launch_collocation_fp64(s, cw, c.coll.n, v.tasks, v.shells, v.shell_list, v.lsh,
@@ -1622,8 +1639,8 @@ int enqueue_fxc(xcq_context_s* ctx, int func) {
                                       0, ctx->max_l)))
       return rc;
     for (int pass = 0; pass < 2; ++pass)
-      if ((rc = launch_density(v, c, XCQ_PREC_FP64, gga, 2.0, pass == 0 ? dp : dt,
-                               pass == 0 ? ctx->d_P : ctx->d_tP)))
+      if ((rc = launch_density(ticket_view(ctx, v, pass), c, XCQ_PREC_FP64, gga, 2.0,
+                               pass == 0 ? dp : dt, pass == 0 ? ctx->d_P : ctx->d_tP)))
         return rc;
     if ((rc = launch_fxc_points(v, c.coll, func, gga, dp, dt, zc))) return rc;
     if ((rc = z_and_vxc(ctx, v, c, gga, zc))) return rc;
@@ -1703,6 +1720,7 @@ int enqueue_fxc_uks(xcq_context_s* ctx, int func) {
   if ((rc = launch_fill(s, ctx->d_vxc, ctx->p_total)) ||
       (rc = launch_fill(s, ctx->d_vxcz, ctx->p_total)))
     return rc;
+  if ((rc = clear_tickets(ctx))) return rc;
   for (const Chunk& c : ctx->chunks) {
     const WorkItem* cw = v.work + c.coll.off;
     if ((rc = launch_collocation_fp64(s, cw, c.coll.n, v.tasks, v.shells, v.shell_list, v.lsh,
@@ -1710,12 +1728,13 @@ int enqueue_fxc_uks(xcq_context_s* ctx, int func) {
                                       0, ctx->max_l)))
       return rc;
     for (int pass = 0; pass < 4; ++pass)
-      if ((rc = launch_density(v, c, XCQ_PREC_FP64, gga, 1.0, dd[pass], mats[pass])))
+      if ((rc = launch_density(ticket_view(ctx, v, pass), c, XCQ_PREC_FP64, gga, 1.0, dd[pass],
+                               mats[pass])))
         return rc;
     if ((rc = launch_fxc_points_uks(v, c.coll, func, gga, dd[0], dd[1], dd[2], dd[3], zs, zz)))
       return rc;
     for (int comp = 0; comp < 2; ++comp) {
-      CtxView vc = v;
+      CtxView vc = ticket_view(ctx, v, comp);
       vc.vxc = comp == 0 ? ctx->d_vxc : ctx->d_vxcz;
       if ((rc = z_and_vxc(ctx, vc, c, gga, comp == 0 ? zs : zz))) return rc;
     }
@@ -1836,6 +1855,7 @@ int enqueue_grad(xcq_context_s* ctx, int func, int weight_derivs) {
   int rc;
   const int64_t gs = grad_stride(ctx->grad_natoms);
   if ((rc = launch_fill(s, ctx->d_grad_part, kGradCopies * gs))) return rc;
+  if ((rc = clear_tickets(ctx))) return rc;
   for (const Chunk& c : ctx->chunks) {
     const WorkItem* cw = v.work + c.coll.off;
     if ((rc = launch_collocation_fp64(s, cw, c.coll.n, v.tasks, v.shells, v.shell_list, v.lsh,
@@ -1881,6 +1901,7 @@ int enqueue_grad_uks(xcq_context_s* ctx, int func, int weight_derivs) {
   int rc;
   const int64_t gs = grad_stride(ctx->grad_natoms);
   if ((rc = launch_fill(s, ctx->d_grad_part, kGradCopies * gs))) return rc;
+  if ((rc = clear_tickets(ctx))) return rc;
   for (const Chunk& c : ctx->chunks) {
     const WorkItem* cw = v.work + c.coll.off;
     if ((rc = launch_collocation_fp64(s, cw, c.coll.n, v.tasks, v.shells, v.shell_list, v.lsh,
@@ -1888,8 +1909,8 @@ int enqueue_grad_uks(xcq_context_s* ctx, int func, int weight_derivs) {
                                       0, ctx->max_l)))
       return rc;
     for (int pass = 0; pass < 2; ++pass)
-      if ((rc = launch_density(v, c, XCQ_PREC_FP64, gga, 1.0, pass == 0 ? ds : dz,
-                               pass == 0 ? ctx->d_P : ctx->d_Pz,
+      if ((rc = launch_density(ticket_view(ctx, v, pass), c, XCQ_PREC_FP64, gga, 1.0,
+                               pass == 0 ? ds : dz, pass == 0 ? ctx->d_P : ctx->d_Pz,
                                gga ? 2 + pass : -1)))
         return rc;
     if ((rc = launch_grad_points_uks(v, c.coll, func, gga, ds, dz, wf))) return rc;

@@ -90,9 +90,10 @@ struct WorkItem {  // (task, a, b): a/b are point-block or pair indices (SYR2K: 
 // when nq >= 8; else 1), sub-list x = items [qoff[x], qoff[x+1]) (queue
 // table at qoff_off of the context's queue array, nx + 1 entries), and a
 // workgroup b takes the next item of sub-list b % nx from that sub-list's
-// ticket counter (counters at cnt_off of the context's counter array) until the
-// sub-list is exhausted.  A launch finds its counters at zero and leaves them
-// so: evaluations launch the same list several times (UKS, FXC, gradients).
+// ticket counter (counters at cnt_off of a counter set) until the sub-list is
+// exhausted.  A launch uses its counters up: an evaluation that launches one list
+// several times (UKS, FXC, gradients) gives each launch a set of its own
+// (CtxView::counters), and all sets are zeroed at the start of every evaluation.
 struct WorkRange {
   int64_t off = 0, n = 0;
   int64_t qoff_off = 0;
@@ -161,7 +162,7 @@ struct CtxView {
   const double *px, *py, *pz, *w;
   const WorkItem* work;
   const int32_t* qoff;
-  unsigned long long* counters;  // ticket counters of the dynamic queues
+  unsigned long long* counters;  // ticket counters of the dynamic queues (one set)
   int64_t* tstamp;  // nullptr unless task timing is on
   const double* P;
   const float* Pf32;  // FP32 copy of P (mixed-precision density stage)
@@ -212,9 +213,7 @@ __device__ __forceinline__ int64_t uniform64(int64_t x) {
 // the workgroup calls it (uniform control flow): one lane takes a ticket
 // with a vector atomic and the item index is broadcast through LDS.  The
 // leading barrier keeps the previous item's readers of the slot ahead of
-// the write.  A sub-list of n items drawn from by w workgroups gives n + w
-// tickets, one past the end to each workgroup; whoever gets the last of them
-// resets the counter for the next launch.
+// the write.
 __device__ __forceinline__ int64_t next_ticket(const QueueArgs& qa) {
   __shared__ int64_t slot;
   __syncthreads();
@@ -223,7 +222,6 @@ __device__ __forceinline__ int64_t next_ticket(const QueueArgs& qa) {
     const unsigned long long t = atomicAdd(qa.counters + x, 1ull);
     const int64_t n = qa.qoff[x + 1] - qa.qoff[x];
     slot = (int64_t)t < n ? qa.qoff[x] + (int64_t)t : kNoItem;
-    if ((int64_t)t == n + (gridDim.x - 1 - x) / (unsigned)qa.nx) atomicExch(qa.counters + x, 0ull);
   }
   __syncthreads();
   return slot;
