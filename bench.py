@@ -11,11 +11,12 @@ Workload (one "step" = one full EXC+VXC evaluation over every task):
 
 Both precisions run on the same resident inputs.  Before timing, the device
 autotuner picks the basis evaluation mode, (FP64) the block-pair threshold and
-the queue count for each precision (untimed); the timed steps replay the captured graph of the evaluation.
+the queue count for each precision (untimed); the timed steps replay the
+captured graph of the evaluation.
 ``value`` is the mixed-precision rate; the FP64 rate, the speed-up and the
 mixed-vs-FP64 |dEXC| / max|dVXC| are reported beside it.
 
-Prints one JSON line (see the driver contract) with a roofline entry for
+Prints one JSON line with a roofline entry for
 the dominant stage (its kernel launches timed with HIP events on the
 context's stream, in an eager step) and a CPU baseline: the oracle (a
 restatement of GauXC's host integrator, its two per-task products through

@@ -190,7 +190,11 @@ struct MolInfo {
 }  // namespace
 
 // The pairs kernel pays where P does not stay in the caches beside the
-// planes (see k_density_wide): it draws level near 3,100 functions, 78 MB.
+// planes (see k_density_wide): it draws level near 3,100 functions, 78 MB.  Its
+// least number of functions is not critical: density stage of 150 and of 90
+// waters with pairs from 128 functions on 125 and 60 ms, 192: 122 and 58, 256:
+// 120 and 57, 320: 119 and 56.5, 384: 120 and 57, 448: 121 and 57, 512: 123 and
+// 57.4, never: 139 and 59.4.
 constexpr int32_t kWideAuto = 1 << 30, kWideNbe = 256;
 constexpr int64_t kWidePBytes = int64_t(64) << 20;
 

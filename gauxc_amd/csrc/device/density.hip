@@ -22,8 +22,8 @@
 // from the planes the collocation stage stored, and so does the Z launch
 // (k_z_from_coeffs); 3 and 4 evaluate them (up to that angular momentum) at
 // the block's points from the shell parameters, as does k_z_in_stage
-// (collocation.hip).  kProductOnly stops at
-// the product, of any stored plane, for the EXC gradient.
+// (collocation.hip).  kProductOnly stops at the product, of any stored plane,
+// for the EXC gradient.
 #include "internal.hpp"
 #include "functional.hpp"
 #include "shell_eval.hpp"
@@ -68,11 +68,12 @@ using Vec4 = T __attribute__((ext_vector_type(4)));
 // which fit the register budget of the GEMM phase).  Row offsets are clamped
 // to a valid row; rows past nbe are not stored.
 // Also records, per granule of 32 functions, max |B| and max |Z| over the
-// block's points (B with its residual; float bits, so unsigned max orders
-// them): LDS atomics into smax, then one device atomic per granule into the
-// task's bound table (direct device atomics when the task has more granules
-// than smax holds).  The B^T Z stage leaves out a block when
-// npts * (max|B_i| max|Z_j| + max|Z_i| max|B_j|) is below the drop tolerance.
+// block's points (the FP32 part of B: its residual is covered by syr_mask's
+// margin; float bits, so unsigned max orders them): LDS atomics into smax, then
+// one device atomic per granule into the task's bound table (direct device
+// atomics when the task has more granules than smax holds).  The B^T Z stage
+// leaves out a block when npts * (max|B_i| max|Z_j| + max|Z_i| max|B_j|) is below
+// the drop tolerance.
 template <typename T, bool GGA, int kZRows = sizeof(T) == 4 ? 4 : 2>
 __device__ __forceinline__ void write_z(const DevTask& t, int m0, int tid, double (*zc)[64],
                                         T* Bm, unsigned (*smax)[2], unsigned* tmax) {
@@ -185,8 +186,8 @@ __device__ __forceinline__ void write_z(const DevTask& t, int m0, int tid, doubl
 // of the first version's 7.9 ms on 24 waters); the rest were chains of
 // dependent loads, barriers and the functional on one wave of four, with two
 // waves per SIMD to cover them.  The functional is now a launch of its own,
-// the shells come from LDS, and four waves fit a SIMD (20 registers spill;
-// three waves without spills: 6.7 ms).  24 waters: 8.9 (64-wide padded
+// the shells come from LDS, and four waves fit a SIMD (21 to 24 registers
+// spill; three waves without spills: 6.7 ms).  24 waters: 8.9 (64-wide padded
 // tiles, 1.4 times the products wanted) -> 6.1 ms; 150 waters: 152 -> 138 ms,
 // there bound by L2 misses (890 GB, 6.5 TB/s); 84 functions: 52 -> 28 us.
 //
@@ -548,7 +549,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void k_density(
 // (2 MB and more) and the blocks' B panels do not stay in L2, P_sub is
 // gathered once per point block and B read once per tile.  Twice the points
 // and twice the functions per workgroup halve both, at two waves per SIMD
-// (128 accumulator registers).  Density stage: 150 waters 137 -> 117 ms, 90
+// (128 accumulator registers; 29 to 35 spill).  Density stage: 150 waters 137 -> 117 ms, 90
 // waters 33.3 -> 30.0, 60 waters 18.6 -> 18.0, 40 waters 8.8 -> 9.1, 24 waters
 // 6.1 -> 6.8; mixed precision (64-function tiles, half the bytes) lost at
 // every size (150 waters 88 -> 95).  Lane (f, q) holds the adjacent points 2f,

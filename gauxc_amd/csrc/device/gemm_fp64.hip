@@ -23,9 +23,9 @@ __device__ __forceinline__ v4d mfma_f64(double a, double b, v4d c) {
 }
 
 // One 1 KiB fragment from memory into LDS: lane l's 16 bytes at base + off
-// go to lds + 16 l.  Inline asm (as the density stage's operand ring) so
-// that the compiler's wait insertion, which cannot tell the two stages
-// apart, adds no wait for it before LDS reads; the K loop waits itself.
+// go to lds + 16 l.  Inline asm so that the compiler's wait insertion, which
+// cannot tell the two stages apart, adds no wait for it before LDS reads; the K
+// loop waits itself.
 __device__ __forceinline__ void frag_to_lds(const double* base, unsigned off, const double* lds) {
   const unsigned m0 = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)lds);
   asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(m0) : "memory");
@@ -38,14 +38,13 @@ __device__ __forceinline__ void frag_to_lds(const double* base, unsigned off, co
 // What bounds it: the matrix cores, once each operand is fetched few enough
 // times.  Padding to 64-wide tiles and 64 points multiplied 1.8 to 2.3 times
 // what is wanted (150 and 24 waters); a first version with one wave per 4 x
-// 3 blocks, its operands straight from memory, multiplied 1.2 times but
-// missed L2 for 28 GB per 24-water call, 4.3 TB/s, with the matrix cores 41%
-// busy.  So four waves share a region's fragments through LDS, and only
-// blocks that hold wanted elements are multiplied: below nbe, on or below
-// the diagonal, not negligible by the bound table.  The wanted blocks are
-// dealt evenly to the waves, each block anywhere in the region; at 64 cycles
-// per MFMA the four fragments a block reads for its four MFMAs take half of
-// the LDS bandwidth.
+// 3 blocks, its operands straight from memory, multiplied 1.2 times but read
+// 23 GB past L2 per 24-water call, with the matrix cores 41% busy.  So four
+// waves share a region's fragments through LDS, and only blocks that hold
+// wanted elements are multiplied: below nbe, on or below the diagonal, not
+// negligible by the bound table.  The wanted blocks are dealt evenly to the
+// waves, each block anywhere in the region; at 64 cycles per MFMA the four
+// fragments a block reads for its four MFMAs take half of the LDS bandwidth.
 //
 // A fragment is 16 functions x 8 points of a plane in lane order: lane (f =
 // l & 15, q = l >> 4) holds points k + 2q, k + 2q + 1 of function row f, the
@@ -53,8 +52,9 @@ __device__ __forceinline__ void frag_to_lds(const double* base, unsigned off, co
 // (Any order of the points serves as long as both operands use it.)  It is
 // one 16-byte load per lane from memory into LDS and one 16-byte LDS read.
 // Two stages of up to 13 blocks (B and Z) fill a third of a CU's LDS: three
-// workgroups per CU, one barrier per eight points.  Now 17 GB of L2 misses
-// per 24-water call, 3.9 TB/s, and the matrix cores 61% busy.
+// workgroups per CU, one barrier per eight points.  Now 12.6 GB past L2 per
+// 24-water call (98 M requests of 128 bytes; the planes hold 9.0 GB) beside 37 M
+// atomic additions, 3.1 TB/s read, and the matrix cores 61% busy.
 //
 // Stage times, 64-wide padded tiles -> this: 24 waters 8.4 -> 4.4 ms, 150
 // waters 94.6 -> 61 ms, 120 functions on 340,000 points 0.66 -> 0.10 ms, 84
@@ -259,8 +259,8 @@ int launch_syr2k(const CtxView& v, const Chunk& c, int precision) {
   }
   if (sum.n)
     hipLaunchKernelGGL(mx ? k_syr2k_reduce<true> : k_syr2k_reduce<false>,
-                       dim3((unsigned)sum.n, mx ? kSyr<true>.blocks() : kSyr<false>.blocks()), dim3(256), 0, v.stream,
-                       v.work + sum.off, v.tasks, v.bfmap, v.syr_part, v.vxc, v.vxc_drop, tm);
+                       dim3((unsigned)sum.n, mx ? kSyr<true>.blocks() : kSyr<false>.blocks()),
+                       dim3(256), 0, v.stream, v.work + sum.off, v.tasks, v.bfmap, v.syr_part, v.vxc, v.vxc_drop, tm);
   XCQ_HIP(hipGetLastError());
   return XCQ_SUCCESS;
 }

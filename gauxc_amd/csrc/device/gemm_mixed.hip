@@ -89,16 +89,18 @@ __global__ __launch_bounds__(256) void k_P_to_f32(int64_t n, const double* __res
 // (f ^ 2q), which keeps the loader's writes (lane 4f + q) and the waves' reads
 // (lane 16 q + f) free of bank conflicts.
 //
-// What bounds it: reading B and Z, 10 bytes per function and point.  24 waters
-// miss L2 for 12.4 GB, about what the planes hold, at 3.5 TB/s, with the
-// matrix cores 18% and the vector units 26% busy.  Tiles of 64 functions,
+// What bounds it: waiting.  24 waters read 7.3 GB past L2 (the planes hold 5.6,
+// 10 bytes per function and point) beside 37 M atomic additions, 2.1 TB/s read,
+// with the matrix cores 18% and the vector units 26% busy: no unit is near its
+// limit, but a K block's split, its products and the barriers around them follow
+// one another, with two workgroups per CU to overlap.  Tiles of 64 functions,
 // padded and with both triangles of the diagonal ones, read and split twice
 // as much: 24 waters 4.7 -> 3.5 ms, 150 waters 58 -> 51 ms.  Regions of 4 x 4
 // blocks take 3.7 and 53 ms, of 4 x 3 at three workgroups per CU 3.9 and 55;
 // blocks in row pairs that share a column's fragments, or fragments loaded a
 // block ahead, spill registers in the K loop (6.5 and 3.9 ms).  The raw
 // operands of the next K block wait in registers; they are local to the loop,
-// so that they are not carried from item to item (18 registers spill, none
+// so that they are not carried from item to item (17 registers spill, none
 // in the K loops; carried 79).
 // Slices and their order as in the FP64 kernel (k_syr2k).
 __global__ __launch_bounds__(256, 2) void k_syr2k_mx(QueueArgs qa,

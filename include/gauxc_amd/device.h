@@ -222,9 +222,10 @@ int xcq_exc_vxc(xcq_context ctx, int functional, int precision, int want_vxc);
  *      spin_dim 2, reference_replicated_xc_host_integrator_exc_vxc.hpp:106-601;
  *      device kernels cuda/kernels/zmat_vxc.cu:62-96,197-274).  P_s = P_a + P_b
  *      goes through xcq_upload_density, P_z = P_a - P_b through
- *      xcq_upload_density_z (single-molecule contexts).  FP64, stored basis
- *      planes, every VXC contribution added.  Synchronous results through
- *      xcq_download_results_uks (vxc_s / vxc_z may be NULL). ---- */
+ *      xcq_upload_density_z (single-molecule contexts).  FP64, the basis
+ *      evaluated in the stages, with the VXC drop tolerance of the energy
+ *      path.  Synchronous results through xcq_download_results_uks (vxc_s /
+ *      vxc_z may be NULL). ---- */
 int xcq_upload_density_z(xcq_context ctx, int32_t nbf, const double* Pz, int64_t ldp);
 int xcq_exc_vxc_uks(xcq_context ctx, int functional, int want_vxc);
 int xcq_download_results_uks(xcq_context ctx, double* exc, double* nel, double* vxc_s,
@@ -260,7 +261,7 @@ int xcq_download_fxc_uks(xcq_context ctx, double* nel, double* fxc_s, double* fx
  *      282-290).  P through xcq_upload_density (single-molecule contexts);
  *      xyz = the natoms atom positions (x, y, z), in the order of the tasks'
  *      parent indices; a shell belongs to the atom at exactly its centre.
- *      FP64, stored basis planes.  weight_derivs = 0 gives the Hellmann-
+ *      FP64, the basis evaluated in the stages.  weight_derivs = 0 gives the Hellmann-
  *      Feynman form (IntegratorSettingsEXC_GRAD::include_weight_derivatives =
  *      false).  xcq_download_exc_grad returns EXC, NEL and grad[3 * natoms]
  *      (atom-major). ---- */
